@@ -576,6 +576,9 @@ struct GemmArgs {
     int M, N, K; void* workspace; int64_t workspace_bytes; hipStream_t stream;
     int batches; GemmBatch batch;   // batches > 1: one launch for that many products, operands `batch` apart (dense A only)
 };
+// gemm_short_k.hip
+int gemm_short_k(const GemmArgs& g, int w_exp_bits, int w_frac_bits);
+inline bool short_k_ok(const GemmArgs& g) { return g.a_dense && !g.bias && g.K <= 128 && g.N <= (1 << 23); }   // (32-bit offsets within 64 rows)
 int gemm_w_e4m3(const GemmArgs& g);
 int gemm_w_e5m2(const GemmArgs& g);
 int gemm_w_e2m3(const GemmArgs& g);
