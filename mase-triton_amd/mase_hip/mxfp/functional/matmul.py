@@ -99,10 +99,20 @@ def _scaled_route(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, oth
     return kernels.scaled_shape_supported(N, K, input.dtype) and L.takes_scaled_route(input.numel() // K, False)
 
 
+def _other_components(other: Tensor, other_meta: MXFPMeta) -> tuple[Tensor, Tensor]:
+    """Components of ``other`` [.., K, N], blocks along K, in [.., N, K] order.  The transposed view of a contiguous tensor (the
+    keys of an attention product) lies in that order already and goes through the flat kernel; a contiguous one through the
+    strided kernel.  (K is a multiple of 32 on this route, so no block straddles two rows either way.)"""
+    lying = other.transpose(-1, -2)
+    if lying.is_contiguous():
+        return kernels.extract_mxfp_components(lying.reshape(-1), other_meta)
+    return kernels.extract_mxfp_components_strided(other, -2, other_meta)
+
+
 def _matmul_through_gemm(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, other_meta: MXFPMeta) -> Tensor:
     if _scaled_route(input, other, input_meta, other_meta):
         K, N = other.shape[-2], other.shape[-1]
-        w_scales, w_elements = kernels.extract_mxfp_components_strided(other.reshape(K, N), -2, other_meta)   # [N, K] order
+        w_scales, w_elements = _other_components(other, other_meta)   # [N, K] order
         w_op = kernels.scaled_operand_from_mxfp(w_scales, w_elements, other_meta, N, K)
         a_op = kernels.scaled_operand_from_dense(input.reshape(-1, K), input_meta)
         y = kernels.mxfp_gemm_scaled(a_op, w_op, None, input.dtype)
@@ -112,7 +122,7 @@ def _matmul_through_gemm(input: Tensor, other: Tensor, input_meta: MXFPMeta | No
     if input_meta is not None:
         # MXFP values are exact in bf16 whatever input.dtype is
         a = quantize_dequantize(input, block_dim=-1, mxfp_meta=input_meta, output_dtype=torch.bfloat16)
-    w_scales, w_elements = kernels.extract_mxfp_components_strided(other, -2, other_meta)  # [.., N, K] order
+    w_scales, w_elements = _other_components(other, other_meta)  # [.., N, K] order
     return gemm_over_batches(a.contiguous(), w_scales, w_elements, other_meta, tuple(other.shape[:-2]), other.shape[-1], input.dtype)
 
 
