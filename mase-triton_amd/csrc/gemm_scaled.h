@@ -366,30 +366,8 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1,
 }
 
 #include "gemm_scaled_rows.h"   // the weight-streaming kernels for up to 64 rows of A
+#include "gemm_scaled_mid.h"    // 128-row tiles for tens to hundreds of rows, and the choice between them and the 256 x 256 ones
 
-
-// K split for few tiles and a long K (a [1024, 4096] output has 64 tiles for 256 CUs): the number of walks per tile, chosen so
-// that the walks about fill the CUs; a walk takes an even number of macro steps, at least 4.  Priced like the bf16 kernels'
-// split: macro steps per walk at about 1 us, rounds of walks over the CUs, and for a split the second launch plus the
-// partial sums written and read once.
-inline int plan_scaled_splits(int M, int N, int K, int cus) {
-    const int64_t tiles = (int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN);
-    const int nmac = K / SMAC;
-    if (tiles * 2 > cus || cus <= 0 || scaled_rows_shape_ok(M, K)) return 1;
-    const double mn_mb = (double)M * N * 4.0 / 1e6;
-    auto price = [&](int s) {
-        const double rounds = (double)((tiles * s + cus - 1) / cus);
-        return rounds * (nmac / s + 3) * 1.0 + (s > 1 ? 4.0 + (2.0 * s + 0.5) * mn_mb * 0.21 : 0.0);
-    };
-    int best = 1;
-    double best_t = price(1);
-    for (int s = 2; s <= 16 && tiles * s <= cus; ++s) {
-        if (nmac % s != 0 || (nmac / s) % 2 != 0 || nmac / s < 4) continue;
-        const double t = price(s);
-        if (t < best_t) { best_t = t; best = s; }
-    }
-    return best;
-}
 
 // a_codes [rows_a, K], w_codes [rows_w, K]: rows padded to multiples of 256; scales [K / 128][rows] dwords.  `workspace`
 // (may be null): room for the fp32 partial sums of a K split, splits * M * N * 4 bytes.
@@ -404,9 +382,11 @@ int launch_gemm_scaled(const uint8_t* a_codes, const uint32_t* a_scales, const u
     if (const int slices = scaled_rows_slices(M, N, K); slices > 0 && workspace && workspace_bytes >= (int64_t)slices * M * N * 4)
         return launch_gemm_scaled_rows_sliced<DT_OUT>(a_codes, a_scales, w_codes, w_scales, bias, bias_dtype, y, M, N, K, static_cast<float*>(workspace), s);
     if (scaled_rows_shape_ok(M, K)) return launch_gemm_scaled_rows<DT_OUT>(a_codes, a_scales, w_codes, w_scales, bias, bias_dtype, y, M, N, K, s);
-    int splits = workspace ? plan_scaled_splits(M, N, K, cus) : 1;
+    ScaledMidPlan plan = plan_scaled(M, N, K, cus, workspace != nullptr);
     const int64_t mn = (int64_t)M * N;
-    if (splits > 1 && workspace_bytes < splits * mn * 4) splits = 1;
+    if (plan.splits > 1 && workspace_bytes < plan.splits * mn * 4) plan = plan_scaled(M, N, K, cus, false);
+    if (plan.bn != 256) return launch_gemm_scaled_mid<DT_OUT>(a_codes, a_scales, w_codes, w_scales, bias, bias_dtype, y, M, N, K, plan, workspace, s);
+    const int splits = plan.splits;
     const int64_t walks = tiles * splits;
     const unsigned grid = (unsigned)(walks < cus ? ((walks + 7) / 8) * 8 : (cus / 8) * 8);
     if (splits > 1) {

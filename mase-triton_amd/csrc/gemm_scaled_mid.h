@@ -1,0 +1,259 @@
+// Block-scaled MXFP GEMM for tens to hundreds of rows of A (a large decode batch, a chunk of a prompt), operands in the prepared
+// form of gemm_scaled.h, on tiles of 128 x 128 or 128 x 64.
+//
+// At these sizes the 256 x 256 tiles of gemm_scaled.h leave most CUs without one (200 x 14336 outputs: 56 tiles for 256 CUs), and
+// splitting K for more of them costs fp32 partial sums of 256-row tiles that are mostly padding.  Smaller tiles give every CU
+// one; what they cost is operand traffic per flop: a 128 x 128 tile takes 32 KB L2 -> LDS and 64 KB LDS -> registers per 128 k for
+// 512 cycles of MFMA.  Both are about what a CU's paths carry in that time, so the kernel is organised to keep them running:
+//   * four wavefronts (2 x 2 of 64 x 64, or 4 x 1 of 32 x 64 when the tile is 64 columns wide), one workgroup per CU;
+//   * codes and scale dwords global -> LDS by DMA into a ring of four stages (one 128-k macro step each), four steps ahead;
+//   * the fragments of macro step s + 1 are read from LDS into the other of two register sets while step s is multiplied: at
+//     the one barrier per step every wavefront has its operands in registers, and the slot of step s is free for step s + 4;
+//   * every MFMA is followed by its share of the step's LDS reads and DMAs and a scheduling barrier, as in gemm_scaled.h.
+// What bounds it: a macro step takes 0.61 us (128 columns; 0.43 with 64), of which MFMAs and LDS are 0.29 (0.18).  The rest is the
+// vector-memory path.  A CU takes in 55 bytes per ns when some of them come from HBM, however deep the ring is (six stages:
+// the same) and whichever wavefronts ask (A and W asked for by different ones: the same): what is in flight is returned in
+// order, and A's L2 hits queue behind W's misses.  With W in L2 as well the step is at its LDS and MFMA time.  With every CU
+// at work HBM's share per CU is the nearer limit (128 x 14336 x 4096: 59 MB of W in 19 us, launch included).
+// N x K = 14336 x 4096: 19.2 / 24.6 / 24.8 us at 128 / 200 / 256 rows, against 28.5 / 35.4 / 43.7 on 256 x 256 tiles; 4096 x 4096: 14 /
+// 16 / 16.5 / 23 at 128 / 256 / 512 / 1024 rows against 21 / 24 / 27 / 42; 4096 x 14336: 22 / 29 at 128 / 256 against 33 / 36.
+// LDS rows are 128 bytes, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7).
+// (included from gemm_impl.h's namespace, after gemm_scaled.h's typedefs)
+
+constexpr int SMD_M = 128, SMD_RING = 4;
+template <int BN> constexpr int smd_stage_bytes() { return (SMD_M + BN) * 128 + 1024; }
+template <int BN> constexpr int smd_lds_bytes() { return SMD_RING * smd_stage_bytes<BN>(); }
+
+__device__ inline void mfma_scaled_v(floatx4& c, const intx8& w, const intx8& a, uint32_t sw, uint32_t sa) {
+    asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]" : "+v"(c) : "v"(w), "v"(a), "v"(sw), "v"(sa));
+}
+// 256 bytes: 4 per lane from (sbase + voff) to LDS lds_addr + 4 * lane
+__device__ inline void dma_64_dwords(uint32_t lds_addr, uint32_t voff, const void* sbase) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
+}
+
+template <int DT_OUT, int BN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mxfp_gemm_scaled_mid_kernel(
+    const uint8_t* __restrict__ a_codes, const uint32_t* __restrict__ a_scales, const uint8_t* __restrict__ w_codes,
+    const uint32_t* __restrict__ w_scales, const void* __restrict__ bias, int bias_dtype, void* __restrict__ y_all, int M, int N, int K,
+    int rows_a, int rows_w, int tiles_m, int splits, int mac_per, int n_walks, int64_t y_split_bytes) {
+    constexpr int WN = BN / 64, WM = 4 / WN, MI = 8 / WM, NJ = 4;       // wavefronts along n and m; 16-row and 16-column tiles of one
+    constexpr int A_BYTES = SMD_M * 128, W_BYTES = BN * 128, STAGE = smd_stage_bytes<BN>(), SC = A_BYTES + W_BYTES;
+    constexpr int RING = SMD_RING;
+    constexpr int W_DMAS = W_BYTES / 4096, OPS = 4 + W_DMAS + 1;        // DMAs per wavefront and step: A, W, scales
+    constexpr int READS = 2 * (MI + NJ) + MI + NJ, MFMAS = MI * NJ;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave_m = wave / WN, wave_n = wave % WN;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+
+    // walk (tile, split of K): m-tile fastest, then the split.  Workgroups are dealt to the 8 XCDs in turn; XCD x takes the x-th
+    // eighth of the walks, so those that share rows of W share an L2.
+    const int walk = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));     // (the grid is a multiple of 8)
+    if (walk >= n_walks) return;
+    const int tile_m = walk % tiles_m, rest = walk / tiles_m;
+    const int z = rest % splits, tile_n = rest / splits, m0 = tile_m * SMD_M, n0 = tile_n * BN;
+    const int mac0 = z * mac_per, nm = min(mac_per, K / 128 - mac0);   // this walk's macro steps (at least one)
+    uint8_t* const y = static_cast<uint8_t*>(y_all) + (size_t)z * (size_t)y_split_bytes;
+
+    // ---- DMA.  Data: lane l fills position l & 7 of row 8 d + (l >> 3) of the wavefront's rows, which must hold the row's piece
+    //      (l & 7) ^ (row >> 1 & 7).  Wavefront w: rows 32 w .. of A, BN / 4 w .. of W, and 64 of the scale dwords (A's 128, then W's).
+    uint32_t voff[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+        voff[d] = (uint32_t)(8 * d + (lane >> 3)) * (uint32_t)K + (uint32_t)(((lane & 7) ^ ((4 * d + (lane >> 4)) & 7)) << 4);
+    const uint32_t sc_voff = (uint32_t)lane * 4u;
+    const int sc_wave = BN == 64 ? min(wave, 2) : wave;                 // (64 columns: the last wavefront repeats W's 64 dwords)
+    const uint8_t* pa = a_codes + (size_t)(m0 + 32 * wave) * K + (size_t)mac0 * 128;
+    const uint8_t* pw = w_codes + (size_t)(n0 + BN / 4 * wave) * K + (size_t)mac0 * 128;
+    const uint32_t* psc = sc_wave < 2 ? a_scales + (size_t)mac0 * rows_a + m0 + 64 * sc_wave : w_scales + (size_t)mac0 * rows_w + n0 + 64 * (sc_wave - 2);
+    const int sc_step = sc_wave < 2 ? rows_a : rows_w;
+    // workgroups of different columns start at different macro steps and wrap around: rows of W (and of A) are K bytes apart, and at
+    // one k all of them would sit on the same few channels of the L2
+    int at = tile_n % nm;                                             // the macro step that is issued next
+    pa += (size_t)at * 128;
+    pw += (size_t)at * 128;
+    psc += (size_t)at * sc_step;
+    auto dma = [&](auto slot_c, auto q_c) __attribute__((always_inline)) {
+        constexpr int slot = decltype(slot_c)::value, q = decltype(q_c)::value;
+        if constexpr (q < 4) dma_1kb(lds_base + (uint32_t)(slot * STAGE + q * 1024) + (uint32_t)wave * 4096u, voff[q], pa);
+        else if constexpr (q < 4 + W_DMAS) dma_1kb(lds_base + (uint32_t)(slot * STAGE + A_BYTES + (q - 4) * 1024) + (uint32_t)wave * (W_DMAS * 1024u), voff[q - 4], pw);
+        else dma_64_dwords(lds_base + (uint32_t)(slot * STAGE + SC) + (uint32_t)sc_wave * 256u, sc_voff, psc);
+    };
+    auto advance = [&]() __attribute__((always_inline)) {
+        const bool wrap = ++at == nm;
+        at = wrap ? 0 : at;
+        pa += wrap ? -(int64_t)(nm - 1) * 128 : 128;
+        pw += wrap ? -(int64_t)(nm - 1) * 128 : 128;
+        psc += wrap ? -(int64_t)(nm - 1) * sc_step : sc_step;
+    };
+
+    // ---- fragments: lane (g = l >> 4, r = l & 15) reads pieces g and g + 4 of row r of its 16-row tile, and the row's scale byte g
+    const uint32_t f_off = (uint32_t)(lane & 15) * 128u + (uint32_t)((((lane >> 4) ^ ((lane >> 1) & 7)) & 7) << 4);
+    const uint8_t* const a_lo = lds + wave_m * (MI * 2048) + f_off;
+    const uint8_t* const a_hi = lds + wave_m * (MI * 2048) + (f_off ^ 64u);
+    const uint8_t* const w_lo = lds + A_BYTES + wave_n * (NJ * 2048) + f_off;
+    const uint8_t* const w_hi = lds + A_BYTES + wave_n * (NJ * 2048) + (f_off ^ 64u);
+    const uint8_t* const a_sc = lds + SC + wave_m * (MI * 64) + (lane & 15) * 4 + (lane >> 4);
+    const uint8_t* const w_sc = lds + SC + 512 + wave_n * (NJ * 64) + (lane & 15) * 4 + (lane >> 4);
+    floatx4 acc[NJ][MI];
+    intx8 af[2][MI], wf[2][NJ];
+    uint32_t as[2][MI], ws[2][NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[j][i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    // read k (0 .. READS - 1) of the stage in `slot` into register set `set`: W fragment 0, A fragment 0, W 1, A 1, ..., then scales
+    auto read = [&](auto slot_c, auto set_c, auto k_c) __attribute__((always_inline)) {
+        constexpr int slot = decltype(slot_c)::value, set = decltype(set_c)::value, k = decltype(k_c)::value;
+        if constexpr (k < 2 * NJ) {
+            constexpr int j = k / 2;
+            if constexpr (k % 2 == 0) wf[set][j].lo = *reinterpret_cast<const intx4*>(w_lo + slot * STAGE + j * 2048);
+            else wf[set][j].hi = *reinterpret_cast<const intx4*>(w_hi + slot * STAGE + j * 2048);
+        } else if constexpr (k < 2 * (NJ + MI)) {
+            constexpr int i = (k - 2 * NJ) / 2;
+            if constexpr (k % 2 == 0) af[set][i].lo = *reinterpret_cast<const intx4*>(a_lo + slot * STAGE + i * 2048);
+            else af[set][i].hi = *reinterpret_cast<const intx4*>(a_hi + slot * STAGE + i * 2048);
+        } else if constexpr (k < 2 * (NJ + MI) + NJ) {
+            constexpr int j = k - 2 * (NJ + MI);
+            ws[set][j] = w_sc[slot * STAGE + j * 64];
+        } else {
+            constexpr int i = k - 2 * (NJ + MI) - NJ;
+            as[set][i] = a_sc[slot * STAGE + i * 64];
+        }
+    };
+
+    static_for<RING>([&](auto s_c) __attribute__((always_inline)) {
+        static_for<OPS>([&](auto q_c) __attribute__((always_inline)) { dma(s_c, q_c); });
+        advance();
+    });
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * OPS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    static_for<READS>([&](auto k_c) __attribute__((always_inline)) { read(IntC<0>{}, IntC<0>{}, k_c); });
+
+    for (int base = 0; base < nm; base += RING) {
+        static_for<RING>([&](auto u_c) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_c)::value, set = u & 1, next = (u + 1) % RING;
+            if (base + u < nm) {
+                // stage s + 1 of this wavefront has landed (those of s + 2 and s + 3 may still fly), step s is in registers
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 2) * OPS) : "memory");
+                lds_barrier();
+                asm volatile("" ::: "memory");
+                static_for<MFMAS>([&](auto t_c) __attribute__((always_inline)) {
+                    constexpr int t = decltype(t_c)::value, i = t / NJ, j = t % NJ;
+                    mfma_scaled_v(acc[j][i], wf[set][j], af[set][i], ws[set][j], as[set][i]);
+                    constexpr int r0 = t * READS / MFMAS, r1 = (t + 1) * READS / MFMAS, d0 = t * OPS / MFMAS, d1 = (t + 1) * OPS / MFMAS;
+                    static_for<r1 - r0>([&](auto k_c) __attribute__((always_inline)) { read(IntC<next>{}, IntC<set ^ 1>{}, IntC<r0 + decltype(k_c)::value>{}); });
+                    static_for<d1 - d0>([&](auto k_c) __attribute__((always_inline)) { dma(IntC<u>{}, IntC<d0 + decltype(k_c)::value>{}); });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                advance();
+            }
+        });
+    }
+    // the look-ahead DMAs still target LDS, which the outputs pass through
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");      // the matrix unit's last results have left its pipeline
+    lds_barrier();
+    asm volatile("" ::: "memory");
+
+    // ---- output: lane holds, for tile (j, i), y[m][n .. n+3] with m = 16 i + lane % 16, n = 16 j + 4 (lane / 16) of the wavefront's
+    //      outputs; staged so that a store instruction writes whole lines (128 bytes of a row: 64 columns, 32 of fp32)
+    constexpr int OB = DT_OUT == F32 ? 4 : 2, PASSES = DT_OUT == F32 ? 2 : 1, JT = NJ / PASSES;
+    uint8_t* const out = lds + wave * (MI * 2048);
+    const int g = lane >> 4, r = lane & 15;
+    const int row0 = m0 + wave_m * (MI * 16), col0 = n0 + wave_n * 64;
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+#pragma unroll
+        for (int jj = 0; jj < JT; ++jj) {
+            const int j = p * JT + jj;
+            float b[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (bias) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) b[v] = load_bias(bias, bias_dtype, min(col0 + 16 * j + 4 * g + v, N - 1));
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                const floatx4 c = acc[j][i];
+                uint8_t* const row = out + (16 * i + r) * 128;
+                if constexpr (DT_OUT == F32)
+                    *reinterpret_cast<float4*>(row + (((4 * jj + g) ^ (r & 7)) * 16)) = make_float4(c[0] + b[0], c[1] + b[1], c[2] + b[2], c[3] + b[3]);
+                else
+                    *reinterpret_cast<uint2*>(row + (((2 * jj + (g >> 1)) ^ (r & 7)) * 16) + (g & 1) * 8) = pack_out4<DT_OUT>(c[0] + b[0], c[1] + b[1], c[2] + b[2], c[3] + b[3]);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the wavefront's own writes)
+        const int col = col0 + p * 32 + (lane & 7) * (16 / OB);
+#pragma unroll
+        for (int t = 0; t < MI * 2; ++t) {
+            const int row = 8 * t + (lane >> 3);
+            const u32x4 v = *reinterpret_cast<const u32x4*>(out + row * 128 + (((lane & 7) ^ (row & 7)) * 16));
+            if (row0 + row < M && col < N) *reinterpret_cast<u32x4*>(y + ((size_t)(row0 + row) * N + col) * OB) = v;
+        }
+        asm volatile("" ::: "memory");
+    }
+}
+
+struct ScaledMidPlan {
+    int bn;        // columns of a tile: 128 or 64; 256: the 256 x 256 kernel of gemm_scaled.h
+    int splits;    // workgroups that share a tile's K, each with its own fp32 [M, N] array of the workspace
+    int mac_per;   // macro steps per split
+};
+
+// Which tile, and how many workgroups share its K.  Every candidate is priced, in us: rounds of workgroups over the CUs x macro
+// steps x time of a step, plus launch, prologue and epilogue, plus, when K is split, the second launch and the partial sums
+// written and read once.  Fitted to both kernels forced on N = 1024 .. 14336, K = 1024 .. 14336, 65 .. 2048 rows: a step takes 1.0 us
+// (256 x 256) with few CUs busy and 1.2 with all, 0.62 (128 x 128) either way, 0.37 and 0.46 (128 x 64); the 256 x 256 kernel walks
+// its tiles as one stream (8 us once), the others pay 2.5 us per round and 2 once.  Where prices are close so are the
+// kernels: 384 x 14336 x 4096 takes 43.4 us on 256 x 256 tiles and 44.0 on 128 x 128 ones, 2048 x 4096 x 4096 41 and 45.
+inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
+    const int nmac = K / SMAC;
+    ScaledMidPlan best{256, 1, nmac};
+    if (cus <= 0) return best;
+    const double mn_mb = (double)M * N * 4.0 / 1e6;
+    double best_t = 1e30;
+    for (int bn = 256; bn >= 64; bn /= 2) {
+        const int64_t tiles = bn == 256 ? (int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN) : (int64_t)((M + 127) / 128) * ((N + bn - 1) / bn);
+        for (int want = 1; want <= 16; ++want) {
+            if (want > 1 && (!may_split || tiles * want > cus)) break;
+            const int per = (nmac + want - 1) / want;
+            if (want > 1 && (per < 4 || (nmac + per - 1) / per != want)) continue;
+            if (bn == 256 && want > 1 && (nmac % want != 0 || per % 2 != 0)) continue;      // that kernel walks equal shares of pairs
+            const int64_t wgs = tiles * want;
+            const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
+            const double step = bn == 256 ? 1.0 + 0.2 * busy : bn == 128 ? 0.62 : 0.37 + 0.09 * busy;
+            const double rounds = (double)((wgs + cus - 1) / cus);
+            const double t = rounds * (per * step + (bn == 256 ? 0.0 : 2.5)) + (bn == 256 ? 8.0 : 2.0) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
+            if (t < best_t) { best_t = t; best = ScaledMidPlan{bn, want, per}; }
+        }
+    }
+    return best;
+}
+
+template <int DT_OUT>
+int launch_gemm_scaled_mid(const uint8_t* a_codes, const uint32_t* a_scales, const uint8_t* w_codes, const uint32_t* w_scales, const void* bias,
+                           int bias_dtype, void* y, int M, int N, int K, const ScaledMidPlan& p, void* workspace, hipStream_t s) {
+    const int rows_a = (M + 255) / 256 * 256, rows_w = (N + 255) / 256 * 256;
+    const int tiles_m = (M + SMD_M - 1) / SMD_M, tiles_n = (N + p.bn - 1) / p.bn;
+    const int64_t walks = (int64_t)tiles_m * tiles_n * p.splits, mn = (int64_t)M * N;
+    if (walks >= (1 << 30)) return fail(ERR_UNSUPPORTED, "too many tiles");
+    auto go = [&](auto kern, int lds_bytes, std::atomic<uint64_t>& allowed, void* out, int64_t split_bytes, const void* b) {
+        if (int rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds_bytes, allowed)) return rc;
+        hipLaunchKernelGGL(kern, dim3((unsigned)((walks + 7) / 8 * 8)), dim3(256), lds_bytes, s, a_codes, a_scales, w_codes, w_scales, b, bias_dtype, out, M,
+                           N, K, rows_a, rows_w, tiles_m, p.splits, p.mac_per, (int)walks, split_bytes);
+        return check_launch("mxfp_gemm_scaled");
+    };
+    static std::atomic<uint64_t> allowed[4] = {{0}, {0}, {0}, {0}};
+    if (p.splits == 1)
+        return p.bn == 128 ? go(mxfp_gemm_scaled_mid_kernel<DT_OUT, 128>, smd_lds_bytes<128>(), allowed[0], y, 0, bias)
+                           : go(mxfp_gemm_scaled_mid_kernel<DT_OUT, 64>, smd_lds_bytes<64>(), allowed[1], y, 0, bias);
+    if (int rc = p.bn == 128 ? go(mxfp_gemm_scaled_mid_kernel<F32, 128>, smd_lds_bytes<128>(), allowed[2], workspace, mn * 4, nullptr)
+                             : go(mxfp_gemm_scaled_mid_kernel<F32, 64>, smd_lds_bytes<64>(), allowed[3], workspace, mn * 4, nullptr))
+        return rc;
+    hipLaunchKernelGGL(split_k_reduce_kernel<DT_OUT>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, s, static_cast<const float*>(workspace), p.splits,
+                       mn, N, bias, bias_dtype, y);
+    return check_launch("mxfp_gemm_scaled");
+}

@@ -436,6 +436,31 @@ def test_scaled_gemm_k_split(mh, MNK):
         assert rel_fro(y, y_one) <= tol
 
 
+@pytest.mark.parametrize("MNK", [(65, 8, 512), (128, 64, 768), (129, 72, 2304), (200, 136, 3840), (257, 520, 7168), (70, 4104, 1024),
+                                 (130, 1032, 4352), (640, 4096, 4096), (200, 14336, 512)])
+def test_scaled_gemm_128_row_tiles(mh, MNK):
+    """The 128 x 128 and 128 x 64 tile kernels around the edges of their tiles (rows, columns), with fewer macro steps than the DMA
+    ring has stages and counts that it does not divide, K split into equal and unequal shares and not split, bias and every output
+    type: every element of the fp32 result against a float64 product of the checker's dequantised operands."""
+    M, N, K = MNK
+    g = torch.Generator().manual_seed(M * 3 + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (0.02 * torch.randn(N, K, generator=g)).to(torch.bfloat16)
+    b = torch.randn(N, generator=g).to(torch.bfloat16)
+    _, _, x_dq = quantised(x, "MXFP8_E4M3_fn")
+    w_sc, w_el, w_dq = quantised(w, "OCP_MXFP6_E3M2")
+    y_ref = x_dq.double() @ w_dq.double().t()
+    a = mh.mxk.scaled_operand_from_dense(x.to(DEV), mh.meta.MXFP8_E4M3_fn)
+    wop = mh.mxk.scaled_operand_from_mxfp(w_sc.to(DEV), w_el.to(DEV), mh.meta.OCP_MXFP6_E3M2, N, K)
+    for split_k in (True, False):
+        y32 = mh.mxk.mxfp_gemm_scaled(a, wop, None, torch.float32, split_k=split_k)
+        assert rel_fro(y32, y_ref) <= F32_TOL
+        assert float((y32.cpu().double() - y_ref).abs().max()) <= 1e-3 * float(y_ref.abs().max())
+        y_b = y_ref + b.double()
+        for odt in (torch.bfloat16, torch.float16):
+            assert rel_fro(mh.mxk.mxfp_gemm_scaled(a, wop, b.to(DEV), odt, split_k=split_k), y_b.to(odt)) <= 1e-3
+
+
 # ---------------------------------------------------------------- the prepared weight on the bf16 kernel
 @pytest.mark.parametrize("MNK", [(512, 256, 512), (1100, 384, 1024), (640, 128, 128)])
 @pytest.mark.parametrize("w_tag", SCALED_TAGS)

@@ -46,3 +46,15 @@ def test_counted_wait_kernels_use_no_scratch(tmp_path):
         # M0 carries the LDS address of the DMAs between inline-asm statements: nothing else may write it
         m0_writes = [ln for ln in text.splitlines() if re.search(r"\bm0\b", ln) and not ln.strip().startswith(";")]
         assert all(re.match(r"\s*s_mov_b32 m0, s\d+", ln) for ln in m0_writes), (unit, m0_writes[:5])
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+@pytest.mark.parametrize("unit,tag", [("gemm_short_k", "gemm_short_k_kernel"), ("gemm_scaled", "gemm_scaled_mid_kernel")])
+def test_counted_wait_kernels_of_one_unit_use_no_scratch(tmp_path, unit, tag):
+    """The same check for the kernels that one translation unit holds for all formats."""
+    text = _assembly(unit, str(tmp_path))
+    sizes = dict(zip(re.findall(r"^(_ZN4mase\w+):\s*; @", text, re.M), re.findall(r"; ScratchSize: (\d+)", text)))
+    sizes = {name: size for name, size in sizes.items() if tag in name}
+    assert sizes and all(int(size) == 0 for size in sizes.values()), sizes
+    m0_writes = [ln for ln in text.splitlines() if re.search(r"\bm0\b", ln) and not ln.strip().startswith(";")]
+    assert all(re.match(r"\s*s_mov_b32 m0, s\d+", ln) for ln in m0_writes), m0_writes[:5]
