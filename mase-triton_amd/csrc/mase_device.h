@@ -58,40 +58,18 @@ template <class F> __host__ __device__ inline uint32_t fmt_sign(const F& f) { re
 __device__ inline uint32_t f32_bits(float v) { return __float_as_uint(v); }
 __device__ inline float bits_f32(uint32_t u) { return __uint_as_float(u); }
 
-__device__ inline uint32_t half_bits_to_f32_bits(uint32_t h) {
-    // exact for every fp16 pattern, including subnormals, without relying on the fp16
-    // denormal mode
-    uint32_t s = (h & 0x8000u) << 16, e = (h >> 10) & 0x1Fu, m = h & 0x3FFu;
-    if (e == 0) {
-        if (m == 0) return s;
-        int lz = __clz(m) - 21;  // m < 2^10: leading zeros within the 11-bit window
-        m = (m << lz) & 0x3FFu;
-        return s | ((uint32_t)(113 - lz) << 23) | (m << 13);
-    }
-    if (e == 31) return s | 0x7F800000u | (m << 13);
-    return s | ((e + 112u) << 23) | (m << 13);
-}
+// The hardware's converts: exact for every fp16 pattern (kernels run with fp16 and fp32 subnormals enabled, the default of the code
+// objects), round to nearest even the other way; a NaN stays a NaN, quieted, which is what every reader of its payload does too.
+__device__ inline uint32_t half_bits_to_f32_bits(uint32_t h) { return f32_bits((float)__builtin_bit_cast(_Float16, (uint16_t)h)); }
 
 __device__ inline uint32_t f32_bits_to_bf16_bits(uint32_t u) {  // RNE; NaN stays NaN
     if ((u & 0x7FFFFFFFu) > 0x7F800000u) return 0x7FC0u | ((u >> 16) & 0x8000u);
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 
-__device__ inline uint32_t f32_bits_to_half_bits(uint32_t u) {  // IEEE RNE, integer only
-    uint32_t s = (u >> 16) & 0x8000u, a = u & 0x7FFFFFFFu;
-    if (a > 0x7F800000u) return s | 0x7E00u;
-    if (a >= 0x47800000u) return s | 0x7C00u;
-    if (a >= 0x38800000u) {
-        uint32_t r = a - 0x38000000u;
-        r = r + 0xFFFu + ((r >> 13) & 1u);
-        return s | (r >> 13);
-    }
-    if (a < 0x33000000u) return s;
-    uint32_t e = a >> 23, m = (a & 0x7FFFFFu) | 0x800000u;
-    int sh = (int)(113 - e) + 13;
-    uint32_t q = m >> sh, rem = m & ((1u << sh) - 1u), half = 1u << (sh - 1);
-    q += (rem > half) || (rem == half && (q & 1u));
-    return s | q;
+__device__ inline uint32_t f32_bits_to_half_bits(uint32_t u) {
+    asm("" : "+v"(u));   // kept apart from the multiply it follows: contracted into one instruction, a product of -0 comes out as +0
+    return __builtin_bit_cast(uint16_t, (_Float16)bits_f32(u));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -264,6 +242,25 @@ __device__ inline uint32_t encode_mxfp_element(uint32_t u, int se, const F& f) {
     // the encoder sees either a subnormal (flushed) or, if rounding reached 2^-126, a value
     // below the range of every format with E <= 7: both give the sign-only code
     return fmt_sign(f);
+}
+
+// The same code without branches, for a compile-time format and a block whose scale byte lies in [bias, 150] and that holds no
+// inf / NaN: `off` = (scale - bias) << 15 puts the quotient's exponent field in the target format above its 15 mantissa bits, as in
+// encode_f32_finite_rn.  (From scale 151 on a quotient can underflow to exactly zero, which drops its sign.)
+template <class F>
+__device__ inline uint32_t encode_mxfp_in_range(uint32_t u, uint32_t off) {
+    static_assert(F::kStatic, "compile-time formats only");
+    static_assert(F{}.finite() && F{}.rmode() == RN, "finite formats, round to nearest even");
+    constexpr int E = F{}.E(), M = F{}.M(), SH = 15 - M;
+    const uint32_t t = __builtin_elementwise_sub_sat((u >> 8) & 0x7FFFFFu, off);
+    const uint32_t q = t >> SH;
+    const uint32_t v = (t + ((1u << (SH - 1)) - 1u) + (q & 1u)) >> SH;
+    const uint32_t ef = q & ~((1u << M) - 1u);
+    const uint32_t code_n = ef | (v - ef);                 // (the block maximum keeps ye within the top field)
+    const uint32_t code_s = ((min(v, 1u) << M) | v) >> 1;
+    const uint32_t mag = q < (1u << M) ? code_s : code_n;
+    const uint32_t code = mag | ((u >> (31 - E - M)) & (1u << (E + M)));
+    return (u & 0x7F800000u) != 0u ? code : 0u;            // flushed inputs: +0, sign included
 }
 
 }  // namespace mase

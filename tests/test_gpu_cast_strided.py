@@ -220,3 +220,56 @@ def test_strided_argument_errors(mh):
     assert lib.mase_hip_extract_mxfp_strided(None, 2, sc.data_ptr(), el.data_ptr(), 1, 64, 8, 32, 4, 3, 1, 0, s) == -1
     assert lib.mase_hip_qdq_mxfp_strided(x.data_ptr(), 2, x.data_ptr(), 0, 1, 64, 8, 32, 4, 3, 1, 0, s) == -1
     assert lib.mase_hip_extract_mxfp_strided(x.data_ptr(), 2, sc.data_ptr(), el.data_ptr(), 0, 64, 8, 32, 4, 3, 1, 0, s) == 0
+
+
+@pytest.mark.parametrize("dt", ["float16", "float32", "bfloat16"])
+@pytest.mark.parametrize("outer,K,inner", [(1, 32, 1), (1, 96, 63), (1, 128, 65), (3, 160, 7), (2, 288, 129), (5, 64, 64)])
+def test_column_tiles_and_the_scale_range_of_the_branch_free_encoder(mh, dt, outer, K, inner):
+    """Tiles of 64 columns x 4 k-blocks with both ends ragged and columns of several outer slices in one tile.  The blocks of a
+    wavefront share one magnitude, 2^-150 .. 2^127 in turn, so that wavefronts on both sides of the encoder's range of scales
+    (scale < bias, 150 / 151, subnormal and zero maxima, inf / NaN) occur, each with elements 2^0 .. 2^-160 below the maximum."""
+    g = torch.Generator().manual_seed(K + inner)
+    x = torch.randn(outer, K, inner, generator=g, dtype=torch.float64)
+    x = x * torch.exp2(-torch.randint(0, 160, x.shape, generator=g).double() * (torch.rand(x.shape, generator=g) < 0.3))
+    exps = (15, 8, 3, 0, -4, -8, -14, -16, -20, -24) if dt == "float16" else (127, 30, 24, 23, 22, 0, -20, -100, -110, -118, -119, -126, -130, -150)
+    column = torch.arange(outer * inner).view(outer, 1, inner) // 64
+    block = (torch.arange(K) // 32).view(1, K, 1)
+    for shift in range(0, len(exps), 3):
+        v = x * torch.exp2(torch.tensor(exps, dtype=torch.float64)[(column * 5 + block + shift) % len(exps)])
+        v[:, :32, 0] = 0.0
+        if shift == 3:
+            v[0, K - 1, inner - 1], v[outer - 1, 0, inner // 2] = float("nan"), float("-inf")
+        v = v.to(getattr(torch, dt))
+        vd, flat = v.to(DEV), rotated(v, 1)
+        for tag, (e, m) in PRESETS.items():
+            meta = mx_meta(mh, e, m)
+            sc_w, el_w = oracle.extract_mxfp(flat, 32, e, m)
+            dq_w = oracle.compose_mxfp(sc_w, el_w, 32, e, m, True, v.dtype)
+            for sc, el in (mh.mxk.extract_mxfp_components_strided(vd, 1, meta), mh.mxk.extract_mxfp_components(flat.to(DEV), meta)):
+                assert_int_equal(sc, sc_w, f"scales {dt} {tag}")
+                assert_int_equal(el, el_w, f"elements {dt} {tag}")
+            assert_bits_equal(mh.mxk.quantize_dequantize_strided(vd, 1, meta, v.dtype), unrotated(dq_w, v.shape, 1), dt, f"qdq {dt} {tag}")
+            assert_bits_equal(mh.mxk.quantize_dequantize(flat.to(DEV), meta, v.dtype), dq_w, dt, f"flat qdq {dt} {tag}")
+
+
+def test_every_fp16_pattern_in_and_out(mh):
+    """The hardware's fp16 converts on all 65536 patterns: through the minifloat pass of formats up to one that holds fp16 (E5 M10) and the
+    MXFP casts (each pattern as an element of blocks of its neighbours)."""
+    import mase_hip.minifloat.functional as MF
+    from mase_hip.minifloat.meta import MinifloatMeta
+
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    for e, m in ((4, 3), (5, 2), (5, 10)):
+        meta = MinifloatMeta(exp_bits=e, frac_bits=m, is_finite=True, round_mode="rn")
+        codes, tm = MF.extract_minifloat_component(x.to(DEV), meta)
+        want = oracle.extract_minifloat(x, e, m)
+        assert_int_equal(codes, want, f"codes E{e}M{m}")
+        assert_bits_equal(MF.compose_minifloat_component(codes, tm), oracle.compose_minifloat(want, e, m, True, torch.float16), "float16", f"E{e}M{m}")
+    for tag, (e, m) in PRESETS.items():
+        meta = mx_meta(mh, e, m)
+        sc_w, el_w = oracle.extract_mxfp(x, 32, e, m)
+        sc, el = mh.mxk.extract_mxfp_components(x.to(DEV), meta)
+        assert_int_equal(sc, sc_w, f"scales {tag}")
+        assert_int_equal(el, el_w, f"elements {tag}")
+        assert_bits_equal(mh.mxk.quantize_dequantize(x.to(DEV), meta, torch.float16), oracle.compose_mxfp(sc_w, el_w, 32, e, m, True, torch.float16),
+                          "float16", f"qdq {tag}")
