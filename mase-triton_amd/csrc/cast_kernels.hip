@@ -136,6 +136,26 @@ __device__ inline void store_val_scalar(void* base, int64_t i, float y) {
 }
 
 // ------------------------------------------------------------------------------ minifloat
+// Codes of a lane's N elements.  A compile-time format takes the branch-free encoder unless an inf / NaN is among the wavefront's
+// elements (a uniform test), which send all of them through the per-element routine.  At 2^24 fp16 / bf16 elements the routine's
+// vector instructions were in the way of the memory: E4M3 fused pass 16.7 / 16.2 -> 15.3 / 14.8 us (67 MB, 4.5 TB/s), codes and back
+// 27.7 / 27.9 -> 26.8 us; a few million elements are bound by the launches either way.
+template <class F, int N>
+__device__ inline void minifloat_encode(const uint32_t (&u)[N], const F& f, uint32_t (&code)[N]) {
+    if constexpr (F::kStatic) {
+        uint32_t amax = 0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) amax = max(amax, u[j] & 0x7FFFFFFFu);
+        if (__builtin_amdgcn_ballot_w64(amax >= 0x7F800000u) == 0) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) code[j] = encode_f32_finite_rn(u[j], f);
+            return;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) code[j] = encode_f32_bits(u[j], f);
+}
+
 template <int DT_IN, class F, int UNROLL>
 __global__ __launch_bounds__(kThreads) void extract_minifloat_kernel(const void* __restrict__ x,
                                                                       uint16_t* __restrict__ codes, int64_t n, F f) {
@@ -152,11 +172,9 @@ __global__ __launch_bounds__(kThreads) void extract_minifloat_kernel(const void*
     for (int r = 0; r < UNROLL; ++r) {
         const int64_t c = chunk0 + (int64_t)r * kThreads;
         if (c < n_chunks) {
-            uint32_t w[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                w[j] = encode_f32_bits(u[r][2 * j], f) | (encode_f32_bits(u[r][2 * j + 1], f) << 16);
-            st128(codes + c * EPT, make_uint4(w[0], w[1], w[2], w[3]));
+            uint32_t code[EPT];
+            minifloat_encode(u[r], f, code);
+            st128(codes + c * EPT, make_uint4(code[0] | (code[1] << 16), code[2] | (code[3] << 16), code[4] | (code[5] << 16), code[6] | (code[7] << 16)));
         }
     }
     if (blockIdx.x == 0 && threadIdx.x < (n % EPT)) {
@@ -216,9 +234,11 @@ __global__ __launch_bounds__(kThreads) void qdq_minifloat_kernel(const void* x, 
     for (int r = 0; r < UNROLL; ++r) {
         const int64_t c = chunk0 + (int64_t)r * kThreads;
         if (c < n_chunks) {
+            uint32_t code[EPT];
             float y[EPT];
+            minifloat_encode(u[r], f, code);
 #pragma unroll
-            for (int j = 0; j < EPT; ++j) y[j] = decode_f32(encode_f32_bits(u[r][j], f), f);
+            for (int j = 0; j < EPT; ++j) y[j] = decode_f32(code[j], f);
             store_vals<DT_OUT, EPT, false>(out, c * EPT, y);
         }
     }
@@ -247,22 +267,7 @@ __global__ __launch_bounds__(kThreads) void minifloat_f32_kernel(const void* x, 
         const uint32_t* p = static_cast<const uint32_t*>(x) + wave_first + 4 * lane;
         const uint4 a = ld128<MASE_QDQ_NT || MODE == 0>(p), b = ld128<MASE_QDQ_NT || MODE == 0>(p + 256);
         const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        // inf / NaN anywhere in the wavefront's 512 elements: the per-element routine for all of them
-        uint32_t amax = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) amax = max(amax, u[j] & 0x7FFFFFFFu);
-        bool fast = false;
-        if constexpr (F::kStatic) {
-            fast = __builtin_amdgcn_ballot_w64(amax >= 0x7F800000u) == 0;
-            if (fast) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) code[j] = encode_f32_finite_rn(u[j], f);
-            }
-        }
-        if (!fast) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) code[j] = encode_f32_bits(u[j], f);
-        }
+        minifloat_encode(u, f, code);
     }
     if (MODE == 0) {
         uint16_t* c = static_cast<uint16_t*>(out) + wave_first + 4 * lane;

@@ -333,3 +333,20 @@ def test_error_codes(mh):
     assert lib.mase_hip_extract_minifloat(x.data_ptr(), 2, el.data_ptr(), 64, 9, 9, 1, 0, None) == -1
     with pytest.raises(ValueError):
         _lib.check(lib.mase_hip_extract_mxfp(None, 2, sc.data_ptr(), el.data_ptr(), 64, 32, 4, 3, 1, 0, None))
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("count", [1, 7, 511, 65536, 65536 + 2053])
+def test_minifloat_16bit_casts_every_pattern(mh, dt, count):
+    """Codes and the fused pass over every pattern in order (wavefronts of 512 elements with only finite values, and with inf / NaN
+    among them), and ragged ends: bit for bit."""
+    import mase_hip.minifloat.functional as MF
+    from mase_hip.minifloat.meta import MinifloatMeta
+
+    x = (torch.arange(count, dtype=torch.int32) * (1 if count >= 65536 else 9973)).to(torch.int16).view(getattr(torch, dt))
+    for e, m in PRESETS.values():
+        meta = MinifloatMeta(exp_bits=e, frac_bits=m, is_finite=True, round_mode="rn")
+        want = oracle.extract_minifloat(x, e, m)
+        codes, _ = MF.extract_minifloat_component(x.to(DEV), meta)
+        assert_int_equal(codes, want, f"codes {dt} E{e}M{m}")
+        assert_bits_equal(MF.quantize_dequantize(x.to(DEV), meta), oracle.compose_minifloat(want, e, m, True, x.dtype), dt, f"qdq {dt} E{e}M{m}")
