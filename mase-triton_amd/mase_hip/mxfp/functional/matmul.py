@@ -103,9 +103,10 @@ def _other_components(other: Tensor, other_meta: MXFPMeta) -> tuple[Tensor, Tens
     """Components of ``other`` [.., K, N], blocks along K, in [.., N, K] order.  The transposed view of a contiguous tensor (the
     keys of an attention product) lies in that order already and goes through the flat kernel; a contiguous one through the
     strided kernel.  (K is a multiple of 32 on this route, so no block straddles two rows either way.)"""
-    lying = other.transpose(-1, -2)
-    if lying.is_contiguous():
-        return kernels.extract_mxfp_components(lying.reshape(-1), other_meta)
+    if not other.is_contiguous():                            # (asked first: a small product is bound by the host)
+        lying = other.transpose(-1, -2)
+        if lying.is_contiguous():
+            return kernels.extract_mxfp_components(lying.reshape(-1), other_meta)
     return kernels.extract_mxfp_components_strided(other, -2, other_meta)
 
 
