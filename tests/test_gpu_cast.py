@@ -350,3 +350,31 @@ def test_minifloat_16bit_casts_every_pattern(mh, dt, count):
         codes, _ = MF.extract_minifloat_component(x.to(DEV), meta)
         assert_int_equal(codes, want, f"codes {dt} E{e}M{m}")
         assert_bits_equal(MF.quantize_dequantize(x.to(DEV), meta), oracle.compose_minifloat(want, e, m, True, x.dtype), dt, f"qdq {dt} E{e}M{m}")
+
+
+@pytest.mark.parametrize("n", [32, 256, 288, 512, 544, 2016, 2048, 2080, 12320])
+def test_mxfp_f32_blocks_of_32_at_the_edges_of_a_wavefront(mh, n):
+    """fp32 casts, whose lanes hold two runs of four 256 elements apart: every remainder of a wavefront's 512 elements that is a number
+    of blocks, an element of its own magnitude at each place of a block in turn (the maximum over eight lanes), zero, subnormal,
+    inf / NaN and out-of-range blocks.  Bit for bit."""
+    import mase_hip.mxfp.kernels as mxk
+    from mase_hip.mxfp.meta import MXFPMeta
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(n // 32, 32, generator=g)
+    b = torch.arange(n // 32)
+    x[b, (b * 5) % 32] *= 300.0
+    for special in (None, 0.0, 1e-39, float("inf"), float("nan"), 3e38, 1e-37):
+        v = x.clone()
+        if special is not None:
+            v[(n // 32) // 2] = torch.full((32,), special) * (1 if special == 0.0 or special != special or special > 1e38 else torch.randn(32, generator=g))
+            v[-1, 31] = -special
+        v = v.reshape(-1)
+        for e, m in PRESETS.values():
+            meta = MXFPMeta(block_size=32, scale_exp_bits=8, element_exp_bits=e, element_frac_bits=m, element_is_finite=True, round_mode="rn")
+            sc_w, el_w = oracle.extract_mxfp(v, 32, e, m)
+            dq_w = oracle.compose_mxfp(sc_w, el_w, 32, e, m, True, torch.float32)
+            sc, el = mxk.extract_mxfp_components(v.to(DEV), meta)
+            assert_int_equal(sc, sc_w, f"scales {n} {special} E{e}M{m}")
+            assert_int_equal(el, el_w, f"elements {n} {special} E{e}M{m}")
+            assert_bits_equal(mxk.quantize_dequantize(v.to(DEV), meta, torch.float32), dq_w, "float32", f"qdq {n} {special} E{e}M{m}")
