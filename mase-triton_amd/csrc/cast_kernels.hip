@@ -1156,8 +1156,10 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_tile_kernel(const void*
     const int64_t unit = (int64_t)(blockIdx.x % 8u) * (gridDim.x / 8u) + blockIdx.x / 8u;
     const int64_t kg = unit / col_tiles, col0 = (unit - kg * col_tiles) * 64, kb0 = kg * 4;
     if (kb0 >= nkb) return;
-    const int64_t col = col0 + lane;
-    if (col < columns && kb0 + q < nkb) {
+    if (kb0 + q < nkb) {                                   // (the whole wavefront)
+        // lanes past the last column redo it: with them masked off, a wavefront of eight lanes or fewer is held up at the issue of its
+        // vector instructions (65 columns x 32 k-blocks: 9.0 us against 4.1 at 81)
+        const int64_t col = min(col0 + lane, columns - 1);
         const int64_t o = col / inner;
         const int64_t first = (o * K + (kb0 + q) * 32) * inner + (col - o * inner);
         uint32_t u[32], amax = 0, code[32], scale;
