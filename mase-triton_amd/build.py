@@ -19,9 +19,9 @@ CSRC = os.path.join(ROOT, "csrc")
 OBJ = os.path.join(ROOT, "build")
 LIB_DIR = os.path.join(ROOT, "mase_hip", "lib")
 LIB = os.path.join(LIB_DIR, "libmase_hip.so")
-# helpers of the benchmark and the tests (a tuned streaming copy as yardstick; the SwiGLU arithmetic on its own); not part of
-# the product's C ABI
-BENCH_SRCS = [os.path.join(CSRC, "bench", f) for f in ("stream_copy.hip", "swiglu_probe.hip")]
+# helpers of the benchmark and the tests (a tuned streaming copy as yardstick; the SwiGLU arithmetic on its own; the rules of the
+# dispatch); not part of the product's C ABI
+BENCH_SRCS = [os.path.join(CSRC, "bench", f) for f in ("stream_copy.hip", "swiglu_probe.hip", "dispatch_probe.hip")]
 BENCH_LIB = os.path.join(LIB_DIR, "libmase_bench.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

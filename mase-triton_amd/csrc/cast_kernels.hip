@@ -1138,13 +1138,14 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_bf16_lines_kernel(const
     }
 }
 
-// Extract for any dtype, format and extents: the same exchange with one column to a lane.  A workgroup takes 64 adjacent columns of
-// the [outer * inner] there are (a lane finds its own place, so a short inner axis fills the wavefronts too) and four
-// consecutive k-blocks, one per wavefront; what lies past the end of either is masked.  Loads are one element per lane: rows of an
-// odd number of elements are at no better alignment.  Needs 16-byte aligned elements.
-// 2976 x 4096 (37 MB to move): fp16 26.5 -> 14.2 us, fp32 18.4 -> 14.8 (49 MB), bf16 with an odd row length 17.1 -> 14.5, against the
-// kernel above that stores a column's 32 codes by itself and takes the general encoder: half of that gain is the encoder's, and
-// vector instructions (about 25 per element) still take as long as the memory.  At 64 x 1000: 11.6 / 6.7 -> 3.9 us.
+// Extract for any dtype and extents and a compile-time format: the same exchange with one column to a lane.  A workgroup takes 64
+// adjacent columns of the [outer * inner] there are (a lane finds its own place, so a short inner axis beside a long outer one fills the
+// wavefronts too; few columns in all do not, see strided_column_tiles) and four consecutive k-blocks, one per wavefront; what
+// lies past the end of either is not stored.  Loads are one element per lane: rows of an odd number of elements are at no
+// better alignment.  Needs 16-byte aligned elements.
+// 2976 x 4096, repeated on one input: fp16 (37 MB to move) 26.5 -> 14.2 us, fp32 (61 MB) 18.4 -> 14.8, bf16 with an odd row length 17.1 ->
+// 14.5, against mxfp_strided_kernel, which stores a column's 32 codes by itself, with the general encoder: half of that gain is the
+// encoder's, and vector instructions (about 25 per element) still take as long as the memory.  At 64 x 1000: 11.6 / 6.7 -> 3.9 us.
 template <int DT_IN, class F>
 __global__ __launch_bounds__(kThreads) void mxfp_strided_tile_kernel(const void* __restrict__ x, uint8_t* __restrict__ scales,
                                                                       uint8_t* __restrict__ elements, int64_t K, int64_t inner,
@@ -1536,10 +1537,10 @@ int mase_hip_extract_mxfp_strided(const void* x, int x_dtype, uint8_t* scales, u
                 return check_launch("extract_mxfp_strided");
             }
         }
-        if (el16) {
+        if constexpr (decltype(f)::kStatic) {   // (the run-time formats' arithmetic hides the stores: level, or up to 12 % slower in tiles)
             const int64_t columns = outer * inner, col_tiles = (columns + 63) / 64, nkb = k_len / 32;
             const int64_t blocks = (col_tiles * ((nkb + 3) / 4) + 7) / 8 * 8;
-            if (blocks <= 0x7FFFFFFFll)
+            if (el16 && blocks <= 0x7FFFFFFFll && strided_column_tiles(columns, nkb, dtype_size(x_dtype)))
                 return dispatch_dtype(x_dtype, [&](auto dt) {
                     hipLaunchKernelGGL((mxfp_strided_tile_kernel<decltype(dt)::value, decltype(f)>), dim3((unsigned)blocks), dim3(kThreads), 0, s,
                                        x, scales, elements, k_len, inner, columns, nkb, col_tiles, f);

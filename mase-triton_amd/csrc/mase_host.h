@@ -82,6 +82,21 @@ inline int check_dtype(int dt, const char* which) {
 
 inline int dtype_size(int dt) { return dt == F32 ? 4 : 2; }
 
+// Extract down the rows of `columns` columns and nkb k-blocks in tiles of 64 columns (one wavefront per tile and k-block)?  A tile that
+// its columns do not fill costs a whole one, which shows once there are more wavefronts than the chip has room to overlap: from
+// then on the kernel whose lanes are blocks of any column.  fp32, tiles / other kernel, us, at 512, 2048, 8192 and 32768 k-blocks: 1 column
+// 4.2 / 6.8, 5.4 / 6.8, 13.9 / 6.9, 48 / 7.0; 16 columns 4.2 / 4.1, 5.5 / 4.3, 14.6 / 6.0, 49 / 24 (fp16 53 / 18); 48 columns 4.4 / 4.4,
+// 5.9 / 6.2, 16.4 / 15.5; 65 columns 4.3 / 4.8, 8.9 / 7.8, 27.3 / 24.8; 96 columns 4.4 / 5.0, 9.1 / 9.4, 28.4 / 28.5 (fp16 28.8 / 24.4); 97 columns
+// 4.4 / 5.2, 9.3 / 10.7, 28.8 / 32.6 (fp16 29.1 / 27.6); fp32 129 columns 22.2 / 23.9 at 4096, fp16 22.4 / 20.2.  Fuller tiles are ahead at every size but the smallest, where they are level.
+// The same for the four k-blocks of a workgroup: with 262144 columns 14.8 / 9.6 at one k-block (fp16 14.5 / 9.5), and 21.1 / 20.4 (21.2 / 19.3)
+// at two; 29.8 / 26.2 (28.9 / 19.9) at five and 131072; at 65536 columns of one or two k-blocks 7.6 / 8.2 and 11.2 / 12.6.
+inline bool strided_column_tiles(int64_t columns, int64_t nkb, int element_bytes) {
+    const int64_t tiles = (columns + 63) / 64, waves = tiles * nkb, groups = (nkb + 3) / 4;
+    if (waves >= 2048 && columns * 2 <= tiles * 64) return false;
+    if (waves >= 4096 && columns * 8 <= tiles * 64 * (element_bytes == 4 ? 5 : 6)) return false;
+    return tiles * groups < 2048 || nkb * 8 > groups * 4 * 5;
+}
+
 // Calls fn(format object): a compile-time format for the five round-to-nearest finite
 // presets, the run-time one otherwise.
 template <class Fn>

@@ -1,0 +1,42 @@
+"""The rules by which a launcher picks a kernel, asked on the CPU through the test helper library (the launchers call the same functions)."""
+import ctypes
+import os
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def lib():
+    path = os.path.join(ROOT, "mase-triton_amd", "mase_hip", "lib", "libmase_bench.so")
+    assert os.path.exists(path), "libmase_bench.so is not built (python mase-triton_amd/build.py)"
+    return ctypes.CDLL(path)
+
+
+def column_tiles(lib, columns, nkb, element_bytes):
+    lib.mase_bench_strided_column_tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    return bool(lib.mase_bench_strided_column_tiles(columns, nkb, element_bytes))
+
+
+@pytest.mark.parametrize("element_bytes", [2, 4])
+def test_few_columns_do_not_go_in_column_tiles(lib, element_bytes):
+    for columns in (1, 3, 8, 16, 31, 32):           # wavefronts at most half full: one per k-block
+        assert column_tiles(lib, columns, 2047, element_bytes)
+        assert not column_tiles(lib, columns, 2048, element_bytes) and not column_tiles(lib, columns, 1 << 20, element_bytes)
+    for columns in (33, 40):                        # five eighths
+        assert column_tiles(lib, columns, 4095, element_bytes) and not column_tiles(lib, columns, 4096, element_bytes)
+    for columns in (65, 80):                        # two wavefronts per k-block
+        assert column_tiles(lib, columns, 2047, element_bytes) and not column_tiles(lib, columns, 2048, element_bytes)
+    for columns in (41, 48, 96, 129):               # up to three quarters: by the element's size
+        assert column_tiles(lib, columns, 1 << 16, element_bytes) == (element_bytes == 4)
+    for columns in (49, 64, 97, 128, 193, 1001, 4096, 1 << 20):
+        assert column_tiles(lib, columns, 3, element_bytes) and column_tiles(lib, columns, 1 << 20, element_bytes)
+
+
+def test_many_columns_of_one_or_two_blocks_do_not_go_in_column_tiles(lib):
+    for nkb in (1, 2):                              # of the four k-blocks of a workgroup
+        assert column_tiles(lib, 1 << 16, nkb, 4) and not column_tiles(lib, 1 << 17, nkb, 4)
+    assert column_tiles(lib, 1 << 15, 5, 2) and not column_tiles(lib, 1 << 16, 5, 2)      # five of eight
+    for nkb in (3, 4, 6, 7, 8, 9, 93):
+        assert column_tiles(lib, 1 << 20, nkb, 2)

@@ -273,3 +273,22 @@ def test_every_fp16_pattern_in_and_out(mh):
         assert_int_equal(el, el_w, f"elements {tag}")
         assert_bits_equal(mh.mxk.quantize_dequantize(x.to(DEV), meta, torch.float16), oracle.compose_mxfp(sc_w, el_w, 32, e, m, True, torch.float16),
                           "float16", f"qdq {tag}")
+
+
+@pytest.mark.parametrize("dt", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("outer,K,inner", [(1, 2047 * 32, 3), (1, 2048 * 32, 3), (1, 4095 * 32, 37), (1, 4096 * 32, 37), (1, 2048 * 32, 65), (43, 2048 * 32, 1),
+                                           (5, 32 * 7, 13), (1, 96, 1), (1, 160, 193), (1, 32, 131071), (3, 64, 43700)])
+def test_few_columns_on_both_sides_of_the_tile_rule(mh, dt, outer, K, inner):
+    """Tiles of 64 columns that few columns fill in part (lanes past the last one redo it), and from 2048 / 4096 wavefronts on the
+    kernel without tiles, as with many columns of one or two blocks: bit for bit."""
+    g = torch.Generator().manual_seed(K + inner)
+    v = torch.randn(outer, K, inner, generator=g)
+    v = (v * torch.exp2(torch.randint(-12, 12, (1, K, 1), generator=g).float())).to(getattr(torch, dt))
+    v[0, :32, 0] = 0.0
+    flat = rotated(v, 1)
+    for tag in ("MXFP8_E4M3_fn", "OCP_MXFP4_E2M1"):
+        e, m = PRESETS[tag]
+        sc_w, el_w = oracle.extract_mxfp(flat, 32, e, m)
+        sc, el = mh.mxk.extract_mxfp_components_strided(v.to(DEV), 1, mx_meta(mh, e, m))
+        assert_int_equal(sc, sc_w, f"scales {dt} {tag}")
+        assert_int_equal(el, el_w, f"elements {dt} {tag}")

@@ -40,3 +40,15 @@ def test_extract_down_the_rows_with_a_last_tile_of_few_columns(dt, columns):
     few, more = (torch.randn(1024, c, device=DEV).to(dt) for c in (columns, columns + 16))
     t_few, t_more = (gpu_us(lambda x=x: mxk.extract_mxfp_components_strided(x, 0, fmt)) for x in (few, more))
     assert t_few <= 1.4 * t_more, (t_few, t_more)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
+def test_extract_down_one_long_column(dt):
+    """One column is the flat tensor: the kernels for blocks down the rows may cost a few times the flat one's time (7 against 3 us),
+    not 15 times (one lane of a wavefront at work: 47 - 54 us)."""
+    import mase_hip.mxfp.kernels as mxk
+    from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
+
+    x = torch.randn(1 << 20, 1, device=DEV).to(dt)
+    t, t_flat = gpu_us(lambda: mxk.extract_mxfp_components_strided(x, 0, fmt)), gpu_us(lambda: mxk.extract_mxfp_components(x.view(-1), fmt))
+    assert t <= 4 * t_flat, (t, t_flat)
