@@ -24,3 +24,8 @@ extern "C" int mase_bench_scaled_plan(int64_t M, int64_t N, int64_t K, int cus, 
 extern "C" int mase_bench_strided_column_tiles(int64_t columns, int64_t nkb, int element_bytes) {
     return mase::strided_column_tiles(columns, nkb, element_bytes) ? 1 : 0;
 }
+
+// does a product without bias go to the kernel for short contractions?
+extern "C" int mase_bench_short_k(int64_t M, int64_t N, int64_t K, int64_t batches) {
+    return mase::short_k_shape_ok((int)M, (int)N, (int)K, (int)batches) ? 1 : 0;
+}

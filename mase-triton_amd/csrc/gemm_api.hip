@@ -46,7 +46,7 @@ static int gemm_entry(const void* a_dense, int a_dtype, const uint8_t* a_scales,
     }
     const GemmArgs g{a_dense, a_scales, a_elements, a_is_dense ? 0 : a_exp_bits, a_frac_bits, w_scales, w_elements, bias, bias_dtype,
                      y, out_dtype, (int)M, (int)N, (int)K, workspace, workspace_bytes, static_cast<hipStream_t>(stream), (int)batches, gb};
-    // a short contraction is bound by its outputs: one kernel for every M and N
+    // a short contraction is bound by its outputs
     if (short_k_ok(g)) return gemm_short_k(g, w_exp_bits, w_frac_bits);
     if (w_exp_bits == 4 && w_frac_bits == 3) return gemm_w_e4m3(g);
     if (w_exp_bits == 5 && w_frac_bits == 2) return gemm_w_e5m2(g);

@@ -578,7 +578,17 @@ struct GemmArgs {
 };
 // gemm_short_k.hip
 int gemm_short_k(const GemmArgs& g, int w_exp_bits, int w_frac_bits);
-inline bool short_k_ok(const GemmArgs& g) { return g.a_dense && !g.bias && g.K <= 128 && g.N <= (1 << 23); }   // (32-bit offsets within 64 rows)
+inline bool short_k_shape_ok(int M, int N, int K, int batches) {
+    if (K > 128 || N > (1 << 23)) return false;             // (32-bit offsets within 64 rows)
+    // Up to 64 rows of A and K = 128: the weight-streaming kernels start faster (their shortest call takes 2.8 us, this one's 6: it composes
+    // 128 x 128 codes before its first product), until there are more rows of W, of all products together, than the chip takes at once.
+    // Old / this one, us, at 4096, 16384 and 32768 rows of W, bf16: M = 1 2.9 / 6.2, 4.8 / 6.4, 7.2 / 6.5; M = 32 3.2 / 6.4, 4.8 - 5.3 / 6.6, 8.1 /
+    // 6.7; M = 64 3.7 / 6.5, 6.4 - 7.3 / 6.7, 11.0 - 12.4 / 6.8; 14336 and 20480 rows: M = 64 6.2 / 6.7, 9.9 / 6.8, M = 32 4.7 / 6.6, 7.0 / 6.7.
+    const bool streams = K == 128 && M <= 64 && ((N % R16_N == 0 && N <= (M <= 16 ? 12288 : 8192)) || N % SK_N == 0);
+    if (streams && (int64_t)N * batches <= (M <= 16 ? 28672 : M <= 32 ? 18432 : 14336)) return false;
+    return true;
+}
+inline bool short_k_ok(const GemmArgs& g) { return g.a_dense && !g.bias && short_k_shape_ok(g.M, g.N, g.K, g.batches); }
 int gemm_w_e4m3(const GemmArgs& g);
 int gemm_w_e5m2(const GemmArgs& g);
 int gemm_w_e2m3(const GemmArgs& g);

@@ -40,3 +40,19 @@ def test_many_columns_of_one_or_two_blocks_do_not_go_in_column_tiles(lib):
     assert column_tiles(lib, 1 << 15, 5, 2) and not column_tiles(lib, 1 << 16, 5, 2)      # five of eight
     for nkb in (3, 4, 6, 7, 8, 9, 93):
         assert column_tiles(lib, 1 << 20, nkb, 2)
+
+
+def short_k(lib, M, N, K, batches=1):
+    lib.mase_bench_short_k.argtypes = [ctypes.c_int64] * 4
+    return bool(lib.mase_bench_short_k(M, N, K, batches))
+
+
+def test_few_rows_of_a_short_contraction_stay_on_the_weight_streaming_kernels(lib):
+    for M, most in ((1, 28672), (16, 28672), (17, 18432), (32, 18432), (33, 14336), (64, 14336)):
+        assert not short_k(lib, M, 32, 128) and not short_k(lib, M, most, 128) and short_k(lib, M, most + 32, 128)
+        assert not short_k(lib, M, 1024, 128, most // 1024) and short_k(lib, M, 1024, 128, most // 1024 + 1)    # rows of W of all products
+        assert short_k(lib, M, 4096, 96) and short_k(lib, M, 4096, 64)      # those kernels take whole 128-k steps
+        assert short_k(lib, M, 1000, 128) and short_k(lib, M, 1001, 128)    # and whole groups of 16 or 32 rows of W
+    assert not short_k(lib, 8, 48, 128) and short_k(lib, 8, 12304, 128) and short_k(lib, 40, 8208, 128)   # 16-row groups up to 12288 / 8192 only
+    assert short_k(lib, 65, 4096, 128) and short_k(lib, 1000, 1000, 128, 64)
+    assert not short_k(lib, 4096, 4096, 160)
