@@ -586,6 +586,14 @@ inline bool short_k_shape_ok(int M, int N, int K, int batches) {
     // 6.7; M = 64 3.7 / 6.5, 6.4 - 7.3 / 6.7, 11.0 - 12.4 / 6.8; 14336 and 20480 rows: M = 64 6.2 / 6.7, 9.9 / 6.8, M = 32 4.7 / 6.6, 7.0 / 6.7.
     const bool streams = K == 128 && M <= 64 && ((N % R16_N == 0 && N <= (M <= 16 ? 12288 : 8192)) || N % SK_N == 0);
     if (streams && (int64_t)N * batches <= (M <= 16 ? 28672 : M <= 32 ? 18432 : 14336)) return false;
+    // One product that gives the 512 x 128 kernel a full round of tiles or more: that one, up to 32768 columns.  (It writes larger pieces of
+    // y, and its walk hides the ends of tiles; products of a batch are grid planes there, whose ends nothing hides: 64 of 1024 x 1024 take
+    // 115 us against 32.)  That kernel / this one, us, bf16 | fp32 out: 1024 x 14336 10.7 / 16.4 | 16.4 / 18.7; 512 x 28672 10.5 / 16.3 | 16.1 /
+    // 18.2; 3000 x 4096 10.1 / 14.5 | 14.6 / 18.0; 16384 x 1024 11.7 / 14.6 | 17.0 / 22.1; 16384 x 4096 35.6 / 34.3 | 53.8 / 76.2; 16384 x 14336 103 /
+    // 113 | 192 / 193; 4096 x 8192 23.1 / 20.4 | 43.5 / 37.2 (the worst for it).  With fewer tiles 2048 x 2048 9.6 / 8.8 | 12.1 / 9.8, 8192 x 1024 11.5 /
+    // 9.6 | 20.3 / 12.8; with more columns 2048 x 65536 78.6 / 57.2 | 137 / 113.
+    const int64_t tall_tiles = (int64_t)((M + UM - 1) / UM) * (N / UN);
+    if (batches == 1 && K == 128 && M >= UM && N % UN == 0 && N <= 32768 && tall_tiles >= 160) return false;
     return true;
 }
 inline bool short_k_ok(const GemmArgs& g) { return g.a_dense && !g.bias && short_k_shape_ok(g.M, g.N, g.K, g.batches); }

@@ -56,3 +56,11 @@ def test_few_rows_of_a_short_contraction_stay_on_the_weight_streaming_kernels(li
     assert not short_k(lib, 8, 48, 128) and short_k(lib, 8, 12304, 128) and short_k(lib, 40, 8208, 128)   # 16-row groups up to 12288 / 8192 only
     assert short_k(lib, 65, 4096, 128) and short_k(lib, 1000, 1000, 128, 64)
     assert not short_k(lib, 4096, 4096, 160)
+
+
+def test_full_rounds_of_large_tiles_stay_on_the_kernel_of_large_tiles(lib):
+    for M, N in ((1024, 14336), (512, 28672), (3000, 4096), (16384, 1024), (16384, 4096), (16384, 14336), (1000, 12288)):   # 160 tiles of 512 x 128 or more
+        assert not short_k(lib, M, N, 128)
+        assert short_k(lib, M, N, 128, 2) and short_k(lib, M, N, 96) and short_k(lib, M, N + 8, 128)
+    for M, N in ((2048, 2048), (8192, 1024), (4096, 2048), (511, 32768), (2048, 65536), (512, 20352)):
+        assert short_k(lib, M, N, 128)

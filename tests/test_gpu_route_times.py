@@ -75,6 +75,19 @@ def test_short_contraction_of_few_rows(M, N):
     assert t <= 1.2 * t_bias, (t, t_bias)
 
 
+@pytest.mark.parametrize("M,N,odt", [(1024, 14336, torch.bfloat16), (512, 28672, torch.bfloat16), (3000, 4096, torch.bfloat16), (16384, 4096, torch.float32)])
+def test_short_contraction_of_a_full_round_of_large_tiles(M, N, odt):
+    """The same for one product of at least 160 tiles of 512 x 128: 10.7 us at 1024 x 14336 with a bias, 16.4 on the kernel for short
+    contractions."""
+    import mase_hip.mxfp.kernels as mxk
+    from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
+
+    a, sc, el = _product(M, N, 128)
+    bias = torch.randn(N, device=DEV).to(torch.bfloat16)
+    t, t_bias = (gpu_us(lambda b=b: mxk.mxfp_gemm(a, None, None, None, sc, el, fmt, b, M, N, 128, odt)) for b in (None, bias))
+    assert t <= 1.2 * t_bias, (t, t_bias)
+
+
 def test_attention_scores_of_one_query():
     """One query per head against 2048 keys of 8 heads: 4.8 us on the weight-streaming kernel, 6.4 on the kernel for short contractions.
     Held to the time of one product with as many rows of W and a bias."""
