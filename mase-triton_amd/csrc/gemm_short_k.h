@@ -192,8 +192,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
                 }
             } else {
                 constexpr int COLS = 128 / ESZ;                  // columns of a staging row
+                const int steps = (int)((min(rows_left, (int64_t)32) * COLS + 63) / 64);   // rows there are (rows past M: none, also below zero)
 #pragma unroll 1
-                for (int i = 0; i < 32 * COLS / 64; ++i) {
+                for (int i = 0; i < steps; ++i) {
                     const int row = i * 64 / COLS + (COLS == 32 ? g2 : 0), b = (lane % COLS) * ESZ;
                     const int col = col0 + lane % COLS;
                     const uint8_t* const s = out + row * 128 + (((b >> 4) ^ ((row >> 1) & 7)) * 16) + (b & 15);
