@@ -583,9 +583,10 @@ inline bool short_k_shape_ok(int M, int N, int K, int batches) {
     // Up to 64 rows of A and K = 128: the weight-streaming kernels start faster (their shortest call takes 2.8 us, this one's 6: it composes
     // 128 x 128 codes before its first product), until there are more rows of W, of all products together, than the chip takes at once.
     // Old / this one, us, at 4096, 16384 and 32768 rows of W, bf16: M = 1 2.9 / 6.2, 4.8 / 6.4, 7.2 / 6.5; M = 32 3.2 / 6.4, 4.8 - 5.3 / 6.6, 8.1 /
-    // 6.7; M = 64 3.7 / 6.5, 6.4 - 7.3 / 6.7, 11.0 - 12.4 / 6.8; 14336 and 20480 rows: M = 64 6.2 / 6.7, 9.9 / 6.8, M = 32 4.7 / 6.6, 7.0 / 6.7.
+    // 6.7; M = 64 3.7 / 6.5, 6.4 - 7.3 / 6.7, 11.0 - 12.4 / 6.8; 14336 and 20480 rows: M = 64 6.2 / 6.7, 9.9 / 6.8, M = 32 4.7 / 6.6, 7.0 / 6.7;
+    // 24576 and 26624 rows: M <= 16 5.5 / 6.6, 7.3 / 6.6.
     const bool streams = K == 128 && M <= 64 && ((N % R16_N == 0 && N <= (M <= 16 ? 12288 : 8192)) || N % SK_N == 0);
-    if (streams && (int64_t)N * batches <= (M <= 16 ? 28672 : M <= 32 ? 18432 : 14336)) return false;
+    if (streams && (int64_t)N * batches <= (M <= 16 ? 24576 : M <= 32 ? 18432 : 14336)) return false;
     // One product that gives the 512 x 128 kernel a full round of tiles or more: that one, up to 32768 columns.  (It writes larger pieces of
     // y, and its walk hides the ends of tiles; products of a batch are grid planes there, whose ends nothing hides: 64 of 1024 x 1024 take
     // 115 us against 32.)  That kernel / this one, us, bf16 | fp32 out: 1024 x 14336 10.7 / 16.4 | 16.4 / 18.7; 512 x 28672 10.5 / 16.3 | 16.1 /
@@ -594,6 +595,13 @@ inline bool short_k_shape_ok(int M, int N, int K, int batches) {
     // 9.6 | 20.3 / 12.8; with more columns 2048 x 65536 78.6 / 57.2 | 137 / 113.
     const int64_t tall_tiles = (int64_t)((M + UM - 1) / UM) * (N / UN);
     if (batches == 1 && K == 128 && M >= UM && N % UN == 0 && N <= 32768 && tall_tiles >= 160) return false;
+    // 129 - 192 rows, three 64-row tiles to a column: with more tiles than workgroups, runs of two that change column compose W
+    // twice.  While the 256 x 128 kernel has a tile for each column and CU (N = 21888 .. 32768) it takes 8.4 - 9.8 us against 12.5.
+    if (batches == 1 && K == 128 && M > 128 && M <= 192 && N % WD_N == 0 && N / WD_N * 3 > 512 && N / WD_N <= 256) return false;
+    // A few rows of any other N at K = 128: the small-tile kernel's one round (256 workgroups of 128 columns; 33 us with one more) starts
+    // faster: 1 row of 1000 .. 20001 columns 5.5 - 5.7 us against 6.1 - 6.4 (fp32 out 6.4 - 6.9), 8 rows 6.2 / 6.7 (6.9); 16 rows 7.0 / 6.2 - 7.5, 40
+    // columns 5.2 / 4.9, K = 96 5.1 - 5.9 / 4.7 - 5.5.  And a few columns that leave element by element: N = 1 3.4 - 5.6 / 3.8 - 6.5, any K.
+    if (!streams && (int64_t)((N + SBN - 1) / SBN) * batches <= 256 && ((M <= 8 && N >= 128 && K == 128) || (M <= 32 && N < 16 && N % 8 != 0))) return false;
     return true;
 }
 inline bool short_k_ok(const GemmArgs& g) { return g.a_dense && !g.bias && short_k_shape_ok(g.M, g.N, g.K, g.batches); }

@@ -48,12 +48,12 @@ def short_k(lib, M, N, K, batches=1):
 
 
 def test_few_rows_of_a_short_contraction_stay_on_the_weight_streaming_kernels(lib):
-    for M, most in ((1, 28672), (16, 28672), (17, 18432), (32, 18432), (33, 14336), (64, 14336)):
-        assert not short_k(lib, M, 32, 128) and not short_k(lib, M, most, 128) and short_k(lib, M, most + 32, 128)
-        assert not short_k(lib, M, 1024, 128, most // 1024) and short_k(lib, M, 1024, 128, most // 1024 + 1)    # rows of W of all products
-        assert short_k(lib, M, 4096, 96) and short_k(lib, M, 4096, 64)      # those kernels take whole 128-k steps
-        assert short_k(lib, M, 1000, 128) and short_k(lib, M, 1001, 128)    # and whole groups of 16 or 32 rows of W
-    assert not short_k(lib, 8, 48, 128) and short_k(lib, 8, 12304, 128) and short_k(lib, 40, 8208, 128)   # 16-row groups up to 12288 / 8192 only
+    for M, most in ((1, 24576), (16, 24576), (17, 18432), (32, 18432), (33, 14336), (64, 14336)):
+        assert not short_k(lib, M, 32, 128) and not short_k(lib, M, most, 128)
+        assert not short_k(lib, M, 1024, 128, most // 1024)
+        assert short_k(lib, M, most + 32, 128) and short_k(lib, M, 1024, 128, most // 1024 + 1)     # rows of W of all products
+        assert short_k(lib, M, 4096, 64)                                    # those kernels take whole 128-k steps
+    assert not short_k(lib, 8, 48, 128) and short_k(lib, 9, 12304, 128) and short_k(lib, 40, 8208, 128)   # 16-row groups up to 12288 / 8192 only
     assert short_k(lib, 65, 4096, 128) and short_k(lib, 1000, 1000, 128, 64)
     assert not short_k(lib, 4096, 4096, 160)
 
@@ -64,3 +64,20 @@ def test_full_rounds_of_large_tiles_stay_on_the_kernel_of_large_tiles(lib):
         assert short_k(lib, M, N, 128, 2) and short_k(lib, M, N, 96) and short_k(lib, M, N + 8, 128)
     for M, N in ((2048, 2048), (8192, 1024), (4096, 2048), (511, 32768), (2048, 65536), (512, 20352)):
         assert short_k(lib, M, N, 128)
+
+
+def test_few_rows_of_any_number_of_columns_stay_on_the_small_tiles(lib):
+    for N in (129, 1000, 1001, 20001, 32767):
+        assert not short_k(lib, 1, N, 128) and not short_k(lib, 8, N, 128)
+        assert short_k(lib, 9, N, 128) and short_k(lib, 8, N, 64) and short_k(lib, 8, N, 96)
+    assert short_k(lib, 1, 32769, 128) and short_k(lib, 1, 1000, 128, 33) and not short_k(lib, 1, 1000, 128, 32)     # 256 workgroups
+    assert short_k(lib, 1, 40, 128) and short_k(lib, 1, 127, 96)
+    assert not short_k(lib, 32, 1, 32) and not short_k(lib, 1, 15, 96) and short_k(lib, 33, 1, 32) and short_k(lib, 32, 8, 32)
+
+
+def test_runs_of_tiles_that_change_column_stay_on_256_row_tiles(lib):
+    for M in (129, 160, 192):
+        for N in (21888, 28672, 32768):
+            assert not short_k(lib, M, N, 128) and short_k(lib, M, N, 128, 2) and short_k(lib, M, N, 96)
+        assert short_k(lib, M, 21760, 128) and short_k(lib, M, 32896, 128) and short_k(lib, M, 28680, 128)
+    assert short_k(lib, 128, 28672, 128) and short_k(lib, 193, 28672, 128)
