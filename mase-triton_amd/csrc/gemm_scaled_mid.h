@@ -209,6 +209,9 @@ struct ScaledMidPlan {
 // (256 x 256) with few CUs busy and 1.2 with all, 0.62 (128 x 128) either way, 0.37 and 0.46 (128 x 64); the 256 x 256 kernel walks
 // its tiles as one stream (8 us once), the others pay 2.5 us per round and 2 once.  Where prices are close so are the
 // kernels: 384 x 14336 x 4096 takes 43.4 us on 256 x 256 tiles and 44.0 on 128 x 128 ones, 2048 x 4096 x 4096 41 and 45.
+// One row of the smaller tiles (up to 128 rows of A) shares nothing of W: a second round adds a wait, up to 1.4 us when it is full (128 x
+// 65536, K = 512 / 1024 / 2048: 14.6 / 19.5 / 29.3 us on 128 x 128 tiles, 12.8 / 17.7 / 27.2 on one round of 256 x 256 ones, fp32 out 18.0 / 23.4 / 33.1
+// and 14.3 / 19.5 / 28.6; K = 4096 53 and 55).
 inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
     const int nmac = K / SMAC;
     ScaledMidPlan best{256, 1, nmac};
@@ -226,7 +229,8 @@ inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
             const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
             const double step = bn == 256 ? 1.0 + 0.2 * busy : bn == 128 ? 0.62 : 0.37 + 0.09 * busy;
             const double rounds = (double)((wgs + cus - 1) / cus);
-            const double t = rounds * (per * step + (bn == 256 ? 0.0 : 2.5)) + (bn == 256 ? 8.0 : 2.0) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
+            const double unshared = bn != 256 && M <= 128 && wgs > cus ? 1.4 * std::min(1.0, (double)(wgs - cus) / cus) : 0.0;
+            const double t = rounds * (per * step + (bn == 256 ? 0.0 : 2.5)) + (bn == 256 ? 8.0 : 2.0 + unshared) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
             if (t < best_t) { best_t = t; best = ScaledMidPlan{bn, want, per}; }
         }
     }

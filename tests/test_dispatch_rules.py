@@ -81,3 +81,35 @@ def test_runs_of_tiles_that_change_column_stay_on_256_row_tiles(lib):
             assert not short_k(lib, M, N, 128) and short_k(lib, M, N, 128, 2) and short_k(lib, M, N, 96)
         assert short_k(lib, M, 21760, 128) and short_k(lib, M, 32896, 128) and short_k(lib, M, 28680, 128)
     assert short_k(lib, 128, 28672, 128) and short_k(lib, 193, 28672, 128)
+
+
+def scaled_plan(lib, M, N, K, may_split=True, cus=256):
+    lib.mase_bench_scaled_plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p]
+    plan = (ctypes.c_int * 3)()
+    assert lib.mase_bench_scaled_plan(M, N, K, cus, may_split, plan) == 0
+    return tuple(plan)
+
+
+def test_the_tile_plan_covers_k(lib):
+    """Every share of a K split has macro steps, the last as well; the 256 x 256 kernel's are equal and even; no more workgroups than CUs."""
+    for M in (65, 128, 200, 256, 300, 511, 1024, 3000, 16384):
+        for N in (8, 264, 1000, 1024, 4096, 4104, 14336, 65536):
+            for K in (512, 768, 1024, 2304, 4096, 4352, 14336, 14080):
+                for cus in (256, 304, 64):
+                    bn, splits, steps = scaled_plan(lib, M, N, K, True, cus)
+                    nmac = K // 128
+                    assert bn in (64, 128, 256) and 1 <= splits <= 16
+                    assert (splits - 1) * steps < nmac <= splits * steps
+                    assert splits == 1 or (steps >= 4 and splits * -(-M // (256 if bn == 256 else 128)) * -(-N // bn) <= cus)
+                    assert bn != 256 or (splits * steps == nmac and steps % 2 == 0)
+                    assert scaled_plan(lib, M, N, K, False, cus)[1:] == (1, nmac)
+
+
+def test_one_full_round_of_large_tiles_is_not_given_to_two_of_small_ones(lib):
+    for M in (65, 96, 128):
+        for K in (512, 1024, 2048):
+            assert scaled_plan(lib, M, 65536, K) == (256, 1, K // 128)
+    # one round of small tiles, a second that large ones would need as well, and several rows of tiles that share W
+    for shape, bn in (((65, 28672, 4096), 128), ((128, 28672, 1024), 128), ((128, 98304, 4096), 128), ((128, 152064, 4096), 128), ((384, 14336, 512), 128),
+                      ((200, 14336, 4096), 128), ((128, 14336, 4096), 64)):
+        assert scaled_plan(lib, *shape)[0] == bn
