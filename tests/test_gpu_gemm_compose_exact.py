@@ -89,3 +89,31 @@ def test_gemm_reproduces_the_compose_table(mh, w_tag, MNK, odt):
             show = [(int(r), int(c), int(scales[c]), hex(int(codes[(r + off) % K])), hex(int(bits_of(y).reshape(-1)[j])),
                      hex(int(want.reshape(-1)[j]))) for r, c, j in zip(rows, cols, i)]
             raise AssertionError(f"offset {off}: {bad.size} of {M * N} differ; first (m, n, scale, code, got, want): {show}")
+
+
+@pytest.mark.parametrize("w_tag", list(PRESETS))
+@pytest.mark.parametrize("MNK", [(128, 256, 128), (64, 264, 64), (100, 257, 96), (32, 256, 32)])
+@pytest.mark.parametrize("odt", [torch.bfloat16, torch.float32])
+def test_short_contractions_reproduce_the_compose_table(mh, w_tag, MNK, odt):
+    """The same for the kernel of K <= 128, whose rows hold fewer columns than FP8 has codes: the rows' codes start at every
+    multiple of K in turn.  (257 columns: element-wise stores, bf16 rows of odd length.)"""
+    M, N, K = MNK
+    e, m = PRESETS[w_tag]
+    n_codes = 1 << (1 + e + m)
+    table = golden("mxfp_compose_table.npz")[f"bfloat16_{w_tag}"]
+    scales = (np.arange(N) * 37 % 256).astype(np.int64)
+    name = "float32" if odt == torch.float32 else "bfloat16"
+    w_sc = torch.from_numpy(np.repeat(scales.astype(np.uint8)[:, None], K // 32, axis=1).copy()).to(DEV)
+    for code0 in range(0, n_codes, K):
+        codes = ((code0 + np.arange(K)) % n_codes).astype(np.int64)
+        w_el = torch.from_numpy(np.repeat(codes.astype(np.uint8)[None, :], N, axis=0).copy()).to(DEV)
+        for off in range(0, K, M):
+            a = torch.zeros(M, K, dtype=torch.bfloat16)
+            a[torch.arange(M), (torch.arange(M) + off) % K] = 1.0
+            y = mh.mxk.mxfp_gemm(a.to(DEV), None, None, None, w_sc, w_el, getattr(mh.meta, w_tag), None, M, N, K, odt)
+            torch.cuda.synchronize()
+            want = expected_bits(table, "bfloat16", scales, codes, M, K, off)
+            if odt == torch.float32:
+                want = want.astype(np.uint32) << 16
+            bad = mismatches(bits_of(y), want, name)
+            assert bad.size == 0, (code0, off, [(int(i // N), int(i % N)) for i in bad[:8]])

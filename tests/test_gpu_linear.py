@@ -287,13 +287,15 @@ def test_gemm_few_rows_special_values(mh, M):
 
 
 @pytest.mark.parametrize("MNK,w_tag,odt,with_bias", [
-    ((129, 128, 128), "MXFP8_E4M3_fn", torch.bfloat16, False),     # two m-tiles (the second holds one row), one macro step
+    ((129, 128, 128), "MXFP8_E4M3_fn", torch.bfloat16, True),      # two m-tiles (the second holds one row), one macro step
+    ((129, 128, 128), "MXFP8_E4M3_fn", torch.bfloat16, False),     # (without a bias K <= 128 is the kernel for short contractions)
     ((256, 256, 256), "OCP_MXFP4_E2M1", torch.float32, True),      # two macro steps: prologue only, fp32 output
     ((200, 384, 896), "OCP_MXFP6_E3M2", torch.bfloat16, True),     # 7 macro steps: the 6-step unrolled loop wraps, ragged M
     ((511, 1024, 1664), "MXFP8_E5M2_fn", torch.float16, False),    # four m-tiles, 13 macro steps, generic decode of E5M2
     ((384, 2048, 2048), "OCP_MXFP6_E2M3", torch.bfloat16, False),  # 48 tiles, K rotation wraps (16 n-tiles = 16 macro steps)
     ((300, 4352, 512), "MXFP8_E4M3_fn", torch.bfloat16, True),     # 34 n-tiles, more than the 4 macro steps: rotation modulo
-    ((257, 128, 64), "MXFP8_E4M3_fn", torch.bfloat16, False),      # 256 x 128 tiles: two m-tiles (one row in the second), one step
+    ((257, 128, 64), "MXFP8_E4M3_fn", torch.bfloat16, True),       # 256 x 128 tiles: two m-tiles (one row in the second), one step
+    ((257, 128, 64), "MXFP8_E4M3_fn", torch.bfloat16, False),      # (short contractions)
     ((512, 256, 320), "OCP_MXFP6_E3M2", torch.float32, True),      # 5 steps of 64 k (K not a multiple of 128), fp32 output
     ((400, 640, 832), "OCP_MXFP4_E2M1", torch.float16, True),      # 13 steps: the 6-step unrolled loop wraps twice
     ((250, 1024, 1152), "MXFP8_E5M2_fn", torch.bfloat16, True),    # 128 x 128 tiles, 9 macro steps
@@ -851,8 +853,12 @@ def test_mxfp_matmul(mh, func_type, backend):
 
 @pytest.mark.parametrize("a_shape,b_shape,dtype", [
     ((3, 40, 256), (256, 192), torch.bfloat16),          # matrix `other`: one GEMM over all rows
-    ((2, 600, 128), (2, 128, 320), torch.bfloat16),      # batched launch, 256 x 256 tiles (N not a multiple of 128)
-    ((40, 16, 64), (40, 64, 96), torch.bfloat16),        # many batches, few rows each (16-row weight-streaming kernel)
+    ((2, 600, 128), (2, 128, 320), torch.bfloat16),      # batched launch of the kernel for short contractions
+    ((2, 600, 160), (2, 160, 320), torch.bfloat16),      # batched launch, small tiles (K and N not multiples of 128)
+    ((2, 3000, 160), (2, 160, 3008), torch.bfloat16),    # batched launch, 256 x 256 tiles (the same with enough of them)
+    ((40, 16, 64), (40, 64, 96), torch.bfloat16),        # many batches, few rows each, short contraction
+    ((40, 16, 256), (40, 256, 96), torch.bfloat16),      # many batches, few rows each (16-row weight-streaming kernel)
+    ((12, 40, 256), (12, 256, 8224), torch.bfloat16),    # 32-row weight-streaming kernel, batched
     ((2, 4, 24, 96), (4, 96, 64), torch.bfloat16),       # `other` broadcast along the first batch axis (its components are expanded)
     ((3, 1, 24, 96), (1, 5, 96, 64), torch.bfloat16),    # both operands broadcast along one axis each
     ((24, 96), (5, 96, 64), torch.bfloat16),             # matrix `input` against batched `other`: A shared (stride 0)
@@ -919,6 +925,7 @@ def test_gemm_batched_entry_point(mh):
     g = torch.Generator(device=DEV).manual_seed(21)
     for (B, M, N, K), a_shared, w_shared, pad in (((8, 128, 512, 1024), False, False, 0), ((5, 16, 256, 256), True, False, 0),
                                                   ((3, 300, 256, 128), False, True, 0), ((4, 640, 1536, 256), False, False, 64),
+                                                  ((3, 300, 256, 256), False, True, 0), ((20, 1, 32, 256), False, False, 32),
                                                   ((20, 1, 32, 32), False, False, 0), ((3, 70, 96, 160), False, False, 32)):
         a_stride = 0 if a_shared else M * K + pad
         w_stride = 0 if w_shared else N * K + pad

@@ -13,6 +13,7 @@ What is checked, against the CPU checker's components of the same inputs:
   * inf / NaN blocks poison exactly the rows (columns) they poison in dequantise-then-matmul;
   * the operand formed from silu(gate) * up inside the kernel equals the one built from torch's two bf16 operations.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -255,7 +256,8 @@ def test_scaled_gemm_vs_checker(mh, MNK, x_tag, w_tag):
 def test_scaled_gemm_many_tiles(mh, MNK):
     """More 256 x 256 tiles than the GPU has compute units, in grids that the workgroups' walk order (patches of 4 x 8
     tiles per group of 32 workgroups) does not divide: every workgroup walks several tiles as one stream and the last
-    patches are partial.  Every output element against the checker's product."""
+    patches are partial (9000 x 520 takes 128 x 128 tiles, more of them than CUs).  Every output element against the
+    checker's product."""
     M, N, K = MNK
     g = torch.Generator().manual_seed(M ^ N)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16)
@@ -308,8 +310,8 @@ def test_scaled_gemm_few_rows(mh, MNK, x_tag, w_tag):
 
 
 def test_scaled_gemm_random_shapes(mh):
-    """A seeded sweep over shapes on every route of the entry point (decode-sized kernel, lone tiles, K split, several
-    tiles per workgroup): M 1 .. 700, N a multiple of 8 up to 1040, K a multiple of 256 up to 3072, format pairs in turn;
+    """A seeded sweep over the weight-streaming kernels and the 128 x 64 tiles, K split and not (what these sizes take; the
+    other tiles have tests of their own below): M 1 .. 700, N a multiple of 8 up to 1040, K a multiple of 256 up to 3072, format pairs in turn;
     every element of the fp32 result against a float64 product of the checker's dequantised operands."""
     import random
 
@@ -410,7 +412,7 @@ def test_special_blocks_poison_the_same_outputs(mh):
 @pytest.mark.parametrize("MNK", [(256, 256, 4096), (300, 520, 2048), (1024, 512, 14336), (700, 264, 7168)])
 def test_scaled_gemm_k_split(mh, MNK):
     """Few tiles and a long K: the launcher splits K over several workgroups per tile (fp32 partial sums in a workspace,
-    a second kernel adds them).  Against the checker and against the unsplit call (which it may equal bit for bit: products
+    a second kernel adds them), on 128 x 64 and 128 x 128 tiles here.  Against the checker and against the unsplit call (which it may equal bit for bit: products
     of two MXFP values have at most eight significant bits, and sums of a few thousand of them are often exact in fp32
     whatever the order)."""
     from mase_hip import _lib
@@ -439,9 +441,9 @@ def test_scaled_gemm_k_split(mh, MNK):
 @pytest.mark.parametrize("MNK", [(65, 8, 512), (128, 64, 768), (129, 72, 2304), (200, 136, 3840), (257, 520, 7168), (70, 4104, 1024),
                                  (130, 1032, 4352), (640, 4096, 4096), (200, 14336, 512)])
 def test_scaled_gemm_128_row_tiles(mh, MNK):
-    """The 128 x 128 and 128 x 64 tile kernels around the edges of their tiles (rows, columns), with fewer macro steps than the DMA
-    ring has stages and counts that it does not divide, K split into equal and unequal shares and not split, bias and every output
-    type: every element of the fp32 result against a float64 product of the checker's dequantised operands."""
+    """The 128 x 64 tile kernel around the edges of its tiles (rows, columns), with fewer macro steps than the DMA ring has stages
+    and counts that it does not divide, K split into equal and unequal shares and not split, and the 128 x 128 kernel on whole
+    columns (its edges: test_scaled_gemm_on_the_tile_it_names); bias and every output type: every element of the fp32 result against a float64 product of the checker's dequantised operands."""
     M, N, K = MNK
     g = torch.Generator().manual_seed(M * 3 + N + K)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16)
@@ -459,6 +461,59 @@ def test_scaled_gemm_128_row_tiles(mh, MNK):
         y_b = y_ref + b.double()
         for odt in (torch.bfloat16, torch.float16):
             assert rel_fro(mh.mxk.mxfp_gemm_scaled(a, wop, b.to(DEV), odt, split_k=split_k), y_b.to(odt)) <= 1e-3
+
+
+def tile_plan(M, N, K, may_split, cus=256):
+    """(columns of a tile, workgroups per tile, 128-k macro steps of each) that the launcher picks on a device with `cus` CUs."""
+    lib = ctypes.CDLL(os.path.join(ROOT, "mase-triton_amd", "mase_hip", "lib", "libmase_bench.so"))
+    lib.mase_bench_scaled_plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p]
+    plan = (ctypes.c_int * 3)()
+    assert lib.mase_bench_scaled_plan(M, N, K, cus, may_split, plan) == 0
+    return tuple(plan)
+
+
+@pytest.mark.parametrize("MNK,split_k,plan", [
+    # 256 x 256, K split
+    ((300, 4096, 14336), True, (256, 8, 14)),      # the second tile row holds 44 rows
+    ((136, 8768, 5120), True, (256, 5, 8)),        # one tile row, the last tile holds 64 columns
+    ((136, 8200, 6912), True, (256, 3, 18)),       # 8 columns in the last tile
+    ((1100, 4096, 4096), True, (256, 2, 16)),
+    # 256 x 256, not split
+    ((65, 33000, 1024), True, (256, 1, 8)),        # a quarter of the tile's rows, 232 columns in the last
+    ((129, 16392, 768), True, (256, 1, 6)),
+    ((777, 4872, 768), False, (256, 1, 6)),
+    # 128 x 128: ragged columns, steps per share that the ring of four does not divide, a shorter last share
+    ((331, 1648, 14080), True, (128, 6, 19)),      # 110 steps: 5 x 19 + 15
+    ((384, 4856, 12288), True, (128, 2, 48)),
+    ((3080, 1200, 3328), True, (128, 1, 26)),
+    ((136, 8768, 5120), False, (128, 1, 40)),
+])
+def test_scaled_gemm_on_the_tile_it_names(mh, MNK, split_k, plan):
+    """Tiles and K splits that the smaller shapes above do not reach, each named: a refit of the launcher's prices that moves a shape
+    to another kernel fails here.  Bias and every output type; every element of the fp32 result against a float64 product of the
+    checker's dequantised operands."""
+    M, N, K = MNK
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if cus != 256:
+        pytest.skip(f"the plans are those of 256 CUs, this device has {cus}")
+    assert tile_plan(M, N, K, split_k) == plan
+    g = torch.Generator().manual_seed(M * 3 + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (0.02 * torch.randn(N, K, generator=g)).to(torch.bfloat16)
+    b = torch.randn(N, generator=g).to(torch.bfloat16)
+    _, _, x_dq = quantised(x, "MXFP8_E4M3_fn")
+    w_sc, w_el, w_dq = quantised(w, "OCP_MXFP6_E3M2")
+    y_ref = x_dq.double() @ w_dq.double().t()
+    a = mh.mxk.scaled_operand_from_dense(x.to(DEV), mh.meta.MXFP8_E4M3_fn)
+    wop = mh.mxk.scaled_operand_from_mxfp(w_sc.to(DEV), w_el.to(DEV), mh.meta.OCP_MXFP6_E3M2, N, K)
+    for bias in (None, b):
+        want = y_ref if bias is None else y_ref + b.double()
+        bd = None if bias is None else b.to(DEV)
+        y32 = mh.mxk.mxfp_gemm_scaled(a, wop, bd, torch.float32, split_k=split_k)
+        assert rel_fro(y32, want) <= F32_TOL
+        assert float((y32.cpu().double() - want).abs().max()) <= 1e-3 * float(want.abs().max())
+        for odt in (torch.bfloat16, torch.float16):
+            assert rel_fro(mh.mxk.mxfp_gemm_scaled(a, wop, bd, odt, split_k=split_k), want.to(odt)) <= 1e-3
 
 
 # ---------------------------------------------------------------- the prepared weight on the bf16 kernel
