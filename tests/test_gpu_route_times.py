@@ -64,15 +64,15 @@ def _product(M, N, K, batches=1):
 
 @pytest.mark.parametrize("M,N", [(1, 4096), (16, 14336), (32, 4096), (64, 1024), (64, 8192)])
 def test_short_contraction_of_few_rows(M, N):
-    """Without a bias the product may not take longer than with one, which always runs on the weight-streaming kernels here (2.9 - 6 us
-    against up to 6.5 on the kernel for short contractions)."""
+    """Without a bias the product may not take longer than with one, which always runs on the weight-streaming kernels here (0.83 - 0.92 of
+    its time, 1.1 - 1.9 times as long on the kernel for short contractions)."""
     import mase_hip.mxfp.kernels as mxk
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
 
     a, sc, el = _product(M, N, 128)
     bias = torch.randn(N, device=DEV).to(torch.bfloat16)
     t, t_bias = (gpu_us(lambda b=b: mxk.mxfp_gemm(a, None, None, None, sc, el, fmt, b, M, N, 128, torch.bfloat16)) for b in (None, bias))
-    assert t <= 1.2 * t_bias, (t, t_bias)
+    assert t <= 1.05 * t_bias, (t, t_bias)
 
 
 @pytest.mark.parametrize("M,N,odt", [(1024, 14336, torch.bfloat16), (512, 28672, torch.bfloat16), (3000, 4096, torch.bfloat16), (16384, 4096, torch.float32)])
@@ -90,7 +90,7 @@ def test_short_contraction_of_a_full_round_of_large_tiles(M, N, odt):
 
 def test_attention_scores_of_one_query():
     """One query per head against 2048 keys of 8 heads: 4.8 us on the weight-streaming kernel, 6.4 on the kernel for short contractions.
-    Held to the time of one product with as many rows of W and a bias."""
+    Held to the time of one product with as many rows of W and a bias (0.82 of it, 1.1 times)."""
     import mase_hip.mxfp.kernels as mxk
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
 
@@ -99,31 +99,32 @@ def test_attention_scores_of_one_query():
     bias = torch.randn(B * N, device=DEV).to(torch.bfloat16)
     t = gpu_us(lambda: mxk.mxfp_gemm_batched(a.view(-1), sc, el, fmt, B, M, N, K, torch.bfloat16, M * K, N * K))
     t_one = gpu_us(lambda: mxk.mxfp_gemm(a[:1], None, None, None, sc, el, fmt, bias, 1, B * N, K, torch.bfloat16))
-    assert t <= 1.2 * t_one, (t, t_one)
+    assert t <= t_one, (t, t_one)
 
 
-@pytest.mark.parametrize("M,N,aligned", [(1, 5001, 5000), (4, 20001, 20008)])
-def test_short_contraction_of_few_rows_and_an_odd_number_of_columns(M, N, aligned):
-    """Rows of y at no alignment leave element by element; only those there are (7.1 and 7.4 us when all 32 rows of a tile were stepped
-    through, 6.2 with whole 16-byte stores).  Held to a multiple of 8 columns (not of 16: that is another kernel)."""
+@pytest.mark.parametrize("N,aligned", [(1001, 1000), (10010, 10008)])
+def test_short_contraction_of_one_row_and_an_odd_number_of_columns(N, aligned):
+    """Rows of y at no alignment leave element by element; only those there are (4.6 us when all 32 rows of a tile were stepped through,
+    3.8 as with whole 16-byte stores).  Held to a multiple of 8 columns."""
     import mase_hip.mxfp.kernels as mxk
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
 
     t = []
     for n in (N, aligned):
-        a, sc, el = _product(M, n, 128)
-        t.append(gpu_us(lambda: mxk.mxfp_gemm(a, None, None, None, sc, el, fmt, None, M, n, 128, torch.bfloat16)))
+        a, sc, el = _product(1, n, 64)
+        t.append(gpu_us(lambda: mxk.mxfp_gemm(a, None, None, None, sc, el, fmt, None, 1, n, 64, torch.bfloat16)))
     assert t[0] <= 1.1 * t[1], t
 
 
-@pytest.mark.parametrize("M,N", [(1, 20008), (129, 28672), (192, 24576)])
-def test_short_contractions_between_the_tile_sizes(M, N):
+@pytest.mark.parametrize("M,N,most", [(1, 20008, 1.03), (129, 28672, 0.9), (192, 24576, 0.85)])
+def test_short_contractions_between_the_tile_sizes(M, N, most):
     """One row of a number of columns that the weight-streaming kernels do not take, and rows whose tiles leave runs that change column:
-    held to the same product with a bias, on the kernels for long contractions (5.7, 8.6 and 9.1 us; 6.4, 12.6 and 12.6 on the other)."""
+    held to the same product with a bias, on the kernels for long contractions (5.7, 8.8 and 9.2 us against 6.0, 11.5 and 12.7 with the
+    bias; 6.6, 12.7 and 12.5 on the other)."""
     import mase_hip.mxfp.kernels as mxk
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
 
     a, sc, el = _product(M, N, 128)
     bias = torch.randn(N, device=DEV).to(torch.bfloat16)
     t, t_bias = (gpu_us(lambda b=b: mxk.mxfp_gemm(a, None, None, None, sc, el, fmt, b, M, N, 128, torch.bfloat16)) for b in (None, bias))
-    assert t <= 1.07 * t_bias, (t, t_bias)
+    assert t <= most * t_bias, (t, t_bias)
