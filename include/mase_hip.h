@@ -284,7 +284,7 @@ int mase_hip_mxfp_gemm_static_ws(const void* a_dense, int a_dtype, const uint8_t
  * K % 256 == 0 and K >= 512; N a multiple of 8 (4 for fp32 output); codes and y 16-byte aligned.  Other shapes: -2,
  * use mase_hip_mxfp_gemm.  Up to 64 rows of A take weight-streaming kernels (the product is a read of W; 17 - 64 rows
  * against a K beyond 4096 only through mase_hip_mxfp_gemm_scaled_ws, which brings the room for their K slices' sums),
- * more rows 256 x 256 tiles.
+ * more rows tiles of 256 x 256, 128 x 128 or 128 x 64, whichever is estimated fastest.
  * Replaces, like mase_hip_mxfp_gemm, the unimplemented backend="fused" of mxfp_linear_XqWq
  *   src/mase_triton/mxfp/functional/linear.py:36-64
  * (extract of x :50-52, the two composes :53-54 and the linear :61 in one prepare call and one GEMM).
@@ -324,10 +324,10 @@ int mase_hip_mxfp_gemm_scaled(const uint8_t* a_codes, const uint32_t* a_scales, 
                               const uint32_t* w_scales, const void* bias, int bias_dtype, void* y,
                               int out_dtype, int64_t M, int64_t N, int64_t K, void* stream);
 /*
- * The same with room for partial sums, as mase_hip_mxfp_gemm_ws: a product with few 256 x 256 tiles and a long K, or with
- * 17 - 64 rows of A and a K beyond 4096, is split over K into fp32 partial sums in `workspace` (mase_hip_mxfp_gemm_scaled_workspace_bytes(M, N, K) bytes, 0 when
- * the shape is not split; 16-byte aligned; NULL or too small: no split), and a second kernel adds them, the bias, and
- * rounds.  Same reference counterpart as mase_hip_mxfp_gemm_scaled.
+ * The same with room for partial sums, as mase_hip_mxfp_gemm_ws: a product with few tiles (of any of the three sizes) for a
+ * long K, or with 17 - 64 rows of A and a K beyond 4096, is split over K into fp32 partial sums in `workspace`
+ * (mase_hip_mxfp_gemm_scaled_workspace_bytes(M, N, K) bytes, up to 16 M * N * 4; 0 when the shape is not split; 16-byte aligned; NULL
+ * or too small: no split, and then perhaps another tile), and a second kernel adds them, the bias, and rounds.  Same reference counterpart as mase_hip_mxfp_gemm_scaled.
  */
 int64_t mase_hip_mxfp_gemm_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mase_hip_mxfp_gemm_scaled_ws(const uint8_t* a_codes, const uint32_t* a_scales, const uint8_t* w_codes,

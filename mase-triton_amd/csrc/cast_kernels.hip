@@ -1145,7 +1145,8 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_bf16_lines_kernel(const
 // better alignment.  Needs 16-byte aligned elements.
 // 2976 x 4096, repeated on one input: fp16 (37 MB to move) 26.5 -> 14.2 us, fp32 (61 MB) 18.4 -> 14.8, bf16 with an odd row length 17.1 ->
 // 14.5, against mxfp_strided_kernel, which stores a column's 32 codes by itself, with the general encoder: half of that gain is the
-// encoder's, and vector instructions (about 25 per element) still take as long as the memory.  At 64 x 1000: 11.6 / 6.7 -> 3.9 us.
+// encoder's, and vector instructions (about 25 per element) still take as long as the memory.  With another input and output on
+// every call: fp16 15.7, fp32 19.1 us.  At 64 x 1000: 11.6 / 6.7 -> 3.9 us.
 template <int DT_IN, class F>
 __global__ __launch_bounds__(kThreads) void mxfp_strided_tile_kernel(const void* __restrict__ x, uint8_t* __restrict__ scales,
                                                                       uint8_t* __restrict__ elements, int64_t K, int64_t inner,

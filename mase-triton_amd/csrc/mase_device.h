@@ -1,9 +1,8 @@
 // Device-side arithmetic shared by the cast kernels and the GEMM: minifloat encode/decode and
 // the MXFP shared-exponent rules, bit-exact with the PyTorch "fake" path of the reference
-// (src/mase_triton/minifloat/fake.py, src/mase_triton/mxfp/fake.py), written as integer
-// operations on IEEE bit patterns so that the result does not depend on the GPU's denormal
-// or rounding mode (the two float multiplies in decode rely on IEEE denormal handling, which
-// is the HIP default on gfx950).
+// (src/mase_triton/minifloat/fake.py, src/mase_triton/mxfp/fake.py).  Encoding is integer operations on IEEE fp32 bit
+// patterns and depends on no mode.  What relies on the modes that HIP sets on gfx950 (fp16 and fp32 subnormals kept, round to
+// nearest even): the converts of fp16 inputs and outputs, which are the hardware's, and the float multiplies of decode.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

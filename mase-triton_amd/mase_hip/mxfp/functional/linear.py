@@ -38,11 +38,12 @@ _GEMM_DTYPES = (torch.bfloat16, torch.float32)
 _BACKENDS = ("separate", "fused", "fused_bf16", "fused_scaled")
 # Which row counts of x backend="fused" sends to the block-scaled kernels.  With the weight operand at hand (a layer keeps
 # it): all of them.  Up to 64 rows the product is a read of W, which the block-scaled weight-streaming kernels do without
-# touching the codes (N x K = 14336 x 4096: 15 / 15.6 / 19.2 us at 16 / 32 / 64 rows against 21 / 23 / 31 us on the bf16
-# kernels; 4096 x 14336: 17.7 / 18.4 / 23.0 against 25.8 / 27.8 / 49.4); beyond, its 256 x 256 tiles, K split over workgroups where
-# they are few, stay ahead (14336 x 4096: 33 / 44 / 45 us at 128 / 256 / 512 rows against 37 / 49 / 73).  When the operand has to
-# be built inside the call (N * K bytes read and written, 25 us at that size) it pays from about 512 rows (71 against 73 us;
-# 72 against 104 at 768).
+# touching the codes; beyond, 128- and 256-row tiles, K split over workgroups where they are few, stay ahead.  GEMMs alone, another W
+# on every call, block-scaled against bf16 kernels, us, at 16 / 32 / 64 / 128 / 256 / 512 / 1024 rows: N x K = 14336 x 4096 15 / 17 / 20 / 22 / 27 /
+# 46 / 50 against 23 / 25 / 31 / 35 / 43 / 72 / 105; 4096 x 14336 19 / 19 / 23 / 25 / 31 / 45 / 66 against 26 / 29 / 50 / 35 / 47 / 77 / 110.
+# When the operand has to be built inside the call (N * K bytes read and written) the whole call takes 50 / 55 / 68 / 72 / 79 us
+# against 39 / 48 / 69 / 78 / 117 on the bf16 kernels at 128 / 256 / 300 / 512 / 1024 rows of 14336 x 4096, and 54 / 60 / 70 / 77 / 102 against 40 / 53 / 77 / 90 / 128
+# of 4096 x 14336: it pays from about 300 rows on.  The line lies at 512, where it paid before there were tiles of 128 rows.
 SCALED_FROM_ROWS_UNPREPARED = 512
 
 
