@@ -14,9 +14,10 @@
 // into each other's way in L2: 33 against 60 us at 1001 rows of the shape below, 56 against 67 at 2048 x 2048.)
 // Any M and N, K a multiple of 32 (short_k_shape_ok in gemm_impl.h says which it is for).  64 products of 1000 x 1000 x 128 (E4M3, bf16
 // out, 152 MB to read and write), repeated on the same buffers: 32 us, 4.7 TB/s (a plain copy of that many bytes reaches 5.2); with other
-// operands and outputs on every call, as in a model, 52 us.  At 1024 x 1024 that is 28 and 30 us (992: 49, 1008: 51): a row that is
-// not whole lines ends and starts in the middle of one, and the halves, written by different workgroups, meet in the caches only while
-// these hold that part of y.  32 products of 2048 x 2048 x 128: 49 and 52 us, 5.6 TB/s.  The kernels that took such shapes before (the
+// operands and outputs on every call, as in a model, 52 us.  At 1024 x 1024 that is 28 and 30 us (992: 49, 1008: 51): rows of whole
+// lines are stored past the caches, others fill these with y, and operands that have to come from memory wait behind its
+// write-back (fresh outputs alone, the operands at hand: 33 us; what reaches memory is y in 64-byte requests in both cases).  32
+// products of 2048 x 2048 x 128: 49 and 52 us, 5.6 TB/s.  The kernels that took such shapes before (the
 // 128 x 128 x 32 single-buffer one, the 512 x 128 one with products as grid planes) take 98, 128 and 259 us on fresh buffers.
 #pragma once
 #include "gemm_impl.h"
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
     // whole 16-byte runs: every row piece starts and ends on a 16-byte boundary
     const bool vec = (N * ESZ) % 16 == 0 && (reinterpret_cast<uintptr_t>(y_all) & 15) == 0 && (gb.y & 15) == 0;
     // rows of whole 128-byte lines go past the caches (the outputs are not read here); others leave half-filled lines, which
-    // the L2 puts together with the neighbours' halves if they come while it holds them
+    // the L2 puts together with the neighbours' halves
     const bool lines = vec && (N * ESZ) % 128 == 0 && (reinterpret_cast<uintptr_t>(y_all) & 127) == 0 && (gb.y & 127) == 0;
 
     bf16x8 wf[2][Q];                                       // W, composed: rows n0 + 32 j + lane % 32, k 16 q + 8 (lane / 32) ..

@@ -491,7 +491,7 @@ def tile_plan(M, N, K, may_split, cus=256):
 def test_scaled_gemm_on_the_tile_it_names(mh, MNK, split_k, plan):
     """Tiles and K splits that the smaller shapes above do not reach, each named: a refit of the launcher's prices that moves a shape
     to another kernel fails here.  Bias and every output type; every element of the fp32 result against a float64 product of the
-    checker's dequantised operands."""
+    oracle's dequantised operands."""
     M, N, K = MNK
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     if cus != 256:

@@ -147,7 +147,7 @@ def test_transposed_right_operand_is_quantised_where_it_lies(shape):
 
 def test_transposed_right_operand_on_the_block_scaled_route():
     """The same where the product takes the block-scaled GEMM (one matrix, 512 rows or more, K a multiple of 256): both layouts of the
-    right operand, with and without unit batch axes, bit for bit, and against the checker's quantisation."""
+    right operand, with and without unit batch axes, bit for bit, and against the oracle's quantisation."""
     import mase_hip.mxfp.functional as F
     import mase_hip.mxfp.kernels as mxk
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn as fmt
