@@ -116,7 +116,7 @@ def test_short_contraction_of_one_row_and_an_odd_number_of_columns(N, aligned):
     assert t[0] <= 1.1 * t[1], t
 
 
-@pytest.mark.parametrize("M,N,most", [(1, 20008, 1.03), (129, 28672, 0.9), (192, 24576, 0.85)])
+@pytest.mark.parametrize("M,N,most", [(1, 20008, 1.05), (129, 28672, 0.9), (192, 24576, 0.85)])
 def test_short_contractions_between_the_tile_sizes(M, N, most):
     """One row of a number of columns that the weight-streaming kernels do not take, and rows whose tiles leave runs that change column:
     held to the same product with a bias, on the kernels for long contractions (5.7, 8.8 and 9.2 us against 6.0, 11.5 and 12.7 with the
