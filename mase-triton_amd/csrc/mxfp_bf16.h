@@ -1,0 +1,244 @@
+// MXFP arithmetic on bfloat16 values, two to a register: blocks of 32 quantised to codes or back to bfloat16, and the re-encoding
+// of codes for the block-scaled matrix instruction.  Shared by the casts (cast_kernels.hip) and the GEMM kernels that quantise an
+// operand on its way in.
+#pragma once
+#include "mase_device.h"
+
+namespace mase {
+
+constexpr int kThreads = 256;   // workgroup of the kernels that use the code tables below
+
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ inline uint32_t pack_bf16(float a, float b) {
+    const bf16x2 r = __builtin_convertvector(floatx2{a, b}, bf16x2);
+    return __builtin_bit_cast(uint32_t, r);
+}
+
+template <class F>
+__device__ inline float mxfp_value(uint32_t code, float scale, const F& f) {
+    return decode_f32(code, f) * scale;
+}
+
+// ------------------------------------------------------------------------------ bf16 fast path
+// bfloat16 input, block size 32, compile-time format.  A lane owns 8 consecutive elements (one
+// 128-bit load), four adjacent lanes own a block.  Two elements are processed per 32-bit
+// register with packed 16-bit integer instructions; there is no per-element branch.
+//
+// With h the bf16 bits, a = h & 0x7FFF and scale the block's biased shared exponent, the value
+//     t = a - ((scale - bias) << 7)        (signed, clamped at 0)
+// is  (ye << 7) | f7 : the element's exponent field in the target format above its 7 mantissa
+// bits.  Rounding to M bits, the reference's "(ye << M) | yf" with its lost carry, the one
+// reachable subnormal binade (ye == 0) and underflow (t < 0) are all functions of t alone.
+// Not covered, and sent to the exact per-element routine by a wave-uniform test: blocks holding
+// inf/NaN, and scales >= 151 (only there can a quotient underflow to exactly zero).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+
+__device__ inline uint32_t as_u32(u16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ inline uint32_t as_u32(i16x2 v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ inline u16x2 as_u16x2(uint32_t v) { return __builtin_bit_cast(u16x2, v); }
+__device__ inline i16x2 as_i16x2(uint32_t v) { return __builtin_bit_cast(i16x2, v); }
+
+template <class F>
+struct PackedBf16 {
+    static constexpr int E = F{}.E(), M = F{}.M(), SH = 7 - M;
+    static constexpr uint32_t LSB = 0x00010001u;
+    // code magnitudes (exponent and mantissa fields, no sign) of two elements, one per 16-bit half,
+    // plus, through `t_q`, the quantised magnitude back in the t domain for the fused QDQ
+    // Packed 16-bit operations written as asm: given the plain expressions the compiler replaces each of them by one
+    // compare and one conditional move per 16-bit half plus a byte permute to put the halves together again.
+    __device__ static inline uint32_t pk_min_u16(uint32_t a, uint32_t b) {
+        uint32_t d;
+        asm("v_pk_min_u16 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+        return d;
+    }
+    // all ones in the halves where a < b (as signed 16-bit numbers whose difference fits 16 bits)
+    __device__ static inline uint32_t pk_less_mask(uint32_t a, uint32_t b) {
+        uint32_t d;
+        asm("v_pk_sub_i16 %0, %1, %2\n\tv_pk_ashrrev_i16 %0, 15, %0 op_sel_hi:[0,1]" : "=&v"(d) : "v"(a), "v"(b));
+        return d;
+    }
+    __device__ static inline uint32_t magnitude(uint32_t a, uint32_t ssb2, uint32_t& t_q) {
+        // t = a - ssb2 clamped at 0 (underflow -> 0); the caller guarantees ssb2 >= 0 in both halves
+        const uint32_t tu = as_u32(__builtin_elementwise_sub_sat(as_u16x2(a), as_u16x2(ssb2)));
+        const uint32_t u = as_u32(as_u16x2(tu) >> (unsigned short)SH);    // (ye << M) | truncated mantissa
+        const uint32_t r = tu + (((1u << (SH - 1)) - 1u) * LSB) + (u & LSB);  // round half to even
+        const uint32_t v = as_u32(as_u16x2(r) >> (unsigned short)SH);     // (ye << M) + rounded mantissa
+        // the reference ORs the exponent field with the rounded mantissa, so a carry out of the mantissa into an odd
+        // exponent field is lost
+        const uint32_t ef = u & (0xFFFFu & ~((1u << M) - 1u)) * LSB;
+        const uint32_t code_n = ef | (v - ef);
+        // ye == 0: the mantissa (with its carry) is shifted down under an explicit leading one; zero stays zero
+        const uint32_t m01 = pk_min_u16(v, LSB);
+        const uint32_t code_s = as_u32(as_u16x2((m01 << M) | v) >> (unsigned short)1);
+        // all ones where ye >= 1, i.e. u >= 2^M
+        const uint32_t is_norm = pk_less_mask(((1u << M) - 1u) * LSB, u);
+        // t-domain value of the code: normal codes keep their fields; subnormal code xf' (>= 2^(M-1))
+        // is 2^-bias * xf' / 2^(M-1), i.e. exponent field 0 and mantissa (xf' << (8 - M)) & 0x7F
+        const uint32_t tq_n = code_n << SH;
+        const uint32_t tq_s = (code_s << (8 - M)) & (0x7Fu * LSB);
+        t_q = (is_norm & tq_n) | (~is_norm & tq_s);
+        return (is_norm & code_n) | (~is_norm & code_s);
+    }
+    // all ones in the halves whose input has a non-zero exponent field (everything else is flushed
+    // to +0.0 by the reference before encoding and gets code 0, sign included)
+    __device__ static inline uint32_t live_mask(uint32_t a) { return as_u32(as_i16x2(a + 0x7F807F80u) >> (short)15); }
+    __device__ static inline uint32_t codes(uint32_t h, uint32_t ssb2) {
+        const uint32_t a = h & 0x7FFF7FFFu;
+        uint32_t t_q;
+        const uint32_t mag = magnitude(a, ssb2, t_q);
+        const uint32_t sgn = (h >> (15 - (E + M))) & ((1u << (E + M)) * LSB);
+        return (mag | sgn) & live_mask(a);
+    }
+    // quantise-dequantise of two bf16 values; valid when every non-zero code lands in the bf16
+    // normal range, i.e. scale > bias (smaller scales give subnormal results: slow path)
+    __device__ static inline uint32_t qdq(uint32_t h, uint32_t ssb2) {
+        const uint32_t a = h & 0x7FFF7FFFu;
+        uint32_t t_q;
+        const uint32_t mag = magnitude(a, ssb2, t_q);
+        const uint32_t nonzero = pk_less_mask(0u, mag);                    // code magnitudes are small positive numbers
+        const uint32_t body = (t_q + ssb2) & nonzero;                      // code 0 -> +-0.0
+        return (body | (h & 0x80008000u)) & live_mask(a);
+    }
+};
+
+// ------------------------------------------------------------------------------ operands of the block-scaled GEMM
+// The block-scaled matrix instruction takes FP8 (E4M3) bytes and one E8M0 scale per 32 of them.  It reads the code
+// S.1111.111 as NaN where the reference's finite E4M3 has +-480, so a block that holds that code is stored one scale
+// step up with every code halved: exact for codes of 16 and more (exponent field - 1) and for even codes below 16
+// (whose value is code * 2^-9 in units of the block scale); an odd code below 16 rounds half to even.  The narrower
+// element formats are embedded into E4M3 bytes with the same value and the same block scale (their subnormals are
+// E4M3 normals).  Scales go out transposed for the GEMM's DMA: dword [k / 128][row], byte (k / 32) % 4.
+__device__ inline uint32_t e4m3_top_bits(uint32_t w) { return ((w & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u; }
+__device__ inline uint32_t e4m3_halve4(uint32_t w) {
+    const uint32_t mag = w & 0x7F7F7F7Fu, sign = w & 0x80808080u;
+    const uint32_t big = (((mag + 0x70707070u) & 0x80808080u) >> 7) * 0xFFu;      // all ones in the bytes with mag >= 16
+    const uint32_t mag_n = ((mag | 0x80808080u) - 0x08080808u) & 0x7F7F7F7Fu;     // exponent field - 1 (the guard bit stops the borrow)
+    const uint32_t q = (mag >> 1) & 0x7F7F7F7Fu;
+    const uint32_t mag_s = q + (mag & q & 0x01010101u);                           // mag / 2, half to even
+    return sign | (big & mag_n) | (~big & mag_s);
+}
+// one code of format F as the E4M3 byte of the same value
+template <class F>
+__device__ inline uint32_t embed_e4m3(uint32_t c, const F& f) {
+    constexpr int E = F{}.E(), M = F{}.M(), bias = (1 << (E - 1)) - 1;
+    if constexpr (E == 4 && M == 3) return c & 0xFFu;
+    const uint32_t s = (c >> (E + M)) & 1u, e = (c >> M) & ((1u << E) - 1u), fr = c & ((1u << M) - 1u);
+    uint32_t mag = 0;
+    if (e != 0) mag = ((e + 7 - bias) << 3) | (fr << (3 - M));
+    else if (fr != 0) {
+        const int p = 31 - __clz(fr);   // value 2^(p - M + 1 - bias) * (1 + rest / 2^p)
+        mag = ((uint32_t)(p - M + 8 - bias) << 3) | ((fr << (3 - p)) & 7u);
+    }
+    return (s << 7) | mag;
+}
+template <class F>
+__device__ inline uint32_t embed_e4m3_x4(uint32_t w, const F& f) {
+    return embed_e4m3(w & 0xFFu, f) | (embed_e4m3((w >> 8) & 0xFFu, f) << 8) | (embed_e4m3((w >> 16) & 0xFFu, f) << 16) |
+           (embed_e4m3(w >> 24, f) << 24);
+}
+// ---- code tables of the bf16 kernels
+// With t as above ((ye << 7) | f7: the element's exponent field in the target format above the 7 mantissa bits of its
+// bf16 magnitude), the code magnitude is a function of t alone: 2^(E + 7) entries, built at compile time by the same steps
+// as PackedBf16::magnitude (round half to even on the M-bit mantissa, the reference's OR that loses a carry into an odd
+// exponent field, the one reachable subnormal binade).  A workgroup copies its format's table into LDS and looks every
+// element up there: half the vector instructions of the arithmetic.
+template <int E, int M>
+struct CodeLut {
+    static constexpr int N = 1 << (E + 7);
+    uint8_t code[N];
+    constexpr CodeLut() : code{} {
+        constexpr int SH = 7 - M;
+        for (int t = 0; t < N; ++t) {
+            const int ye = t >> 7, f7 = t & 127;
+            const int q = f7 >> SH, r = f7 & ((1 << SH) - 1), half = 1 << (SH - 1);
+            const int yf = q + ((r > half || (r == half && (q & 1))) ? 1 : 0);   // in [0, 2^M]
+            const int c = ye != 0 ? ((ye << M) | yf) : (yf != 0 ? ((yf | (1 << M)) >> 1) : 0);
+            code[t] = (uint8_t)c;
+        }
+    }
+};
+template <int E, int M>
+__device__ const CodeLut<E, M> kCodeLut{};
+
+// LDS copy of the table (the code-producing modes; the fused quantise-dequantise pass does not use one: BYTES = 16 there);
+// all threads of the workgroup call it, before the first bf16_block_step.
+template <class F, bool QDQ>
+struct LdsLut {
+    static constexpr int E = F{}.E(), M = F{}.M();
+    static constexpr int BYTES = QDQ ? 16 : (1 << (E + 7));
+    __device__ static inline void fill(uint8_t* lds) {
+        if (QDQ) return;
+        for (int i = threadIdx.x * 16; i < BYTES; i += kThreads * 16)
+            *reinterpret_cast<uint4*>(lds + i) = *reinterpret_cast<const uint4*>(kCodeLut<E, M>.code + i);
+        __syncthreads();
+    }
+};
+
+// two table entries, for the t values in the halves of `t2` (issued here, valid after the caller's s_waitcnt; plain loads into
+// two registers: a load into half a register does not keep the other half on this hardware)
+template <bool UNUSED>
+__device__ inline void lut_pair(uint32_t& lo, uint32_t& hi, uint32_t lds_base, uint32_t t2) {
+    const uint32_t a_lo = lds_base + (t2 & 0xFFFFu), a_hi = lds_base + (t2 >> 16);
+    asm volatile("ds_read_u8 %0, %2\n\tds_read_u8 %1, %3" : "=&v"(lo), "=&v"(hi) : "v"(a_lo), "v"(a_hi));
+}
+
+// The arithmetic of one 128-bit step of the bf16 kernels below: 8 elements of a lane whose three quad neighbours hold the
+// rest of the block.  QDQ false: o[j] = two codes in the low bytes of the halves; true: two quantised bf16 values.
+// `lut`: LDS address of the table (LdsLut<F, QDQ>).  Every lane of a quad must call it (DPP).
+template <class F, bool QDQ>
+__device__ inline void bf16_block_step(const uint4& raw, const F& f, uint32_t (&o)[4], uint32_t& scale, uint32_t lut) {
+    constexpr int E = F{}.E(), M = F{}.M();
+    const uint32_t h[4] = {raw.x, raw.y, raw.z, raw.w};
+    // block maximum of |x| bits: packed max over the lane's four registers, then the two halves,
+    // then the four lanes of the block (DPP quad permutes)
+    u16x2 m2 = __builtin_elementwise_max(__builtin_elementwise_max(as_u16x2(h[0] & 0x7FFF7FFFu), as_u16x2(h[1] & 0x7FFF7FFFu)),
+                                         __builtin_elementwise_max(as_u16x2(h[2] & 0x7FFF7FFFu), as_u16x2(h[3] & 0x7FFF7FFFu)));
+    uint32_t amax = max((uint32_t)m2[0], (uint32_t)m2[1]);
+    amax = max(amax, (uint32_t)__builtin_amdgcn_mov_dpp((int)amax, 0xB1, 0xF, 0xF, true));  // lane ^ 1
+    amax = max(amax, (uint32_t)__builtin_amdgcn_mov_dpp((int)amax, 0x4E, 0xF, 0xF, true));  // lane ^ 2
+    const int ef_max = (int)(amax >> 7);
+    const int scale_n = max(ef_max - fmt_emax_unb(f), 0);  // amax == 0 gives 0: the all-flushed rule
+    // (scale_n < bias: the packed arithmetic subtracts (scale_n - bias) << 7 with unsigned saturation)
+    const bool hard = amax >= 0x7F80u || scale_n >= 151 || (amax != 0u && scale_n < fmt_bias(f) + (QDQ ? 1 : 0));
+    scale = (uint32_t)scale_n;
+    if (__builtin_amdgcn_ballot_w64(hard) == 0) {
+        const uint32_t ssb = (uint32_t)((scale_n - fmt_bias(f)) << 7) & 0xFFFFu;
+        const uint32_t ssb2 = ssb | (ssb << 16);
+        if constexpr (QDQ) {
+            // (the fused pass stays on the packed arithmetic: a lane has as many stores as loads to hide it under, and a
+            // workgroup would copy a table half the size of its input; measured slower with the table)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = PackedBf16<F>::qdq(h[j], ssb2);
+            return;
+        }
+        uint32_t hl[4], lo[4], hi[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            // inputs with a zero exponent field are flushed to +0.0 before encoding (code 0, sign included): clear them here
+            hl[j] = h[j] & PackedBf16<F>::live_mask(h[j] & 0x7FFF7FFFu);
+            const uint32_t t2 = as_u32(__builtin_elementwise_sub_sat(as_u16x2(hl[j] & 0x7FFF7FFFu), as_u16x2(ssb2)));
+            lut_pair<false>(lo[j], hi[j], lut, t2);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo[0]), "+v"(lo[1]), "+v"(lo[2]), "+v"(lo[3]), "+v"(hi[0]), "+v"(hi[1]), "+v"(hi[2]), "+v"(hi[3]));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            o[j] = lo[j] | (hi[j] << 16) | ((hl[j] >> (15 - (E + M))) & ((1u << (E + M)) * 0x00010001u));
+        }
+    } else {
+        // exact per-element routine (the block's lanes agree on amax, so they agree on the result)
+        const uint32_t amax32 = amax << 16;
+        const int se = shared_exponent<F, true>(amax32, f);
+        scale = amax32 < 0x00800000u ? 0u : (uint32_t)(se + 127);
+        const float sc = scale_f32(scale);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t c0 = encode_mxfp_element(h[j] << 16, se, f), c1 = encode_mxfp_element(h[j] & 0xFFFF0000u, se, f);
+            o[j] = QDQ ? pack_bf16(mxfp_value(c0, sc, f), mxfp_value(c1, sc, f)) : (c0 | (c1 << 16));
+        }
+    }
+}
+
+}  // namespace mase

@@ -34,6 +34,7 @@ SIGNATURES = {
     "mase_hip_mxfp_gemm_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64]),
     "mase_hip_mxfp_gemm_batched": (_i32, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i64, _i32,
                                           _i64, _i64, _i64, _i64, _vp]),
+    "mase_hip_mxfp_scores": (_i32, [_vp, _i32, _i32, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
     "mase_hip_mxfp_gemm_static_ws": (_i32, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _i32,
                                             _vp, _i32, _i64, _i64, _i64, _i32, _vp]),
     "mase_hip_scaled_padded_rows": (_i64, [_i64]),

@@ -8,7 +8,8 @@ backend="fused" (NotImplementedError in the reference, :21-22) quantises ``other
 along its second-to-last axis (no transposed copy).  When ``other`` is quantised it stays in MXFP
 form: its codes come out as [.., N, K], the layout the GEMM kernels read, and all leading batch
 axes (broadcast ones included) go into ONE batched GEMM launch that composes the codes to bf16
-on their way to the MFMA units.  A product of two quantised bfloat16 operands against ONE matrix
+on their way to the MFMA units.  Products of queries and keys (``other`` the transposed view of a contiguous bfloat16 tensor, K up to
+128) quantise their operands inside the GEMM: one launch, or two.  A product of two quantised bfloat16 operands against ONE matrix
 (``other`` without batch axes) with enough rows takes the block-scaled FP8 matrix instruction instead, as
 ``mxfp_linear`` does (functional/linear.py).  Everything else goes through the one-pass quantise-dequantise
 kernels and ``torch.matmul``.
@@ -110,6 +111,36 @@ def _other_components(other: Tensor, other_meta: MXFPMeta) -> tuple[Tensor, Tens
     return kernels.extract_mxfp_components_strided(other, -2, other_meta)
 
 
+# The keys are quantised inside the product, once for every 128 rows of queries, up to this many such panels x K; beyond, a pass over
+# them comes first.  Inside / before, us: 32 products of 512 x 512 x 128 (4 panels) 14.6 / 18.1, 64 of 256 x 256 x 128 11.5 / 18.2; 64 of 1000 x
+# 1000 x 128 (8) 55 / 47, 32 of 1464 x 1464 x 64 (12) 39 / 36.
+SCORES_QUANTISE_W_UP_TO = 512
+
+
+def _scores(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, other_meta: MXFPMeta) -> Tensor | None:
+    """The product of queries and keys in one or two launches, or None where it is not one: ``other`` the transposed view of a
+    contiguous bfloat16 tensor, K up to 128."""
+    K, N = other.shape[-2], other.shape[-1]
+    if (input.dtype != torch.bfloat16 or not kernels.scores_shape_supported(N, K) or other.is_contiguous()
+            or not kernels.scores_format_supported(other_meta) or not (input_meta is None or kernels.scores_format_supported(input_meta))):
+        return None
+    lying = other.transpose(-1, -2)
+    if not lying.is_contiguous():
+        return None
+    bi, bo = tuple(input.shape[:-2]), tuple(other.shape[:-2])
+    M = input.shape[-2]
+    if _prod(bo) == 1:
+        batch, M = (), input.numel() // K                     # one matrix: all rows of the input are rows of one product
+    else:
+        batch = tuple(torch.broadcast_shapes(bi, bo))
+        if _prod(bi) != 1 and bi != batch or bo != batch:
+            return None                                         # broadcast along some axes only
+    quantise_w = input_meta is not None and input_meta == other_meta and -(-M // 128) * K <= SCORES_QUANTISE_W_UP_TO
+    w = lying if quantise_w else kernels.quantize_dequantize(lying.reshape(-1), other_meta, torch.bfloat16)
+    y = kernels.mxfp_scores(input, input_meta, w, quantise_w, _prod(batch), M, N, K, 0 if _prod(bi) == 1 else M * K, N * K)
+    return y.view(*torch.broadcast_shapes(bi, bo), input.shape[-2], N)
+
+
 def _matmul_through_gemm(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, other_meta: MXFPMeta) -> Tensor:
     if _scaled_route(input, other, input_meta, other_meta):
         K, N = other.shape[-2], other.shape[-1]
@@ -119,6 +150,9 @@ def _matmul_through_gemm(input: Tensor, other: Tensor, input_meta: MXFPMeta | No
         y = kernels.mxfp_gemm_scaled(a_op, w_op, None, input.dtype)
         lead = torch.broadcast_shapes(tuple(input.shape[:-2]), tuple(other.shape[:-2]))
         return y.view(*lead, input.shape[-2], N)
+    y = _scores(input, other, input_meta, other_meta)
+    if y is not None:
+        return y
     a = input
     if input_meta is not None:
         # MXFP values are exact in bf16 whatever input.dtype is

@@ -224,6 +224,32 @@ def mxfp_gemm_batched(a: Tensor, w_scales: Tensor, w_elements: Tensor, w_meta: M
     return y
 
 
+def scores_format_supported(meta: MXFPMeta) -> bool:
+    return meta.block_size == 32 and meta.element_is_finite and meta.scale_exp_bits == 8 and meta.round_mode == "rn"
+
+
+def scores_shape_supported(N: int, K: int) -> bool:
+    return K % 32 == 0 and K <= 128 and N % 8 == 0 and N <= 1 << 23
+
+
+def mxfp_scores(a: Tensor, meta: MXFPMeta | None, w: Tensor, quantise_w: bool, batches: int, M: int, N: int, K: int,
+                a_batch_stride: int, w_batch_stride: int) -> Tensor:
+    """``batches`` products y[b] = Q(A[b]) @ W[b]^T in one launch, K <= 128: ``a`` and ``w`` hold bfloat16 [M, K] and [N, K] matrices
+    ``a_batch_stride`` and ``w_batch_stride`` elements apart (0 shares the operand).  A is quantised in format ``meta`` on the way
+    in (None: used as it is), W too if ``quantise_w``.  Returns y [batches, M, N]."""
+    _lib.require_gpu(a, "activations")
+    assert a.dtype == w.dtype == torch.bfloat16 and a.device == w.device and scores_shape_supported(N, K)
+    assert meta is None or scores_format_supported(meta)
+    a, w = _lib.dense(a), _lib.dense(w)
+    assert a.numel() >= (batches - 1) * a_batch_stride + M * K and w.numel() >= (batches - 1) * w_batch_stride + N * K
+    y = torch.empty((batches, M, N), dtype=torch.bfloat16, device=a.device)
+    e, f = (0, 0) if meta is None else (meta.element_exp_bits, meta.element_frac_bits)
+    with _lib.on_device(a.device):
+        _lib.check(_lib.load().mase_hip_mxfp_scores(a.data_ptr(), e, f, w.data_ptr(), int(quantise_w), y.data_ptr(), M, N, K, batches,
+                                                    a_batch_stride, w_batch_stride, M * N, _lib.stream_ptr(a.device)))
+    return y
+
+
 # ---- the block-scaled matrix instruction route (FP8 bytes and E8M0 scales straight into the matrix unit)
 _SCALED_FORMATS = {(4, 3), (2, 3), (3, 2), (2, 1)}
 
