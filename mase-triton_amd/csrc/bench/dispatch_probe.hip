@@ -6,6 +6,13 @@
 // of K there), 128-k macro steps of each but a shorter last one}.  `may_split`: the caller brings room for partial sums.
 extern "C" int mase_bench_scaled_plan(int64_t M, int64_t N, int64_t K, int cus, int may_split, int* plan) {
     if (!plan || M < 1 || N < 1 || K < 512 || K % 256 != 0 || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K >= ((int64_t)1 << 27) || cus < 8) return -1;
+    const mase::ScaledMidPlan few = mase::plan_scaled_few((int)M, (int)N, (int)K, cus, may_split != 0);
+    if (few.bn != 0) {
+        plan[0] = few.bn;
+        plan[1] = few.splits;
+        plan[2] = few.mac_per;
+        return 0;
+    }
     const int slices = may_split ? mase::scaled_rows_slices((int)M, (int)N, (int)K) : 0;
     if (slices > 0 || mase::scaled_rows_shape_ok((int)M, (int)K)) {
         plan[0] = 0;

@@ -1,14 +1,14 @@
 // Block-scaled MXFP GEMM for tens to hundreds of rows of A (a large decode batch, a chunk of a prompt), operands in the prepared
-// form of gemm_scaled.h, on tiles of 128 x 128 or 128 x 64.
+// form of gemm_scaled.h, on tiles of 128 x 128 or 128 x 64; and of 64 x 64 for 17 - 64 rows.
 //
 // At these sizes the 256 x 256 tiles of gemm_scaled.h leave most CUs without one (200 x 14336 outputs: 56 tiles for 256 CUs), and
 // splitting K for more of them costs fp32 partial sums of 256-row tiles that are mostly padding.  Smaller tiles give every CU
 // one; what they cost is operand traffic per flop: a 128 x 128 tile takes 32 KB L2 -> LDS and 64 KB LDS -> registers per 128 k for
 // 512 cycles of MFMA.  Both are about what a CU's paths carry in that time, so the kernel is organised to keep them running:
 //   * four wavefronts (2 x 2 of 64 x 64, or 4 x 1 of 32 x 64 when the tile is 64 columns wide), one workgroup per CU;
-//   * codes and scale dwords global -> LDS by DMA into a ring of four stages (one 128-k macro step each), four steps ahead;
+//   * codes and scale dwords global -> LDS by DMA into a ring of four stages (64 x 64: eight) of one 128-k macro step each, as many steps ahead;
 //   * the fragments of macro step s + 1 are read from LDS into the other of two register sets while step s is multiplied: at
-//     the one barrier per step every wavefront has its operands in registers, and the slot of step s is free for step s + 4;
+//     the one barrier per step every wavefront has its operands in registers, and the slot of step s is free for the step a ring ahead;
 //   * every MFMA is followed by its share of the step's LDS reads and DMAs and a scheduling barrier, as in gemm_scaled.h.
 // What bounds it: a macro step takes 0.61 us (128 columns; 0.43 with 64), of which MFMAs and LDS are 0.29 (0.18).  The rest is the
 // vector-memory path.  A CU takes in 55 bytes per ns when some of them come from HBM, however deep the ring is (six stages:
@@ -20,9 +20,10 @@
 // LDS rows are 128 bytes, the 16-byte piece c of row r at position c ^ ((r >> 1) & 7).
 // (included from gemm_impl.h's namespace, after gemm_scaled.h's typedefs)
 
-constexpr int SMD_M = 128, SMD_RING = 4;
-template <int BN> constexpr int smd_stage_bytes() { return (SMD_M + BN) * 128 + 1024; }
-template <int BN> constexpr int smd_lds_bytes() { return SMD_RING * smd_stage_bytes<BN>(); }
+// bytes of one ring stage, stages of the ring (as many as LDS holds, at most eight), bytes of LDS
+template <int BM, int BN> constexpr int smd_stage_bytes() { return (BM + BN) * 128 + 1024; }
+template <int BM, int BN> constexpr int smd_ring() { return BM == 128 ? 4 : 8; }
+template <int BM, int BN> constexpr int smd_lds_bytes() { return smd_ring<BM, BN>() * smd_stage_bytes<BM, BN>(); }
 
 __device__ inline void mfma_scaled_v(floatx4& c, const intx8& w, const intx8& a, uint32_t sw, uint32_t sa) {
     asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]" : "+v"(c) : "v"(w), "v"(a), "v"(sw), "v"(sa));
@@ -32,15 +33,15 @@ __device__ inline void dma_64_dwords(uint32_t lds_addr, uint32_t voff, const voi
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
 
-template <int DT_OUT, int BN>
+template <int DT_OUT, int BM, int BN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mxfp_gemm_scaled_mid_kernel(
     const uint8_t* __restrict__ a_codes, const uint32_t* __restrict__ a_scales, const uint8_t* __restrict__ w_codes,
     const uint32_t* __restrict__ w_scales, const void* __restrict__ bias, int bias_dtype, void* __restrict__ y_all, int M, int N, int K,
     int rows_a, int rows_w, int tiles_m, int splits, int mac_per, int n_walks, int64_t y_split_bytes) {
-    constexpr int WN = BN / 64, WM = 4 / WN, MI = 8 / WM, NJ = 4;       // wavefronts along n and m; 16-row and 16-column tiles of one
-    constexpr int A_BYTES = SMD_M * 128, W_BYTES = BN * 128, STAGE = smd_stage_bytes<BN>(), SC = A_BYTES + W_BYTES;
-    constexpr int RING = SMD_RING;
-    constexpr int W_DMAS = W_BYTES / 4096, OPS = 4 + W_DMAS + 1;        // DMAs per wavefront and step: A, W, scales
+    constexpr int WN = BN / 64, WM = 4 / WN, MI = BM / 16 / WM, NJ = 4;       // wavefronts along n and m; 16-row and 16-column tiles of one
+    constexpr int A_BYTES = BM * 128, W_BYTES = BN * 128, STAGE = smd_stage_bytes<BM, BN>(), SC = A_BYTES + W_BYTES;
+    constexpr int RING = smd_ring<BM, BN>();
+    constexpr int A_DMAS = A_BYTES / 4096, W_DMAS = W_BYTES / 4096, OPS = A_DMAS + W_DMAS + 1;        // DMAs per wavefront and step: A, W, scales
     constexpr int READS = 2 * (MI + NJ) + MI + NJ, MFMAS = MI * NJ;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     const int lane = threadIdx.x & 63;
@@ -53,22 +54,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int walk = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));     // (the grid is a multiple of 8)
     if (walk >= n_walks) return;
     const int tile_m = walk % tiles_m, rest = walk / tiles_m;
-    const int z = rest % splits, tile_n = rest / splits, m0 = tile_m * SMD_M, n0 = tile_n * BN;
+    const int z = rest % splits, tile_n = rest / splits, m0 = tile_m * BM, n0 = tile_n * BN;
     const int mac0 = z * mac_per, nm = min(mac_per, K / 128 - mac0);   // this walk's macro steps (at least one)
     uint8_t* const y = static_cast<uint8_t*>(y_all) + (size_t)z * (size_t)y_split_bytes;
 
     // ---- DMA.  Data: lane l fills position l & 7 of row 8 d + (l >> 3) of the wavefront's rows, which must hold the row's piece
-    //      (l & 7) ^ (row >> 1 & 7).  Wavefront w: rows 32 w .. of A, BN / 4 w .. of W, and 64 of the scale dwords (A's 128, then W's).
+    //      (l & 7) ^ (row >> 1 & 7).  Wavefront w: rows BM / 4 w .. of A, BN / 4 w .. of W, and 64 of the scale dwords (A's, then W's).
     uint32_t voff[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d)
         voff[d] = (uint32_t)(8 * d + (lane >> 3)) * (uint32_t)K + (uint32_t)(((lane & 7) ^ ((4 * d + (lane >> 4)) & 7)) << 4);
     const uint32_t sc_voff = (uint32_t)lane * 4u;
-    const int sc_wave = BN == 64 ? min(wave, 2) : wave;                 // (64 columns: the last wavefront repeats W's 64 dwords)
-    const uint8_t* pa = a_codes + (size_t)(m0 + 32 * wave) * K + (size_t)mac0 * 128;
+    const int sc_wave = min(wave, BM / 64 + BN / 64 - 1);               // (fewer than 256 dwords: the last wavefronts repeat W's)
+    constexpr int SC_A = BM / 64;
+    const uint8_t* pa = a_codes + (size_t)(m0 + BM / 4 * wave) * K + (size_t)mac0 * 128;
     const uint8_t* pw = w_codes + (size_t)(n0 + BN / 4 * wave) * K + (size_t)mac0 * 128;
-    const uint32_t* psc = sc_wave < 2 ? a_scales + (size_t)mac0 * rows_a + m0 + 64 * sc_wave : w_scales + (size_t)mac0 * rows_w + n0 + 64 * (sc_wave - 2);
-    const int sc_step = sc_wave < 2 ? rows_a : rows_w;
+    const uint32_t* psc = sc_wave < SC_A ? a_scales + (size_t)mac0 * rows_a + m0 + 64 * sc_wave : w_scales + (size_t)mac0 * rows_w + n0 + 64 * (sc_wave - SC_A);
+    const int sc_step = sc_wave < SC_A ? rows_a : rows_w;
     // workgroups of different columns start at different macro steps and wrap around: rows of W (and of A) are K bytes apart, and at
     // one k all of them would sit on the same few channels of the L2
     int at = tile_n % nm;                                             // the macro step that is issued next
@@ -77,8 +79,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     psc += (size_t)at * sc_step;
     auto dma = [&](auto slot_c, auto q_c) __attribute__((always_inline)) {
         constexpr int slot = decltype(slot_c)::value, q = decltype(q_c)::value;
-        if constexpr (q < 4) dma_1kb(lds_base + (uint32_t)(slot * STAGE + q * 1024) + (uint32_t)wave * 4096u, voff[q], pa);
-        else if constexpr (q < 4 + W_DMAS) dma_1kb(lds_base + (uint32_t)(slot * STAGE + A_BYTES + (q - 4) * 1024) + (uint32_t)wave * (W_DMAS * 1024u), voff[q - 4], pw);
+        if constexpr (q < A_DMAS) dma_1kb(lds_base + (uint32_t)(slot * STAGE + q * 1024) + (uint32_t)wave * (A_DMAS * 1024u), voff[q], pa);
+        else if constexpr (q < A_DMAS + W_DMAS) dma_1kb(lds_base + (uint32_t)(slot * STAGE + A_BYTES + (q - A_DMAS) * 1024) + (uint32_t)wave * (W_DMAS * 1024u), voff[q - A_DMAS], pw);
         else dma_64_dwords(lds_base + (uint32_t)(slot * STAGE + SC) + (uint32_t)sc_wave * 256u, sc_voff, psc);
     };
     auto advance = [&]() __attribute__((always_inline)) {
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const uint8_t* const w_lo = lds + A_BYTES + wave_n * (NJ * 2048) + f_off;
     const uint8_t* const w_hi = lds + A_BYTES + wave_n * (NJ * 2048) + (f_off ^ 64u);
     const uint8_t* const a_sc = lds + SC + wave_m * (MI * 64) + (lane & 15) * 4 + (lane >> 4);
-    const uint8_t* const w_sc = lds + SC + 512 + wave_n * (NJ * 64) + (lane & 15) * 4 + (lane >> 4);
+    const uint8_t* const w_sc = lds + SC + BM * 4 + wave_n * (NJ * 64) + (lane & 15) * 4 + (lane >> 4);
     floatx4 acc[NJ][MI];
     intx8 af[2][MI], wf[2][NJ];
     uint32_t as[2][MI], ws[2][NJ];
@@ -198,6 +200,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 
 struct ScaledMidPlan {
+    int bm;        // rows of a tile: 64, 128; 256: the 256 x 256 kernel of gemm_scaled.h
     int bn;        // columns of a tile: 128 or 64; 256: the 256 x 256 kernel of gemm_scaled.h
     int splits;    // workgroups that share a tile's K, each with its own fp32 [M, N] array of the workspace
     int mac_per;   // macro steps per split
@@ -214,7 +217,7 @@ struct ScaledMidPlan {
 // and 14.3 / 19.5 / 28.6; K = 4096 53 and 55).
 inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
     const int nmac = K / SMAC;
-    ScaledMidPlan best{256, 1, nmac};
+    ScaledMidPlan best{256, 256, 1, nmac};
     if (cus <= 0) return best;
     const double mn_mb = (double)M * N * 4.0 / 1e6;
     double best_t = 1e30;
@@ -231,8 +234,47 @@ inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
             const double rounds = (double)((wgs + cus - 1) / cus);
             const double unshared = bn != 256 && M <= 128 && wgs > cus ? 1.4 * std::min(1.0, (double)(wgs - cus) / cus) : 0.0;
             const double t = rounds * (per * step + (bn == 256 ? 0.0 : 2.5)) + (bn == 256 ? 8.0 : 2.0 + unshared) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
-            if (t < best_t) { best_t = t; best = ScaledMidPlan{bn, want, per}; }
+            if (t < best_t) { best_t = t; best = ScaledMidPlan{bn == 256 ? 256 : 128, bn, want, per}; }
         }
+    }
+    return best;
+}
+
+// Up to 64 rows: tiles of 64 x 64 against the weight-streaming kernel that keeps A in its registers.  The latter's prologue and the MFMAs
+// of a unit grow with the 16-row tiles of A (every CU takes in all of A), and a unit of a short K is too few bytes in flight; these
+// tiles read 64 rows of A per 64 of W whatever M is, from a grid of N / 64.  Prices in us with W from memory.  GEMMs alone, W from memory |
+// W in the memory-side cache, tiles / the other kernel: 14336 x 4096 32 rows 16.7 / 16.0 | 12.9 / 15.4, 48 rows 16.8 / 17.5 | 13.0 / 17.0, 64 rows
+// 16.9 / 19.5 | 13.0 / 19.3; 4096 x 14336, K in four, 32 rows 19.2 / 18.5 | 17.4 / 18.3, 48 rows 19.5 / 20.5 | 17.6 / 20.4, 64 rows 19.8 / 23.0 | 17.7 / 23.1;
+// 8192 x 2048 16 rows 7.1 / 7.8 | 7.1 / 7.5, 64 rows 7.1 / 12.1 | 7.1 / 11.8; 4096 x 4096 32 rows 9.4 / 8.1 | 9.4 / 7.5, 64 rows 9.4 / 10.3 | 9.4 / 9.7.  Layer calls
+// of 48 rows, before and now: 14336 x 768 18.2 / 8.7, 8192 x 8192 27.3 / 21.5, 2176 x 10752 18.1 / 15.6.  (Tiles of 64 x 128 are never ahead: 14336 x
+// 4096 21.2 | 13.8.)  bn == 0: a weight-streaming kernel.
+inline ScaledMidPlan plan_scaled_few(int M, int N, int K, int cus, bool may_split) {
+    const int nmac = K / SMAC;
+    ScaledMidPlan best{0, 0, 1, nmac};
+    if (M > 64 || cus <= 0) return best;
+    // 17 - 32 rows of a long K: level at best (896 x 14336 13.4 / 14.7); up to 16 rows, or with no room for sums, the chunked kernel
+    if (M <= 32 && K > 4096) return best;
+    const double mn_mb = (double)M * N * 4.0 / 1e6;
+    auto split_cost = [&](int splits) { return splits > 1 ? 3.0 + (2.0 * splits + 0.5) * mn_mb * 0.16 : 0.0; };
+    // the other kernel: prologue, then units of 16 rows of W x (a slice of) K, the last as half units; a unit takes its latency at least
+    const int slices = K > 4096 ? (may_split ? scaled_rows_slices(M, N, K) : 0) : 1;
+    double best_t = 1e30;                                   // (33 rows and more without room for its sums: these tiles, or 128-row ones)
+    if (slices > 0) {
+        const int mt = (M + 15) / 16, groups = (N + 15) / 16, per_slice = std::max(1, std::min(groups, cus / slices));
+        const double units = slices > 1 ? (groups + per_slice - 1) / per_slice : std::max(1.0, std::ceil(2.0 * groups / cus) / 2.0);
+        const double busy = std::min(1.0, (double)groups * slices / cus);
+        best_t = 3.8 + 0.9 * mt * (0.5 + 0.5 * busy) + units * (std::max(1.6, (double)nmac / slices / 32.0 * 2.15) * (0.4 + 0.6 * busy) + 0.25 * mt) +
+                 split_cost(slices) - 0.5;
+    }
+    const int64_t tiles = (N + 63) / 64;
+    for (int want = 1; want <= 16; ++want) {
+        if (want > 1 && (!may_split || tiles * want > cus || N % 4 != 0)) break;
+        const int per = (nmac + want - 1) / want;
+        if (want > 1 && (per < 12 || (nmac + per - 1) / per != want)) continue;
+        const int64_t wgs = tiles * want;
+        const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
+        const double t = (double)((wgs + cus - 1) / cus) * (per * (0.15 + 0.28 * busy) + 1.2) + 2.0 + split_cost(want);
+        if (t < best_t) { best_t = t; best = ScaledMidPlan{64, 64, want, per}; }
     }
     return best;
 }
@@ -241,7 +283,7 @@ template <int DT_OUT>
 int launch_gemm_scaled_mid(const uint8_t* a_codes, const uint32_t* a_scales, const uint8_t* w_codes, const uint32_t* w_scales, const void* bias,
                            int bias_dtype, void* y, int M, int N, int K, const ScaledMidPlan& p, void* workspace, hipStream_t s) {
     const int rows_a = (M + 255) / 256 * 256, rows_w = (N + 255) / 256 * 256;
-    const int tiles_m = (M + SMD_M - 1) / SMD_M, tiles_n = (N + p.bn - 1) / p.bn;
+    const int tiles_m = (M + p.bm - 1) / p.bm, tiles_n = (N + p.bn - 1) / p.bn;
     const int64_t walks = (int64_t)tiles_m * tiles_n * p.splits, mn = (int64_t)M * N;
     if (walks >= (1 << 30)) return fail(ERR_UNSUPPORTED, "too many tiles");
     auto go = [&](auto kern, int lds_bytes, std::atomic<uint64_t>& allowed, void* out, int64_t split_bytes, const void* b) {
@@ -250,13 +292,16 @@ int launch_gemm_scaled_mid(const uint8_t* a_codes, const uint32_t* a_scales, con
                            N, K, rows_a, rows_w, tiles_m, p.splits, p.mac_per, (int)walks, split_bytes);
         return check_launch("mxfp_gemm_scaled");
     };
-    static std::atomic<uint64_t> allowed[4] = {{0}, {0}, {0}, {0}};
-    if (p.splits == 1)
-        return p.bn == 128 ? go(mxfp_gemm_scaled_mid_kernel<DT_OUT, 128>, smd_lds_bytes<128>(), allowed[0], y, 0, bias)
-                           : go(mxfp_gemm_scaled_mid_kernel<DT_OUT, 64>, smd_lds_bytes<64>(), allowed[1], y, 0, bias);
-    if (int rc = p.bn == 128 ? go(mxfp_gemm_scaled_mid_kernel<F32, 128>, smd_lds_bytes<128>(), allowed[2], workspace, mn * 4, nullptr)
-                             : go(mxfp_gemm_scaled_mid_kernel<F32, 64>, smd_lds_bytes<64>(), allowed[3], workspace, mn * 4, nullptr))
-        return rc;
+    static std::atomic<uint64_t> allowed[2][2][2] = {};
+    auto pick = [&](auto dt, void* out, int64_t split_bytes, const void* b) {
+        constexpr int DT = decltype(dt)::value;
+        std::atomic<uint64_t>* const done = allowed[split_bytes != 0][p.bm == 64];
+        if (p.bm == 64) return go(mxfp_gemm_scaled_mid_kernel<DT, 64, 64>, smd_lds_bytes<64, 64>(), done[0], out, split_bytes, b);
+        return p.bn == 128 ? go(mxfp_gemm_scaled_mid_kernel<DT, 128, 128>, smd_lds_bytes<128, 128>(), done[0], out, split_bytes, b)
+                           : go(mxfp_gemm_scaled_mid_kernel<DT, 128, 64>, smd_lds_bytes<128, 64>(), done[1], out, split_bytes, b);
+    };
+    if (p.splits == 1) return pick(IntC<DT_OUT>{}, y, 0, bias);
+    if (int rc = pick(IntC<F32>{}, workspace, mn * 4, nullptr)) return rc;
     hipLaunchKernelGGL(split_k_reduce_kernel<DT_OUT>, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, s, static_cast<const float*>(workspace), p.splits,
                        mn, N, bias, bias_dtype, y);
     return check_launch("mxfp_gemm_scaled");
