@@ -1,4 +1,5 @@
 // C-ABI entry point of the products with a short contraction that quantise on the way in; the kernel is in gemm_scores.h.
+#include "../../include/mase_hip_scores.h"
 #include "gemm_scores.h"
 
 using namespace mase;

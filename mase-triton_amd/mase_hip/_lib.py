@@ -1,8 +1,11 @@
-"""ctypes binding of lib/libmase_hip.so (declarations: include/mase_hip.h at the repo root)."""
+"""ctypes binding of lib/libmase_hip.so (declarations: include/mase_hip.h and mase_hip_scores.h at the repo root), and the extension module beside it
+(csrc/host/bindings.cpp) through which the most frequent calls go."""
 from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -34,7 +37,6 @@ SIGNATURES = {
     "mase_hip_mxfp_gemm_workspace_bytes": (_i64, [_i32, _i64, _i64, _i64]),
     "mase_hip_mxfp_gemm_batched": (_i32, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _i32, _i64, _i64, _i64, _i32,
                                           _i64, _i64, _i64, _i64, _vp]),
-    "mase_hip_mxfp_scores": (_i32, [_vp, _i32, _i32, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
     "mase_hip_mxfp_gemm_static_ws": (_i32, [_vp, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _i32,
                                             _vp, _i32, _i64, _i64, _i64, _i32, _vp]),
     "mase_hip_scaled_padded_rows": (_i64, [_i64]),
@@ -48,6 +50,11 @@ SIGNATURES = {
     "mase_hip_mxfp_linear_scaled_scratch_bytes": (_i64, [_i64, _i64, _i64]),
     "mase_hip_mxfp_linear_scaled": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i64, _i64, _vp, _i64, _vp]),
     "mase_hip_mxfp_gemm_prepared_w": (_i32, [_vp, _i32, _vp, _vp, _vp, _i32, _vp, _i32, _i64, _i64, _i64, _vp]),
+}
+
+# include/mase_hip_scores.h
+SCORES_SIGNATURES = {
+    "mase_hip_mxfp_scores": (_i32, [_vp, _i32, _i32, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
 }
 
 
@@ -64,11 +71,30 @@ def load() -> ctypes.CDLL:
                 f"{_LIB_PATH} is missing: build it with `python mase-triton_amd/build.py` "
                 "(mase_hip has no other implementation to fall back to)")
         lib = ctypes.CDLL(_LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **SCORES_SIGNATURES}.items():
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = res, args
         _lib = lib
     return _lib
+
+
+_HOST_PATH = os.path.join(os.path.dirname(_LIB_PATH), "_mase_host.so")
+_host = None
+
+
+def host():
+    """The extension module: functions that take a plain call (contiguous, aligned tensors on the current GPU) in one step and
+    return None for any other, which then goes through the wrappers of this package."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(_HOST_PATH):
+            raise RuntimeError(f"{_HOST_PATH} is missing: build it with `python mase-triton_amd/build.py`")
+        loader = importlib.machinery.ExtensionFileLoader("_mase_host", _HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_mase_host", _HOST_PATH, loader=loader))
+        loader.exec_module(module)
+        _host = module
+    return _host
 
 
 class MaseHipError(RuntimeError):
