@@ -24,6 +24,10 @@ LIB = os.path.join(LIB_DIR, "libmase_hip.so")
 BENCH_SRCS = [os.path.join(CSRC, "bench", f) for f in ("stream_copy.hip", "swiglu_probe.hip", "dispatch_probe.hip")]
 BENCH_LIB = os.path.join(LIB_DIR, "libmase_bench.so")
 
+# the native side of the Python calls: plain C++ against torch's headers
+HOST_SRC = os.path.join(CSRC, "host", "bindings.cpp")
+HOST_LIB = os.path.join(LIB_DIR, "_mase_host.so")
+
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -84,7 +88,24 @@ def build_library(force: bool = False, save_temps: bool = False, verbose: bool =
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
+    if force or _stale(HOST_LIB, [HOST_SRC, *_includes(HOST_SRC), LIB]):
+        build_host(verbose)
     return LIB
+
+
+def build_host(verbose: bool = True) -> None:
+    import sysconfig
+
+    import torch
+
+    torch_dir = os.path.dirname(os.path.abspath(torch.__file__))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(torch_dir, "include"), "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           "-isystem", sysconfig.get_paths()["include"], HOST_SRC, "-o", HOST_LIB, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-L", LIB_DIR, "-lmase_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.run(cmd, check=True)
 
 
 if __name__ == "__main__":

@@ -1,0 +1,287 @@
+// Native side of the calls that a program makes most often: argument checks, output allocation and the call into libmase_hip.so in one
+// step from Python.  A small cast takes 3 us on the GPU and as long to launch; through ctypes and Python wrappers it took 8 - 13 us of
+// host time, now 4.5 - 6.
+//
+// Every function takes the call only where it is plain: exact torch tensors on the current GPU, contiguous, 16-byte aligned, of
+// a type that the kernels read, no dispatch or function mode active.  Anything else (and any error that the library reports) returns
+// None, and the Python wrapper does what it always did: it copies, converts, switches the device, or raises the error.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/ops/empty.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../../include/mase_hip.h"
+#include "../../../include/mase_hip_scores.h"
+
+namespace {
+
+PyObject* g_raw_stream = nullptr;   // torch._C._cuda_getCurrentRawStream
+
+int dtype_code(at::ScalarType t) {
+    return t == at::kFloat ? 0 : t == at::kHalf ? 1 : t == at::kBFloat16 ? 2 : -1;
+}
+const at::ScalarType kDtypes[3] = {at::kFloat, at::kHalf, at::kBFloat16};
+
+// an exact tensor on a GPU that owns its data as it lies
+const at::Tensor* gpu_tensor(PyObject* o) {
+    if (!THPVariable_CheckExact(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || !t.unsafeGetTensorImpl()->has_storage() || t.is_neg() || t._is_zerotensor()) return nullptr;
+    return &t;
+}
+bool dense(const at::Tensor& t) { return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// stream of the current device if `t` is on it and nothing wants to see the calls; false: not a plain call
+bool stream_of(const at::Tensor& t, void** stream) {
+    static const c10::impl::VirtualGuardImpl guard(c10::DeviceType::CUDA);
+    if (c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::PythonTorchFunctionTLS::stack_len() > 0) return false;
+    const auto device = t.device().index();
+    if (guard.getDevice().index() != device) return false;
+    PyObject* const index = PyLong_FromLong(device);
+    if (!index) return PyErr_Clear(), false;
+    PyObject* const raw = PyObject_CallOneArg(g_raw_stream, index);
+    Py_DECREF(index);
+    if (!raw) return PyErr_Clear(), false;
+    *stream = PyLong_AsVoidPtr(raw);
+    Py_DECREF(raw);
+    if (PyErr_Occurred()) return PyErr_Clear(), false;
+    return true;
+}
+
+// (block_size, exp_bits, frac_bits, finite, round mode or -1) of MXFP formats, (exp_bits, frac_bits, finite, round mode) of minifloat ones
+template <int N>
+bool ints(PyObject* tuple, long (&v)[N]) {
+    if (!PyTuple_CheckExact(tuple) || PyTuple_GET_SIZE(tuple) != N) return false;
+    for (int i = 0; i < N; ++i) {
+        v[i] = PyLong_AsLong(PyTuple_GET_ITEM(tuple, i));
+        if (v[i] == -1 && PyErr_Occurred()) return PyErr_Clear(), false;
+    }
+    return v[N - 1] >= 0;
+}
+// code of the output type: None (that of `t`) or a code
+int out_code(PyObject* o, const at::Tensor& t) {
+    if (o == Py_None) return dtype_code(t.scalar_type());
+    const long c = PyLong_AsLong(o);
+    if (c == -1 && PyErr_Occurred()) return PyErr_Clear(), -1;
+    return c >= 0 && c < 3 ? (int)c : -1;
+}
+
+// blocks along axis `dim` of a contiguous tensor: [outer, k, inner]; false: not an axis
+bool extents(const at::Tensor& t, long dim, int64_t& outer, int64_t& k, int64_t& inner) {
+    const int64_t nd = t.dim();
+    if (dim < -nd || dim >= nd) return false;
+    if (dim < 0) dim += nd;
+    outer = inner = 1;
+    for (int64_t i = 0; i < dim; ++i) outer *= t.size(i);
+    for (int64_t i = dim + 1; i < nd; ++i) inner *= t.size(i);
+    k = t.size(dim);
+    return dim == nd - 1 || k % 32 == 0;
+}
+
+at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor& like) { return at::empty(sizes, at::TensorOptions().dtype(dtype).device(like.device())); }
+
+#define PLAIN(cond) \
+    if (!(cond)) Py_RETURN_NONE
+
+// extract_mxfp(x, block_dim, format) -> (scales [n / B, 1], elements [n / B, B])
+PyObject* extract_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 3);
+    const at::Tensor* const x = gpu_tensor(a[0]);
+    long f[5];
+    PLAIN(x && dense(*x) && ints(a[2], f));
+    const long dim = PyLong_AsLong(a[1]);
+    int64_t outer, k, inner;
+    void* stream;
+    const int dt = dtype_code(x->scalar_type());
+    const int64_t n = x->numel(), B = f[0];
+    if (PyErr_Occurred()) PyErr_Clear();
+    PLAIN(dt >= 0 && n > 0 && B > 0 && n % B == 0 && extents(*x, dim, outer, k, inner) && stream_of(*x, &stream));
+    const bool last = dim == -1 || dim == x->dim() - 1;
+    PLAIN(last || B == 32);
+    at::Tensor scales = empty({n / B, 1}, at::kByte, *x), elements = empty({n / B, B}, at::kByte, *x);
+    const int rc = last ? mase_hip_extract_mxfp(x->data_ptr(), dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
+                        : mase_hip_extract_mxfp_strided(x->data_ptr(), dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3],
+                                                        (int)f[4], stream);
+    PLAIN(rc == 0);
+    PyObject* const s = THPVariable_Wrap(std::move(scales));
+    PyObject* const e = s ? THPVariable_Wrap(std::move(elements)) : nullptr;
+    PyObject* const r = e ? PyTuple_New(2) : nullptr;
+    if (!r) {
+        Py_XDECREF(s);
+        Py_XDECREF(e);
+        return nullptr;
+    }
+    PyTuple_SET_ITEM(r, 0, s);
+    PyTuple_SET_ITEM(r, 1, e);
+    return r;
+    END_HANDLE_TH_ERRORS
+}
+
+// qdq_mxfp(x, block_dim, format, output code or None) -> tensor of x's shape
+PyObject* qdq_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 4);
+    const at::Tensor* const x = gpu_tensor(a[0]);
+    long f[5];
+    PLAIN(x && dense(*x) && ints(a[2], f));
+    const long dim = PyLong_AsLong(a[1]);
+    if (PyErr_Occurred()) PyErr_Clear();
+    int64_t outer, k, inner;
+    void* stream;
+    const int dt = dtype_code(x->scalar_type()), od = out_code(a[3], *x);
+    const int64_t n = x->numel(), B = f[0];
+    PLAIN(dt >= 0 && od >= 0 && n > 0 && B > 0 && n % B == 0 && extents(*x, dim, outer, k, inner) && stream_of(*x, &stream));
+    const bool last = dim == -1 || dim == x->dim() - 1;
+    PLAIN(last || B == 32);
+    at::Tensor out = empty(x->sizes(), kDtypes[od], *x);
+    const int rc = last ? mase_hip_qdq_mxfp(x->data_ptr(), dt, out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
+                        : mase_hip_qdq_mxfp_strided(x->data_ptr(), dt, out.data_ptr(), od, outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream);
+    PLAIN(rc == 0);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// compose_mxfp(scales, elements, format, output code, shape of the tensor with its block axis last) -> tensor of that shape
+PyObject* compose_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 5);
+    const at::Tensor *const scales = gpu_tensor(a[0]), *const elements = gpu_tensor(a[1]);
+    long f[5];
+    PLAIN(scales && elements && dense(*scales) && dense(*elements) && ints(a[2], f) && PyTuple_Check(a[4]));
+    const int od = out_code(a[3], *elements);
+    const int64_t n = elements->numel(), B = f[0];
+    PLAIN(od >= 0 && n > 0 && B > 0 && n % B == 0 && scales->numel() == n / B && scales->scalar_type() == at::kByte && elements->scalar_type() == at::kByte &&
+          scales->device() == elements->device());
+    c10::SmallVector<int64_t, 6> shape;
+    int64_t total = 1;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[4]); ++i) {
+        const long d = PyLong_AsLong(PyTuple_GET_ITEM(a[4], i));
+        if (PyErr_Occurred()) PyErr_Clear();
+        PLAIN(d > 0);
+        shape.push_back(d);
+        PLAIN(!__builtin_mul_overflow(total, (int64_t)d, &total));
+    }
+    void* stream;
+    PLAIN(total == n && stream_of(*elements, &stream));
+    at::Tensor out = empty(shape, kDtypes[od], *elements);
+    PLAIN(mase_hip_compose_mxfp(scales->data_ptr<uint8_t>(), elements->data_ptr<uint8_t>(), out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], stream) == 0);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// minifloat(kind, x, format, output code or None): kind 0 extract (uint16 codes), 1 compose (x: codes), 2 quantise-dequantise
+PyObject* minifloat(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 4);
+    const long kind = PyLong_AsLong(a[0]);
+    if (PyErr_Occurred()) PyErr_Clear();
+    const at::Tensor* const x = gpu_tensor(a[1]);
+    long f[4];
+    PLAIN(x && dense(*x) && ints(a[2], f));
+    const int dt = dtype_code(x->scalar_type()), od = kind == 0 ? 0 : out_code(a[3], *x);
+    const int64_t n = x->numel();
+    void* stream;
+    PLAIN(kind >= 0 && kind <= 2 && n > 0 && od >= 0 && (kind == 1 ? x->scalar_type() == at::kUInt16 : dt >= 0) && stream_of(*x, &stream));
+    at::Tensor out = empty(x->sizes(), kind == 0 ? at::kUInt16 : kDtypes[od], *x);
+    const int E = (int)f[0], M = (int)f[1], fin = (int)f[2], rm = (int)f[3];
+    const int rc = kind == 0   ? mase_hip_extract_minifloat(x->data_ptr(), dt, static_cast<uint16_t*>(out.data_ptr()), n, E, M, fin, rm, stream)
+                   : kind == 1 ? mase_hip_compose_minifloat(static_cast<const uint16_t*>(x->data_ptr()), out.data_ptr(), od, n, E, M, fin, stream)
+                               : mase_hip_qdq_minifloat(x->data_ptr(), dt, out.data_ptr(), od, n, E, M, fin, rm, stream);
+    PLAIN(rc == 0);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// linear_scaled(x [.., K] bf16, exp_bits, frac_bits, minifloat, w_codes, w_scales, N, bias or None) -> [.., N]
+PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 8);
+    const at::Tensor *const x = gpu_tensor(a[0]), *const codes = gpu_tensor(a[4]), *const w_sc = gpu_tensor(a[5]);
+    PLAIN(x && codes && w_sc && dense(*x) && x->dim() > 0 && x->scalar_type() == at::kBFloat16 && codes->device() == x->device() && w_sc->device() == x->device());
+    PLAIN(codes->is_contiguous() && w_sc->is_contiguous() && codes->scalar_type() == at::kByte && w_sc->scalar_type() == at::kInt && codes->dim() == 2);
+    const long e = PyLong_AsLong(a[1]), m = PyLong_AsLong(a[2]), mini = PyLong_AsLong(a[3]), N = PyLong_AsLong(a[6]);
+    if (PyErr_Occurred()) PyErr_Clear();
+    const int64_t K = x->size(-1), M = K > 0 ? x->numel() / K : 0;
+    PLAIN(M > 0 && N > 0 && codes->size(1) == K && codes->size(0) >= N && w_sc->numel() >= K / 128 * codes->size(0));
+    const void* b_ptr = nullptr;
+    int b_dt = 0;
+    if (a[7] != Py_None) {
+        const at::Tensor* const b = THPVariable_Check(a[7]) ? &THPVariable_Unpack(a[7]) : nullptr;
+        PLAIN(b && b->is_cuda() && b->device() == x->device() && b->unsafeGetTensorImpl()->has_storage() && b->is_contiguous() && b->numel() == N);
+        b_dt = dtype_code(b->scalar_type());
+        PLAIN(b_dt >= 0);
+        b_ptr = b->data_ptr();
+    }
+    void* stream;
+    PLAIN(stream_of(*x, &stream));
+    const int64_t bytes = mase_hip_mxfp_linear_scaled_scratch_bytes(M, N, K);
+    PLAIN(bytes > 0);
+    at::Tensor scratch = empty({bytes}, at::kByte, *x);
+    c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
+    shape.back() = N;
+    at::Tensor y = empty(shape, at::kBFloat16, *x);
+    PLAIN(mase_hip_mxfp_linear_scaled(x->data_ptr(), 2, (int)e, (int)m, (int)mini, codes->data_ptr<uint8_t>(), reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>()), b_ptr, b_dt,
+                                      y.data_ptr(), 2, M, N, K, scratch.data_ptr(), bytes, stream) == 0);
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+// scores(left [.., M, K], right [.., K, N], format of left, the same of right, panels x K up to which right is quantised inside): left @ right where
+// both are bf16 with the same leading axes, quantised in one format, and right is the transposed view of a contiguous tensor
+PyObject* scores(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+    HANDLE_TH_ERRORS
+    PLAIN(n_args == 4);
+    const at::Tensor *const l = gpu_tensor(a[0]), *const r = gpu_tensor(a[1]);
+    long f[5];
+    PLAIN(l && r && ints(a[2], f) && f[0] == 32 && f[3] == 1 && f[4] == 0);
+    const int64_t nd = l->dim();
+    PLAIN(nd >= 2 && r->dim() == nd && l->scalar_type() == at::kBFloat16 && r->scalar_type() == at::kBFloat16 && l->device() == r->device() && dense(*l) &&
+          reinterpret_cast<uintptr_t>(r->data_ptr()) % 16 == 0);
+    const int64_t M = l->size(-2), K = l->size(-1), N = r->size(-1);
+    PLAIN(r->size(-2) == K && K > 0 && K <= 128 && K % 32 == 0 && N > 0 && N % 8 == 0 && N <= (1 << 23) && M > 0 && l->numel() > 0);
+    PLAIN(r->stride(-2) == 1 && (r->stride(-1) == K || N == 1));
+    int64_t batches = 1;
+    for (int64_t i = nd - 3; i >= 0; --i) {
+        PLAIN(l->size(i) == r->size(i) && (l->size(i) == 1 || r->stride(i) == batches * N * K));
+        batches *= l->size(i);
+    }
+    const long inside = PyLong_AsLong(a[3]);
+    if (PyErr_Occurred()) PyErr_Clear();
+    void* stream;
+    PLAIN(stream_of(*l, &stream));
+    const bool quantise_w = (M + 127) / 128 * K <= inside;
+    at::Tensor w;
+    if (!quantise_w) {
+        w = empty({batches * N * K}, at::kBFloat16, *l);
+        PLAIN(mase_hip_qdq_mxfp(r->data_ptr(), 2, w.data_ptr(), 2, batches * N * K, 32, (int)f[1], (int)f[2], 1, 0, stream) == 0);
+    }
+    c10::SmallVector<int64_t, 6> shape(l->sizes().begin(), l->sizes().end());
+    shape.back() = N;
+    at::Tensor y = empty(shape, at::kBFloat16, *l);
+    PLAIN(mase_hip_mxfp_scores(l->data_ptr(), (int)f[1], (int)f[2], quantise_w ? r->data_ptr() : w.data_ptr(), quantise_w, y.data_ptr(), M, N, K, batches, M * K, N * K, M * N,
+                               stream) == 0);
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
+}
+
+#define FN(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(name)), METH_FASTCALL, nullptr}
+PyMethodDef kMethods[] = {FN(extract_mxfp), FN(qdq_mxfp), FN(compose_mxfp), FN(minifloat), FN(linear_scaled), FN(scores), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_mase_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__mase_host(void) {
+    PyObject* const c = PyImport_ImportModule("torch._C");
+    if (!c) return nullptr;
+    g_raw_stream = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");
+    Py_DECREF(c);
+    if (!g_raw_stream) return nullptr;
+    return PyModule_Create(&kModule);
+}

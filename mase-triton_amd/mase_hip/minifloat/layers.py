@@ -7,6 +7,7 @@ from typing import Literal
 import torch
 from torch import Tensor, nn
 
+from .. import _lib
 from ..utils.qlayer import ChangeDtypeError
 from . import functional as MinifloatF
 from .meta import MinifloatMeta, MinifloatTensorMeta
@@ -139,8 +140,20 @@ class MinifloatLinearPTQ(nn.Module):
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_minifloat_meta)
 
-    @torch.no_grad()
     def forward(self, input: Tensor) -> Tensor:
+        # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
+        if self._fast_sig is not None and self._fast_sig == self._call_signature(input):
+            w, op = self._parameters["w_element"], self._scaled_w
+            if self._scaled_w_key == (w.data_ptr(), w._version, w.device):
+                xm = self.x_minifloat_meta
+                y = _lib.host().linear_scaled(input, xm.exp_bits, xm.frac_bits, 1, op.codes, op.scales, self.out_features,
+                                              None if self.layer_type.endswith("Bq") else self.bias)
+                if y is not None:
+                    return y
+        return self._forward(input)
+
+    @torch.no_grad()
+    def _forward(self, input: Tensor) -> Tensor:
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the codes
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.

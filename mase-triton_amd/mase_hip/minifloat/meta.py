@@ -12,6 +12,7 @@ from typing import Literal
 
 import torch
 
+from ..dtype import ROUND_MODE_TO_CODE
 from ..utils.meta import device_str, dtype_str, shape_tuple
 
 
@@ -27,6 +28,11 @@ class MinifloatMeta:
         assert self.exp_bits > 0
         assert self.frac_bits > 0
         assert self.exp_bits + self.frac_bits < 16  # codes travel as uint16
+
+    @functools.cached_property
+    def _codes(self) -> tuple[int, int, int, int]:
+        """The format in the numbers of the C ABI; an unknown round mode is -1."""
+        return self.exp_bits, self.frac_bits, int(self.is_finite), ROUND_MODE_TO_CODE.get(self.round_mode, -1)
 
     @property
     def _bias(self) -> int:

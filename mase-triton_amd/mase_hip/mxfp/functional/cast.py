@@ -4,7 +4,9 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
-from ...utils.meta import device_str, dtype_str, shape_tuple
+from ... import _lib
+from ...dtype import TORCH_DTYPE_TO_CODE
+from ...utils.meta import shape_tuple
 from .. import kernels
 from ..helpers import flatten_for_quantize, permute_for_dequantize
 from ..meta import MXFPMeta, MXFPTensorMeta
@@ -19,9 +21,10 @@ def extract_mxfp_components(tensor: Tensor, block_dim: int, mxfp_meta: MXFPMeta)
     """
     ndim = tensor.ndim
     assert -ndim <= block_dim < ndim
-    tensor_meta = MXFPTensorMeta(
-        device=device_str(tensor.device), dtype=dtype_str(tensor.dtype), shape=shape_tuple(tensor.shape),
-        block_dim=block_dim, meta=mxfp_meta)
+    tensor_meta = MXFPTensorMeta.of(tensor, block_dim, mxfp_meta)
+    plain = _lib.host().extract_mxfp(tensor, block_dim, mxfp_meta._codes)
+    if plain is not None:
+        return plain[0], plain[1], tensor_meta
     if tensor.device.type == "cuda" and kernels.strided_blocks_supported(tensor_meta.shape, block_dim, mxfp_meta):
         # blocks along an inner axis are read in place: same outputs as the permuted copy below
         scales, elements = kernels.extract_mxfp_components_strided(tensor, block_dim, mxfp_meta)
@@ -39,9 +42,14 @@ def compose_mxfp_tensor(scales: Tensor, elements: Tensor, tensor_meta: MXFPTenso
     """Dequantise to the original shape; ``output_dtype`` defaults to the recorded dtype."""
     if output_dtype is None:
         output_dtype = getattr(torch, tensor_meta.dtype)
+    shape, block_dim = tensor_meta.shape, tensor_meta.block_dim
+    if block_dim in (-1, len(shape) - 1):
+        plain = _lib.host().compose_mxfp(scales, elements, tensor_meta.meta._codes, TORCH_DTYPE_TO_CODE.get(output_dtype, -1), shape)
+        if plain is not None:
+            return plain
     flat = kernels.compose_mxfp_tensor(scales=scales, elements=elements, mxfp_meta=tensor_meta.meta,
                                        output_dtype=output_dtype)
-    return permute_for_dequantize(flat, ori_shape=tensor_meta.shape, block_dim=tensor_meta.block_dim)
+    return permute_for_dequantize(flat, ori_shape=shape, block_dim=block_dim)
 
 
 def quantize_dequantize(tensor: Tensor, block_dim: int, mxfp_meta: MXFPMeta,
@@ -50,6 +58,9 @@ def quantize_dequantize(tensor: Tensor, block_dim: int, mxfp_meta: MXFPMeta,
     one fused kernel without materialising scales or elements."""
     ndim = tensor.ndim
     assert -ndim <= block_dim < ndim
+    plain = _lib.host().qdq_mxfp(tensor, block_dim, mxfp_meta._codes, None if output_dtype is None else TORCH_DTYPE_TO_CODE.get(output_dtype, -1))
+    if plain is not None:
+        return plain
     if output_dtype is None:
         output_dtype = tensor.dtype
     if tensor.device.type == "cuda" and kernels.strided_blocks_supported(shape_tuple(tensor.shape), block_dim, mxfp_meta):

@@ -21,6 +21,7 @@ from typing import Literal
 import torch
 from torch import Tensor
 
+from ... import _lib
 from .. import kernels
 from ..meta import MXFPMeta
 from .cast import compose_mxfp_tensor, extract_mxfp_components, quantize_dequantize
@@ -177,6 +178,10 @@ def mxfp_matmul(
         assert input_meta is not None
     if quantised_other:
         assert other_meta is not None
+    if fused and quantised_input and quantised_other and (input_meta is other_meta or input_meta == other_meta):
+        plain = _lib.host().scores(input, other, other_meta._codes, SCORES_QUANTISE_W_UP_TO)     # queries and keys, as a model has them
+        if plain is not None:
+            return plain
     if fused and quantised_other and _gemm_route(input, other, quantised_input, other_meta):
         return _matmul_through_gemm(input, other, input_meta if quantised_input else None, other_meta)
     if quantised_input:

@@ -10,6 +10,7 @@ import functools
 from dataclasses import dataclass
 from typing import Literal
 
+from ..dtype import ROUND_MODE_TO_CODE
 from ..minifloat.meta import MinifloatMeta
 from ..utils.meta import device_str, dtype_str, shape_tuple
 
@@ -36,6 +37,12 @@ class MXFPMeta:
             f"Legal values are: {LEGAL_ELEMENT_EXP_FRAC_BITS}.")
 
     @functools.cached_property
+    def _codes(self) -> tuple[int, int, int, int, int]:
+        """The format in the numbers of the C ABI; an unknown round mode is -1."""
+        return (self.block_size, self.element_exp_bits, self.element_frac_bits, int(self.element_is_finite),
+                ROUND_MODE_TO_CODE.get(self.round_mode, -1))
+
+    @functools.cached_property
     def element_meta(self) -> MinifloatMeta:
         """The minifloat format of one element."""
         return MinifloatMeta(exp_bits=self.element_exp_bits, frac_bits=self.element_frac_bits,
@@ -56,6 +63,13 @@ class MXFPTensorMeta:
         object.__setattr__(self, "device", device_str(self.device))
         object.__setattr__(self, "dtype", dtype_str(self.dtype))
         object.__setattr__(self, "shape", shape_tuple(self.shape))
+
+    @classmethod
+    def of(cls, tensor, block_dim: int, meta: MXFPMeta) -> "MXFPTensorMeta":
+        """The meta of ``tensor`` (what the constructor makes of its device, dtype and shape, without the frozen class's setters)."""
+        self = object.__new__(cls)
+        self.__dict__.update(device=device_str(tensor.device), dtype=dtype_str(tensor.dtype), shape=tuple(tensor.shape), block_dim=block_dim, meta=meta)
+        return self
 
     def create(self, device=None, dtype=None, shape=None, block_dim: int | None = None,
                meta: MXFPMeta | None = None) -> "MXFPTensorMeta":
