@@ -97,6 +97,17 @@ inline bool strided_column_tiles(int64_t columns, int64_t nkb, int element_bytes
     return tiles * groups < 2048 || nkb * 8 > groups * 4 * 5;
 }
 
+// The same for the kernel that takes two columns of 16-bit elements to a lane, 128 columns and four k-blocks to a workgroup.  bf16, against the
+// kernel that stores a column's codes by itself, us: 2976 x 4096 11.2 / 12.6, 65536 x 200 12.5 / 15.6, 1024 x 2050 4.8 / 6.1; tiles that the columns or k-blocks
+// leave half empty cost once there are many: 160 x 65536 (five k-blocks) 13.5 / 10.8, 32 x 262144 level without it.  fp16, against one column to a lane:
+// 2976 x 4096 12.5 / 14.7, 65536 x 200 13.6 / 17.5, 256 x 9000 5.2 / 6.0; with fewer wavefronts the other kernel's shorter lanes are ahead: 96 x 14336 4.9 / 4.5,
+// 64 x 1000 4.6 / 4.2.
+inline bool strided_pair_tiles(int64_t columns, int64_t nkb, bool bf16) {
+    const int64_t tiles = (columns + 127) / 128, groups = (nkb + 3) / 4, waves = tiles * groups * 4;
+    const bool filled = columns * nkb * 10 >= tiles * 128 * groups * 4 * 7;
+    return bf16 ? filled || waves < 2048 : filled && waves >= 512;
+}
+
 // Calls fn(format object): a compile-time format for the five round-to-nearest finite
 // presets, the run-time one otherwise.
 template <class Fn>
