@@ -290,18 +290,29 @@ __device__ inline uint32_t block_max(uint32_t amax, int lpb) {
 // Scale byte and codes of N elements of one block whose largest |x| has bits `amax` (the block's lanes agree on it).  A compile-time
 // format takes the branch-free encoder unless some block of the wavefront is out of its range (a uniform test): with the general
 // routine the vector instructions and not the memory bound the casts (4096 x 4096, blocks along the rows: fp16 extract 22.4 -> 15.1 us,
-// fused pass 29.8 -> 17.3, fp32 extract 18.4 -> 16.9; fused pass of [2976, 4096] down the rows: fp16 33.2 -> 15.0, fp32 20.5 -> 17.5).
+// fused pass 29.8 -> 17.3, fp32 extract 18.4 -> 16.9; fused pass of [2976, 4096] down the rows: fp16 33.2 -> 15.0, fp32 20.5 -> 17.5).  A block
+// that holds inf or NaN has scale 255, the NaN code where they are and 0 elsewhere: set behind a uniform test (the general routine
+// for all elements of such a wavefront was the last thing a launch waited for).
 template <int DT_IN, class F, int N>
 __device__ inline void mxfp_encode(const uint32_t (&u)[N], uint32_t amax, const F& f, uint32_t (&code)[N], uint32_t& scale) {
     if constexpr (F::kStatic) {
         const int top = DT_IN != F32 ? (int)(amax >> 23) : floor_log2_fp32(amax) + 127;
         const int sc = amax < 0x00800000u ? 0 : max(top - fmt_emax_unb(f), 0);   // largest |x| flushed: scale 0, every code 0
-        const bool hard = amax >= 0x7F800000u || sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f));
+        const bool nonfinite = amax >= 0x7F800000u;
+        const bool hard = !nonfinite && (sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f)));
         if (__builtin_amdgcn_ballot_w64(hard) == 0) {
             const uint32_t off = (uint32_t)max(sc - fmt_bias(f), 0) << 15;
-            scale = (uint32_t)sc;
+            scale = nonfinite ? 255u : (uint32_t)sc;
 #pragma unroll
             for (int j = 0; j < N; ++j) code[j] = encode_mxfp_in_range<F>(u[j], off);
+            if (__builtin_amdgcn_ballot_w64(nonfinite) != 0) {
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    const bool e = (u[j] & 0x7FFFFFFFu) >= 0x7F800000u;
+                    if (nonfinite) code[j] = 0u;
+                    if (__builtin_amdgcn_ballot_w64(e) != 0 && e) code[j] = encode_nonfinite(false, true, u[j] & 0x7FFFFFu, f);
+                }
+            }
             return;
         }
     }
@@ -767,6 +778,25 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_kernel(const void* x, u
 // 16-bit half.  Needs inner % 2 == 0 and 4-byte aligned x / out.
 // One block of 32 rows for the lane's two columns, read at x + first (+ j * inner).  res[j]: MODE 0 the two codes
 // of row j (low byte of each 16-bit half), MODE 1 the two bf16 results; scale[t]: the scale byte of column t.
+// Codes of the blocks of inf / NaN among a lane's two columns (halves in `poisoned`): scale 255, the NaN code where an element is inf / NaN
+// itself and 0 elsewhere.  bits(j, c): fp32 bits of row j, column c.  (The general routine for all 64 elements of such a lane was what
+// a launch waited for last: 2976 x 4096 fp16 with one inf 19.6 us, without 12.4.)
+template <class F, class Bits>
+__device__ inline void set_poisoned_blocks(uint32_t poisoned, uint32_t (&scale)[2], uint32_t (&res)[32], Bits&& bits, const F& f) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) scale[c] = (poisoned >> (16 * c)) & 1u ? 255u : scale[c];
+#pragma unroll
+    for (int j = 0; j < 32; ++j) {
+        res[j] &= ~poisoned;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const uint32_t u = bits(j, c);
+            const bool e = (u & 0x7FFFFFFFu) >= 0x7F800000u;
+            if (__builtin_amdgcn_ballot_w64(e) != 0 && e) res[j] |= encode_nonfinite(false, true, u & 0x7FFFFFu, f) << (16 * c);
+        }
+    }
+}
+
 template <class F, int MODE>
 __device__ inline void strided_bf16_block(const uint16_t* x, int64_t first, int64_t inner, const F& f, uint32_t (&res)[32],
                                           uint32_t (&scale)[2]) {
@@ -777,13 +807,14 @@ __device__ inline void strided_bf16_block(const uint16_t* x, int64_t first, int6
         h[j] = *reinterpret_cast<const uint32_t*>(x + first + j * inner);
         m = __builtin_elementwise_max(m, as_u16x2(h[j] & 0x7FFF7FFFu));
     }
-    uint32_t amax[2];
+    uint32_t amax[2], poisoned = 0;                        // `poisoned`: the halves whose block holds inf / NaN
     bool hard = false;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         amax[c] = m[c];
         const int scale_n = max((int)(amax[c] >> 7) - fmt_emax_unb(f), 0);  // amax == 0 gives 0: the all-flushed rule
-        hard |= amax[c] >= 0x7F80u || scale_n >= 151 || (amax[c] != 0u && scale_n < fmt_bias(f) + (MODE == 1 ? 1 : 0));
+        hard |= (MODE == 1 || amax[c] < 0x7F80u) && (amax[c] >= 0x7F80u || scale_n >= 151 || (amax[c] != 0u && scale_n < fmt_bias(f) + (MODE == 1 ? 1 : 0)));
+        poisoned |= MODE == 0 && amax[c] >= 0x7F80u ? 0xFFFFu << (16 * c) : 0u;
         scale[c] = (uint32_t)scale_n;
     }
     if (__builtin_amdgcn_ballot_w64(hard) == 0) {
@@ -792,6 +823,8 @@ __device__ inline void strided_bf16_block(const uint16_t* x, int64_t first, int6
         const uint32_t ssb2 = lo | (hi << 16);
 #pragma unroll
         for (int j = 0; j < 32; ++j) res[j] = MODE == 0 ? PackedBf16<F>::codes(h[j], ssb2) : PackedBf16<F>::qdq(h[j], ssb2);
+        if (MODE == 0 && __builtin_amdgcn_ballot_w64(poisoned != 0u) != 0)
+            set_poisoned_blocks(poisoned, scale, res, [&](int j, int c) { return ((h[j] >> (16 * c)) & 0xFFFFu) << 16; }, f);
     } else {
         // exact per-element routine
         int se[2];
@@ -1002,24 +1035,18 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_pair_kernel(const uint1
                 amax[c] = half_bits_to_f32_bits(m[c]);
                 scale[c] = (uint32_t)max((int)(amax[c] >> 23) - fmt_emax_unb(f), 0);   // nothing but zeros: 0, every code 0
             }
+            const uint32_t poisoned = (m[0] >= 0x7C00u ? 0xFFFFu : 0u) | (m[1] >= 0x7C00u ? 0xFFFF0000u : 0u);
             // (a scale of fp16 values lies between bias and 150)
-            if (__builtin_amdgcn_ballot_w64(max((uint32_t)m[0], (uint32_t)m[1]) >= 0x7C00u) == 0) {
-                const uint32_t lo = ((uint32_t)max((int)scale[0] - fmt_bias(f), 0) << 7) & 0xFFFFu, hi = ((uint32_t)max((int)scale[1] - fmt_bias(f), 0) << 7) & 0xFFFFu;
-                const uint32_t ssb2 = lo | (hi << 16);
+            const uint32_t lo = ((uint32_t)max((int)scale[0] - fmt_bias(f), 0) << 7) & 0xFFFFu, hi = ((uint32_t)max((int)scale[1] - fmt_bias(f), 0) << 7) & 0xFFFFu;
+            const uint32_t ssb2 = lo | (hi << 16);
 #pragma unroll
-                for (int j = 0; j < 32; ++j) {
-                    const uint32_t u0 = half_bits_to_f32_bits(h[j] & 0xFFFFu), u1 = half_bits_to_f32_bits(h[j] >> 16);
-                    const uint32_t top = __builtin_amdgcn_perm(u1, u0, 0x07060302u), rest = __builtin_amdgcn_perm(u1, u0, 0x05040100u);
-                    res[j] = PackedBf16<F>::codes(top | PackedBf16<F>::pk_min_u16(rest, 0x00010001u), ssb2);
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < 2; ++c) scale[c] = amax[c] < 0x00800000u ? 0u : (uint32_t)(shared_exponent<F, true>(amax[c], f) + 127);
-                const int se0 = shared_exponent<F, true>(amax[0], f), se1 = shared_exponent<F, true>(amax[1], f);
-#pragma unroll
-                for (int j = 0; j < 32; ++j)
-                    res[j] = encode_mxfp_element(half_bits_to_f32_bits(h[j] & 0xFFFFu), se0, f) | (encode_mxfp_element(half_bits_to_f32_bits(h[j] >> 16), se1, f) << 16);
+            for (int j = 0; j < 32; ++j) {
+                const uint32_t u0 = half_bits_to_f32_bits(h[j] & 0xFFFFu), u1 = half_bits_to_f32_bits(h[j] >> 16);
+                const uint32_t top = __builtin_amdgcn_perm(u1, u0, 0x07060302u), rest = __builtin_amdgcn_perm(u1, u0, 0x05040100u);
+                res[j] = PackedBf16<F>::codes(top | PackedBf16<F>::pk_min_u16(rest, 0x00010001u), ssb2);
             }
+            if (__builtin_amdgcn_ballot_w64(poisoned != 0u) != 0)
+                set_poisoned_blocks(poisoned, scale, res, [&](int j, int c) { return half_bits_to_f32_bits((h[j] >> (16 * c)) & 0xFFFFu); }, f);
         }
         gather_column_codes(res, cd);
 #pragma unroll
