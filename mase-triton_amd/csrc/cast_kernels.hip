@@ -291,21 +291,22 @@ __device__ inline uint32_t block_max(uint32_t amax, int lpb) {
 // format takes the branch-free encoder unless some block of the wavefront is out of its range (a uniform test): with the general
 // routine the vector instructions and not the memory bound the casts (4096 x 4096, blocks along the rows: fp16 extract 22.4 -> 15.1 us,
 // fused pass 29.8 -> 17.3, fp32 extract 18.4 -> 16.9; fused pass of [2976, 4096] down the rows: fp16 33.2 -> 15.0, fp32 20.5 -> 17.5).  A block
-// that holds inf or NaN has scale 255, the NaN code where they are and 0 elsewhere: set behind a uniform test (the general routine
-// for all elements of such a wavefront was the last thing a launch waited for).
-template <int DT_IN, class F, int N>
+// that holds inf or NaN has scale 255, the NaN code where they are and 0 elsewhere: POISONED sets these behind a uniform test, where a lane
+// has a whole block of 32 (the general routine for such a wavefront was the last thing a launch waited for: extract of one inf
+// 7.6 -> 4.8 us); the fused pass down the rows keeps the general routine, with whose registers it is 8 % faster.
+template <int DT_IN, class F, int N, bool POISONED = false>
 __device__ inline void mxfp_encode(const uint32_t (&u)[N], uint32_t amax, const F& f, uint32_t (&code)[N], uint32_t& scale) {
     if constexpr (F::kStatic) {
         const int top = DT_IN != F32 ? (int)(amax >> 23) : floor_log2_fp32(amax) + 127;
         const int sc = amax < 0x00800000u ? 0 : max(top - fmt_emax_unb(f), 0);   // largest |x| flushed: scale 0, every code 0
-        const bool nonfinite = amax >= 0x7F800000u;
-        const bool hard = !nonfinite && (sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f)));
+        const bool nonfinite = POISONED && amax >= 0x7F800000u;
+        const bool hard = !nonfinite && (amax >= 0x7F800000u || sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f)));
         if (__builtin_amdgcn_ballot_w64(hard) == 0) {
             const uint32_t off = (uint32_t)max(sc - fmt_bias(f), 0) << 15;
             scale = nonfinite ? 255u : (uint32_t)sc;
 #pragma unroll
             for (int j = 0; j < N; ++j) code[j] = encode_mxfp_in_range<F>(u[j], off);
-            if (__builtin_amdgcn_ballot_w64(nonfinite) != 0) {
+            if (POISONED && __builtin_amdgcn_ballot_w64(nonfinite) != 0) {
 #pragma unroll
                 for (int j = 0; j < N; ++j) {
                     const bool e = (u[j] & 0x7FFFFFFFu) >= 0x7F800000u;
@@ -973,7 +974,7 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_tile_kernel(const void*
         for (int j = 0; j < 32; ++j) u[j] = load_bits_scalar<DT_IN>(x, first + j * inner);
 #pragma unroll
         for (int j = 0; j < 32; ++j) amax = max(amax, u[j] & 0x7FFFFFFFu);
-        mxfp_encode<DT_IN, F, 32>(u, amax, f, code, scale);
+        mxfp_encode<DT_IN, F, 32, true>(u, amax, f, code, scale);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             uint32_t w[4];
