@@ -107,7 +107,9 @@ extern "C" int mase_hip_mxfp_gemm_static_ws(const void* a_dense, int a_dtype, co
                                             int a_exp_bits, int a_frac_bits, const uint8_t* w_scales, const uint8_t* w_elements,
                                             int w_exp_bits, int w_frac_bits, const void* bias, int bias_dtype, void* y, int out_dtype,
                                             int64_t M, int64_t N, int64_t K, int block_size, void* stream) {
-    const int64_t need = mase_hip_mxfp_gemm_workspace_bytes(a_dense != nullptr, M, N, K);
+    // (ragged shapes are not split here: such calls have never used the array)
+    const bool ragged = M >= 1 && N >= 1 && K >= 1 && M <= 0x7FFFFFFF && N <= 0x7FFFFFFF && K <= 0x7FFFFFFF && ragged_shape((int)M, (int)N, (int)K);
+    const int64_t need = ragged ? 0 : mase_hip_mxfp_gemm_workspace_bytes(a_dense != nullptr, M, N, K);
     if (need > (int64_t)MASE_HIP_STATIC_WORKSPACE_BYTES)
         return fail(ERR_UNSUPPORTED, "this shape splits K into " + std::to_string(need) + " bytes of partial sums, more than the " +
                                          std::to_string((long long)MASE_HIP_STATIC_WORKSPACE_BYTES) +

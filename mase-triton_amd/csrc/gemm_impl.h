@@ -328,14 +328,6 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1,
     }  // tile loop
 }
 
-#include "gemm_tall.h"
-#include "gemm_skinny.h"
-#include "gemm_rows16.h"
-#include "gemm_mid.h"
-#include "gemm_wide.h"
-#include "gemm_split_k.h"
-#include "gemm_scaled.h"
-
 // ---------------------------------------------------------------------------------------------
 // Small-shape kernel: 128 x 128 x 32 tiles, single LDS buffer.  Used when the problem cannot
 // fill the chip with 256 x 256 tiles.
@@ -343,12 +335,13 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(1,
 constexpr int SBM = 128, SBN = 128, SBK = 32;
 constexpr int S_STRIDE = SBK + 8;  // bf16 elements per tile row: 80 bytes
 
-template <int A_MODE, class FA, class FW, int DT_OUT>
+template <int A_MODE, class FA, class FW, int DT_OUT, bool SPLIT>
 __global__ __launch_bounds__(kGemmThreads) void mxfp_gemm_small_kernel(
     const uint16_t* __restrict__ a_dense0, const uint8_t* __restrict__ a_scales, const uint8_t* __restrict__ a_elements,
     const uint8_t* __restrict__ w_scales0, const uint8_t* __restrict__ w_elements0, const void* __restrict__ bias,
-    int bias_dtype, void* __restrict__ y0, int M, int N, int K, GemmBatch gb) {
-    // batched launches: workgroups of grid plane z work on product z (offsets are zero for a single product)
+    int bias_dtype, void* __restrict__ y0, int M, int N, int K, int steps_per, GemmBatch gb) {
+    // batched launches: workgroups of grid plane z work on product z (offsets are zero for a single product); K split (SPLIT):
+    // on steps z * steps_per .. of the product, into plane z of the sums
     const uint16_t* __restrict__ const a_dense = a_dense0 + (int64_t)blockIdx.z * gb.a;
     const uint8_t* __restrict__ const w_scales = w_scales0 + (int64_t)blockIdx.z * gb.ws;
     const uint8_t* __restrict__ const w_elements = w_elements0 + (int64_t)blockIdx.z * gb.we;
@@ -393,9 +386,10 @@ __global__ __launch_bounds__(kGemmThreads) void mxfp_gemm_small_kernel(
         }
     };
 
-    const int ktiles = K / SBK;
-    fetch(0);
-    for (int kt = 0; kt < ktiles; ++kt) {
+    const int kt0 = SPLIT ? (int)blockIdx.z * steps_per : 0;
+    const int ktiles = SPLIT ? min(kt0 + steps_per, K / SBK) : K / SBK;
+    fetch(kt0);
+    for (int kt = kt0; kt < ktiles; ++kt) {
         __syncthreads();  // everyone finished reading the previous slab
         {
             uint4 lo, hi;
@@ -440,6 +434,14 @@ __global__ __launch_bounds__(kGemmThreads) void mxfp_gemm_small_kernel(
             }
         }
 }
+
+#include "gemm_tall.h"
+#include "gemm_skinny.h"
+#include "gemm_rows16.h"
+#include "gemm_mid.h"
+#include "gemm_wide.h"
+#include "gemm_split_k.h"
+#include "gemm_scaled.h"
 
 template <int A_MODE, class FA, class FW, int DT_OUT>
 int launch_gemm(const void* a_dense, const uint8_t* a_scales, const uint8_t* a_elements, const uint8_t* w_scales,
@@ -536,9 +538,9 @@ int launch_gemm(const void* a_dense, const uint8_t* a_scales, const uint8_t* a_e
     } else {
         const dim3 grid((unsigned)((N + SBN - 1) / SBN), (unsigned)((M + SBM - 1) / SBM), (unsigned)batches);
         if (grid.y > 65535u) return fail(ERR_UNSUPPORTED, "M too large for the launch grid");
-        hipLaunchKernelGGL((mxfp_gemm_small_kernel<A_MODE, FA, FW, DT_OUT>), grid, dim3(kGemmThreads), 0, s,
+        hipLaunchKernelGGL((mxfp_gemm_small_kernel<A_MODE, FA, FW, DT_OUT, false>), grid, dim3(kGemmThreads), 0, s,
                            static_cast<const uint16_t*>(a_dense), a_scales, a_elements, w_scales, w_elements, bias, bias_dtype, y, M,
-                           N, K, gb);
+                           N, K, 0, gb);
     }
     return check_launch("mxfp_gemm");
 }

@@ -7,8 +7,10 @@
 struct SplitPlan {
     int splits;  // 1: do not split
     int k_len;   // k per split, a multiple of 128
-    int kind;    // 0: 128 x 128 tiles, 1: 256 x 128 tiles, 2: 512 x 128 tiles
-    int64_t workspace_bytes(int M, int N) const { return splits > 1 ? (int64_t)splits * M * N * 4 : 0; }
+    int kind;    // 0: 128 x 128 tiles, 1: 256 x 128 tiles, 2: 512 x 128 tiles, 3: 128 x 128 tiles of any shape (mxfp_gemm_small_kernel)
+    // (any shape: the arrays lie a multiple of four sums apart)
+    int64_t sums(int M, int N) const { return kind == 3 ? ((int64_t)M * N + 3) / 4 * 4 : (int64_t)M * N; }
+    int64_t workspace_bytes(int M, int N) const { return splits > 1 ? splits * sums(M, N) * 4 : 0; }
 };
 
 // Estimated time of one 128-k macro step of a 128 x 128 tile, in us, by the share of the CUs that have a workgroup
@@ -20,6 +22,35 @@ inline double split_step_us(int64_t wgs, int cus) {
     return 1.1 + 0.5 * (share - 0.25) / 0.75;
 }
 
+// Products that none of the tile kernels with K in whole macro steps takes (N or K ragged) and that are too small for 256 x 256 tiles go to
+// the 128 x 128 x 32 single-buffer kernel (launch_gemm).  A step of that kernel is the latency of its loads, 0.8 us, whatever else the CU does,
+// so it wants several workgroups on a CU as well as shares of K.  Unsplit and now, us: 79 x 1673 x 3040 (M x N x K) 53 / 25, 316 x 699 x 7488 171 / 32,
+// 120 x 4080 x 6848 155 / 33, 1 x 8001 x 8160 172 / 45, 700 x 1000 x 4096 98 / 32, 120 x 501 x 800 20.9 / 15.5; a split is taken where it is priced 15 % below
+// the whole product (700 x 1029 x 512: 18.7 unsplit, 20.6 in shares).  The sums are kept within 32 MB.
+inline bool ragged_shape(int M, int N, int K) {
+    if (K % 32 != 0 || K < 256 || (int64_t)M * N >= (int64_t)4096 * 4096) return false;
+    if ((int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 128) return false;
+    if (M <= 64 && N % 16 == 0 && N <= (M <= 16 ? 12288 : 8192) && K % 128 == 0) return false;
+    if (M <= 128 && N % 32 == 0 && K % 128 == 0) return false;
+    return !(M > 128 && N % 128 == 0 && K % 64 == 0);
+}
+inline SplitPlan plan_split_ragged(int M, int N, int K, int cus) {
+    SplitPlan p{1, K, 3};
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const int steps = K / 32;
+    const double mn_mb = (double)M * N * 4.0 / 1e6;
+    double best = 1e30;
+    for (int want = 1; want <= 16; ++want) {
+        const int per = (steps + want - 1) / want;
+        if (want > 1 && (per < 4 || (steps + per - 1) / per != want || want * mn_mb > 33.0)) continue;
+        const int64_t per_cu = (tiles * want + cus - 1) / cus;
+        const double together = (double)std::min<int64_t>(per_cu, 4);
+        const double t = (double)((per_cu + 3) / 4) * per * 0.8 * (1.0 + 0.3 * (together - 1.0)) + (want > 1 ? 4.0 + (2.0 * want + 0.5) * mn_mb * 0.21 : 0.0);
+        if (t < (want > 1 ? best : 1e30)) { best = want > 1 ? t : 0.85 * t; p.splits = want; p.k_len = per * 32; }
+    }
+    return p;
+}
+
 // The same plan for the size query and the launch: it depends on the shape and the CU count only.  Every candidate
 // (tile kind, number of splits) is priced as rounds x macro steps per split x step time x (1.0 / 1.4 / 2.05 for 128 / 256 /
 // 512-row tiles), plus, when split, 4 us for the second launch and the partial sums written and read once at 4.7 TB/s
@@ -27,6 +58,7 @@ inline double split_step_us(int64_t wgs, int cus) {
 // an unsplit one the plan says so.
 inline SplitPlan plan_split_k(int M, int N, int K, int cus, bool allow_tall = true) {
     SplitPlan p{1, K, 0};
+    if (cus > 0 && ragged_shape(M, N, K)) return plan_split_ragged(M, N, K, cus);
     // up to 64 rows the weight-streaming kernels are as fast or faster (64 x 4096 x 4096: 14.5 us against 20.4 us split)
     if (M <= 64 || N % 128 != 0 || K % 128 != 0 || cus <= 0) return p;
     const int nmac = K / 128;
@@ -90,10 +122,40 @@ __global__ __launch_bounds__(256) void split_k_reduce_kernel(const float* __rest
     store_out4<DT_OUT>(y, o, r, (reinterpret_cast<uintptr_t>(y) & 15) == 0, 4);
 }
 
+// the same for any M and N: `pitch` sums (a multiple of four) from one split's array to the next
+template <int DT_OUT>
+__global__ __launch_bounds__(256) void split_k_reduce_any_kernel(const float* __restrict__ partial, int splits, int64_t mn, int64_t pitch, int N,
+                                                                 const void* __restrict__ bias, int bias_dtype, void* __restrict__ y) {
+    const int64_t o = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (o >= mn) return;
+    float4 acc = *reinterpret_cast<const float4*>(partial + o);
+    for (int z = 1; z < splits; ++z) {
+        const float4 v = *reinterpret_cast<const float4*>(partial + (size_t)z * pitch + o);
+        acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+    }
+    float r[4] = {acc.x, acc.y, acc.z, acc.w};
+    const int valid = (int)min((int64_t)4, mn - o);
+    if (bias)
+        for (int t = 0; t < valid; ++t) r[t] += load_bias(bias, bias_dtype, (int)((o + t) % N));
+    store_out4<DT_OUT>(y, o, r, (reinterpret_cast<uintptr_t>(y) & 15) == 0, valid);
+}
+
 template <class FW, int DT_OUT>
 int launch_gemm_split_k(const void* a_dense, const uint8_t* w_scales, const uint8_t* w_elements, const void* bias, int bias_dtype,
                         void* y, int M, int N, int K, const SplitPlan& plan, void* workspace, hipStream_t s) {
     const int64_t mn = (int64_t)M * N;
+    if (plan.kind == 3) {
+        const int64_t pitch = plan.sums(M, N);
+        const dim3 grid((unsigned)((N + SBN - 1) / SBN), (unsigned)((M + SBM - 1) / SBM), (unsigned)plan.splits);
+        if (grid.y > 65535u) return fail(ERR_UNSUPPORTED, "M too large for the launch grid");
+        hipLaunchKernelGGL((mxfp_gemm_small_kernel<0, SFmt<4, 3>, FW, F32, true>), grid, dim3(kGemmThreads), 0, s, static_cast<const uint16_t*>(a_dense),
+                           static_cast<const uint8_t*>(nullptr), static_cast<const uint8_t*>(nullptr), w_scales, w_elements, static_cast<const void*>(nullptr), 0,
+                           workspace, M, N, K, plan.k_len / SBK, GemmBatch{0, 0, 0, pitch * 4});
+        if (int rc = check_launch("mxfp_gemm")) return rc;
+        hipLaunchKernelGGL(split_k_reduce_any_kernel<DT_OUT>, dim3((unsigned)((mn + 1023) / 1024)), dim3(256), 0, s, static_cast<const float*>(workspace), plan.splits,
+                           mn, pitch, N, bias, bias_dtype, y);
+        return check_launch("mxfp_gemm");
+    }
     if (plan.kind == 0) {
         auto kern = mxfp_gemm_mid_kernel<FW, F32, 2>;
         static std::atomic<uint64_t> lds_allowed{0};
