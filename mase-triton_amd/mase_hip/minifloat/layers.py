@@ -69,6 +69,7 @@ class MinifloatLinearPTQ(nn.Module):
         self.b_element = self.b_tensor_meta = None
         self._narrowed = self._narrowed_key = None
         self._scaled_w = self._scaled_w_key = None
+        self._no_operand_sig = None   # what the last call that had no use for the operand looked like
         self._fast_sig = None   # what the last call on the block-scaled route looked like (see forward)
 
         if "Wq" in layer_type:
@@ -142,7 +143,8 @@ class MinifloatLinearPTQ(nn.Module):
 
     def forward(self, input: Tensor) -> Tensor:
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
-        if self._fast_sig is not None and self._fast_sig == self._call_signature(input):
+        sig = self._call_signature(input)
+        if self._fast_sig is not None and self._fast_sig == sig:
             w, op = self._parameters["w_element"], self._scaled_w
             if self._scaled_w_key == (w.data_ptr(), w._version, w.device):
                 xm = self.x_minifloat_meta
@@ -150,14 +152,14 @@ class MinifloatLinearPTQ(nn.Module):
                                               None if self.layer_type.endswith("Bq") else self.bias)
                 if y is not None:
                     return y
-        return self._forward(input)
+        return self._forward(input, sig)
 
     @torch.no_grad()
-    def _forward(self, input: Tensor) -> Tensor:
+    def _forward(self, input: Tensor, sig: tuple) -> Tensor:
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the codes
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._fast_sig is not None and self._fast_sig == self._call_signature(input):
+        if self._fast_sig is not None and self._fast_sig == sig:
             w = self.w_element
             if self._scaled_w_key == (w.data_ptr(), w._version, w.device):
                 from ..mxfp import kernels
@@ -170,8 +172,10 @@ class MinifloatLinearPTQ(nn.Module):
                 else:
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense_minifloat(x2, xm.exp_bits, xm.frac_bits), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
-        w_operand = self._weight_operand(input)
-        self._fast_sig = self._call_signature(input) if w_operand is not None else None
+        # (a call that looks like the last one that no kernel took the operand for is not asked about again)
+        w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
+        self._no_operand_sig = sig if w_operand is None else None
+        self._fast_sig = sig if w_operand is not None else None
         return MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,

@@ -70,6 +70,7 @@ class MXFPLinearPTQ(nn.Module):
         self.dtype, self.device = dtype, device
 
         self._scaled_w = self._scaled_w_key = None   # the weight in the block-scaled GEMM's form, and what it was built from
+        self._no_operand_sig = None                  # what the last call that had no use for it looked like
         self._fast_sig = None                        # what the last call on the block-scaled route looked like (see forward)
         self.weight = self.bias = None
         self.w_scales = self.w_elements = self.w_tensor_meta = None
@@ -155,7 +156,8 @@ class MXFPLinearPTQ(nn.Module):
 
     def forward(self, input: Tensor) -> Tensor:
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
-        if self._fast_sig is not None and self._fast_sig == self._call_signature(input):
+        sig = self._call_signature(input)
+        if self._fast_sig is not None and self._fast_sig == sig:
             params, w = self._parameters, self._scaled_w
             w_elements, w_scales = params["w_elements"], params["w_scales"]
             if self._scaled_w_key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
@@ -164,14 +166,14 @@ class MXFPLinearPTQ(nn.Module):
                                               None if self.layer_type.endswith("Bq") else self.bias)
                 if y is not None:
                     return y
-        return self._forward(input)
+        return self._forward(input, sig)
 
     @torch.no_grad()
-    def _forward(self, input: Tensor) -> Tensor:
+    def _forward(self, input: Tensor, sig: tuple) -> Tensor:
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the weight
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._fast_sig is not None and self._fast_sig == self._call_signature(input):
+        if self._fast_sig is not None and self._fast_sig == sig:
             w_elements, w_scales = self.w_elements, self.w_scales
             if self._scaled_w_key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
                 from . import kernels
@@ -184,8 +186,10 @@ class MXFPLinearPTQ(nn.Module):
                 else:
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense(x2, meta), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
-        w_operand = self._weight_operand(input)
-        self._fast_sig = self._call_signature(input) if w_operand is not None and self._takes_scaled_route(input) else None
+        # (a call that looks like the last one that no kernel took the operand for is not asked about again)
+        w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
+        self._no_operand_sig = sig if w_operand is None else None
+        self._fast_sig = sig if w_operand is not None and self._takes_scaled_route(input) else None
         return MXFP_F.mxfp_linear(
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
