@@ -26,6 +26,7 @@ class MinifloatLinearPTQ(nn.Module):
     in_features: int
     out_features: int
     _CODE_PARAMS = ("w_element", "b_element")
+    _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
     def __init__(
         self,
@@ -69,7 +70,6 @@ class MinifloatLinearPTQ(nn.Module):
         self.b_element = self.b_tensor_meta = None
         self._narrowed = self._narrowed_key = None
         self._scaled_w = self._scaled_w_key = None
-        self._no_operand_sig = None   # what the last call that had no use for the operand looked like
         self._fast_sig = None   # what the last call on the block-scaled route looked like (see forward)
 
         if "Wq" in layer_type:
@@ -94,7 +94,7 @@ class MinifloatLinearPTQ(nn.Module):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
         self._narrowed = self._narrowed_key = None
-        self._scaled_w = self._scaled_w_key = self._fast_sig = None
+        self._scaled_w = self._scaled_w_key = self._fast_sig = self._no_operand_sig = None
         for name, dt in before.items():
             now = getattr(self, name).dtype
             if now != dt:
@@ -145,8 +145,8 @@ class MinifloatLinearPTQ(nn.Module):
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
         sig = self._call_signature(input)
         if self._fast_sig is not None and self._fast_sig == sig:
-            w, op = self._parameters["w_element"], self._scaled_w
-            if self._scaled_w_key == (w.data_ptr(), w._version, w.device):
+            w, op = self._parameters.get("w_element"), self._scaled_w     # (none: held otherwise, by a parametrisation)
+            if w is not None and self._scaled_w_key == (w.data_ptr(), w._version, w.device):
                 xm = self.x_minifloat_meta
                 y = _lib.host().linear_scaled(input, xm.exp_bits, xm.frac_bits, 1, op.codes, op.scales, self.out_features,
                                               None if self.layer_type.endswith("Bq") else self.bias)
@@ -172,15 +172,17 @@ class MinifloatLinearPTQ(nn.Module):
                 else:
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense_minifloat(x2, xm.exp_bits, xm.frac_bits), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
-        # (a call that looks like the last one that no kernel took the operand for is not asked about again)
+        # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
         w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
-        self._no_operand_sig = sig if w_operand is None else None
+        self._no_operand_sig = None
         self._fast_sig = sig if w_operand is not None else None
-        return MinifloatF.minifloat_linear(
+        y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             _narrowed=self._narrowed_weight(), _w_operand=w_operand)
+        self._no_operand_sig = sig if w_operand is None else None
+        return y
 
     def extra_repr(self) -> str:
         return (f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}, "

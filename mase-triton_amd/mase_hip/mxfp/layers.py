@@ -30,6 +30,7 @@ class MXFPLinearPTQ(nn.Module):
     in_features: int
     out_features: int
     _CODE_PARAMS = ("w_scales", "w_elements", "b_scales", "b_elements")
+    _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
     def __init__(
         self,
@@ -70,7 +71,6 @@ class MXFPLinearPTQ(nn.Module):
         self.dtype, self.device = dtype, device
 
         self._scaled_w = self._scaled_w_key = None   # the weight in the block-scaled GEMM's form, and what it was built from
-        self._no_operand_sig = None                  # what the last call that had no use for it looked like
         self._fast_sig = None                        # what the last call on the block-scaled route looked like (see forward)
         self.weight = self.bias = None
         self.w_scales = self.w_elements = self.w_tensor_meta = None
@@ -101,6 +101,7 @@ class MXFPLinearPTQ(nn.Module):
     def _apply(self, fn, recurse=True):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
+        self._no_operand_sig = None
         for name, dt in before.items():
             now = getattr(self, name).dtype
             if now != dt:
@@ -115,7 +116,7 @@ class MXFPLinearPTQ(nn.Module):
         """Drop the cached block-scaled form of the weight.  Writes to ``w_scales`` / ``w_elements`` that torch records
         (``copy_`` under ``no_grad``, ``load_state_dict``, moving the module) are noticed without this call; writes
         through ``.data`` are not."""
-        self._scaled_w = self._scaled_w_key = self._fast_sig = None
+        self._scaled_w = self._scaled_w_key = self._fast_sig = self._no_operand_sig = None
 
     def _takes_scaled_route(self, input: Tensor) -> bool:
         """Does ``forward(input)`` run on the block-scaled GEMM?"""
@@ -159,8 +160,8 @@ class MXFPLinearPTQ(nn.Module):
         sig = self._call_signature(input)
         if self._fast_sig is not None and self._fast_sig == sig:
             params, w = self._parameters, self._scaled_w
-            w_elements, w_scales = params["w_elements"], params["w_scales"]
-            if self._scaled_w_key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
+            w_elements, w_scales = params.get("w_elements"), params.get("w_scales")     # (none: held otherwise, by a parametrisation)
+            if w_elements is not None and w_scales is not None and self._scaled_w_key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
                 meta = self.x_mxfp_meta
                 y = _lib.host().linear_scaled(input, meta.element_exp_bits, meta.element_frac_bits, 0, w.codes, w.scales, self.out_features,
                                               None if self.layer_type.endswith("Bq") else self.bias)
@@ -186,15 +187,17 @@ class MXFPLinearPTQ(nn.Module):
                 else:
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense(x2, meta), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
-        # (a call that looks like the last one that no kernel took the operand for is not asked about again)
+        # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
         w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
-        self._no_operand_sig = sig if w_operand is None else None
+        self._no_operand_sig = None
         self._fast_sig = sig if w_operand is not None and self._takes_scaled_route(input) else None
-        return MXFP_F.mxfp_linear(
+        y = MXFP_F.mxfp_linear(
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             w_operand=w_operand)
+        self._no_operand_sig = sig if w_operand is None else None
+        return y
 
     @torch.no_grad()
     def forward_swiglu(self, gate: Tensor, up: Tensor) -> Tensor:
