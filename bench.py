@@ -38,8 +38,9 @@ TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "hbm_counters_gemm_c4_c5_casts_
 CSRC = os.path.join(ROOT, "mase-triton_amd", "csrc")
 GEMM_SOURCES = ("gemm_tall.h", "gemm_impl.h", "mxfp_compose.h", "mase_device.h")
 SCALED_SOURCES = ("gemm_scaled.h", "gemm_tall.h", "mase_device.h")
-CAST_SOURCES = ("cast_kernels.hip", "swiglu.h", "mxfp_compose.h", "mase_device.h")
+CAST_SOURCES = ("cast_kernels.hip", "mxfp_bf16.h", "swiglu.h", "mxfp_compose.h", "mase_device.h")
 ROWS_SOURCES = ("gemm_scaled_rows.h", "mase_device.h")
+MID_SOURCES = ("gemm_scaled_mid.h", "mase_device.h")
 
 
 def sources_fingerprint(names) -> str:
@@ -445,7 +446,7 @@ def bench_hbm(torch, with_cpu):
     del xs, ys, cs
 
     # Decode-sized mxfp_linear is a read of W: C4's weight against the first 16 rows of C4's x, both as the operands a layer
-    # keeps / builds, on the block-scaled weight-streaming kernel; the weight rotates through seven copies (424 MB) so that
+    # keeps / builds, on the block-scaled kernels for few rows; the weight rotates through seven copies (424 MB) so that
     # none of it is served from the 256 MB memory-side cache.  The bf16 weight-streaming kernel on the same data beside it.
     from mase_hip.mxfp import kernels
     from mase_hip.mxfp.meta import MXFP8_E4M3_fn
@@ -458,7 +459,7 @@ def bench_hbm(torch, with_cpu):
     comps = [(w_sc, w_el)] + [(w_sc.clone(), w_el.clone()) for _ in range(6)]
     wops = [kernels.scaled_operand_from_mxfp(sc, el, MXFP8_E4M3_fn, N, K) for sc, el in comps]
     w_bytes = N * K * (1 + 1 / 32)
-    for rows in (16, 64):      # one and four operand tiles of x in the wavefronts' registers
+    for rows in (16, 64):      # the weight-streaming kernel, 64 x 64 tiles
         xr = x64[:rows].contiguous()
         a_op = kernels.scaled_operand_from_dense(xr, MXFP8_E4M3_fn)
         a_dq = kernels.quantize_dequantize(xr.view(-1), MXFP8_E4M3_fn, torch.bfloat16).view(rows, K)
@@ -470,11 +471,11 @@ def bench_hbm(torch, with_cpu):
         def rows_gemm_bf16(i):
             kernels.mxfp_gemm(a_dq, None, None, None, comps[i][0], comps[i][1], MXFP8_E4M3_fn, None, rows, N, K, torch.bfloat16, out=y)
 
-        for name, fn in (("mxfp_gemm_scaled_rows", rows_gemm), ("mxfp_gemm_skinny (bf16)", rows_gemm_bf16)):
+        for name, fn in (("mxfp_gemm_scaled_rows" if rows == 16 else "mxfp_gemm_scaled_mid", rows_gemm), ("mxfp_gemm_skinny (bf16)", rows_gemm_bf16)):
             avg, best = time_kernel(torch, fn, len(wops))
             cavg, _ = time_kernel(torch, lambda i: fn(0), 1)
             roof(name, f"C4 W x {rows} rows", f"decode: {rows} rows of C4's x against W [{N},{K}] MXFP8 E4M3, bf16 out (bytes = W's codes and scales)", w_bytes,
-                 avg, best, cavg, ROWS_SOURCES if fn is rows_gemm else GEMM_SOURCES)
+                 avg, best, cavg, (ROWS_SOURCES if rows == 16 else MID_SOURCES) if fn is rows_gemm else GEMM_SOURCES)
     return out
 
 
@@ -704,7 +705,7 @@ COUNTER_ROWS = (
     ("mxfp_gemm_tall_kernel", "mxfp_gemm_tall_kernel C4", _M4 * _K4 * 2 + _N4 * _K4 * 33 // 32, _M4 * _N4 * 2, GEMM_SOURCES),
     ("mxfp_gemm_scaled_kernel", "mxfp_gemm_scaled_kernel C5 gate+up", (_M5 + 2 * _I5) * _H5 * 33 // 32, _M5 * 2 * _I5 * 2, SCALED_SOURCES),
     ("mxfp_gemm_scaled_kernel", "mxfp_gemm_scaled_kernel C5 down", (_M5 + _H5) * _I5 * 33 // 32, _M5 * _H5 * 2, SCALED_SOURCES),
-    ("mxfp_gemm_scaled_rows_regs_kernel<2, 4, 8>", "mxfp_gemm_scaled_rows C4 W x 64 rows", _N4 * _K4 * 33 // 32 + 64 * _K4 * 33 // 32, 64 * _N4 * 2, ROWS_SOURCES),
+    ("mxfp_gemm_scaled_mid_kernel<2, 64, 64>", "mxfp_gemm_scaled_mid C4 W x 64 rows", _N4 * _K4 * 33 // 32 + 64 * _K4 * 33 // 32, 64 * _N4 * 2, MID_SOURCES),
     ("scaled_from_dense_kernel|0>, 1>(", "scaled_operand_from_swiglu C5", _M5 * _I5 * 4, _M5 * _I5 * 33 // 32, CAST_SOURCES),
     ("scaled_from_dense_kernel|0>, 0>(", "scaled_operand_from_dense C4 x", _M4 * _K4 * 2, _M4 * _K4 * 33 // 32, CAST_SOURCES),
     ("scaled_operand_kernel<mase::SFmt<4, 3", "scaled_operand_from_mxfp C4 W", _N4 * _K4 * 33 // 32, _N4 * _K4 * 33 // 32, CAST_SOURCES),
