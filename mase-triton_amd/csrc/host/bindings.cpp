@@ -54,22 +54,26 @@ bool stream_of(const at::Tensor& t, void** stream) {
     return true;
 }
 
+// the whole number that `o` stands for; false: none that a long holds (a block axis of 1.0 is for the wrappers to refuse)
+bool whole(PyObject* o, long& v) {
+    v = PyLong_AsLong(o);
+    if (v == -1 && PyErr_Occurred()) return PyErr_Clear(), false;
+    return true;
+}
+
 // (block_size, exp_bits, frac_bits, finite, round mode or -1) of MXFP formats, (exp_bits, frac_bits, finite, round mode) of minifloat ones
 template <int N>
 bool ints(PyObject* tuple, long (&v)[N]) {
     if (!PyTuple_CheckExact(tuple) || PyTuple_GET_SIZE(tuple) != N) return false;
-    for (int i = 0; i < N; ++i) {
-        v[i] = PyLong_AsLong(PyTuple_GET_ITEM(tuple, i));
-        if (v[i] == -1 && PyErr_Occurred()) return PyErr_Clear(), false;
-    }
+    for (int i = 0; i < N; ++i)
+        if (!whole(PyTuple_GET_ITEM(tuple, i), v[i])) return false;
     return v[N - 1] >= 0;
 }
 // code of the output type: None (that of `t`) or a code
 int out_code(PyObject* o, const at::Tensor& t) {
     if (o == Py_None) return dtype_code(t.scalar_type());
-    const long c = PyLong_AsLong(o);
-    if (c == -1 && PyErr_Occurred()) return PyErr_Clear(), -1;
-    return c >= 0 && c < 3 ? (int)c : -1;
+    long c;
+    return whole(o, c) && c >= 0 && c < 3 ? (int)c : -1;
 }
 
 // blocks along axis `dim` of a contiguous tensor: [outer, k, inner]; false: not an axis
@@ -94,14 +98,12 @@ PyObject* extract_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
     PLAIN(n_args == 3);
     const at::Tensor* const x = gpu_tensor(a[0]);
-    long f[5];
-    PLAIN(x && dense(*x) && ints(a[2], f));
-    const long dim = PyLong_AsLong(a[1]);
+    long f[5], dim;
+    PLAIN(x && dense(*x) && ints(a[2], f) && whole(a[1], dim));
     int64_t outer, k, inner;
     void* stream;
     const int dt = dtype_code(x->scalar_type());
     const int64_t n = x->numel(), B = f[0];
-    if (PyErr_Occurred()) PyErr_Clear();
     PLAIN(dt >= 0 && n > 0 && B > 0 && n % B == 0 && extents(*x, dim, outer, k, inner) && stream_of(*x, &stream));
     const bool last = dim == -1 || dim == x->dim() - 1;
     PLAIN(last || B == 32);
@@ -129,10 +131,8 @@ PyObject* qdq_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
     PLAIN(n_args == 4);
     const at::Tensor* const x = gpu_tensor(a[0]);
-    long f[5];
-    PLAIN(x && dense(*x) && ints(a[2], f));
-    const long dim = PyLong_AsLong(a[1]);
-    if (PyErr_Occurred()) PyErr_Clear();
+    long f[5], dim;
+    PLAIN(x && dense(*x) && ints(a[2], f) && whole(a[1], dim));
     int64_t outer, k, inner;
     void* stream;
     const int dt = dtype_code(x->scalar_type()), od = out_code(a[3], *x);
@@ -162,9 +162,8 @@ PyObject* compose_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     c10::SmallVector<int64_t, 6> shape;
     int64_t total = 1;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[4]); ++i) {
-        const long d = PyLong_AsLong(PyTuple_GET_ITEM(a[4], i));
-        if (PyErr_Occurred()) PyErr_Clear();
-        PLAIN(d > 0);
+        long d;
+        PLAIN(whole(PyTuple_GET_ITEM(a[4], i), d) && d > 0);
         shape.push_back(d);
         PLAIN(!__builtin_mul_overflow(total, (int64_t)d, &total));
     }
@@ -180,11 +179,9 @@ PyObject* compose_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
 PyObject* minifloat(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
     PLAIN(n_args == 4);
-    const long kind = PyLong_AsLong(a[0]);
-    if (PyErr_Occurred()) PyErr_Clear();
     const at::Tensor* const x = gpu_tensor(a[1]);
-    long f[4];
-    PLAIN(x && dense(*x) && ints(a[2], f));
+    long kind, f[4];
+    PLAIN(whole(a[0], kind) && x && dense(*x) && ints(a[2], f));
     const int dt = dtype_code(x->scalar_type()), od = kind == 0 ? 0 : out_code(a[3], *x);
     const int64_t n = x->numel();
     void* stream;
@@ -206,8 +203,8 @@ PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const at::Tensor *const x = gpu_tensor(a[0]), *const codes = gpu_tensor(a[4]), *const w_sc = gpu_tensor(a[5]);
     PLAIN(x && codes && w_sc && dense(*x) && x->dim() > 0 && x->scalar_type() == at::kBFloat16 && codes->device() == x->device() && w_sc->device() == x->device());
     PLAIN(codes->is_contiguous() && w_sc->is_contiguous() && codes->scalar_type() == at::kByte && w_sc->scalar_type() == at::kInt && codes->dim() == 2);
-    const long e = PyLong_AsLong(a[1]), m = PyLong_AsLong(a[2]), mini = PyLong_AsLong(a[3]), N = PyLong_AsLong(a[6]);
-    if (PyErr_Occurred()) PyErr_Clear();
+    long e, m, mini, N;
+    PLAIN(whole(a[1], e) && whole(a[2], m) && whole(a[3], mini) && whole(a[6], N));
     const int64_t K = x->size(-1), M = K > 0 ? x->numel() / K : 0;
     PLAIN(M > 0 && N > 0 && codes->size(1) == K && codes->size(0) >= N && w_sc->numel() >= K / 128 * codes->size(0));
     const void* b_ptr = nullptr;
@@ -252,10 +249,9 @@ PyObject* scores(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         PLAIN(l->size(i) == r->size(i) && (l->size(i) == 1 || r->stride(i) == batches * N * K));
         batches *= l->size(i);
     }
-    const long inside = PyLong_AsLong(a[3]);
-    if (PyErr_Occurred()) PyErr_Clear();
+    long inside;
     void* stream;
-    PLAIN(stream_of(*l, &stream));
+    PLAIN(whole(a[3], inside) && stream_of(*l, &stream));
     const bool quantise_w = (M + 127) / 128 * K <= inside;
     at::Tensor w;
     if (!quantise_w) {

@@ -43,7 +43,7 @@ def compose_mxfp_tensor(scales: Tensor, elements: Tensor, tensor_meta: MXFPTenso
     if output_dtype is None:
         output_dtype = getattr(torch, tensor_meta.dtype)
     shape, block_dim = tensor_meta.shape, tensor_meta.block_dim
-    if block_dim in (-1, len(shape) - 1):
+    if isinstance(block_dim, int) and block_dim in (-1, len(shape) - 1):     # (1.0 compares equal too, and names no axis)
         plain = _lib.host().compose_mxfp(scales, elements, tensor_meta.meta._codes, TORCH_DTYPE_TO_CODE.get(output_dtype, -1), shape)
         if plain is not None:
             return plain

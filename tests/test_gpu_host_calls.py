@@ -1,6 +1,8 @@
 """Calls through the extension module against the same calls through the Python wrappers (the module replaced by one that takes no
 call): the same values, types, shapes and layouts, or the same error, over contiguous and strided, aligned and misaligned, empty and
 0-d inputs, every block axis, dtype, format, round mode and output type; and the calls that the module must leave to the wrappers."""
+from fractions import Fraction
+
 import pytest
 import torch
 
@@ -97,6 +99,25 @@ def test_casts_either_way(monkeypatch, dtype):
                 _same(*_both(monkeypatch, lambda: MF.compose_minifloat_component(a[0].view(torch.int16), a[1], torch.float32)))
             else:
                 _same(a, b)
+
+
+@pytest.mark.parametrize("dim", [0.0, 1.0, -1.0, 0.5, torch.tensor(1.0), Fraction(1), True, torch.tensor(1)])
+def test_axes_that_are_no_whole_numbers(monkeypatch, dim):
+    """An axis that is no integer is refused, whatever it compares equal to; True and a 0-d integer tensor are integers."""
+    import mase_hip.mxfp.functional as MX
+    from mase_hip import _lib
+    from mase_hip.mxfp.meta import MXFP8_E4M3_fn as m
+
+    x = torch.randn(64, 64, device=DEV)
+    sc, el, tm = MX.extract_mxfp_components(x, -1, m)
+    tm = tm.create(block_dim=dim)
+    for fn in (lambda: MX.extract_mxfp_components(x, dim, m), lambda: MX.quantize_dequantize(x, dim, m), lambda: MX.compose_mxfp_tensor(sc, el, tm)):
+        plain, general = _both(monkeypatch, fn)
+        _same(plain, general)
+        whole = not isinstance(dim, (float, Fraction)) and not (isinstance(dim, torch.Tensor) and dim.is_floating_point())
+        assert whole != (plain is TypeError)
+    if not whole:
+        assert _lib.host().extract_mxfp(x, dim, m._codes) is None and _lib.host().qdq_mxfp(x, dim, m._codes, None) is None
 
 
 def test_layers_either_way(monkeypatch):
