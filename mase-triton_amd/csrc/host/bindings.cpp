@@ -76,6 +76,9 @@ int out_code(PyObject* o, const at::Tensor& t) {
     return whole(o, c) && c >= 0 && c < 3 ? (int)c : -1;
 }
 
+using Sizes = c10::SmallVector<int64_t, 6>;
+Sizes sizes_of(const at::Tensor& t) { return Sizes(t.sizes().begin(), t.sizes().end()); }
+
 // blocks along axis `dim` of a contiguous tensor: [outer, k, inner]; false: not an axis
 bool extents(const at::Tensor& t, long dim, int64_t& outer, int64_t& k, int64_t& inner) {
     const int64_t nd = t.dim();
@@ -88,7 +91,16 @@ bool extents(const at::Tensor& t, long dim, int64_t& outer, int64_t& k, int64_t&
     return dim == nd - 1 || k % 32 == 0;
 }
 
-at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, const at::Tensor& like) { return at::empty(sizes, at::TensorOptions().dtype(dtype).device(like.device())); }
+at::Tensor empty(at::IntArrayRef sizes, at::ScalarType dtype, at::Device device) { return at::empty(sizes, at::TensorOptions().dtype(dtype).device(device)); }
+
+// Other Python threads run while one allocates (which can wait for the GPU) and launches (which waits where the queue is full), as they do
+// beside torch's own calls.  What such a thread could change (sizes, data) is read before; nothing of Python's is touched in its scope.
+struct WithoutGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    WithoutGil() = default;
+    WithoutGil(const WithoutGil&) = delete;
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
 
 #define PLAIN(cond) \
     if (!(cond)) Py_RETURN_NONE
@@ -107,10 +119,18 @@ PyObject* extract_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     PLAIN(dt >= 0 && n > 0 && B > 0 && n % B == 0 && extents(*x, dim, outer, k, inner) && stream_of(*x, &stream));
     const bool last = dim == -1 || dim == x->dim() - 1;
     PLAIN(last || B == 32);
-    at::Tensor scales = empty({n / B, 1}, at::kByte, *x), elements = empty({n / B, B}, at::kByte, *x);
-    const int rc = last ? mase_hip_extract_mxfp(x->data_ptr(), dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
-                        : mase_hip_extract_mxfp_strided(x->data_ptr(), dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3],
-                                                        (int)f[4], stream);
+    const void* const data = x->data_ptr();
+    const at::Device device = x->device();
+    at::Tensor scales, elements;
+    int rc;
+    {
+        const WithoutGil released;
+        scales = empty({n / B, 1}, at::kByte, device);
+        elements = empty({n / B, B}, at::kByte, device);
+        rc = last ? mase_hip_extract_mxfp(data, dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
+                  : mase_hip_extract_mxfp_strided(data, dt, scales.data_ptr<uint8_t>(), elements.data_ptr<uint8_t>(), outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3], (int)f[4],
+                                                  stream);
+    }
     PLAIN(rc == 0);
     PyObject* const s = THPVariable_Wrap(std::move(scales));
     PyObject* const e = s ? THPVariable_Wrap(std::move(elements)) : nullptr;
@@ -140,9 +160,17 @@ PyObject* qdq_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     PLAIN(dt >= 0 && od >= 0 && n > 0 && B > 0 && n % B == 0 && extents(*x, dim, outer, k, inner) && stream_of(*x, &stream));
     const bool last = dim == -1 || dim == x->dim() - 1;
     PLAIN(last || B == 32);
-    at::Tensor out = empty(x->sizes(), kDtypes[od], *x);
-    const int rc = last ? mase_hip_qdq_mxfp(x->data_ptr(), dt, out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
-                        : mase_hip_qdq_mxfp_strided(x->data_ptr(), dt, out.data_ptr(), od, outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream);
+    const Sizes sizes = sizes_of(*x);
+    const void* const data = x->data_ptr();
+    const at::Device device = x->device();
+    at::Tensor out;
+    int rc;
+    {
+        const WithoutGil released;
+        out = empty(sizes, kDtypes[od], device);
+        rc = last ? mase_hip_qdq_mxfp(data, dt, out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream)
+                  : mase_hip_qdq_mxfp_strided(data, dt, out.data_ptr(), od, outer, k, inner, 32, (int)f[1], (int)f[2], (int)f[3], (int)f[4], stream);
+    }
     PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -159,7 +187,7 @@ PyObject* compose_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t n = elements->numel(), B = f[0];
     PLAIN(od >= 0 && n > 0 && B > 0 && n % B == 0 && scales->numel() == n / B && scales->scalar_type() == at::kByte && elements->scalar_type() == at::kByte &&
           scales->device() == elements->device());
-    c10::SmallVector<int64_t, 6> shape;
+    Sizes shape;
     int64_t total = 1;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[4]); ++i) {
         long d;
@@ -169,8 +197,16 @@ PyObject* compose_mxfp(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     void* stream;
     PLAIN(total == n && stream_of(*elements, &stream));
-    at::Tensor out = empty(shape, kDtypes[od], *elements);
-    PLAIN(mase_hip_compose_mxfp(scales->data_ptr<uint8_t>(), elements->data_ptr<uint8_t>(), out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], stream) == 0);
+    const uint8_t *const scale_data = scales->data_ptr<uint8_t>(), *const element_data = elements->data_ptr<uint8_t>();
+    const at::Device device = elements->device();
+    at::Tensor out;
+    int rc;
+    {
+        const WithoutGil released;
+        out = empty(shape, kDtypes[od], device);
+        rc = mase_hip_compose_mxfp(scale_data, element_data, out.data_ptr(), od, n, (int)B, (int)f[1], (int)f[2], (int)f[3], stream);
+    }
+    PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -186,11 +222,19 @@ PyObject* minifloat(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t n = x->numel();
     void* stream;
     PLAIN(kind >= 0 && kind <= 2 && n > 0 && od >= 0 && (kind == 1 ? x->scalar_type() == at::kUInt16 : dt >= 0) && stream_of(*x, &stream));
-    at::Tensor out = empty(x->sizes(), kind == 0 ? at::kUInt16 : kDtypes[od], *x);
+    const Sizes sizes = sizes_of(*x);
+    const void* const data = x->data_ptr();
+    const at::Device device = x->device();
     const int E = (int)f[0], M = (int)f[1], fin = (int)f[2], rm = (int)f[3];
-    const int rc = kind == 0   ? mase_hip_extract_minifloat(x->data_ptr(), dt, static_cast<uint16_t*>(out.data_ptr()), n, E, M, fin, rm, stream)
-                   : kind == 1 ? mase_hip_compose_minifloat(static_cast<const uint16_t*>(x->data_ptr()), out.data_ptr(), od, n, E, M, fin, stream)
-                               : mase_hip_qdq_minifloat(x->data_ptr(), dt, out.data_ptr(), od, n, E, M, fin, rm, stream);
+    at::Tensor out;
+    int rc;
+    {
+        const WithoutGil released;
+        out = empty(sizes, kind == 0 ? at::kUInt16 : kDtypes[od], device);
+        rc = kind == 0   ? mase_hip_extract_minifloat(data, dt, static_cast<uint16_t*>(out.data_ptr()), n, E, M, fin, rm, stream)
+             : kind == 1 ? mase_hip_compose_minifloat(static_cast<const uint16_t*>(data), out.data_ptr(), od, n, E, M, fin, stream)
+                         : mase_hip_qdq_minifloat(data, dt, out.data_ptr(), od, n, E, M, fin, rm, stream);
+    }
     PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -218,14 +262,24 @@ PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     void* stream;
     PLAIN(stream_of(*x, &stream));
-    const int64_t bytes = mase_hip_mxfp_linear_scaled_scratch_bytes(M, N, K);
-    PLAIN(bytes > 0);
-    at::Tensor scratch = empty({bytes}, at::kByte, *x);
-    c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
+    Sizes shape = sizes_of(*x);
     shape.back() = N;
-    at::Tensor y = empty(shape, at::kBFloat16, *x);
-    PLAIN(mase_hip_mxfp_linear_scaled(x->data_ptr(), 2, (int)e, (int)m, (int)mini, codes->data_ptr<uint8_t>(), reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>()), b_ptr, b_dt,
-                                      y.data_ptr(), 2, M, N, K, scratch.data_ptr(), bytes, stream) == 0);
+    const void* const data = x->data_ptr();
+    const uint8_t* const code_data = codes->data_ptr<uint8_t>();
+    const uint32_t* const scale_data = reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>());
+    const at::Device device = x->device();
+    at::Tensor scratch, y;
+    int rc = -1;
+    {
+        const WithoutGil released;
+        const int64_t bytes = mase_hip_mxfp_linear_scaled_scratch_bytes(M, N, K);
+        if (bytes > 0) {
+            scratch = empty({bytes}, at::kByte, device);
+            y = empty(shape, at::kBFloat16, device);
+            rc = mase_hip_mxfp_linear_scaled(data, 2, (int)e, (int)m, (int)mini, code_data, scale_data, b_ptr, b_dt, y.data_ptr(), 2, M, N, K, scratch.data_ptr(), bytes, stream);
+        }
+    }
+    PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -253,16 +307,24 @@ PyObject* scores(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     void* stream;
     PLAIN(whole(a[3], inside) && stream_of(*l, &stream));
     const bool quantise_w = (M + 127) / 128 * K <= inside;
-    at::Tensor w;
-    if (!quantise_w) {
-        w = empty({batches * N * K}, at::kBFloat16, *l);
-        PLAIN(mase_hip_qdq_mxfp(r->data_ptr(), 2, w.data_ptr(), 2, batches * N * K, 32, (int)f[1], (int)f[2], 1, 0, stream) == 0);
-    }
-    c10::SmallVector<int64_t, 6> shape(l->sizes().begin(), l->sizes().end());
+    Sizes shape = sizes_of(*l);
     shape.back() = N;
-    at::Tensor y = empty(shape, at::kBFloat16, *l);
-    PLAIN(mase_hip_mxfp_scores(l->data_ptr(), (int)f[1], (int)f[2], quantise_w ? r->data_ptr() : w.data_ptr(), quantise_w, y.data_ptr(), M, N, K, batches, M * K, N * K, M * N,
-                               stream) == 0);
+    const void *const left = l->data_ptr(), *const right = r->data_ptr();
+    const at::Device device = l->device();
+    at::Tensor w, y;
+    int rc = 0;
+    {
+        const WithoutGil released;
+        if (!quantise_w) {
+            w = empty({batches * N * K}, at::kBFloat16, device);
+            rc = mase_hip_qdq_mxfp(right, 2, w.data_ptr(), 2, batches * N * K, 32, (int)f[1], (int)f[2], 1, 0, stream);
+        }
+        if (rc == 0) {
+            y = empty(shape, at::kBFloat16, device);
+            rc = mase_hip_mxfp_scores(left, (int)f[1], (int)f[2], quantise_w ? right : w.data_ptr(), quantise_w, y.data_ptr(), M, N, K, batches, M * K, N * K, M * N, stream);
+        }
+    }
+    PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }

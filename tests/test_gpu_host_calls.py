@@ -1,6 +1,9 @@
 """Calls through the extension module against the same calls through the Python wrappers (the module replaced by one that takes no
 call): the same values, types, shapes and layouts, or the same error, over contiguous and strided, aligned and misaligned, empty and
 0-d inputs, every block axis, dtype, format, round mode and output type; and the calls that the module must leave to the wrappers."""
+import sys
+import threading
+import time
 from fractions import Fraction
 
 import pytest
@@ -213,6 +216,59 @@ def test_left_to_the_wrappers():
         MX.quantize_dequantize(x.cpu(), -1, m)
     with pytest.raises(Exception):
         torch.vmap(lambda t: MX.quantize_dequantize(t, -1, m))(x)
+
+
+def _plain_calls():
+    """Each function of the module once, its arguments plain; outputs of at least 32 MB."""
+    import mase_hip.minifloat.functional as MF
+    import mase_hip.minifloat.meta as mf
+    import mase_hip.mxfp.functional as MX
+    import mase_hip.mxfp.kernels as mxk
+    from mase_hip import _lib
+    from mase_hip.mxfp.meta import MXFP8_E4M3_fn as m
+
+    host, f8 = _lib.host(), mf.FP8_E4M3_fn
+    x = torch.randn(4096, 8192, device=DEV)
+    sc, el, _ = MX.extract_mxfp_components(x, -1, m)
+    codes, _ = MF.extract_minifloat_component(x, f8)
+    a = torch.randn(4096, 512, device=DEV).to(torch.bfloat16)
+    w = mxk.scaled_operand_from_mxfp(*MX.extract_mxfp_components(a, -1, m)[:2], m, 4096, 512)
+    q, k = (torch.randn(32, 1024, 64, device=DEV).to(torch.bfloat16) for _ in range(2))
+    return {"extract_mxfp": lambda: host.extract_mxfp(x, -1, m._codes), "extract_mxfp, rows": lambda: host.extract_mxfp(x, 0, m._codes),
+            "qdq_mxfp": lambda: host.qdq_mxfp(x, -1, m._codes, None), "compose_mxfp": lambda: host.compose_mxfp(sc, el, m._codes, 0, (4096, 8192)),
+            "minifloat, extract": lambda: host.minifloat(0, x, f8._codes, None), "minifloat, compose": lambda: host.minifloat(1, codes, f8._codes, 0),
+            "minifloat, both": lambda: host.minifloat(2, x, f8._codes, None),
+            "linear_scaled": lambda: host.linear_scaled(a, 4, 3, 0, w.codes, w.scales, 4096, None),
+            "scores": lambda: host.scores(q, k.transpose(-1, -2), m._codes, 512)}
+
+
+def test_other_threads_run_beside_a_call():
+    """A call lets go of the interpreter while it allocates and launches: with the interpreter's own switching put off, another thread gets
+    on only where a call lets it.  Every output is kept, so every call waits for the driver to allocate."""
+    calls = _plain_calls()
+    ticks, stop = [0], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            ticks[0] += 1
+            time.sleep(1e-4)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        sys.setswitchinterval(1000.0)
+        for name, call in calls.items():
+            torch.cuda.empty_cache()
+            before, kept = ticks[0], [call() for _ in range(16)]
+            seen = ticks[0] - before
+            assert seen > 0, name
+            assert all(y is not None for y in kept), name
+            del kept
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
 
 
 def test_streams_and_capture():
