@@ -22,6 +22,14 @@ int mase_hip_mxfp_scores(const void* a, int a_exp_bits, int a_frac_bits, const v
                          int64_t N, int64_t K, int64_t batches, int64_t a_batch_stride, int64_t w_batch_stride,
                          int64_t y_batch_stride, void* stream);
 
+/*
+ * The way that is fastest for such a product (M, N, K, batches as above): 2: mase_hip_mxfp_scores with quantise_w, 1: W through
+ * mase_hip_qdq_mxfp first, 0: neither (mase_hip_extract_mxfp of W, mase_hip_qdq_mxfp of A, mase_hip_mxfp_gemm_batched; also for shapes
+ * that mase_hip_mxfp_scores refuses).  one_format != 0: A and W are quantised in the same format (else never 2).  Depends on its
+ * arguments only.
+ */
+int mase_hip_mxfp_scores_plan(int64_t M, int64_t N, int64_t K, int64_t batches, int one_format);
+
 #ifdef __cplusplus
 }
 #endif

@@ -32,3 +32,29 @@ extern "C" int mase_hip_mxfp_scores(const void* a, int a_exp_bits, int a_frac_bi
         return fail(ERR_INVALID, "MXFP element (exp_bits, frac_bits) must be one of (4,3) (5,2) (2,3) (3,2) (2,1)");
     });
 }
+
+// Which way a product of short contraction goes.  The general route is a pass over each operand and the kernels that compose codes
+// (gemm_short_k.h, a weight-streaming one for few rows).  GPU time in us on other operands each call, general / W in a pass before / W
+// inside:
+//   K = 96 pays for 128 (zeros), without the L2 prefetch of W.  Many outputs, more than one panel: 23 of 2048 x 513 27 / 31 / 37, 10 of 8192 x
+//   640 41 / 45 / 53, 12 of 2048 x 384 18.6 / 24 / 24; few outputs 11.3 / 9.9 / 9.6 (one of 2048 x 1000); rows of y off the 128-byte lines or
+//   short ones 58 / 42 (50 of 1000 x 1000), 60 / 51 (136 x 200 x 2048 down to 64 columns); one panel 54 / 45 inside (473 of 512 x 128), but 76 / 92 / 95
+//   where rows of y are a few lines (2507 of 200 x 16);
+//   K = 128, long rows of whole lines, three to twelve panels: 6 of 2048 x 768 18.6 / 24 / 24, 65536 x 768 35 / 50 / 51; outside that 64.0 / 41.7 (25 of 1000 x
+//   2048), 44.6 / 40.4 (7 of 2048 x 4096);
+//   K <= 64: inside up to twelve panels (2 of 8192 x 1464 19.1 / 21.9 / 18.5), before beyond that (54 / 34 with 27 of 1000 x 2048 x 64).
+// A dense A, or formats that differ, rules "inside" out, and a pass over W writes twice the bytes of its codes.  Dense A, general / before: 26.1 /
+// 33.4 (99 of 512 x 1000 x 64), 22.5 / 34.8 (360 of 512 x 1), 61.7 / 69.6 (32 of 2048 x 2048 x 128); 0.6 - 0.9 of the time with many rows off the lines,
+// and with few outputs, where both are bound by their launches.
+extern "C" int mase_hip_mxfp_scores_plan(int64_t M, int64_t N, int64_t K, int64_t batches, int one_format) {
+    if (M < 1 || N < 1 || K < 1 || batches < 1 || K % 32 != 0 || K > SCO_MAX_K || N % 8 != 0 || N > (1 << 23) || M > 0x7FFFFFFF - SCO_M) return 0;
+    const int64_t panels = (M + SCO_M - 1) / SCO_M;
+    const double y_mb = (double)batches * (double)M * (double)N * 2e-6, w_mb = (double)batches * (double)N * (double)K * 2e-6;
+    const bool few = y_mb < 9.0, many = y_mb >= 48.0, lines = N % 64 == 0;
+    if (!one_format) return (few && w_mb < 9.0) || (many && !lines && panels > 2) ? 1 : 0;
+    if (few) return 2;
+    if (K == 96 && panels > 1) return many && panels > 2 && (!lines || N <= 512) ? 1 : 0;
+    if (K == 96 && N <= 256) return 0;
+    if (K == 128 && lines && N >= 2048 && panels > 2 && panels <= 12) return 0;
+    return panels * (K <= 64 ? 64 : 128) <= (K <= 64 ? 768 : 512) ? 2 : 1;
+}

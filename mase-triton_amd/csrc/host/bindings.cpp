@@ -284,11 +284,11 @@ PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
-// scores(left [.., M, K], right [.., K, N], format of left, the same of right, panels x K up to which right is quantised inside): left @ right where
-// both are bf16 with the same leading axes, quantised in one format, and right is the transposed view of a contiguous tensor
+// scores(left [.., M, K], right [.., K, N], format of both): left @ right where both are bf16 with the same leading axes and right is the
+// transposed view of a contiguous tensor, K up to 128, whichever way is the fastest
 PyObject* scores(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
-    PLAIN(n_args == 4);
+    PLAIN(n_args == 3);
     const at::Tensor *const l = gpu_tensor(a[0]), *const r = gpu_tensor(a[1]);
     long f[5];
     PLAIN(l && r && ints(a[2], f) && f[0] == 32 && f[3] == 1 && f[4] == 0);
@@ -303,25 +303,37 @@ PyObject* scores(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         PLAIN(l->size(i) == r->size(i) && (l->size(i) == 1 || r->stride(i) == batches * N * K));
         batches *= l->size(i);
     }
-    long inside;
+    const int way = mase_hip_mxfp_scores_plan(M, N, K, batches, 1), E = (int)f[1], m = (int)f[2];
     void* stream;
-    PLAIN(whole(a[3], inside) && stream_of(*l, &stream));
-    const bool quantise_w = (M + 127) / 128 * K <= inside;
+    PLAIN((way != 0 || batches <= 65535) && stream_of(*l, &stream));
     Sizes shape = sizes_of(*l);
     shape.back() = N;
     const void *const left = l->data_ptr(), *const right = r->data_ptr();
     const at::Device device = l->device();
-    at::Tensor w, y;
+    const int64_t n_a = l->numel(), n_w = batches * N * K;
+    at::Tensor a_q, w_q, scales, y;
     int rc = 0;
     {
         const WithoutGil released;
-        if (!quantise_w) {
-            w = empty({batches * N * K}, at::kBFloat16, device);
-            rc = mase_hip_qdq_mxfp(right, 2, w.data_ptr(), 2, batches * N * K, 32, (int)f[1], (int)f[2], 1, 0, stream);
-        }
-        if (rc == 0) {
+        if (way == 0) {
+            a_q = empty({n_a}, at::kBFloat16, device);
+            scales = empty({n_w / 32}, at::kByte, device);
+            w_q = empty({n_w}, at::kByte, device);
             y = empty(shape, at::kBFloat16, device);
-            rc = mase_hip_mxfp_scores(left, (int)f[1], (int)f[2], quantise_w ? right : w.data_ptr(), quantise_w, y.data_ptr(), M, N, K, batches, M * K, N * K, M * N, stream);
+            rc = mase_hip_qdq_mxfp(left, 2, a_q.data_ptr(), 2, n_a, 32, E, m, 1, 0, stream);
+            if (rc == 0) rc = mase_hip_extract_mxfp(right, 2, scales.data_ptr<uint8_t>(), w_q.data_ptr<uint8_t>(), n_w, 32, E, m, 1, 0, stream);
+            if (rc == 0)
+                rc = mase_hip_mxfp_gemm_batched(a_q.data_ptr(), 2, scales.data_ptr<uint8_t>(), w_q.data_ptr<uint8_t>(), E, m, y.data_ptr(), 2, M, N, K, 32, batches, M * K, N * K, M * N,
+                                                stream);
+        } else {
+            if (way == 1) {
+                w_q = empty({n_w}, at::kBFloat16, device);
+                rc = mase_hip_qdq_mxfp(right, 2, w_q.data_ptr(), 2, n_w, 32, E, m, 1, 0, stream);
+            }
+            if (rc == 0) {
+                y = empty(shape, at::kBFloat16, device);
+                rc = mase_hip_mxfp_scores(left, E, m, way == 2 ? right : w_q.data_ptr(), way == 2, y.data_ptr(), M, N, K, batches, M * K, N * K, M * N, stream);
+            }
         }
     }
     PLAIN(rc == 0);

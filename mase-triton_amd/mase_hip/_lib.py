@@ -55,6 +55,7 @@ SIGNATURES = {
 # include/mase_hip_scores.h
 SCORES_SIGNATURES = {
     "mase_hip_mxfp_scores": (_i32, [_vp, _i32, _i32, _vp, _i32, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp]),
+    "mase_hip_mxfp_scores_plan": (_i32, [_i64, _i64, _i64, _i64, _i32]),
 }
 
 

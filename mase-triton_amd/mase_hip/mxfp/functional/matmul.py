@@ -9,7 +9,7 @@ along its second-to-last axis (no transposed copy).  When ``other`` is quantised
 form: its codes come out as [.., N, K], the layout the GEMM kernels read, and all leading batch
 axes (broadcast ones included) go into ONE batched GEMM launch that composes the codes to bf16
 on their way to the MFMA units.  Products of queries and keys (``other`` the transposed view of a contiguous bfloat16 tensor, K up to
-128) quantise their operands inside the GEMM: one launch, or two.  A product of two quantised bfloat16 operands against ONE matrix
+128) quantise their operands inside the GEMM where that is faster: one launch, or two.  A product of two quantised bfloat16 operands against ONE matrix
 (``other`` without batch axes) with enough rows takes the block-scaled FP8 matrix instruction instead, as
 ``mxfp_linear`` does (functional/linear.py).  Everything else goes through the one-pass quantise-dequantise
 kernels and ``torch.matmul``.
@@ -112,15 +112,9 @@ def _other_components(other: Tensor, other_meta: MXFPMeta) -> tuple[Tensor, Tens
     return kernels.extract_mxfp_components_strided(other, -2, other_meta)
 
 
-# The keys are quantised inside the product, once for every 128 rows of queries, up to this many such panels x K; beyond, a pass over
-# them comes first.  Inside / before, us: 32 products of 512 x 512 x 128 (4 panels) 14.6 / 18.1, 64 of 256 x 256 x 128 11.5 / 18.2; 64 of 1000 x
-# 1000 x 128 (8) 55 / 47, 32 of 1464 x 1464 x 64 (12) 39 / 36.
-SCORES_QUANTISE_W_UP_TO = 512
-
-
 def _scores(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, other_meta: MXFPMeta) -> Tensor | None:
-    """The product of queries and keys in one or two launches, or None where it is not one: ``other`` the transposed view of a
-    contiguous bfloat16 tensor, K up to 128."""
+    """The product of queries and keys in one or two launches, or None where it is not one (``other`` the transposed view of a
+    contiguous bfloat16 tensor, K up to 128) or the general kernels are ahead."""
     K, N = other.shape[-2], other.shape[-1]
     if (input.dtype != torch.bfloat16 or not kernels.scores_shape_supported(N, K) or other.is_contiguous()
             or not kernels.scores_format_supported(other_meta) or not (input_meta is None or kernels.scores_format_supported(input_meta))):
@@ -136,7 +130,10 @@ def _scores(input: Tensor, other: Tensor, input_meta: MXFPMeta | None, other_met
         batch = tuple(torch.broadcast_shapes(bi, bo))
         if _prod(bi) != 1 and bi != batch or bo != batch:
             return None                                         # broadcast along some axes only
-    quantise_w = input_meta is not None and input_meta == other_meta and -(-M // 128) * K <= SCORES_QUANTISE_W_UP_TO
+    plan = kernels.scores_plan(M, N, K, _prod(batch), input_meta is not None and input_meta == other_meta)
+    if plan == 0:
+        return None
+    quantise_w = plan == 2
     w = lying if quantise_w else kernels.quantize_dequantize(lying.reshape(-1), other_meta, torch.bfloat16)
     y = kernels.mxfp_scores(input, input_meta, w, quantise_w, _prod(batch), M, N, K, 0 if _prod(bi) == 1 else M * K, N * K)
     return y.view(*torch.broadcast_shapes(bi, bo), input.shape[-2], N)
@@ -179,7 +176,7 @@ def mxfp_matmul(
     if quantised_other:
         assert other_meta is not None
     if fused and quantised_input and quantised_other and (input_meta is other_meta or input_meta == other_meta):
-        plain = _lib.host().scores(input, other, other_meta._codes, SCORES_QUANTISE_W_UP_TO)     # queries and keys, as a model has them
+        plain = _lib.host().scores(input, other, other_meta._codes)     # queries and keys, as a model has them
         if plain is not None:
             return plain
     if fused and quantised_other and _gemm_route(input, other, quantised_input, other_meta):

@@ -232,6 +232,11 @@ def scores_shape_supported(N: int, K: int) -> bool:
     return K % 32 == 0 and K <= 128 and N % 8 == 0 and N <= 1 << 23
 
 
+def scores_plan(M: int, N: int, K: int, batches: int, one_format: bool) -> int:
+    """The fastest way for such products: 2: ``mxfp_scores`` with W quantised inside, 1: with W quantised before, 0: not ``mxfp_scores``."""
+    return _lib.load().mase_hip_mxfp_scores_plan(M, N, K, batches, int(one_format))
+
+
 def mxfp_scores(a: Tensor, meta: MXFPMeta | None, w: Tensor, quantise_w: bool, batches: int, M: int, N: int, K: int,
                 a_batch_stride: int, w_batch_stride: int) -> Tensor:
     """``batches`` products y[b] = Q(A[b]) @ W[b]^T in one launch, K <= 128: ``a`` and ``w`` hold bfloat16 [M, K] and [N, K] matrices

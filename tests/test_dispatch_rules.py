@@ -113,3 +113,27 @@ def test_one_full_round_of_large_tiles_is_not_given_to_two_of_small_ones(lib):
     for shape, bn in (((65, 28672, 4096), 128), ((128, 28672, 1024), 128), ((128, 98304, 4096), 128), ((128, 152064, 4096), 128), ((384, 14336, 512), 128),
                       ((200, 14336, 4096), 128), ((128, 14336, 4096), 64)):
         assert scaled_plan(lib, *shape)[0] == bn
+
+
+def test_ways_of_a_product_of_short_contraction():
+    """2: queries and keys quantised inside the kernel of whole rows, 1: keys in a pass before it, 0: the general kernels."""
+    from mase_hip.mxfp.kernels import scores_plan as plan
+
+    for K in (32, 64, 96, 128):                     # few outputs: inside, whatever the shape
+        assert plan(1, 8, K, 1, True) == plan(4096, 64, K, 17, True) == plan(1, 65536, K, 64, True) == plan(2000, 2000, K, 1, True) == 2
+    assert plan(1536, 2048, 64, 8, True) == 2 and plan(1537, 2048, 64, 8, True) == 1      # twelve panels
+    assert plan(512, 1000, 128, 48, True) == 2 and plan(513, 1000, 128, 48, True) == 1    # four
+    # K = 96: zeros up to 128 and no prefetch
+    assert plan(129, 8192, 96, 28, True) == plan(513, 2048, 96, 46, True) == plan(640, 8192, 96, 10, True) == plan(1000, 1000, 96, 10, True) == 0
+    assert plan(128, 2048, 96, 127, True) == 2 and plan(16, 200, 96, 2507, True) == 0
+    assert plan(1000, 1000, 96, 50, True) == plan(2048, 512, 96, 46, True) == 1
+    # K = 128: long rows of whole lines, three to twelve panels
+    assert plan(257, 2048, 128, 20, True) == plan(768, 65536, 128, 1, True) == plan(1464, 8192, 128, 5, True) == 0
+    assert plan(256, 2048, 128, 20, True) == 2 and plan(768, 2040, 128, 31, True) == plan(768, 1984, 128, 31, True) == plan(2048, 2048, 128, 13, True) == 1
+    # a dense A, or two formats: never inside
+    for K in (32, 64, 96, 128):
+        assert plan(1, 1000, K, 8, False) == plan(1000, 1000, K, 48, False) == plan(256, 512, K, 4, False) == 1
+        assert plan(1, 1000, K, 400, False) == plan(2048, 2048, K, 32, False) == plan(513, 2048, K, 10, False) == plan(256, 1000, K, 200, False) == 0
+    # what the kernel does not take, and empty products
+    assert plan(64, 60, 64, 1, True) == plan(64, 64, 160, 1, True) == plan(64, 64, 48, 1, True) == plan(0, 64, 64, 1, True) == plan(64, 64, 64, 0, True) == 0
+    assert plan(64, (1 << 23) + 8, 64, 1, True) == 0 and plan(2 ** 31 - 1, 8, 32, 1, True) == 0

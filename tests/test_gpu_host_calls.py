@@ -176,6 +176,26 @@ def test_scores_either_way(monkeypatch):
             assert plain is general
 
 
+@pytest.mark.parametrize("shape,N,K,way", [((2, 3, 200), 200, 64, 2), ((300,), 72, 32, 2), ((1, 1, 5), 1000, 128, 2), ((20, 513), 2504, 64, 2), ((9, 640), 1000, 128, 1),
+                                           ((2, 24, 300), 512, 96, 0), ((1, 700), 16384, 128, 0), ((2000,), 8192, 96, 0), ((2500, 1), 2000, 96, 2), ((66000, 16), 200, 96, 0)])
+def test_scores_each_way(monkeypatch, shape, N, K, way):
+    """Each of the three ways through the module and through the wrappers: the same kernels, so the same bits."""
+    import mase_hip.mxfp.functional as MX
+    import mase_hip.mxfp.kernels as mxk
+    from mase_hip import _lib
+    from mase_hip.mxfp.meta import OCP_MXFP6_E2M3 as m
+
+    batches = 1
+    for d in shape[:-1]:
+        batches *= d
+    assert mxk.scores_plan(shape[-1], N, K, batches, True) == way
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    q, k = (torch.randn(*s, K, generator=g, device=DEV, dtype=torch.bfloat16) for s in (shape, (*shape[:-1], N)))
+    k = k.transpose(-1, -2)
+    assert (_lib.host().scores(q, k, m._codes) is None) == (batches > 65535 and way == 0)      # (more products than a launch of the general kernels takes)
+    _same(*_both(monkeypatch, lambda: MX.mxfp_matmul(q, k, m, m, "XqWq", "fused")))
+
+
 def test_left_to_the_wrappers():
     """Function and dispatch modes, vmap and other devices see what they saw: the module takes none of these calls."""
     from torch.overrides import TorchFunctionMode
@@ -239,7 +259,7 @@ def _plain_calls():
             "minifloat, extract": lambda: host.minifloat(0, x, f8._codes, None), "minifloat, compose": lambda: host.minifloat(1, codes, f8._codes, 0),
             "minifloat, both": lambda: host.minifloat(2, x, f8._codes, None),
             "linear_scaled": lambda: host.linear_scaled(a, 4, 3, 0, w.codes, w.scales, 4096, None),
-            "scores": lambda: host.scores(q, k.transpose(-1, -2), m._codes, 512)}
+            "scores": lambda: host.scores(q, k.transpose(-1, -2), m._codes)}
 
 
 def test_other_threads_run_beside_a_call():
