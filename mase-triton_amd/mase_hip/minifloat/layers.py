@@ -173,15 +173,18 @@ class MinifloatLinearPTQ(nn.Module):
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense_minifloat(x2, xm.exp_bits, xm.frac_bits), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
         # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
+        # (written to the instance's dict: nn.Module's own assignment costs a microsecond, on every call whose shape changes)
         w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
-        self._no_operand_sig = None
-        self._fast_sig = sig if w_operand is not None else None
+        notes = self.__dict__
+        notes["_no_operand_sig"] = None
+        notes["_fast_sig"] = sig if w_operand is not None else None
         y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             _narrowed=self._narrowed_weight(), _w_operand=w_operand)
-        self._no_operand_sig = sig if w_operand is None else None
+        if w_operand is None:
+            notes["_no_operand_sig"] = sig
         return y
 
     def extra_repr(self) -> str:

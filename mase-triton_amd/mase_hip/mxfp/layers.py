@@ -188,15 +188,18 @@ class MXFPLinearPTQ(nn.Module):
                     y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense(x2, meta), self._scaled_w, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
         # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
+        # (written to the instance's dict: nn.Module's own assignment costs a microsecond, on every call whose shape changes)
         w_operand = None if self._no_operand_sig == sig else self._weight_operand(input)
-        self._no_operand_sig = None
-        self._fast_sig = sig if w_operand is not None and self._takes_scaled_route(input) else None
+        notes = self.__dict__
+        notes["_no_operand_sig"] = None
+        notes["_fast_sig"] = sig if w_operand is not None and self._takes_scaled_route(input) else None
         y = MXFP_F.mxfp_linear(
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             w_operand=w_operand)
-        self._no_operand_sig = sig if w_operand is None else None
+        if w_operand is None:
+            notes["_no_operand_sig"] = sig
         return y
 
     @torch.no_grad()
