@@ -137,3 +137,23 @@ def test_ways_of_a_product_of_short_contraction():
     # what the kernel does not take, and empty products
     assert plan(64, 60, 64, 1, True) == plan(64, 64, 160, 1, True) == plan(64, 64, 48, 1, True) == plan(0, 64, 64, 1, True) == plan(64, 64, 64, 0, True) == 0
     assert plan(64, (1 << 23) + 8, 64, 1, True) == 0 and plan(2 ** 31 - 1, 8, 32, 1, True) == 0
+
+
+def test_ragged_products_of_a_short_contraction_bring_no_room():
+    """Their second launch would cost a call from Python more than sharing K saves on the GPU (the library splits them for who brings the room)."""
+    from mase_hip.mxfp import kernels
+
+    class Library:
+        mase_hip_mxfp_gemm_workspace_bytes = staticmethod(lambda dense, M, N, K: 4096)
+
+    def room(M, N, K):
+        return kernels._workspace_bytes(Library, "no device", True, M, N, K)
+
+    try:
+        for M, N, K in ((1, 1000, 512), (16, 4001, 1312), (64, 1024, 1280), (65, 300, 992), (1000, 1673, 800), (200, 1024, 992), (129, 40, 896)):
+            assert room(M, N, K) == 0, (M, N, K)
+        for M, N, K in ((1, 1000, 1344), (64, 40, 4096), (65, 300, 1024), (1000, 1673, 2048), (65, 1024, 768), (512, 256, 512)):
+            assert room(M, N, K) == 4096, (M, N, K)
+    finally:
+        for key in [k for k in kernels._WS_BYTES if k[0] == "no device"]:
+            del kernels._WS_BYTES[key]
