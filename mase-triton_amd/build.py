@@ -27,6 +27,7 @@ BENCH_LIB = os.path.join(LIB_DIR, "libmase_bench.so")
 # the native side of the Python calls: plain C++ against torch's headers
 HOST_SRC = os.path.join(CSRC, "host", "bindings.cpp")
 HOST_LIB = os.path.join(LIB_DIR, "_mase_host.so")
+HOST_BUILT_FOR = os.path.join(OBJ, "_mase_host.built_for")    # the torch and the Python that the extension was compiled against
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -88,9 +89,23 @@ def build_library(force: bool = False, save_temps: bool = False, verbose: bool =
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
-    if force or _stale(HOST_LIB, [HOST_SRC, *_includes(HOST_SRC), LIB]):
+    if force or _stale(HOST_LIB, [HOST_SRC, *_includes(HOST_SRC), LIB]) or _read(HOST_BUILT_FOR) != host_built_for():
         build_host(verbose)
     return LIB
+
+
+def _read(path: str) -> str | None:
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        return f.read()
+
+
+def host_built_for() -> str:
+    """What the extension's binary interface depends on (mase_hip/_lib.py compares it when it loads the extension)."""
+    import torch
+
+    return f"torch {torch.__version__}, Python {sys.version_info.major}.{sys.version_info.minor}"
 
 
 def build_host(verbose: bool = True) -> None:
@@ -99,13 +114,17 @@ def build_host(verbose: bool = True) -> None:
     import torch
 
     torch_dir = os.path.dirname(os.path.abspath(torch.__file__))
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f'-DMASE_BUILT_FOR="{host_built_for()}"',
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-isystem", os.path.join(torch_dir, "include"), "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
            "-isystem", sysconfig.get_paths()["include"], HOST_SRC, "-o", HOST_LIB, "-L", os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
            "-L", LIB_DIR, "-lmase_hip", "-Wl,-rpath,$ORIGIN"]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
+    os.makedirs(OBJ, exist_ok=True)
+    with open(HOST_BUILT_FOR, "w") as f:
+        f.write(host_built_for())
 
 
 if __name__ == "__main__":

@@ -353,5 +353,10 @@ PyMODINIT_FUNC PyInit__mase_host(void) {
     g_raw_stream = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");
     Py_DECREF(c);
     if (!g_raw_stream) return nullptr;
-    return PyModule_Create(&kModule);
+    PyObject* const module = PyModule_Create(&kModule);
+    if (module && PyModule_AddStringConstant(module, "built_for", MASE_BUILT_FOR) < 0) {
+        Py_DECREF(module);
+        return nullptr;
+    }
+    return module;
 }

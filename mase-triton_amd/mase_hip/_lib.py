@@ -7,6 +7,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
 
 import torch
 
@@ -94,6 +95,9 @@ def host():
         loader = importlib.machinery.ExtensionFileLoader("_mase_host", _HOST_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("_mase_host", _HOST_PATH, loader=loader))
         loader.exec_module(module)
+        here = f"torch {torch.__version__}, Python {sys.version_info.major}.{sys.version_info.minor}"
+        if module.built_for != here:                       # (tensors cross the boundary as C++ objects)
+            raise RuntimeError(f"{_HOST_PATH} was built for {module.built_for} and this is {here}: build it again with `python mase-triton_amd/build.py`")
         _host = module
     return _host
 
