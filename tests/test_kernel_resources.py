@@ -58,3 +58,15 @@ def test_counted_wait_kernels_of_one_unit_use_no_scratch(tmp_path, unit, tag):
     assert sizes and all(int(size) == 0 for size in sizes.values()), sizes
     m0_writes = [ln for ln in text.splitlines() if re.search(r"\bm0\b", ln) and not ln.strip().startswith(";")]
     assert all(re.match(r"\s*s_mov_b32 m0, s\d+", ln) for ln in m0_writes), m0_writes[:5]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_counted_waits_of_the_scores_kernel_use_no_scratch(tmp_path):
+    """Of the attention-scores kernel (template arguments: format, quantise A, quantise W, K) the builds whose W is quantised before fetch it by
+    DMA and count their operations; those that quantise W wait with the compiler's own counts (at K = 128 they do use scratch)."""
+    text = _assembly("gemm_scores", str(tmp_path))
+    sizes = dict(zip(re.findall(r"^(_ZN4mase\w+):\s*; @", text, re.M), re.findall(r"; ScratchSize: (\d+)", text)))
+    counted = {name: size for name, size in sizes.items() if re.search(r"mxfp_scores_kernelI.*Lb[01]ELb0ELi(64|128)EE", name)}
+    assert len(counted) == 12 and all(int(size) == 0 for size in counted.values()), counted      # five formats and A as it is, two lengths of K
+    m0_writes = [ln for ln in text.splitlines() if re.search(r"\bm0\b", ln) and not ln.strip().startswith(";")]
+    assert all(re.match(r"\s*s_mov_b32 m0, s\d+", ln) for ln in m0_writes), m0_writes[:5]
