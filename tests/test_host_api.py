@@ -25,8 +25,8 @@ def lib():
     return _lib.load()
 
 
-def declared_symbols():
-    text = open(os.path.join(ROOT, "include", "mase_hip.h")).read()
+def declared_symbols(header="mase_hip.h"):
+    text = open(os.path.join(ROOT, "include", header)).read()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     return sorted(set(re.findall(r"\b(mase_hip_\w+)\s*\(", text)))
 
@@ -40,6 +40,38 @@ def test_library_exports_every_declared_symbol(lib):
         assert hasattr(lib, n), f"{n} declared in include/mase_hip.h but not exported"
     assert sorted(_lib.SIGNATURES) == names, "ctypes signatures out of step with the header"
     assert lib.mase_hip_abi_version() == 1
+
+
+def test_library_exports_the_scores_header(lib):
+    """include/mase_hip_scores.h, the second half of the interface."""
+    from mase_hip import _lib
+
+    names = declared_symbols("mase_hip_scores.h")
+    assert sorted(_lib.SCORES_SIGNATURES) == names and not set(names) & set(_lib.SIGNATURES)
+    text = open(os.path.join(ROOT, "include", "mase_hip_scores.h")).read()
+    text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
+    for n in names:
+        assert hasattr(lib, n), f"{n} declared in include/mase_hip_scores.h but not exported"
+        declared = re.search(rf"\b{n}\s*\(([^)]*)\)", text).group(1).split(",")
+        as_ctypes = [ctypes.c_void_p if "*" in a else ctypes.c_int64 if "int64_t" in a else ctypes.c_int for a in declared]
+        assert _lib.SCORES_SIGNATURES[n] == (ctypes.c_int, as_ctypes), n
+
+
+def test_scores_arguments_without_a_gpu(lib):
+    buf = (ctypes.c_uint8 * 256)()
+    p = ctypes.addressof(buf)
+    p += (-p) % 16
+
+    def call(a=p, e=4, m=3, w=p, qw=0, y=p, M=4, N=64, K=128, Z=1, sa=0, sw=0, sy=256):
+        return lib.mase_hip_mxfp_scores(a, e, m, w, qw, y, M, N, K, Z, sa, sw, sy, None)
+
+    assert call(M=0, a=None, w=None, y=None) == 0                                             # no rows
+    assert call(M=-1) == call(N=0) == call(K=0) == call(K=48) == call(a=None) == call(w=None) == call(y=None) == -1
+    assert call(K=160) == call(N=60) == call(N=(1 << 23) + 8) == call(M=2 ** 31 - 1) == -2
+    assert call(a=p + 2) == call(w=p + 8) == call(y=p + 4) == call(Z=0) == call(Z=2 ** 31) == -1
+    assert call(e=0, m=0, qw=1) == -1 and b"A's format" in lib.mase_hip_last_error()
+    assert call(Z=2, sa=8) == call(Z=2, sw=64) == call(Z=2, sy=8) == call(Z=2, sy=260) == call(Z=2, sa=516) == -1
+    assert call(e=4, m=2) == -1
 
 
 def test_argument_errors_without_a_gpu(lib):
