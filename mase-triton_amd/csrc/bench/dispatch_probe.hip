@@ -32,6 +32,11 @@ extern "C" int mase_bench_strided_column_tiles(int64_t columns, int64_t nkb, int
     return mase::strided_column_tiles(columns, nkb, element_bytes) ? 1 : 0;
 }
 
+// does an extract of 16-bit elements down the rows go two columns to a lane?  (bf16 whose extents are multiples of 128 goes before that)
+extern "C" int mase_bench_strided_pair_tiles(int64_t columns, int64_t nkb, int bf16) {
+    return mase::strided_pair_tiles(columns, nkb, bf16 != 0) ? 1 : 0;
+}
+
 // does a product without bias go to the kernel for short contractions?
 extern "C" int mase_bench_short_k(int64_t M, int64_t N, int64_t K, int64_t batches) {
     return mase::short_k_shape_ok((int)M, (int)N, (int)K, (int)batches) ? 1 : 0;

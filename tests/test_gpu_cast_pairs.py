@@ -1,6 +1,10 @@
-"""Extract down the rows of 16-bit matrices with an even inner axis, two columns to a lane: columns and k-blocks that fill tiles of 128 x 4
-and that do not, several outer matrices in one tile, every fp16 and bf16 bit pattern as an element and as the largest of its block, inf
-and NaN blocks beside ordinary ones; codes and scales against the checker bit for bit."""
+"""Extract down the rows of 16-bit matrices with an even inner axis, codes and scales against the checker bit for bit: sizes on both sides
+of the rule that takes them two columns to a lane, and, on that kernel by the rule's own answer, columns and k-blocks that fill tiles of
+128 x 4 and that do not, several outer matrices in one tile, every fp16 and bf16 bit pattern as an element and as the largest of its block, inf
+and NaN blocks beside ordinary ones."""
+import ctypes
+import os
+
 import pytest
 import torch
 
@@ -10,6 +14,20 @@ from helpers import PRESETS
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _two_columns_to_a_lane(shape, dim, dtype):
+    """Is mxfp_strided_pair_kernel what an extract of such a tensor runs?"""
+    lib = ctypes.CDLL(os.path.join(ROOT, "mase-triton_amd", "mase_hip", "lib", "libmase_bench.so"))
+    lib.mase_bench_strided_pair_tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    k, inner, columns = shape[dim], 1, 1
+    for i, d in enumerate(shape):
+        inner *= d if i > dim else 1
+        columns *= d if i != dim else 1
+    bf16 = dtype == torch.bfloat16
+    whole_lines = bf16 and inner % 128 == 0 and k % 128 == 0           # a kernel of their own
+    return inner % 2 == 0 and not whole_lines and bool(lib.mase_bench_strided_pair_tiles(columns, k // 32, bf16))
 
 
 def _check(x, block_dim, tag):
@@ -51,3 +69,46 @@ def test_every_pattern(dtype, tag):
         x.view(-1, 32, 512)[:, 5] = torch.tensor(2.0 ** top * 1.5, dtype=torch.float64).to(dtype)
         _check(x, 0, tag)
         _check(x.repeat(4, 1), 0, tag)
+
+
+PAIR_SHAPES = [((1024, 2050), 0), ((1056, 2048), 0), ((1056, 2050), 0), ((992, 2174), 0), ((3, 1056, 700), 1), ((6, 352, 1030), 1), ((350, 1056, 6), 1), ((2, 1088, 5, 206), 1)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,dim", PAIR_SHAPES)
+def test_two_columns_to_a_lane(dtype, shape, dim):
+    """Last tiles of 2 to 126 columns and of one to three k-blocks, outer matrices that end inside a tile; inf and NaN in some blocks."""
+    assert _two_columns_to_a_lane(shape, dim, dtype)
+    g = torch.Generator().manual_seed(sum(shape))
+    x = (torch.randn(*shape, generator=g) * torch.exp(3 * torch.randn(*shape[:-1], 1, generator=g))).to(dtype)
+    flat = x.view(-1)
+    for i, v in enumerate((float("inf"), float("-inf"), float("nan"))):
+        flat[torch.randint(0, flat.numel(), (200,), generator=g)] = v
+        flat[-1 - 5 * i] = v
+    for tag in PRESETS:
+        _check(x, dim, tag)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("tag", list(PRESETS))
+def test_every_pattern_two_columns_to_a_lane(dtype, tag):
+    """1056 x 2050 on that kernel: every bit pattern among its neighbours; every one in random company (fp16: inf or NaN in two blocks of
+    three); every finite one below block maxima of several binades."""
+    rows, columns = 1056, 2050
+    assert _two_columns_to_a_lane((rows, columns), 0, dtype)
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.int16)
+    g = torch.Generator().manual_seed(11)
+    near = torch.cat([bits.view(2048, 32).t(), bits[:64].view(32, 2)], 1)                 # 32 neighbours to a column
+    _check(torch.cat([near.roll(i, 1) for i in range(rows // 32)]).view(dtype).contiguous(), 0, tag)
+
+    def mixed(patterns):
+        n = -(-rows * columns // patterns.numel())
+        return torch.cat([patterns[torch.randperm(patterns.numel(), generator=g)] for _ in range(n)])[:rows * columns].view(rows, columns).contiguous()
+
+    _check(mixed(bits).view(dtype), 0, tag)
+    finite = bits[bits.view(dtype).isfinite()]
+    for top in ([-14, -2, 3, 15] if dtype == torch.float16 else [-100, -14, 0, 20, 127]):
+        x = mixed(finite).view(dtype)
+        x = torch.where(x.abs().double() < 2.0 ** top, x, torch.zeros_like(x))
+        x.view(-1, 32, columns)[:, 5] = torch.tensor(2.0 ** top * 1.5, dtype=torch.float64).to(dtype)
+        _check(x, 0, tag)
