@@ -291,6 +291,46 @@ def test_other_threads_run_beside_a_call():
         thread.join()
 
 
+@pytest.mark.parametrize("take", range(9))
+def test_the_module_takes_plain_calls(take):
+    """(Where it took none, both sides of the comparisons above would be the wrappers.)"""
+    name, call = list(_plain_calls().items())[take]
+    assert call() is not None, name
+
+
+@pytest.mark.parametrize("kind", ["mxfp", "minifloat"])
+def test_layers_go_through_the_module(monkeypatch, kind):
+    """From the second call of a kind on; again after a call of another look."""
+    import mase_hip.minifloat.layers as ML
+    import mase_hip.minifloat.meta as mf
+    import mase_hip.mxfp.layers as XL
+    import mase_hip.mxfp.meta as mx
+    from mase_hip import _lib
+
+    w = torch.randn(520, 512, device=DEV).to(torch.bfloat16)
+    layer = (XL.MXFPLinearPTQ(w, None, mx.MXFP8_E4M3_fn, mx.OCP_MXFP6_E3M2, None, "XqWqB", "fused") if kind == "mxfp" else
+             ML.MinifloatLinearPTQ(weight=w, bias=None, x_minifloat_meta=mf.FP8_E4M3_fn, w_minifloat_meta=mf.FP6_E2M3_fn, b_minifloat_meta=None, layer_type="XqWqB",
+                                   backend="fused"))
+    host, seen = _lib.host(), []
+
+    class Watched:
+        def __getattr__(self, name):
+            def call(*args):
+                y = getattr(host, name)(*args)
+                if name == "linear_scaled":
+                    seen.append(y)
+                return y
+            return call
+
+    monkeypatch.setattr(_lib, "_host", Watched())
+    for rows, calls in ((3, 0), (3, 1), (3, 2), (70, 2), (70, 3), (3, 3), (3, 4)):
+        y = layer(torch.randn(rows, 512, device=DEV).to(torch.bfloat16))
+        assert len(seen) == calls
+        assert seen == [] or all(t is not None for t in seen)
+        if calls and rows == 3 and calls in (1, 2, 4):
+            assert y is seen[-1]
+
+
 def test_streams_and_capture():
     """The call runs on the current stream, also while it is captured."""
     import mase_hip.mxfp.functional as MX
