@@ -1,5 +1,5 @@
 // Block-scaled MXFP GEMM for tens to hundreds of rows of A (a large decode batch, a chunk of a prompt), operands in the prepared
-// form of gemm_scaled.h, on tiles of 128 x 128 or 128 x 64; and of 64 x 64 for 17 - 64 rows.
+// form of gemm_scaled.h, on tiles of 128 x 128 or 128 x 64; and of 64 x 64 for up to 64 rows (plan_scaled_few).
 //
 // At these sizes the 256 x 256 tiles of gemm_scaled.h leave most CUs without one (200 x 14336 outputs: 56 tiles for 256 CUs), and
 // splitting K for more of them costs fp32 partial sums of 256-row tiles that are mostly padding.  Smaller tiles give every CU
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         static_for<RING>([&](auto u_c) __attribute__((always_inline)) {
             constexpr int u = decltype(u_c)::value, set = u & 1, next = (u + 1) % RING;
             if (base + u < nm) {
-                // stage s + 1 of this wavefront has landed (those of s + 2 and s + 3 may still fly), step s is in registers
+                // stage s + 1 of this wavefront has landed (the RING - 2 stages behind it may still fly), step s is in registers
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 2) * OPS) : "memory");
                 lds_barrier();
                 asm volatile("" ::: "memory");
@@ -248,6 +248,11 @@ inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
 // 8192 x 2048 16 rows 7.1 / 7.8 | 7.1 / 7.5, 64 rows 7.1 / 12.1 | 7.1 / 11.8; 4096 x 4096 32 rows 9.4 / 8.1 | 9.4 / 7.5, 64 rows 9.4 / 10.3 | 9.4 / 9.7.  Layer calls
 // of 48 rows, before and now: 14336 x 768 18.2 / 8.7, 8192 x 8192 27.3 / 21.5, 2176 x 10752 18.1 / 15.6.  (Tiles of 64 x 128 are never ahead: 14336 x
 // 4096 21.2 | 13.8.)  bn == 0: a weight-streaming kernel.
+// The tiles' price for K up to 4096 is fitted to the operand of x and the product, another W on every call (where the tiles lose more than
+// alone), by the other kernel's operand tiles: of 2100 shapes eight come out more than 2 % slower than on the other kernel (worst 49 x 4096 x
+// 3072, 14.8 / 13.3), 145 with the price of a longer K for all.  Tiles / the other kernel, us: 17 x 8192 x 2560 14.6 / 12.3, 1 x 8192 x 2048
+// 11.7 / 10.1, 32 x 32768 x 2560 29.2 / 25.2, 5 x 93008 x 1792 50.7 / 43.9, 64 x 65536 x 3072 58.4 / 52.4, but 16 x 14336 x 768 9.0 / 13.0, 17 x 65536 x 512
+// 22 / 35, 64 x 14336 x 4096 20.6 / 23.9.
 inline ScaledMidPlan plan_scaled_few(int M, int N, int K, int cus, bool may_split) {
     const int nmac = K / SMAC;
     ScaledMidPlan best{0, 0, 1, nmac};
@@ -258,7 +263,7 @@ inline ScaledMidPlan plan_scaled_few(int M, int N, int K, int cus, bool may_spli
     auto split_cost = [&](int splits) { return splits > 1 ? 3.0 + (2.0 * splits + 0.5) * mn_mb * 0.16 : 0.0; };
     // the other kernel: prologue, then units of 16 rows of W x (a slice of) K, the last as half units; a unit takes its latency at least
     const int slices = K > 4096 ? (may_split ? scaled_rows_slices(M, N, K) : 0) : 1;
-    double best_t = 1e30;                                   // (33 rows and more without room for its sums: these tiles, or 128-row ones)
+    double best_t = 1e30;                                   // (33 rows and more without room for its sums: these tiles)
     if (slices > 0) {
         const int mt = (M + 15) / 16, groups = (N + 15) / 16, per_slice = std::max(1, std::min(groups, cus / slices));
         const double units = slices > 1 ? (groups + per_slice - 1) / per_slice : std::max(1.0, std::ceil(2.0 * groups / cus) / 2.0);
@@ -266,6 +271,12 @@ inline ScaledMidPlan plan_scaled_few(int M, int N, int K, int cus, bool may_spli
         best_t = 3.8 + 0.9 * mt * (0.5 + 0.5 * busy) + units * (std::max(1.6, (double)nmac / slices / 32.0 * 2.15) * (0.4 + 0.6 * busy) + 0.25 * mt) +
                  split_cost(slices) - 0.5;
     }
+    struct Price { double step, busy, round, launch; };
+    const Price price = K > 4096  ? Price{0.15, 0.28, 1.2, 2.0}
+                        : M <= 16 ? Price{0.24, 0.36, 1.2, 2.0}
+                        : M <= 32 ? Price{0.21, 0.36, 1.2, 1.5}
+                        : M <= 48 ? Price{0.15, 0.28, 2.1, 1.1}
+                                  : Price{0.19, 0.32, 1.8, 0.5};
     const int64_t tiles = (N + 63) / 64;
     for (int want = 1; want <= 16; ++want) {
         if (want > 1 && (!may_split || tiles * want > cus || N % 4 != 0)) break;
@@ -273,7 +284,7 @@ inline ScaledMidPlan plan_scaled_few(int M, int N, int K, int cus, bool may_spli
         if (want > 1 && (per < 12 || (nmac + per - 1) / per != want)) continue;
         const int64_t wgs = tiles * want;
         const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
-        const double t = (double)((wgs + cus - 1) / cus) * (per * (0.15 + 0.28 * busy) + 1.2) + 2.0 + split_cost(want);
+        const double t = (double)((wgs + cus - 1) / cus) * (per * (price.step + price.busy * busy) + price.round) + price.launch + split_cost(want);
         if (t < best_t) { best_t = t; best = ScaledMidPlan{64, 64, want, per}; }
     }
     return best;

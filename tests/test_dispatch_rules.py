@@ -157,3 +157,12 @@ def test_ragged_products_of_a_short_contraction_bring_no_room():
     finally:
         for key in [k for k in kernels._WS_BYTES if k[0] == "no device"]:
             del kernels._WS_BYTES[key]
+
+
+def test_few_rows_stay_with_the_weight_streaming_kernel_where_it_is_ahead(lib):
+    """K of 1280 to 3584: tiles of 64 x 64 took 1.06 - 1.19 times as long for these (operand of x and product, another W on every call)."""
+    for shape in ((1, 8192, 2048), (16, 8192, 2048), (1, 24576, 1536), (16, 20480, 1280), (5, 93008, 1792), (16, 48848, 2048), (1, 1536, 1280), (10, 1096, 1280),
+                  (17, 8192, 2560), (32, 32768, 2560), (26, 4424, 2560), (17, 16384, 3072), (64, 4096, 3584), (64, 65536, 3072)):
+        assert scaled_plan(lib, *shape)[0] == 0, shape
+    for shape in ((1, 12288, 1024), (16, 14336, 768), (17, 65536, 512), (32, 8192, 1536), (33, 8192, 2048), (64, 8192, 2048), (48, 4096, 14336), (64, 14336, 4096)):
+        assert scaled_plan(lib, *shape)[0] == 64, shape
