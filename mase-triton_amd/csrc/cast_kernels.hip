@@ -290,30 +290,18 @@ __device__ inline uint32_t block_max(uint32_t amax, int lpb) {
 // Scale byte and codes of N elements of one block whose largest |x| has bits `amax` (the block's lanes agree on it).  A compile-time
 // format takes the branch-free encoder unless some block of the wavefront is out of its range (a uniform test): with the general
 // routine the vector instructions and not the memory bound the casts (4096 x 4096, blocks along the rows: fp16 extract 22.4 -> 15.1 us,
-// fused pass 29.8 -> 17.3, fp32 extract 18.4 -> 16.9; fused pass of [2976, 4096] down the rows: fp16 33.2 -> 15.0, fp32 20.5 -> 17.5).  A block
-// that holds inf or NaN has scale 255, the NaN code where they are and 0 elsewhere: POISONED sets these behind a uniform test, where a lane
-// has a whole block of 32 (the general routine for such a wavefront was the last thing a launch waited for: extract of one inf
-// 7.6 -> 4.8 us); the fused pass down the rows keeps the general routine, with whose registers it is 8 % faster.
-template <int DT_IN, class F, int N, bool POISONED = false>
+// fused pass 29.8 -> 17.3, fp32 extract 18.4 -> 16.9; fused pass of [2976, 4096] down the rows: fp16 33.2 -> 15.0, fp32 20.5 -> 17.5).
+template <int DT_IN, class F, int N>
 __device__ inline void mxfp_encode(const uint32_t (&u)[N], uint32_t amax, const F& f, uint32_t (&code)[N], uint32_t& scale) {
     if constexpr (F::kStatic) {
         const int top = DT_IN != F32 ? (int)(amax >> 23) : floor_log2_fp32(amax) + 127;
         const int sc = amax < 0x00800000u ? 0 : max(top - fmt_emax_unb(f), 0);   // largest |x| flushed: scale 0, every code 0
-        const bool nonfinite = POISONED && amax >= 0x7F800000u;
-        const bool hard = !nonfinite && (amax >= 0x7F800000u || sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f)));
+        const bool hard = amax >= 0x7F800000u || sc >= 151 || (amax >= 0x00800000u && sc < fmt_bias(f));
         if (__builtin_amdgcn_ballot_w64(hard) == 0) {
             const uint32_t off = (uint32_t)max(sc - fmt_bias(f), 0) << 15;
-            scale = nonfinite ? 255u : (uint32_t)sc;
+            scale = (uint32_t)sc;
 #pragma unroll
             for (int j = 0; j < N; ++j) code[j] = encode_mxfp_in_range<F>(u[j], off);
-            if (POISONED && __builtin_amdgcn_ballot_w64(nonfinite) != 0) {
-#pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    const bool e = (u[j] & 0x7FFFFFFFu) >= 0x7F800000u;
-                    if (nonfinite) code[j] = 0u;
-                    if (__builtin_amdgcn_ballot_w64(e) != 0 && e) code[j] = encode_nonfinite(false, true, u[j] & 0x7FFFFFu, f);
-                }
-            }
             return;
         }
     }
@@ -943,6 +931,24 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_bf16_lines_kernel(const
     }
 }
 
+// A block that holds inf or NaN has scale 255, the NaN code where they are and 0 elsewhere.  The general routine for such a lane's 32
+// elements would be the last thing that a launch waits for (extract of one inf 7.6 us, so 4.8): what is not finite becomes the number below one
+// that a finite format's NaN code stands for (exponent -1, quiet bit set), the rest zero, and the block a block of scale 1 that is encoded like any
+// other.  Before the encoder, so that it costs no registers: setting the codes afterwards kept 32 more alive (fp16 tiles 74 -> 103 registers,
+// bf16 137), and 2976 x 4095 without any inf went from 15.0 to 17.4 us (bf16), 14.9 -> 16.0 (fp16), 18.4 -> 19.6 (fp32).
+// true: the lane's block is one; its scale byte is 255.
+template <class F, int N>
+__device__ inline bool replace_nonfinite(uint32_t (&u)[N], uint32_t& amax, const F& f) {
+    static_assert(F::kStatic, "finite formats");
+    const bool poisoned = amax >= 0x7F800000u;
+    if (__builtin_amdgcn_ballot_w64(poisoned) != 0 && poisoned) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) u[j] = (u[j] & 0x7FFFFFFFu) >= 0x7F800000u ? 0x3F400000u | (u[j] & 0x7FFFFFu) : 0u;
+        amax = (uint32_t)(127 + fmt_emax_unb(f)) << 23;
+    }
+    return poisoned;
+}
+
 // Extract for any dtype and extents and a compile-time format: the same exchange with one column to a lane.  A workgroup takes 64
 // adjacent columns of the [outer * inner] there are (a lane finds its own place, so a short inner axis beside a long outer one fills the
 // wavefronts too; few columns in all do not, see strided_column_tiles) and four consecutive k-blocks, one per wavefront; what
@@ -974,7 +980,9 @@ __global__ __launch_bounds__(kThreads) void mxfp_strided_tile_kernel(const void*
         for (int j = 0; j < 32; ++j) u[j] = load_bits_scalar<DT_IN>(x, first + j * inner);
 #pragma unroll
         for (int j = 0; j < 32; ++j) amax = max(amax, u[j] & 0x7FFFFFFFu);
-        mxfp_encode<DT_IN, F, 32, true>(u, amax, f, code, scale);
+        const bool poisoned = replace_nonfinite(u, amax, f);
+        mxfp_encode<DT_IN, F, 32>(u, amax, f, code, scale);
+        if (poisoned) scale = 255u;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             uint32_t w[4];

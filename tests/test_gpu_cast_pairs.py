@@ -112,3 +112,29 @@ def test_every_pattern_two_columns_to_a_lane(dtype, tag):
         x = torch.where(x.abs().double() < 2.0 ** top, x, torch.zeros_like(x))
         x.view(-1, 32, columns)[:, 5] = torch.tensor(2.0 ** top * 1.5, dtype=torch.float64).to(dtype)
         _check(x, 0, tag)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tag", list(PRESETS))
+def test_nonfinite_blocks_one_column_to_a_lane(dtype, tag):
+    """An odd number of columns: blocks of inf and of NaN with every payload beside ordinary blocks, zeros and blocks for the general routine
+    (scales below the format's bias or past 150) in one wavefront."""
+    g = torch.Generator().manual_seed(13)
+    rows, columns = 128, 513
+    if dtype == torch.float32:
+        x = torch.randn(rows, columns, generator=g)
+        bits = x.view(torch.int32).view(-1)
+        some = torch.randperm(rows * columns, generator=g)[:3000]
+        bits[some] = 0x7F800000 | (torch.randint(0, 1 << 23, (3000,), generator=g).to(torch.int32) << torch.randint(0, 23, (3000,), generator=g).to(torch.int32) & 0x7FFFFF)
+        bits[some[::2]] |= -(1 << 31)
+    else:
+        x = torch.arange(65536, dtype=torch.int32).to(torch.int16)[torch.randperm(65536, generator=g)].view(dtype)
+        x = torch.cat([x, x[:rows * columns - 65536]]).view(rows, columns).contiguous()
+    _check(x, 0, tag)
+    sparse = torch.randn(rows, columns, generator=g).to(dtype)
+    sparse[:, ::7] = 0.0
+    if dtype != torch.float16:
+        sparse[:, 3::11] *= 1e30
+        sparse[:, 4::13] *= 1e-37
+    sparse[5, ::5], sparse[77, 1::9], sparse[100, 2::17] = float("inf"), float("nan"), float("-inf")
+    _check(sparse, 0, tag)

@@ -70,3 +70,13 @@ def test_counted_waits_of_the_scores_kernel_use_no_scratch(tmp_path):
     assert len(counted) == 12 and all(int(size) == 0 for size in counted.values()), counted      # five formats and A as it is, two lengths of K
     m0_writes = [ln for ln in text.splitlines() if re.search(r"\bm0\b", ln) and not ln.strip().startswith(";")]
     assert all(re.match(r"\s*s_mov_b32 m0, s\d+", ln) for ln in m0_writes), m0_writes[:5]
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_extract_down_the_rows_leaves_room_for_six_wavefronts(tmp_path):
+    """mxfp_strided_tile_kernel waits for memory with up to six wavefronts per SIMD: with code that kept a block's values alive beside its codes it had
+    three or four and took up to 17 % longer."""
+    text = _assembly("cast_kernels", str(tmp_path))
+    occupancy = dict(zip(re.findall(r"^(_ZN4mase\w+):\s*; @", text, re.M), re.findall(r"; Occupancy: (\d+)", text)))
+    occupancy = {name: int(n) for name, n in occupancy.items() if "mxfp_strided_tile_kernel" in name}
+    assert len(occupancy) == 15 and min(occupancy.values()) >= 6, occupancy
