@@ -33,8 +33,8 @@ extern "C" int mase_bench_strided_column_tiles(int64_t columns, int64_t nkb, int
 }
 
 // does an extract of 16-bit elements down the rows go two columns to a lane?  (bf16 whose extents are multiples of 128 goes before that)
-extern "C" int mase_bench_strided_pair_tiles(int64_t columns, int64_t nkb, int bf16) {
-    return mase::strided_pair_tiles(columns, nkb, bf16 != 0) ? 1 : 0;
+extern "C" int mase_bench_strided_pair_tiles(int64_t inner, int64_t columns, int64_t nkb, int bf16) {
+    return mase::strided_pair_tiles(inner, columns, nkb, bf16 != 0) ? 1 : 0;
 }
 
 // does a product without bias go to the kernel for short contractions?

@@ -1424,7 +1424,7 @@ int mase_hip_extract_mxfp_strided(const void* x, int x_dtype, uint8_t* scales, u
             if (x_dtype != F32 && inner % 2 == 0 && aligned(x, 4) && el16) {
                 const int64_t columns = outer * inner, nkb = k_len / 32, tiles = (columns + kStridedTCols - 1) / kStridedTCols;
                 const int64_t blocks = (tiles * ((nkb + 3) / 4) + 7) / 8 * 8;
-                if (blocks <= 0x7FFFFFFFll && strided_pair_tiles(columns, nkb, x_dtype == BF16)) {
+                if (blocks <= 0x7FFFFFFFll && strided_pair_tiles(inner, columns, nkb, x_dtype == BF16)) {
                     auto go = [&](auto dt) {
                         hipLaunchKernelGGL((mxfp_strided_pair_kernel<decltype(dt)::value, decltype(f)>), dim3((unsigned)blocks), dim3(kThreads), 0, s,
                                            static_cast<const uint16_t*>(x), scales, elements, k_len, inner, columns, nkb, tiles, f);

@@ -101,11 +101,17 @@ inline bool strided_column_tiles(int64_t columns, int64_t nkb, int element_bytes
 // kernel that stores a column's codes by itself, us: 2976 x 4096 11.2 / 12.6, 65536 x 200 12.5 / 15.6, 1024 x 2050 4.8 / 6.1; tiles that the columns or k-blocks
 // leave half empty cost once there are many: 160 x 65536 (five k-blocks) 13.5 / 10.8, 32 x 262144 level without it.  fp16, against one column to a lane:
 // 2976 x 4096 12.5 / 14.7, 65536 x 200 13.6 / 17.5, 256 x 9000 5.2 / 6.0; with fewer wavefronts the other kernel's shorter lanes are ahead: 96 x 14336 4.9 / 4.5,
-// 64 x 1000 4.6 / 4.2.
-inline bool strided_pair_tiles(int64_t columns, int64_t nkb, bool bf16) {
+// 64 x 1000 4.6 / 4.2, 64 matrices of 512 x 64 5.3 / 4.9.
+// Rows (the inner axis) of a few columns behind a longer outer axis: a load then takes pieces of many matrices.  bf16 rows of fewer than 80 columns:
+// filled tiles are behind (1000 matrices of 2080 x 2 15.5 / 10.4, 32 of 87360 x 6 26.2 / 19.0, 128 of 10912 x 12 20.0 / 17.0, 3 of 2048 or 8192 x 32 7.3 / 6.8
+// and 17.7 / 17.1; at best 3 % ahead), a few columns in all are what the other kernel leaves its lanes idle for (65536 x 2 4.1 / 6.9, 8 x 4096 x 8 4.4 /
+// 4.8) until their wavefronts are many (36832 x 64 6.4 / 5.7, 11 of 27776 x 12 8.6 / 6.7).  fp16: rows of 4 (32 matrices of 32768 or 131072: 9.2 / 7.5, 26.9 /
+// 19.6) and 12 columns (9.1 / 8.4, level when many); 2, 6, 8 and longer ones are ahead (10.6 / 12.3, 6.8 / 7.3).
+inline bool strided_pair_tiles(int64_t inner, int64_t columns, int64_t nkb, bool bf16) {
     const int64_t tiles = (columns + 127) / 128, groups = (nkb + 3) / 4, waves = tiles * groups * 4;
     const bool filled = columns * nkb * 10 >= tiles * 128 * groups * 4 * 7;
-    return bf16 ? filled || waves < 2048 : filled && waves >= 512;
+    if (!bf16) return filled && waves > 512 && inner != 4 && inner != 12;
+    return inner < 80 ? !filled && waves <= 1024 : filled || waves < 2048;
 }
 
 // Calls fn(format object): a compile-time format for the five round-to-nearest finite

@@ -115,6 +115,24 @@ def test_one_full_round_of_large_tiles_is_not_given_to_two_of_small_ones(lib):
         assert scaled_plan(lib, *shape)[0] == bn
 
 
+def test_short_rows_behind_an_outer_axis_do_not_go_two_columns_to_a_lane(lib):
+    """(matrices, rows, columns): a tenth to half slower than the other kernels there."""
+    rule = lib.mase_bench_strided_pair_tiles
+    rule.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int]
+
+    def pair(outer, k, inner, bf16):
+        return bool(rule(inner, outer * inner, k // 32, bf16))
+
+    for shape in ((1000, 2080, 2), (32, 87360, 6), (1000, 672, 6), (128, 10912, 12), (8, 26208, 20), (11, 27776, 12), (1, 36832, 64), (29, 102272, 4), (128, 3584, 40)):
+        assert not pair(*shape, 1), shape
+    for shape in ((29, 69888, 4), (32, 131072, 4), (1000, 1024, 4), (1000, 352, 12), (64, 512, 64), (32, 1024, 64)):
+        assert not pair(*shape, 0), shape
+    for shape in ((1, 2976, 4096), (1, 65536, 200), (1, 1024, 2050), (4, 4096, 320), (1, 32768, 2), (8, 4096, 8), (3, 4096, 12)):
+        assert pair(*shape, 1), shape
+    for shape in ((1, 2976, 4096), (1, 65536, 200), (1, 1024, 2050), (128, 16384, 2), (32, 87360, 6), (32, 65536, 8), (64, 2048, 64)):
+        assert pair(*shape, 0), shape
+
+
 def test_ways_of_a_product_of_short_contraction():
     """2: queries and keys quantised inside the kernel of whole rows, 1: keys in a pass before it, 0: the general kernels."""
     from mase_hip.mxfp.kernels import scores_plan as plan

@@ -20,14 +20,14 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 def _two_columns_to_a_lane(shape, dim, dtype):
     """Is mxfp_strided_pair_kernel what an extract of such a tensor runs?"""
     lib = ctypes.CDLL(os.path.join(ROOT, "mase-triton_amd", "mase_hip", "lib", "libmase_bench.so"))
-    lib.mase_bench_strided_pair_tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    lib.mase_bench_strided_pair_tiles.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int]
     k, inner, columns = shape[dim], 1, 1
     for i, d in enumerate(shape):
         inner *= d if i > dim else 1
         columns *= d if i != dim else 1
     bf16 = dtype == torch.bfloat16
     whole_lines = bf16 and inner % 128 == 0 and k % 128 == 0           # a kernel of their own
-    return inner % 2 == 0 and not whole_lines and bool(lib.mase_bench_strided_pair_tiles(columns, k // 32, bf16))
+    return inner % 2 == 0 and not whole_lines and bool(lib.mase_bench_strided_pair_tiles(inner, columns, k // 32, bf16))
 
 
 def _check(x, block_dim, tag):
@@ -71,11 +71,12 @@ def test_every_pattern(dtype, tag):
         _check(x.repeat(4, 1), 0, tag)
 
 
-PAIR_SHAPES = [((1024, 2050), 0), ((1056, 2048), 0), ((1056, 2050), 0), ((992, 2174), 0), ((3, 1056, 700), 1), ((6, 352, 1030), 1), ((350, 1056, 6), 1), ((2, 1088, 5, 206), 1)]
+PAIR_SHAPES = [(s, d, t) for t in (torch.float16, torch.bfloat16) for s, d in
+               (((1024, 2050), 0), ((1056, 2048), 0), ((1056, 2050), 0), ((992, 2174), 0), ((3, 1056, 700), 1), ((6, 352, 1030), 1), ((2, 1088, 5, 206), 1))]
+PAIR_SHAPES += [((350, 1056, 6), 1, torch.float16), ((8, 1056, 6), 1, torch.bfloat16), ((3, 2080, 20), 1, torch.bfloat16), ((1056, 2), 0, torch.bfloat16)]
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("shape,dim", PAIR_SHAPES)
+@pytest.mark.parametrize("shape,dim,dtype", PAIR_SHAPES)
 def test_two_columns_to_a_lane(dtype, shape, dim):
     """Last tiles of 2 to 126 columns and of one to three k-blocks, outer matrices that end inside a tile; inf and NaN in some blocks."""
     assert _two_columns_to_a_lane(shape, dim, dtype)
