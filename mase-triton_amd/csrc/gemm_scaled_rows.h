@@ -197,9 +197,9 @@ __device__ inline RowsUnit rows_unit(int b, int u, int grid, int full_rounds, in
 // bytes of a row at a time, every cache line is fetched twice, and with every CU of an XCD asking its L2 for the same A
 // that is what the prologue costs: 22 against 19 us at 64 rows, N x K = 14336 x 4096).  The wavefronts' partial sums meet
 // in LDS; wavefront t adds and stores tile t.  Eight wavefronts: 15.6 against 18.4 us with four at 32 rows (sixteen: the
-// same, and the registers of four tiles no longer fit).  N x K = 14336 x 4096: 14.0 / 15.6 / 19.2 us at 16 / 32 / 64 rows against
-// 20.9 / 23.2 / 30.8 on the bf16 weight-streaming kernels (23.8 / 26.9 at 32 / 64 rows on the chunked and the tile kernel); 4096 x
-// 4096: 6.8 / 7.6 / 10.0 against 9.7 / 10.7 / 16.9.  (A build that kept 16 rows of A in LDS instead, four wavefronts: 14.8 us at
+// same, and the registers of four tiles no longer fit).  N x K = 14336 x 4096: 14.0 / 15.6 us at 16 / 32 rows against 20.9 / 23.2 on the
+// bf16 weight-streaming kernels (32 rows on the chunked kernel: 23.8); 4096 x 4096: 6.8 / 7.6 / 10.0 at 16 / 32 / 64 rows against 9.7 / 10.7 /
+// 16.9.  (64 rows of 14336 x 4096 take 19.2 us here and 16.9 on the 64 x 64 tiles of gemm_scaled_mid.h, which plan_scaled_few picks.)  (A build that kept 16 rows of A in LDS instead, four wavefronts: 14.8 us at
 // 16 rows where this one takes 14.0, same box.)
 // W by DMA into two LDS units, the next but one asked for before the wait for the next (one to two units in flight per CU,
 // no registers on the way), measured 15.1 / 16.4 / 19.9 us at 16 / 32 / 64 rows: no faster, so the time is not in a pipe that runs
@@ -357,9 +357,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WAVE
 inline bool scaled_rows_shape_ok(int M, int K) { return K >= 128 && (M <= 32 || (M <= 64 && K <= 4096)); }
 
 // K beyond what a wavefront's registers hold of A in one piece, 17 - 64 rows: slices of at most 32 macro steps, their sums added
-// by a second kernel (room for them: slices * M * N * 4 bytes).  0: not a shape for this.  N x K = 4096 x 14336: 18.4 / 23.0 us
-// at 32 / 64 rows against 23.3 (the chunked kernel) / 31.0 (the tile kernel, K split) and 27.8 / 49.4 on the bf16 kernels; 8192 x
-// 8192: 19.4 / 24.4 against 23.2 / 30.2 and 29.5 / 42.6.  (Up to 16 rows the chunked kernel is level: 17.7 us, one launch.)
+// by a second kernel (room for them: slices * M * N * 4 bytes).  0: not a shape for this.  From 33 rows on plan_scaled_few prices it against
+// 64 x 64 tiles.  32 rows of 4096 x 14336 (N x K): 18.4 us against 23.3 on the chunked kernel and 27.8 on the bf16 ones; of 8192 x 8192 19.4
+// against 23.2 and 29.5.  (Up to 16 rows the chunked kernel is level: 17.7 us, one launch.)
 inline int scaled_rows_slices(int M, int N, int K) {
     if (M <= 16 || M > 64 || K <= 4096 || K % 128 != 0 || N % 4 != 0) return 0;
     return (K / 128 + 31) / 32;

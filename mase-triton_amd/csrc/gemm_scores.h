@@ -47,7 +47,8 @@ struct ScoresArgs {
 // QA / QW: quantise A / W in format F on the way in.  KP: the K the loops are built for (64 or 128); a smaller K is filled with zeros.
 // Wavefronts 0 - 3 multiply and store, the others (one, or four that quantise) bring W.  A wavefront's memory operations complete
 // in order, and a store takes microseconds to be acknowledged while the memory is busy writing: a wavefront that stored and
-// waited for loads as well would wait for its stores.
+// waited for loads as well would wait for its stores.  (The builds of KP = 128 that quantise W do: 128 registers are all that four wavefronts
+// per SIMD leave them, and 72 - 80 bytes per lane go through scratch.  They wait with the compiler's counts only; mase_hip_mxfp_scores_plan has their times.)
 template <class F, bool QA, bool QW, int KP>
 __global__ __launch_bounds__(sco_threads<QW>()) __attribute__((amdgpu_waves_per_eu(QW ? 4 : 2))) void mxfp_scores_kernel(const ScoresArgs p) {
     constexpr int Q = KP / 16;                             // 16-k steps

@@ -37,8 +37,8 @@ _LAYER_TYPES = ("XWB", "XWBq", "XWqB", "XWqBq", "XqWB", "XqWBq", "XqWqB", "XqWqB
 _GEMM_DTYPES = (torch.bfloat16, torch.float32)
 _BACKENDS = ("separate", "fused", "fused_bf16", "fused_scaled")
 # Which row counts of x backend="fused" sends to the block-scaled kernels.  With the weight operand at hand (a layer keeps
-# it): all of them.  Up to 64 rows the product is a read of W, which the block-scaled weight-streaming kernels do without
-# touching the codes; beyond, 128- and 256-row tiles, K split over workgroups where they are few, stay ahead.  GEMMs alone, another W
+# it): all of them.  Up to 64 rows the product is a read of W, which the block-scaled weight-streaming kernels and 64-row tiles do
+# without touching the codes; beyond, 128- and 256-row tiles, K split over workgroups where they are few, stay ahead.  GEMMs alone, another W
 # on every call, block-scaled against bf16 kernels, us, at 16 / 32 / 64 / 128 / 256 / 512 / 1024 rows: N x K = 14336 x 4096 15 / 17 / 20 / 22 / 27 /
 # 46 / 50 against 23 / 25 / 31 / 35 / 43 / 72 / 105; 4096 x 14336 19 / 19 / 23 / 25 / 31 / 45 / 66 against 26 / 29 / 50 / 35 / 47 / 77 / 110.
 # When the operand has to be built inside the call (N * K bytes read and written) the whole call takes 50 / 55 / 68 / 72 / 79 us
