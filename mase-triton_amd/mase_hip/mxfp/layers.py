@@ -105,6 +105,15 @@ class MXFPLinearPTQ(nn.Module):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
         self._no_operand_sig = None
+        if self.w_scales is not None:
+            # (a move that moved nothing keeps the weight's other forms)
+            key = (self.w_elements.data_ptr(), self.w_elements._version, self.w_scales.data_ptr(), self.w_scales._version)
+            if self._scaled_w_key != key:
+                self._scaled_w = self._scaled_w_key = None
+            if self._packed_w_key != key:
+                self._packed_w = self._packed_w_key = None
+            if self._scaled_w is None or self._packed_w is None:
+                self._fast_sig = None
         for name, dt in before.items():
             now = getattr(self, name).dtype
             if now != dt:
