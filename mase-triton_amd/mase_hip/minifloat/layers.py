@@ -8,14 +8,14 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm
 from . import functional as MinifloatF
 from .meta import MinifloatMeta, MinifloatTensorMeta
 
 LayerType = Literal["XWB", "XWBq", "XWqB", "XWqBq", "XqWB", "XqWBq", "XqWqB", "XqWqBq"]
 
 
-class MinifloatLinearPTQ(nn.Module):
+class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
     """``y = x W^T + b`` with any of x / W / b held or rounded in a minifloat format.
 
     Quantised weights and biases are stored as uint16 code tensors (``w_element``,
@@ -26,7 +26,9 @@ class MinifloatLinearPTQ(nn.Module):
     in_features: int
     out_features: int
     _CODE_PARAMS = ("w_element", "b_element")
-    _packed_w = _packed_w_key = None   # the weight packed at its own width, and what it was built from
+    _FORMS = ("_narrowed", "_scaled_w", "_packed_w")      # the codes in one byte each, in the block-scaled GEMM's form, and packed at their own width
+    _FORM_COMPONENTS = ("w_element",)
+    _narrowed = _scaled_w = _packed_w = None
     _fast_packed = 0         # was the call that _fast_sig notes one on the packed weight (1: x quantised, 2: dense) or on the one-byte codes (3)?
     _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
@@ -70,8 +72,6 @@ class MinifloatLinearPTQ(nn.Module):
         self.weight = self.bias = None
         self.w_element = self.w_tensor_meta = None
         self.b_element = self.b_tensor_meta = None
-        self._narrowed = self._narrowed_key = None
-        self._scaled_w = self._scaled_w_key = None
         self._fast_sig = None   # what the last call on the block-scaled route looked like (see forward)
 
         if "Wq" in layer_type:
@@ -95,9 +95,8 @@ class MinifloatLinearPTQ(nn.Module):
     def _apply(self, fn, recurse=True):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
-        self._narrowed = self._narrowed_key = None
-        self._scaled_w = self._scaled_w_key = self._fast_sig = self._no_operand_sig = None
-        self._packed_w = self._packed_w_key = None
+        self._drop_forms(moved_only=True)
+        self._no_operand_sig = None
         for name, dt in before.items():
             now = getattr(self, name).dtype
             if now != dt:
@@ -115,13 +114,20 @@ class MinifloatLinearPTQ(nn.Module):
         if (self.backend == "separate" or w is None or w.device.type != "cuda"
                 or not MinifloatF.gemm_weight_eligible(self.w_tensor_meta)):
             return None
-        key = (w.data_ptr(), w._version, w.device)
-        if self._narrowed_key != key:
-            self._narrowed = MinifloatF.narrow_weight_codes(w, self.w_tensor_meta)
-            self._narrowed_key = key
-        return self._narrowed
+        return self._weight_form("_narrowed").value
 
-    def _weight_operand(self, input: Tensor):
+    def _build_form(self, name: str, w_element: Tensor):
+        from ..mxfp import kernels
+        from .functional import linear as L
+
+        tm = self.w_tensor_meta
+        if name == "_narrowed":
+            return MinifloatF.narrow_weight_codes(w_element, tm)
+        if name == "_scaled_w":
+            return L.scaled_weight_operand(w_element, tm, self._narrowed_weight())
+        return kernels.packed_weight_from_mxfp(*self._narrowed_weight(), tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features)
+
+    def _weight_operand(self, input: Tensor) -> WeightForm | None:
         """The weight in the block-scaled GEMM's form when this call takes that GEMM (quantised bfloat16 activations, see
         ``minifloat_linear``), else None.  Not part of ``state_dict``; rebuilt like the one-byte copy."""
         from ..mxfp.functional.linear import takes_scaled_route
@@ -135,13 +141,9 @@ class MinifloatLinearPTQ(nn.Module):
         if not ((self.backend == "fused_scaled" or takes_scaled_route(rows, True))
                 and L._scaled_eligible(input, self.x_minifloat_meta, self.w_tensor_meta, bias)):
             return None
-        key = (w.data_ptr(), w._version, w.device)
-        if self._scaled_w_key != key:
-            self._scaled_w = L.scaled_weight_operand(w, self.w_tensor_meta, self._narrowed_weight())
-            self._scaled_w_key = key
-        return self._scaled_w
+        return self._weight_form("_scaled_w")
 
-    def _packed_weight(self, input: Tensor):
+    def _packed_weight(self, input: Tensor) -> tuple[WeightForm, bool] | None:
         """The weight packed at its own width when that is the fastest form for this call, and whether the activations are dense (``MXFPLinearPTQ``);
         else None."""
         from ..mxfp import kernels
@@ -159,12 +161,7 @@ class MinifloatLinearPTQ(nn.Module):
         elif not (self.layer_type.startswith("XqWq") and kernels.packed_pays(rows, self.out_features, self.in_features, E, M, input.device)
                   and L._scaled_eligible(input, self.x_minifloat_meta, tm, bias)):
             return None
-        key = (w.data_ptr(), w._version, w.device)
-        if self._packed_w_key != key:
-            scales, codes = self._narrowed_weight()
-            self._packed_w = kernels.packed_weight_from_mxfp(scales, codes, E, M, self.out_features, self.in_features)
-            self._packed_w_key = key
-        return self._packed_w, dense
+        return self._weight_form("_packed_w"), dense
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_minifloat_meta)
@@ -174,17 +171,14 @@ class MinifloatLinearPTQ(nn.Module):
         sig = self._call_signature(input)
         if self._fast_sig is not None and self._fast_sig == sig:
             w, packed = self._parameters.get("w_element"), self._fast_packed     # (none: held otherwise, by a parametrisation)
-            op, built_from = (self._packed_w, self._packed_w_key) if packed else (self._scaled_w, self._scaled_w_key)
-            if packed == 3:
-                if w is not None and self._narrowed_key == (w.data_ptr(), w._version, w.device):
-                    (scales, codes), m = self._narrowed, self.w_tensor_meta.meta
-                    y = _lib.host().linear_plain(input, self.x_minifloat_meta._codes if self.layer_type.startswith("Xq") else None, 1, scales, codes, m.exp_bits,
-                                                 m.frac_bits, self.out_features, None if self.layer_type.endswith("Bq") else self.bias)
-                    if y is not None:
-                        return y
-            elif w is not None and built_from == (w.data_ptr(), w._version, w.device):
-                xm, bias = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias
-                if packed == 2:
+            form = self._narrowed if packed == 3 else self._packed_w if packed else self._scaled_w
+            if form is not None and w is not None and form.key == (w.data_ptr(), w._version):
+                xm, bias, op = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, form.value
+                if packed == 3:
+                    (scales, codes), m = op, self.w_tensor_meta.meta
+                    y = _lib.host().linear_plain(input, xm._codes if self.layer_type.startswith("Xq") else None, 1, scales, codes, m.exp_bits, m.frac_bits,
+                                                 self.out_features, bias)
+                elif packed == 2:
                     y = _lib.host().linear_packed_dense(input, op.codes, op.scales, op.exp_bits, op.frac_bits, self.out_features, bias)
                 elif packed:
                     y = _lib.host().linear_packed(input, xm.exp_bits, xm.frac_bits, 1, op.codes, op.scales, op.exp_bits, op.frac_bits, self.out_features, bias)
@@ -200,17 +194,17 @@ class MinifloatLinearPTQ(nn.Module):
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
         if self._fast_sig is not None and self._fast_sig == sig and not self._fast_packed:
-            w = self.w_element
-            if self._scaled_w_key == (w.data_ptr(), w._version, w.device):
+            form, w = self._scaled_w, self.w_element
+            if form is not None and form.key == (w.data_ptr(), w._version):
                 from ..mxfp import kernels
 
                 xm = self.x_minifloat_meta
                 x2 = input.reshape(-1, self.in_features)
                 bias = None if self.layer_type.endswith("Bq") else self.bias
                 if x2.is_contiguous() and x2.data_ptr() % 16 == 0 and x2.shape[0] > 0 and (bias is None or bias.is_contiguous()):
-                    y = kernels.linear_scaled(x2, xm.exp_bits, xm.frac_bits, True, self._scaled_w, bias)
+                    y = kernels.linear_scaled(x2, xm.exp_bits, xm.frac_bits, True, form.value, bias)
                 else:
-                    y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense_minifloat(x2, xm.exp_bits, xm.frac_bits), self._scaled_w, bias, input.dtype)
+                    y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense_minifloat(x2, xm.exp_bits, xm.frac_bits), form.value, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
         # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
         # (written to the instance's dict: nn.Module's own assignment costs a microsecond, on every call whose shape changes)
@@ -220,7 +214,7 @@ class MinifloatLinearPTQ(nn.Module):
         if packed is not None:
             from ..mxfp import kernels
 
-            w, dense = packed
+            w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_fast_sig"], notes["_fast_packed"] = None, sig, 2 if dense else 1
             xm, bias, x2 = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
@@ -237,7 +231,7 @@ class MinifloatLinearPTQ(nn.Module):
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
-            _narrowed=self._narrowed_weight(), _w_operand=w_operand)
+            _narrowed=self._narrowed_weight(), _w_operand=None if w_operand is None else w_operand.value)
         if w_operand is None:
             notes["_no_operand_sig"] = sig
             from .functional import linear as L

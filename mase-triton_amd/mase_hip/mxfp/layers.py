@@ -8,14 +8,14 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm
 from . import functional as MXFP_F
 from .meta import MXFPMeta, MXFPTensorMeta
 
 LayerType = Literal["XWB", "XWBq", "XWqB", "XWqBq", "XqWB", "XqWBq", "XqWqB", "XqWqBq"]
 
 
-class MXFPLinearPTQ(nn.Module):
+class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
     """``y = x W^T + b`` with any of x / W / b held or rounded in an MXFP format.
 
     A quantised weight is stored as two frozen uint8 parameters, ``w_scales`` [N*K/B, 1] and
@@ -31,7 +31,9 @@ class MXFPLinearPTQ(nn.Module):
     in_features: int
     out_features: int
     _CODE_PARAMS = ("w_scales", "w_elements", "b_scales", "b_elements")
-    _packed_w = _packed_w_key = None   # the weight packed at its own width, and what it was built from
+    _FORMS = ("_scaled_w", "_packed_w")      # the weight in the block-scaled GEMM's form, and packed at its own width
+    _FORM_COMPONENTS = ("w_elements", "w_scales")
+    _scaled_w = _packed_w = None
     _fast_packed = 0         # was the call that _fast_sig notes one on the packed weight (1: x quantised, 2: dense) or on the components (3)?
     _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
@@ -73,7 +75,6 @@ class MXFPLinearPTQ(nn.Module):
         self.backend = backend
         self.dtype, self.device = dtype, device
 
-        self._scaled_w = self._scaled_w_key = None   # the weight in the block-scaled GEMM's form, and what it was built from
         self._fast_sig = None                        # what the last call on the block-scaled route looked like (see forward)
         self.weight = self.bias = None
         self.w_scales = self.w_elements = self.w_tensor_meta = None
@@ -105,15 +106,7 @@ class MXFPLinearPTQ(nn.Module):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
         self._no_operand_sig = None
-        if self.w_scales is not None:
-            # (a move that moved nothing keeps the weight's other forms)
-            key = (self.w_elements.data_ptr(), self.w_elements._version, self.w_scales.data_ptr(), self.w_scales._version)
-            if self._scaled_w_key != key:
-                self._scaled_w = self._scaled_w_key = None
-            if self._packed_w_key != key:
-                self._packed_w = self._packed_w_key = None
-            if self._scaled_w is None or self._packed_w is None:
-                self._fast_sig = None
+        self._drop_forms(moved_only=True)
         for name, dt in before.items():
             now = getattr(self, name).dtype
             if now != dt:
@@ -128,8 +121,17 @@ class MXFPLinearPTQ(nn.Module):
         """Drop the cached block-scaled form of the weight.  Writes to ``w_scales`` / ``w_elements`` that torch records
         (``copy_`` under ``no_grad``, ``load_state_dict``, moving the module) are noticed without this call; writes
         through ``.data`` are not."""
-        self._scaled_w = self._scaled_w_key = self._fast_sig = self._no_operand_sig = None
-        self._packed_w = self._packed_w_key = None
+        self._drop_forms()
+        self._fast_sig = self._no_operand_sig = None
+
+    def _build_form(self, name: str, w_elements: Tensor, w_scales: Tensor):
+        from . import kernels
+        from .functional import linear as L
+
+        if name == "_scaled_w":
+            return L.scaled_weight_operand(w_scales, w_elements, self.w_tensor_meta)
+        m = self.w_tensor_meta.meta
+        return kernels.packed_weight_from_mxfp(w_scales, w_elements, m.element_exp_bits, m.element_frac_bits, self.out_features, self.in_features)
 
     def _takes_scaled_route(self, input: Tensor) -> bool:
         """Does ``forward(input)`` run on the block-scaled GEMM?"""
@@ -142,7 +144,7 @@ class MXFPLinearPTQ(nn.Module):
         return ((self.backend == "fused_scaled" or L.takes_scaled_route(rows, True))
                 and L._scaled_eligible(input, self.x_mxfp_meta, self.w_tensor_meta, bias))
 
-    def _weight_operand(self, input: Tensor):
+    def _weight_operand(self, input: Tensor) -> WeightForm | None:
         """The weight in the block-scaled GEMM's form when this call has a kernel that reads it (the block-scaled GEMM for
         quantised bfloat16 activations, the large-tile bf16 kernel from 512 rows on), else None."""
         from . import kernels
@@ -159,19 +161,9 @@ class MXFPLinearPTQ(nn.Module):
                     and kernels.prepared_w_shape_supported(rows, tm.shape[0], tm.shape[1]))
             if not bf16:
                 return None
-        return self._prepared_weight()
+        return self._weight_form("_scaled_w")
 
-    def _prepared_weight(self):
-        """The weight in the block-scaled GEMM's form, built once and again after a change."""
-        from .functional import linear as L
-
-        key = (self.w_elements.data_ptr(), self.w_elements._version, self.w_scales.data_ptr(), self.w_scales._version)
-        if self._scaled_w is None or self._scaled_w_key != key:
-            self._scaled_w = L.scaled_weight_operand(self.w_scales, self.w_elements, self.w_tensor_meta)
-            self._scaled_w_key = key
-        return self._scaled_w
-
-    def _packed_weight(self, input: Tensor, scaled: bool = False):
+    def _packed_weight(self, input: Tensor, scaled: bool = False) -> tuple[WeightForm, bool] | None:
         """The weight packed at its own width when that is the fastest form for this call, and whether the call is one of dense activations
         (weight-only layers) or of quantised ones; else None.  ``scaled``: the caller knows that the call takes the block-scaled route."""
         from . import kernels
@@ -192,11 +184,7 @@ class MXFPLinearPTQ(nn.Module):
         elif not (kernels.packed_pays(rows, self.out_features, self.in_features, m.element_exp_bits, m.element_frac_bits, input.device)
                   and (scaled or self._takes_scaled_route(input))):
             return None
-        key = (self.w_elements.data_ptr(), self.w_elements._version, self.w_scales.data_ptr(), self.w_scales._version)
-        if self._packed_w is None or self._packed_w_key != key:
-            self._packed_w = kernels.packed_weight_from_mxfp(self.w_scales, self.w_elements, m.element_exp_bits, m.element_frac_bits, self.out_features, self.in_features)
-            self._packed_w_key = key
-        return self._packed_w, dense
+        return self._weight_form("_packed_w"), dense
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta)
@@ -206,7 +194,7 @@ class MXFPLinearPTQ(nn.Module):
         sig = self._call_signature(input)
         if self._fast_sig is not None and self._fast_sig == sig:
             params, packed = self._parameters, self._fast_packed
-            w, built_from = (self._packed_w, self._packed_w_key) if packed else (self._scaled_w, self._scaled_w_key)
+            form = self._packed_w if packed else self._scaled_w
             w_elements, w_scales = params.get("w_elements"), params.get("w_scales")     # (none: held otherwise, by a parametrisation)
             if packed == 3:
                 if w_elements is not None and w_scales is not None:
@@ -215,8 +203,9 @@ class MXFPLinearPTQ(nn.Module):
                                                  m.element_exp_bits, m.element_frac_bits, self.out_features, None if self.layer_type.endswith("Bq") else self.bias)
                     if y is not None:
                         return y
-            elif w_elements is not None and w_scales is not None and built_from == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
-                meta = self.x_mxfp_meta
+            elif (form is not None and w_elements is not None and w_scales is not None
+                  and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version)):
+                meta, w = self.x_mxfp_meta, form.value
                 bias = None if self.layer_type.endswith("Bq") else self.bias
                 if packed == 2:
                     y = _lib.host().linear_packed_dense(input, w.codes, w.scales, w.exp_bits, w.frac_bits, self.out_features, bias)
@@ -235,17 +224,17 @@ class MXFPLinearPTQ(nn.Module):
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
         if self._fast_sig is not None and self._fast_sig == sig and not self._fast_packed:
-            w_elements, w_scales = self.w_elements, self.w_scales
-            if self._scaled_w_key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
+            form, w_elements, w_scales = self._scaled_w, self.w_elements, self.w_scales
+            if form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
                 from . import kernels
 
                 x2 = input.reshape(-1, self.in_features)
                 bias = None if self.layer_type.endswith("Bq") else self.bias
                 meta = self.x_mxfp_meta
                 if x2.is_contiguous() and x2.data_ptr() % 16 == 0 and x2.shape[0] > 0 and (bias is None or bias.is_contiguous()):
-                    y = kernels.linear_scaled(x2, meta.element_exp_bits, meta.element_frac_bits, False, self._scaled_w, bias)
+                    y = kernels.linear_scaled(x2, meta.element_exp_bits, meta.element_frac_bits, False, form.value, bias)
                 else:
-                    y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense(x2, meta), self._scaled_w, bias, input.dtype)
+                    y = kernels.mxfp_gemm_scaled(kernels.scaled_operand_from_dense(x2, meta), form.value, bias, input.dtype)
                 return y.view(*input.shape[:-1], self.out_features)
         # (a call that looks like the last one that ran and that no kernel took the operand for is not asked about again)
         # (written to the instance's dict: nn.Module's own assignment costs a microsecond, on every call whose shape changes)
@@ -255,7 +244,7 @@ class MXFPLinearPTQ(nn.Module):
         if packed is not None:
             from . import kernels
 
-            w, dense = packed
+            w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_fast_sig"], notes["_fast_packed"] = None, sig, 2 if dense else 1
             meta, bias, x2 = self.x_mxfp_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
@@ -272,7 +261,7 @@ class MXFPLinearPTQ(nn.Module):
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
-            w_operand=w_operand)
+            w_operand=None if w_operand is None else w_operand.value)
         if w_operand is None:
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
@@ -295,10 +284,10 @@ class MXFPLinearPTQ(nn.Module):
         if (gate.shape == up.shape and gate.dtype == up.dtype and gate.device == up.device and gate.shape[-1] == self.in_features
                 and self.layer_type == "XqWqB" and self._takes_scaled_route(gate)):
             packed = self._packed_weight(gate, True)
-            w_op = self._prepared_weight() if packed is None else None
+            w_op = self._weight_form("_scaled_w").value if packed is None else packed[0].value
             a_op = kernels.scaled_operand_from_swiglu(gate.reshape(-1, self.in_features) if gate.ndim != 2 else gate,
                                                       up.reshape(-1, self.in_features) if up.ndim != 2 else up, self.x_mxfp_meta)
-            y = kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype) if packed is None else kernels.mxfp_gemm_packed(a_op, packed[0], self.bias)
+            y = kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype) if packed is None else kernels.mxfp_gemm_packed(a_op, w_op, self.bias)
             return y.view(*gate.shape[:-1], self.out_features)
         return self.forward(torch.nn.functional.silu(gate) * up)
 

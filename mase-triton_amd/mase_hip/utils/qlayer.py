@@ -1,4 +1,4 @@
-"""Helpers for the PTQ layers (same contract as src/mase_triton/utils/qlayer.py:4-21)."""
+"""Helpers for the PTQ layers (the first two: same contract as src/mase_triton/utils/qlayer.py:4-21)."""
 import torch
 
 
@@ -18,3 +18,56 @@ def _canonical(device) -> torch.device:
 def devices_equal(device1, device2) -> bool:
     """True if both name the same device; a bare "cuda" means "cuda:0"."""
     return _canonical(device1) == _canonical(device2)
+
+
+class WeightForm:
+    """A quantised weight in another form than its stored components.
+
+    ``key`` names the components that it was built from, by address and version.  An address names a tensor only until its memory is handed out
+    again, so the form holds an alias of each: whatever replaces a component while the form is kept lies elsewhere."""
+
+    __slots__ = ("value", "key", "components")
+
+    def __init__(self, value, key: tuple, components: tuple):
+        self.value, self.key, self.components = value, key, components
+
+
+def weight_key(components) -> tuple:
+    return tuple(v for c in components for v in (c.data_ptr(), c._version))
+
+
+class KeepsWeightForms:
+    """What the PTQ layers have in common that keep their weight in further forms (attributes named by ``_FORMS``) beside the components
+    (``_FORM_COMPONENTS``).  Forms are built on the first call that reads them and again after a change of the components, and are part of
+    neither ``state_dict`` nor a copy or pickle of the layer."""
+
+    _FORMS: tuple[str, ...] = ()
+    _FORM_COMPONENTS: tuple[str, ...] = ()
+
+    def _build_form(self, name: str, *components: torch.Tensor):
+        raise NotImplementedError
+
+    def _weight_form(self, name: str) -> WeightForm:
+        """The form ``name`` of the weight as it is now."""
+        components = tuple(getattr(self, c) for c in self._FORM_COMPONENTS)
+        kept, key = getattr(self, name), weight_key(components)
+        if kept is None or kept.key != key:
+            kept = WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
+            self.__dict__[name] = kept
+        return kept
+
+    def _drop_forms(self, moved_only: bool = False) -> None:
+        """Forget the forms, or those whose components are not the layer's any more."""
+        components = [getattr(self, c) for c in self._FORM_COMPONENTS]
+        key = None if any(c is None for c in components) else weight_key(components)
+        for name in self._FORMS:
+            kept = getattr(self, name)
+            if kept is not None and not (moved_only and kept.key == key):
+                self.__dict__[name] = None
+                self.__dict__["_fast_sig"] = None
+
+    def __getstate__(self):
+        return {**self.__dict__, **dict.fromkeys(self._FORMS), "_fast_sig": None}
+
+    def __setstate__(self, state):
+        super().__setstate__({**state, **dict.fromkeys(self._FORMS), "_fast_sig": None})     # (older pickles hold forms without a key)

@@ -1,5 +1,8 @@
-"""The other forms of a quantised weight that a layer keeps, with stand-ins for the kernels that build and read them: what becomes of them when the
+"""The further forms of a quantised weight that a layer keeps, with stand-ins for the kernels that build and read them: what becomes of them when the
 components move or change."""
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -43,7 +46,7 @@ class OnGpu:
 
 
 def both_forms(layer):
-    return layer._prepared_weight(), layer._packed_weight(OnGpu(), True)[0]
+    return layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
 
 
 def test_forms_go_with_the_components_that_move(layer):
@@ -54,3 +57,26 @@ def test_forms_go_with_the_components_that_move(layer):
     assert (layer._scaled_w, layer._packed_w) == kept
     layer.to("meta")
     assert layer._scaled_w is None and layer._packed_w is None
+
+
+def test_components_at_a_former_address_are_not_the_former_components(layer):
+    """A freed component's memory goes to the next one of its size, whose version is 0 again."""
+    seen = set()
+    for seed in range(1, 30):
+        assert [f.value.sum for f in both_forms(layer)] == [int(layer.w_elements.sum(dtype=torch.int64))] * 2
+        seen.add(layer._scaled_w.key)
+        layer.w_elements = layer.w_scales = None
+        scales, elements = components(seed)
+        layer.w_scales, layer.w_elements = (torch.nn.Parameter(t, requires_grad=False) for t in (scales, elements))
+    assert len(seen) > 1
+
+
+def test_a_copy_builds_its_own_forms(layer):
+    both_forms(layer)
+    for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
+        assert other._scaled_w is None and other._packed_w is None and layer._scaled_w is not None
+    state = layer.__getstate__()
+    state.update(_scaled_w=object(), _fast_sig=())                       # as a layer was pickled that kept forms without their components
+    other = MXFPLinearPTQ.__new__(MXFPLinearPTQ)
+    other.__setstate__(state)
+    assert other._scaled_w is None and other._fast_sig is None
