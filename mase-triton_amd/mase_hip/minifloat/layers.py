@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm, capturing
 from . import functional as MinifloatF
 from .meta import MinifloatMeta, MinifloatTensorMeta
 
@@ -161,7 +161,8 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         elif not (self.layer_type.startswith("XqWq") and kernels.packed_pays(rows, self.out_features, self.in_features, E, M, input.device)
                   and L._scaled_eligible(input, self.x_minifloat_meta, tm, bias)):
             return None
-        return self._weight_form("_packed_w"), dense
+        form = self._weight_form("_packed_w", needed=False)
+        return None if form is None else (form, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_minifloat_meta)
@@ -232,7 +233,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             _narrowed=self._narrowed_weight(), _w_operand=None if w_operand is None else w_operand.value)
-        if w_operand is None:
+        if w_operand is None and not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm, capturing
 from . import functional as MXFP_F
 from .meta import MXFPMeta, MXFPTensorMeta
 
@@ -161,7 +161,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                     and kernels.prepared_w_shape_supported(rows, tm.shape[0], tm.shape[1]))
             if not bf16:
                 return None
-        return self._weight_form("_scaled_w")
+        return self._weight_form("_scaled_w", needed=scaled)
 
     def _packed_weight(self, input: Tensor, scaled: bool = False) -> tuple[WeightForm, bool] | None:
         """The weight packed at its own width when that is the fastest form for this call, and whether the call is one of dense activations
@@ -184,7 +184,8 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         elif not (kernels.packed_pays(rows, self.out_features, self.in_features, m.element_exp_bits, m.element_frac_bits, input.device)
                   and (scaled or self._takes_scaled_route(input))):
             return None
-        return self._weight_form("_packed_w"), dense
+        form = self._weight_form("_packed_w", needed=False)
+        return None if form is None else (form, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta)
@@ -262,7 +263,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             w_operand=None if w_operand is None else w_operand.value)
-        if w_operand is None:
+        if w_operand is None and not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

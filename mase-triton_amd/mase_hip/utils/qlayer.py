@@ -1,6 +1,8 @@
 """Helpers for the PTQ layers (the first two: same contract as src/mase_triton/utils/qlayer.py:4-21)."""
 import torch
 
+from .. import _lib
+
 
 class ChangeDtypeError(Exception):
     """Raised when ``.to(dtype=...)`` would change the dtype of stored integer codes."""
@@ -36,6 +38,14 @@ def weight_key(components) -> tuple:
     return tuple(v for c in components for v in (c.data_ptr(), c._version))
 
 
+def capturing(device: torch.device) -> bool:
+    """Is the current stream of ``device`` being captured into a graph?  (What is launched then runs when the graph does, not now.)"""
+    if device.type != "cuda":
+        return False
+    with _lib.on_device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class KeepsWeightForms:
     """What the PTQ layers have in common that keep their weight in further forms (attributes named by ``_FORMS``) beside the components
     (``_FORM_COMPONENTS``).  Forms are built on the first call that reads them and again after a change of the components, and are part of
@@ -47,14 +57,20 @@ class KeepsWeightForms:
     def _build_form(self, name: str, *components: torch.Tensor):
         raise NotImplementedError
 
-    def _weight_form(self, name: str) -> WeightForm:
-        """The form ``name`` of the weight as it is now."""
+    def _weight_form(self, name: str, needed: bool = True) -> WeightForm | None:
+        """The form ``name`` of the weight as it is now.  One that is built while the stream is captured belongs to that graph, which writes it on every
+        replay; with ``needed`` false, for a call that has another way, None in its place."""
         components = tuple(getattr(self, c) for c in self._FORM_COMPONENTS)
         kept, key = getattr(self, name), weight_key(components)
-        if kept is None or kept.key != key:
-            kept = WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
-            self.__dict__[name] = kept
-        return kept
+        if kept is not None and kept.key == key:
+            return kept
+        in_graph = capturing(components[0].device)
+        if in_graph and not needed:
+            return None
+        form = WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
+        if not in_graph:
+            self.__dict__[name] = form
+        return form
 
     def _drop_forms(self, moved_only: bool = False) -> None:
         """Forget the forms, or those whose components are not the layer's any more."""

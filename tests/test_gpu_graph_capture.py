@@ -41,3 +41,50 @@ def test_fused_layer_replays_from_a_graph(M, K, N):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(static_y.view(torch.int16), want.view(torch.int16)), f"replay {i}"
+
+
+@pytest.mark.parametrize("family", ["mxfp", "minifloat"])
+@pytest.mark.parametrize("layer_type,rows,warm_rows", [("XqWqB", 48, 2000),   # the packed weight's rows, warmed up at the block-scaled form's
+                                                       ("XWqB", 12, 40),      # weight only: warmed up on the components
+                                                       ("XWqB", 3000, 12),    # ... and the bf16 kernel's prepared form
+                                                       ("XqWqB", 48, None)])  # no warm-up but of another layer
+def test_forms_that_a_capture_meets_first(family, layer_type, rows, warm_rows):
+    """A layer captured at a row count whose form of the weight it has not built: eager calls before the first replay, and of other streams, are right, and
+    so is every replay."""
+    import mase_hip.minifloat.meta as mf
+    import mase_hip.mxfp.meta as mx
+    from mase_hip.minifloat.layers import MinifloatLinearPTQ
+    from mase_hip.mxfp.layers import MXFPLinearPTQ
+
+    K, N = 4096, 2048
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    w = (0.5 * torch.randn(N, K, generator=g, device=DEV)).to(torch.bfloat16)
+
+    def make(backend):
+        if family == "mxfp":
+            return MXFPLinearPTQ(w, None, mx.MXFP8_E4M3_fn if layer_type == "XqWqB" else None, mx.OCP_MXFP4_E2M1, None, layer_type, backend)
+        return MinifloatLinearPTQ(weight=w, bias=None, x_minifloat_meta=mf.FP8_E4M3_fn if layer_type == "XqWqB" else None, w_minifloat_meta=mf.FP4_E2M1_fn,
+                                  b_minifloat_meta=None, layer_type=layer_type, backend=backend)
+
+    def close(y, ref):
+        return ((y.double() - ref.double()).norm() / ref.double().norm()).item() <= 1e-3
+
+    layer, separate, other = make("fused"), make("separate"), make("fused")
+    x = torch.randn(rows, K, generator=g, device=DEV).to(torch.bfloat16)
+    want = separate(x)
+    if warm_rows is not None:
+        layer(torch.randn(warm_rows, K, generator=g, device=DEV).to(torch.bfloat16))
+    other(x)                                       # the kernels' first launches are not captured
+    torch.cuda.synchronize()
+    static_x, graph = x.clone(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        static_y = layer(static_x)
+    assert close(layer(x), want) and close(layer(x), want)
+    for i in range(3):
+        scale = 2.0 ** i
+        static_x.copy_(x * scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert close(static_y, separate(x * scale)), i
+        assert close(layer(x), want), i
+    assert close(other(x), want)

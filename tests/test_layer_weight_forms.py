@@ -80,3 +80,16 @@ def test_a_copy_builds_its_own_forms(layer):
     other = MXFPLinearPTQ.__new__(MXFPLinearPTQ)
     other.__setstate__(state)
     assert other._scaled_w is None and other._fast_sig is None
+
+
+def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
+    """What a captured stream is given runs on the replays: nothing is written yet for the calls between."""
+    from mase_hip.utils import qlayer
+
+    monkeypatch.setattr(qlayer, "capturing", lambda device: True)
+    assert layer._packed_weight(OnGpu(), True) is None and layer._weight_form("_scaled_w").value.sum > 0
+    assert layer._scaled_w is None and layer._packed_w is None
+    monkeypatch.setattr(qlayer, "capturing", lambda device: False)
+    kept = both_forms(layer)
+    monkeypatch.setattr(qlayer, "capturing", lambda device: True)
+    assert both_forms(layer) == kept == (layer._scaled_w, layer._packed_w)
