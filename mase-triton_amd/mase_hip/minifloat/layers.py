@@ -107,14 +107,14 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             self.b_tensor_meta = self.b_tensor_meta.create(device=self.b_element.device)
         return result
 
-    def _narrowed_weight(self):
+    def _narrowed_weight(self) -> WeightForm | None:
         """One-byte copy of the weight codes for the fused GEMM (not part of ``state_dict``),
         rebuilt when ``w_element`` is replaced, written in place or moved."""
         w = self.w_element
         if (self.backend == "separate" or w is None or w.device.type != "cuda"
                 or not MinifloatF.gemm_weight_eligible(self.w_tensor_meta)):
             return None
-        return self._weight_form("_narrowed").value
+        return self._weight_form("_narrowed")
 
     def _build_form(self, name: str, w_element: Tensor):
         from ..mxfp import kernels
@@ -123,9 +123,14 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         tm = self.w_tensor_meta
         if name == "_narrowed":
             return MinifloatF.narrow_weight_codes(w_element, tm)
+        narrowed = self._narrowed_weight()
         if name == "_scaled_w":
-            return L.scaled_weight_operand(w_element, tm, self._narrowed_weight())
-        return kernels.packed_weight_from_mxfp(*self._narrowed_weight(), tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features)
+            value = L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value)
+        else:
+            value = kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features)
+        if narrowed is not None:
+            self._keep_form("_narrowed", narrowed)
+        return value
 
     def _weight_operand(self, input: Tensor) -> WeightForm | None:
         """The weight in the block-scaled GEMM's form when this call takes that GEMM (quantised bfloat16 activations, see
@@ -223,17 +228,23 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:
                 y = kernels.linear_packed(_lib.dense(x2), xm.exp_bits, xm.frac_bits, True, w, None if bias is None else bias.contiguous())
+            self._keep_form("_packed_w", packed[0])
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
         notes["_fast_packed"] = 0
         notes["_fast_sig"] = sig if w_operand is not None else None
+        narrowed = self._narrowed_weight()
         y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
-            _narrowed=self._narrowed_weight(), _w_operand=None if w_operand is None else w_operand.value)
-        if w_operand is None and not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
+            _narrowed=None if narrowed is None else narrowed.value, _w_operand=None if w_operand is None else w_operand.value)
+        if narrowed is not None:
+            self._keep_form("_narrowed", narrowed)
+        if w_operand is not None:
+            self._keep_form("_scaled_w", w_operand)
+        elif not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

@@ -253,6 +253,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:
                 y = kernels.linear_packed(_lib.dense(x2), meta.element_exp_bits, meta.element_frac_bits, False, w, None if bias is None else bias.contiguous())
+            self._keep_form("_packed_w", packed[0])
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
@@ -263,7 +264,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             w_operand=None if w_operand is None else w_operand.value)
-        if w_operand is None and not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
+        if w_operand is not None:
+            self._keep_form("_scaled_w", w_operand)
+        elif not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 
@@ -285,10 +288,12 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         if (gate.shape == up.shape and gate.dtype == up.dtype and gate.device == up.device and gate.shape[-1] == self.in_features
                 and self.layer_type == "XqWqB" and self._takes_scaled_route(gate)):
             packed = self._packed_weight(gate, True)
-            w_op = self._weight_form("_scaled_w").value if packed is None else packed[0].value
+            form = self._weight_form("_scaled_w") if packed is None else packed[0]
             a_op = kernels.scaled_operand_from_swiglu(gate.reshape(-1, self.in_features) if gate.ndim != 2 else gate,
                                                       up.reshape(-1, self.in_features) if up.ndim != 2 else up, self.x_mxfp_meta)
-            y = kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype) if packed is None else kernels.mxfp_gemm_packed(a_op, w_op, self.bias)
+            y = (kernels.mxfp_gemm_scaled(a_op, form.value, self.bias, gate.dtype) if packed is None
+                 else kernels.mxfp_gemm_packed(a_op, form.value, self.bias))
+            self._keep_form("_scaled_w" if packed is None else "_packed_w", form)
             return y.view(*gate.shape[:-1], self.out_features)
         return self.forward(torch.nn.functional.silu(gate) * up)
 

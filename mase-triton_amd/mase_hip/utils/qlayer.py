@@ -46,10 +46,20 @@ def capturing(device: torch.device) -> bool:
         return torch.cuda.is_current_stream_capturing()
 
 
+def finish(device: torch.device, every_stream: bool) -> None:
+    """Wait for the current stream of ``device``, or for all its streams."""
+    with _lib.on_device(device):
+        torch.cuda.synchronize(device) if every_stream else torch.cuda.current_stream(device).synchronize()
+
+
 class KeepsWeightForms:
     """What the PTQ layers have in common that keep their weight in further forms (attributes named by ``_FORMS``) beside the components
     (``_FORM_COMPONENTS``).  Forms are built on the first call that reads them and again after a change of the components, and are part of
-    neither ``state_dict`` nor a copy or pickle of the layer."""
+    neither ``state_dict`` nor a copy or pickle of the layer.
+
+    A form is built on the stream of the call and read by calls on any stream and of any thread.  So a call uses what it has built in its stream's
+    order, and once its product is launched waits for the stream and only then shows the form to others (``_keep_form``): once in a form's life,
+    where an event would have to be asked about on every call, and cannot be under capture."""
 
     _FORMS: tuple[str, ...] = ()
     _FORM_COMPONENTS: tuple[str, ...] = ()
@@ -58,19 +68,25 @@ class KeepsWeightForms:
         raise NotImplementedError
 
     def _weight_form(self, name: str, needed: bool = True) -> WeightForm | None:
-        """The form ``name`` of the weight as it is now.  One that is built while the stream is captured belongs to that graph, which writes it on every
-        replay; with ``needed`` false, for a call that has another way, None in its place."""
+        """The form ``name`` of the weight as it is now: the kept one, or a new one for ``_keep_form``.  One that is built while the stream is captured
+        belongs to that graph, which writes it on every replay; with ``needed`` false, for a call that has another way, None in its place."""
         components = tuple(getattr(self, c) for c in self._FORM_COMPONENTS)
         kept, key = getattr(self, name), weight_key(components)
         if kept is not None and kept.key == key:
             return kept
-        in_graph = capturing(components[0].device)
-        if in_graph and not needed:
+        if not needed and capturing(components[0].device):
             return None
-        form = WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
-        if not in_graph:
-            self.__dict__[name] = form
-        return form
+        return WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
+
+    def _keep_form(self, name: str, form: WeightForm) -> None:
+        """Keep a form that ``_weight_form`` gave, for calls on every stream."""
+        kept = getattr(self, name)
+        if form is kept or capturing(form.components[0].device):
+            return
+        if any(isinstance(getattr(type(self), c, None), property) for c in self._FORM_COMPONENTS):
+            return                                            # (a parametrisation makes another tensor for every call)
+        finish(form.components[0].device, every_stream=kept is not None)      # (calls on other streams may still read the one that goes)
+        self.__dict__[name] = form
 
     def _drop_forms(self, moved_only: bool = False) -> None:
         """Forget the forms, or those whose components are not the layer's any more."""

@@ -5,11 +5,14 @@ import pickle
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 import mase_hip.mxfp.functional as MX
 import mase_hip.mxfp.meta as mx
+from mase_hip import _lib
 from mase_hip.mxfp import kernels
 from mase_hip.mxfp.layers import MXFPLinearPTQ
+from mase_hip.utils import qlayer
 
 N, K = 2048, 4096        # (freshly mapped pages, which an allocator hands out again at once)
 
@@ -31,6 +34,7 @@ def layer(monkeypatch):
     monkeypatch.setattr("mase_hip.mxfp.functional.linear.scaled_weight_operand", lambda scales, elements, meta: Form(elements))
     monkeypatch.setattr(kernels, "packed_weight_from_mxfp", lambda scales, elements, e, m, rows, k: Form(elements))
     monkeypatch.setattr(kernels, "packed_pays", lambda *a: True)
+    monkeypatch.setattr(qlayer, "finish", lambda device, every_stream: None)
     scales, elements = components(0)
     meta = mx.MXFPTensorMeta(device="cpu", dtype="bfloat16", shape=(N, K), block_dim=1, meta=mx.OCP_MXFP4_E2M1)
     return MXFPLinearPTQ.from_quantized(scales, elements, meta, None, None, None, None, mx.MXFP8_E4M3_fn, "XqWqB", "fused")
@@ -44,9 +48,15 @@ class OnGpu:
     def numel(self):
         return 4 * K
 
+    def reshape(self, *shape):
+        return self
+
 
 def both_forms(layer):
-    return layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
+    forms = layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
+    layer._keep_form("_scaled_w", forms[0])
+    layer._keep_form("_packed_w", forms[1])
+    return forms
 
 
 def test_forms_go_with_the_components_that_move(layer):
@@ -84,12 +94,40 @@ def test_a_copy_builds_its_own_forms(layer):
 
 def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
     """What a captured stream is given runs on the replays: nothing is written yet for the calls between."""
-    from mase_hip.utils import qlayer
-
     monkeypatch.setattr(qlayer, "capturing", lambda device: True)
-    assert layer._packed_weight(OnGpu(), True) is None and layer._weight_form("_scaled_w").value.sum > 0
+    form = layer._weight_form("_scaled_w")
+    layer._keep_form("_scaled_w", form)
+    assert layer._packed_weight(OnGpu(), True) is None and form.value.sum > 0
     assert layer._scaled_w is None and layer._packed_w is None
     monkeypatch.setattr(qlayer, "capturing", lambda device: False)
     kept = both_forms(layer)
     monkeypatch.setattr(qlayer, "capturing", lambda device: True)
     assert both_forms(layer) == kept == (layer._scaled_w, layer._packed_w)
+
+
+def test_forms_are_shown_to_other_streams_when_they_are_written(layer, monkeypatch):
+    """The call that builds a form uses it in its stream's order; others see it when that stream has run."""
+    order = []
+    monkeypatch.setattr(_lib, "dense", lambda t: t)
+    monkeypatch.setattr(kernels, "linear_packed", lambda *a: (order.append("product"), torch.zeros(4, N))[1])
+    monkeypatch.setattr(qlayer, "finish", lambda device, every_stream: order.append((layer._packed_w, every_stream)))
+    layer(OnGpu())
+    first = layer._packed_w
+    assert order == ["product", (None, False)] and first is not None
+    with torch.no_grad():
+        layer.w_elements.add_(1)
+    order.clear()
+    layer._forward(OnGpu(), ())
+    assert order == ["product", (first, True)] and layer._packed_w is not first      # (a call on another stream may still read the first)
+
+
+def test_components_that_a_parametrisation_makes_have_no_kept_forms(layer):
+    class Same(torch.nn.Module):
+        def forward(self, t):
+            return t.clone()
+
+    torch.nn.utils.parametrize.register_parametrization(layer, "w_elements", Same(), unsafe=True)
+    for delta in (0, 1, 1):
+        layer.parametrizations.w_elements.original.data.add_(delta)
+        assert [f.value.sum for f in both_forms(layer)] == [int(layer.w_elements.sum(dtype=torch.int64))] * 2
+        assert layer._scaled_w is None and layer._packed_w is None
