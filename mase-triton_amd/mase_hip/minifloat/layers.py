@@ -29,7 +29,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
     _FORMS = ("_narrowed", "_scaled_w", "_packed_w")      # the codes in one byte each, in the block-scaled GEMM's form, and packed at their own width
     _FORM_COMPONENTS = ("w_element",)
     _narrowed = _scaled_w = _packed_w = None
-    _fast_packed = 0         # was the call that _fast_sig notes one on the packed weight (1: x quantised, 2: dense) or on the one-byte codes (3)?
+    # (_note: 0 the block-scaled form, 1 the packed weight with x quantised, 2 with x dense, 3 the one-byte codes)
     _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
     def __init__(
@@ -72,7 +72,6 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         self.weight = self.bias = None
         self.w_element = self.w_tensor_meta = None
         self.b_element = self.b_tensor_meta = None
-        self._fast_sig = None   # what the last call on the block-scaled route looked like (see forward)
 
         if "Wq" in layer_type:
             if w_element is None:
@@ -175,8 +174,9 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
     def forward(self, input: Tensor) -> Tensor:
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
         sig = self._call_signature(input)
-        if self._fast_sig is not None and self._fast_sig == sig:
-            w, packed = self._parameters.get("w_element"), self._fast_packed     # (none: held otherwise, by a parametrisation)
+        note = self._note
+        if note is not None and note[0] == sig:
+            w, packed = self._parameters.get("w_element"), note[1]     # (none: held otherwise, by a parametrisation)
             form = self._narrowed if packed == 3 else self._packed_w if packed else self._scaled_w
             if form is not None and w is not None and form.key == (w.data_ptr(), w._version):
                 xm, bias, op = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, form.value
@@ -199,7 +199,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the codes
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._fast_sig is not None and self._fast_sig == sig and not self._fast_packed:
+        if self._note == (sig, 0):
             form, w = self._scaled_w, self.w_element
             if form is not None and form.key == (w.data_ptr(), w._version):
                 from ..mxfp import kernels
@@ -222,7 +222,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
 
             w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
-            notes["_no_operand_sig"], notes["_fast_sig"], notes["_fast_packed"] = None, sig, 2 if dense else 1
+            notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
             xm, bias, x2 = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
             if dense:
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
@@ -232,8 +232,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
-        notes["_fast_packed"] = 0
-        notes["_fast_sig"] = sig if w_operand is not None else None
+        notes["_note"] = None if w_operand is None else (sig, 0)
         narrowed = self._narrowed_weight()
         y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
@@ -250,7 +249,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
 
             if ("Wq" in self.layer_type and self.backend in ("fused", "fused_bf16") and input.numel() > 0
                     and L._gemm_eligible(input, self.x_minifloat_meta if self.layer_type.startswith("Xq") else None, self.w_tensor_meta, self.bias)):
-                notes["_fast_sig"], notes["_fast_packed"] = sig, 3
+                notes["_note"] = sig, 3
         return y
 
     def extra_repr(self) -> str:

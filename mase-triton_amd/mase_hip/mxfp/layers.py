@@ -34,7 +34,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
     _FORMS = ("_scaled_w", "_packed_w")      # the weight in the block-scaled GEMM's form, and packed at its own width
     _FORM_COMPONENTS = ("w_elements", "w_scales")
     _scaled_w = _packed_w = None
-    _fast_packed = 0         # was the call that _fast_sig notes one on the packed weight (1: x quantised, 2: dense) or on the components (3)?
+    # (_note: 0 the block-scaled form, 1 the packed weight with x quantised, 2 with x dense, 3 the components)
     _no_operand_sig = None   # what the last call that had no use for the block-scaled weight looked like (layers unpickled from before it have none)
 
     def __init__(
@@ -75,7 +75,6 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         self.backend = backend
         self.dtype, self.device = dtype, device
 
-        self._fast_sig = None                        # what the last call on the block-scaled route looked like (see forward)
         self.weight = self.bias = None
         self.w_scales = self.w_elements = self.w_tensor_meta = None
         self.b_scales = self.b_elements = self.b_tensor_meta = None
@@ -122,7 +121,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         (``copy_`` under ``no_grad``, ``load_state_dict``, moving the module) are noticed without this call; writes
         through ``.data`` are not."""
         self._drop_forms()
-        self._fast_sig = self._no_operand_sig = None
+        self._note = self._no_operand_sig = None
 
     def _build_form(self, name: str, w_elements: Tensor, w_scales: Tensor):
         from . import kernels
@@ -193,8 +192,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
     def forward(self, input: Tensor) -> Tensor:
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)
         sig = self._call_signature(input)
-        if self._fast_sig is not None and self._fast_sig == sig:
-            params, packed = self._parameters, self._fast_packed
+        note = self._note
+        if note is not None and note[0] == sig:
+            params, packed = self._parameters, note[1]
             form = self._packed_w if packed else self._scaled_w
             w_elements, w_scales = params.get("w_elements"), params.get("w_scales")     # (none: held otherwise, by a parametrisation)
             if packed == 3:
@@ -224,7 +224,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the weight
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._fast_sig is not None and self._fast_sig == sig and not self._fast_packed:
+        if self._note == (sig, 0):
             form, w_elements, w_scales = self._scaled_w, self.w_elements, self.w_scales
             if form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
                 from . import kernels
@@ -247,7 +247,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
 
             w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
-            notes["_no_operand_sig"], notes["_fast_sig"], notes["_fast_packed"] = None, sig, 2 if dense else 1
+            notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
             meta, bias, x2 = self.x_mxfp_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
             if dense:
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
@@ -257,8 +257,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
-        notes["_fast_packed"] = 0
-        notes["_fast_sig"] = sig if w_operand is not None and self._takes_scaled_route(input) else None
+        notes["_note"] = (sig, 0) if w_operand is not None and self._takes_scaled_route(input) else None
         y = MXFP_F.mxfp_linear(
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
@@ -272,7 +271,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
 
             if ("Wq" in self.layer_type and self.backend in ("fused", "fused_bf16") and input.numel() > 0
                     and L._gemm_eligible(input, self.layer_type.startswith("Xq"), self.w_tensor_meta, self.bias)):
-                notes["_fast_sig"], notes["_fast_packed"] = sig, 3
+                notes["_note"] = sig, 3
         return y
 
     @torch.no_grad()

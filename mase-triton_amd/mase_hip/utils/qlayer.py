@@ -63,6 +63,17 @@ class KeepsWeightForms:
 
     _FORMS: tuple[str, ...] = ()
     _FORM_COMPONENTS: tuple[str, ...] = ()
+    # What the last call looked like that a call of the same look may follow without the checks, and the way that it went.  One tuple, read once and
+    # written once: a thread's call can lie between any two steps of another's.
+    _note: tuple[tuple, int] | None = None
+
+    @property
+    def _fast_sig(self):
+        return None if (note := self._note) is None else note[0]
+
+    @property
+    def _fast_packed(self) -> int:
+        return 0 if (note := self._note) is None else note[1]
 
     def _build_form(self, name: str, *components: torch.Tensor):
         raise NotImplementedError
@@ -95,11 +106,10 @@ class KeepsWeightForms:
         for name in self._FORMS:
             kept = getattr(self, name)
             if kept is not None and not (moved_only and kept.key == key):
-                self.__dict__[name] = None
-                self.__dict__["_fast_sig"] = None
+                self.__dict__[name] = self.__dict__["_note"] = None
 
     def __getstate__(self):
-        return {**self.__dict__, **dict.fromkeys(self._FORMS), "_fast_sig": None}
+        return {**self.__dict__, **dict.fromkeys(self._FORMS), "_note": None}
 
     def __setstate__(self, state):
-        super().__setstate__({**state, **dict.fromkeys(self._FORMS), "_fast_sig": None})     # (older pickles hold forms without a key)
+        super().__setstate__({**state, **dict.fromkeys(self._FORMS), "_note": None})         # (older pickles hold forms without a key)

@@ -1,5 +1,7 @@
-"""A layer that is called on several streams: the forms of its weight that the first call builds on its own stream are whole
+"""A layer that is called on several streams and from several threads: the forms of its weight that the first call builds on its own stream are whole
 for every other."""
+import threading
+
 import pytest
 import torch
 
@@ -48,3 +50,34 @@ def test_forms_built_behind_other_work_of_their_stream(family, layer_type, rows)
                 outs.append(layer(x))
         torch.cuda.synchronize()
         assert all(torch.equal(y, expect) for y in outs)
+
+
+@pytest.mark.parametrize("family", ["mxfp", "minifloat"])
+def test_threads_with_streams_of_their_own(family):
+    """Decode-sized and prefill-sized calls of the same fresh layers, each thread with its own mix."""
+    K, N, rows = 4096, 2048, (1, 12, 48, 600, 3000)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    xs = [torch.randn(r, K, generator=g, device=DEV).to(torch.bfloat16) for r in rows]
+    for layer_type in ("XqWqB", "XWqB"):
+        w = (0.5 * torch.randn(N, K, generator=g, device=DEV)).to(torch.bfloat16)
+        warm = _make(family, layer_type, w)
+        want = [warm(x) for x in xs]
+        for _ in range(5):
+            layer, bad = _make(family, layer_type, w), []
+            torch.cuda.synchronize()
+
+            def calls(first):
+                try:
+                    with torch.cuda.stream(torch.cuda.Stream()):
+                        ys = [(i, layer(xs[i])) for k in range(10) for i in [(first + k * (first + 1)) % len(xs)]]
+                        torch.cuda.current_stream().synchronize()
+                    bad.extend(rows[i] for i, y in ys if not torch.equal(y, want[i]))
+                except Exception as e:      # noqa: BLE001
+                    bad.append(repr(e))
+
+            threads = [threading.Thread(target=calls, args=(t,)) for t in range(4)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            assert not bad, (layer_type, bad)

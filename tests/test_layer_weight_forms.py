@@ -25,6 +25,8 @@ def components(seed, dtype=torch.uint8):
 class Form:
     """What a stand-in builds: the sum of the codes that it was given."""
 
+    codes = scales = exp_bits = frac_bits = None
+
     def __init__(self, elements):
         self.sum = int(elements.sum(dtype=torch.int64))
 
@@ -86,7 +88,7 @@ def test_a_copy_builds_its_own_forms(layer):
     for other in (copy.deepcopy(layer), pickle.loads(pickle.dumps(layer))):
         assert other._scaled_w is None and other._packed_w is None and layer._scaled_w is not None
     state = layer.__getstate__()
-    state.update(_scaled_w=object(), _fast_sig=())                       # as a layer was pickled that kept forms without their components
+    state.update(_scaled_w=object(), _fast_sig=(), _fast_packed=1)      # as a layer was pickled that kept forms without their components
     other = MXFPLinearPTQ.__new__(MXFPLinearPTQ)
     other.__setstate__(state)
     assert other._scaled_w is None and other._fast_sig is None
@@ -131,3 +133,27 @@ def test_components_that_a_parametrisation_makes_have_no_kept_forms(layer):
         layer.parametrizations.w_elements.original.data.add_(delta)
         assert [f.value.sum for f in both_forms(layer)] == [int(layer.w_elements.sum(dtype=torch.int64))] * 2
         assert layer._scaled_w is None and layer._packed_w is None
+
+
+def test_a_call_between_the_steps_of_another(layer, monkeypatch):
+    """A weight-only layer shared by a prefill and a decode thread: a decode call that lands where the prefill call asks for its route."""
+    layer.layer_type, layer.x_mxfp_meta = "XWqB", None
+    small, large, taken = OnGpu(), OnGpu(), []
+    large.shape = torch.Size((600, K))
+
+    class Host:
+        linear_packed_dense = staticmethod(lambda *a: taken.append("dense") or torch.zeros(4, N))
+
+    monkeypatch.setattr(_lib, "_host", Host)
+    monkeypatch.setattr(kernels, "packed_dense_pays", lambda rows, *a: rows <= 32)
+    monkeypatch.setattr(kernels, "mxfp_gemm_packed_dense", lambda *a: torch.zeros(4, N))
+    monkeypatch.setattr(kernels, "prepared_w_shape_supported", lambda *a: True)
+    monkeypatch.setattr(kernels, "prepared_w_pays", lambda *a: True)
+    monkeypatch.setattr(MX, "mxfp_linear", lambda **kw: torch.zeros(600, N))
+    monkeypatch.setattr(OnGpu, "numel", lambda self: self.shape.numel())
+    layer(large)                                      # both forms are there
+    layer(small)
+    asked = MXFPLinearPTQ._takes_scaled_route
+    monkeypatch.setattr(MXFPLinearPTQ, "_takes_scaled_route", lambda self, x: asked(self, x) if x is small else (layer(small), asked(self, x))[1])
+    layer(large)
+    assert taken and set(taken) == {"dense"}
