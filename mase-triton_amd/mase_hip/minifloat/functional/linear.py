@@ -43,15 +43,20 @@ _GEMM_WEIGHT_FORMATS = ((4, 3), (5, 2), (2, 3), (3, 2), (2, 1))
 _UNIT_SCALE = 127  # E8M0 code of 2^0
 
 
-def narrow_weight_codes(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta) -> tuple[Tensor, Tensor]:
+def narrow_weight_codes(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta, into: tuple[Tensor, Tensor] | None = None) -> tuple[Tensor, Tensor]:
     """uint16 minifloat codes [N, K] -> (uint8 unit scales [N*K/32], uint8 codes [N, K]) for the
     MXFP GEMM.  Only the low ``1 + exp_bits + frac_bits`` bits of a code carry meaning, as in
-    the decode of the reference (src/mase_triton/minifloat/fake.py:97-123)."""
+    the decode of the reference (src/mase_triton/minifloat/fake.py:97-123).  ``into``: an earlier result whose memory this one takes."""
     assert w_element.dtype == torch.uint16
-    codes = w_element.contiguous().view(torch.uint8).view(*w_element.shape, 2)[..., 0].contiguous()
+    low = w_element.contiguous().view(torch.uint8).view(*w_element.shape, 2)[..., 0]
+    if into is not None and (into[1].shape != low.shape or into[1].device != low.device):
+        into = None
+    codes = low.contiguous() if into is None else into[1].copy_(low)
     n_bits = w_tensor_meta.meta.n_bits
     if n_bits < 8:
         codes &= (1 << n_bits) - 1
+    if into is not None:
+        return into
     scales = torch.full((w_element.numel() // 32,), _UNIT_SCALE, dtype=torch.uint8, device=w_element.device)
     return scales, codes
 
@@ -97,7 +102,7 @@ def _scaled_eligible(x: Tensor, x_meta: MinifloatMeta | None, w_tensor_meta: Min
 
 
 def scaled_weight_operand(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta,
-                          narrowed: tuple[Tensor, Tensor] | None = None) -> "mxfp_kernels.ScaledOperand":
+                          narrowed: tuple[Tensor, Tensor] | None = None, into: "mxfp_kernels.ScaledOperand | None" = None) -> "mxfp_kernels.ScaledOperand":
     """The weight codes in the block-scaled GEMM's form (a copy: N * K bytes of codes, N * K / 32 of unit scales).
     A layer builds it once and passes it to ``minifloat_linear(..., _w_operand=...)``."""
     scales, codes = narrowed if narrowed is not None else narrow_weight_codes(w_element, w_tensor_meta)
@@ -105,7 +110,7 @@ def scaled_weight_operand(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta,
     wm = w_tensor_meta.meta
     as_mxfp = MXFPMeta(block_size=32, scale_exp_bits=8, element_exp_bits=wm.exp_bits, element_frac_bits=wm.frac_bits,
                        element_is_finite=True, round_mode="rn")
-    return mxfp_kernels.scaled_operand_from_mxfp(scales, codes, as_mxfp, out_features, in_features)
+    return mxfp_kernels.scaled_operand_from_mxfp(scales, codes, as_mxfp, out_features, in_features, into)
 
 
 _BACKENDS = ("separate", "fused", "fused_bf16", "fused_scaled")

@@ -115,18 +115,18 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             return None
         return self._weight_form("_narrowed")
 
-    def _build_form(self, name: str, w_element: Tensor):
+    def _build_form(self, name: str, into, w_element: Tensor):
         from ..mxfp import kernels
         from .functional import linear as L
 
         tm = self.w_tensor_meta
         if name == "_narrowed":
-            return MinifloatF.narrow_weight_codes(w_element, tm)
+            return MinifloatF.narrow_weight_codes(w_element, tm, into)
         narrowed = self._narrowed_weight()
         if name == "_scaled_w":
-            value = L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value)
+            value = L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value, into)
         else:
-            value = kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features)
+            value = kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features, into)
         if narrowed is not None:
             self._keep_form("_narrowed", narrowed)
         return value

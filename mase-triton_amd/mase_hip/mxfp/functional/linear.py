@@ -98,11 +98,12 @@ def _scaled_eligible(x: Tensor, x_meta: MXFPMeta | None, w_tensor_meta: MXFPTens
     return b is None or b.dtype in (torch.bfloat16, torch.float16, torch.float32)
 
 
-def scaled_weight_operand(w_scales: Tensor, w_elements: Tensor, w_tensor_meta: MXFPTensorMeta) -> "kernels.ScaledOperand":
+def scaled_weight_operand(w_scales: Tensor, w_elements: Tensor, w_tensor_meta: MXFPTensorMeta,
+                          into: "kernels.ScaledOperand | None" = None) -> "kernels.ScaledOperand":
     """The weight components in the block-scaled GEMM's form (a copy: N * K bytes of codes and N * K / 32 of scales).
-    A layer builds it once and passes it to ``mxfp_linear(..., w_operand=...)``."""
+    A layer builds it once and passes it to ``mxfp_linear(..., w_operand=...)``.  ``into``: an earlier one whose memory it takes."""
     out_features, in_features = w_tensor_meta.shape
-    return kernels.scaled_operand_from_mxfp(w_scales, w_elements, w_tensor_meta.meta, out_features, in_features)
+    return kernels.scaled_operand_from_mxfp(w_scales, w_elements, w_tensor_meta.meta, out_features, in_features, into)
 
 
 def mxfp_linear(

@@ -351,14 +351,17 @@ def scaled_operand_from_swiglu(gate: Tensor, up: Tensor, meta: MXFPMeta) -> Scal
     return ScaledOperand(codes, scales, rows, K)
 
 
-def scaled_operand_from_mxfp(scales: Tensor, elements: Tensor, meta: MXFPMeta, rows: int, K: int) -> ScaledOperand:
-    """MXFP components of a row-major [rows, K] matrix, blocked along K -> block-scaled GEMM operand."""
+def scaled_operand_from_mxfp(scales: Tensor, elements: Tensor, meta: MXFPMeta, rows: int, K: int, into: ScaledOperand | None = None) -> ScaledOperand:
+    """MXFP components of a row-major [rows, K] matrix, blocked along K -> block-scaled GEMM operand (in the memory of ``into`` if that has the size)."""
     assert scaled_format_supported(meta)
     assert scales.dtype == torch.uint8 and elements.dtype == torch.uint8
     _lib.require_gpu(elements, "elements")
     scales, elements = _lib.dense(scales), _lib.dense(elements)
     assert elements.numel() == rows * K and scales.numel() == rows * K // 32
-    codes, out_scales = _scaled_buffers(rows, K, elements.device)
+    if into is not None and (into.rows, into.K, into.codes.device) == (rows, K, elements.device):
+        codes, out_scales = into.codes, into.scales
+    else:
+        codes, out_scales = _scaled_buffers(rows, K, elements.device)
     with _lib.on_device(elements.device):
         _lib.check(_lib.load().mase_hip_scaled_operand_from_mxfp(
             scales.data_ptr(), elements.data_ptr(), meta.element_exp_bits, meta.element_frac_bits, rows, K,
@@ -457,15 +460,18 @@ def _packed_plan(M: int, N: int, K: int, exp_bits: int, frac_bits: int, device: 
         return bool(_lib.load().mase_hip_mxfp_packed_plan(M, N, K, exp_bits, frac_bits))
 
 
-def packed_weight_from_mxfp(scales: Tensor, elements: Tensor, exp_bits: int, frac_bits: int, rows: int, K: int) -> PackedWeight:
-    """MXFP components (one byte per code) of a row-major [rows, K] matrix, blocked along K, packed."""
+def packed_weight_from_mxfp(scales: Tensor, elements: Tensor, exp_bits: int, frac_bits: int, rows: int, K: int, into: PackedWeight | None = None) -> PackedWeight:
+    """MXFP components (one byte per code) of a row-major [rows, K] matrix, blocked along K, packed (in the memory of ``into`` if that has the format and size)."""
     assert scales.dtype == torch.uint8 and elements.dtype == torch.uint8
     _lib.require_gpu(elements, "elements")
     scales, elements = _lib.dense(scales), _lib.dense(elements)
     assert elements.numel() == rows * K and scales.numel() == rows * K // 32
     lib, dev = _lib.load(), elements.device
-    codes = torch.empty(lib.mase_hip_packed_weight_bytes(rows, K, exp_bits, frac_bits), dtype=torch.uint8, device=dev)
-    out_scales = torch.empty((K // 128, (rows + 255) // 256 * 256), dtype=torch.int32, device=dev)
+    if into is not None and (into.rows, into.K, into.exp_bits, into.frac_bits, into.codes.device) == (rows, K, exp_bits, frac_bits, dev):
+        codes, out_scales = into.codes, into.scales
+    else:
+        codes = torch.empty(lib.mase_hip_packed_weight_bytes(rows, K, exp_bits, frac_bits), dtype=torch.uint8, device=dev)
+        out_scales = torch.empty((K // 128, (rows + 255) // 256 * 256), dtype=torch.int32, device=dev)
     with _lib.on_device(dev):
         _lib.check(lib.mase_hip_packed_weight_from_mxfp(scales.data_ptr(), elements.data_ptr(), exp_bits, frac_bits, rows, K, codes.data_ptr(),
                                                         out_scales.data_ptr(), _lib.stream_ptr(dev)))

@@ -123,14 +123,14 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         self._drop_forms()
         self._note = self._no_operand_sig = None
 
-    def _build_form(self, name: str, w_elements: Tensor, w_scales: Tensor):
+    def _build_form(self, name: str, into, w_elements: Tensor, w_scales: Tensor):
         from . import kernels
         from .functional import linear as L
 
         if name == "_scaled_w":
-            return L.scaled_weight_operand(w_scales, w_elements, self.w_tensor_meta)
+            return L.scaled_weight_operand(w_scales, w_elements, self.w_tensor_meta, into)
         m = self.w_tensor_meta.meta
-        return kernels.packed_weight_from_mxfp(w_scales, w_elements, m.element_exp_bits, m.element_frac_bits, self.out_features, self.in_features)
+        return kernels.packed_weight_from_mxfp(w_scales, w_elements, m.element_exp_bits, m.element_frac_bits, self.out_features, self.in_features, into)
 
     def _takes_scaled_route(self, input: Tensor) -> bool:
         """Does ``forward(input)`` run on the block-scaled GEMM?"""

@@ -59,7 +59,11 @@ class KeepsWeightForms:
 
     A form is built on the stream of the call and read by calls on any stream and of any thread.  So a call uses what it has built in its stream's
     order, and once its product is launched waits for the stream and only then shows the form to others (``_keep_form``): once in a form's life,
-    where an event would have to be asked about on every call, and cannot be under capture."""
+    where an event would have to be asked about on every call, and cannot be under capture.
+
+    A captured call reads the forms that were kept then, where they lie.  So components that are written in place are built into the same memory again,
+    by the next call or by ``load_state_dict`` itself, and replays follow; a graph is captured again after the components were replaced or moved or
+    ``invalidate_weight_operand`` was called."""
 
     _FORMS: tuple[str, ...] = ()
     _FORM_COMPONENTS: tuple[str, ...] = ()
@@ -75,7 +79,8 @@ class KeepsWeightForms:
     def _fast_packed(self) -> int:
         return 0 if (note := self._note) is None else note[1]
 
-    def _build_form(self, name: str, *components: torch.Tensor):
+    def _build_form(self, name: str, into, *components: torch.Tensor):
+        """The value of form ``name``, in the memory of the value ``into`` if that is given."""
         raise NotImplementedError
 
     def _weight_form(self, name: str, needed: bool = True) -> WeightForm | None:
@@ -85,9 +90,11 @@ class KeepsWeightForms:
         kept, key = getattr(self, name), weight_key(components)
         if kept is not None and kept.key == key:
             return kept
-        if not needed and capturing(components[0].device):
+        in_graph = capturing(components[0].device)
+        if in_graph and not needed:
             return None
-        return WeightForm(self._build_form(name, *components), key, tuple(c.detach() for c in components))
+        into = kept.value if kept is not None and kept.key[::2] == key[::2] and not in_graph else None      # (the same tensors, written since)
+        return WeightForm(self._build_form(name, into, *components), key, tuple(c.detach() for c in components))
 
     def _keep_form(self, name: str, form: WeightForm) -> None:
         """Keep a form that ``_weight_form`` gave, for calls on every stream."""
@@ -107,6 +114,13 @@ class KeepsWeightForms:
             kept = getattr(self, name)
             if kept is not None and not (moved_only and kept.key == key):
                 self.__dict__[name] = self.__dict__["_note"] = None
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        super()._load_from_state_dict(*args, **kwargs)
+        for name in self._FORMS:
+            kept = getattr(self, name)
+            if kept is not None and kept.key[::2] == weight_key([getattr(self, c) for c in self._FORM_COMPONENTS])[::2]:
+                self._keep_form(name, self._weight_form(name))
 
     def __getstate__(self):
         return {**self.__dict__, **dict.fromkeys(self._FORMS), "_note": None}

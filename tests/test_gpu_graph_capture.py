@@ -88,3 +88,47 @@ def test_forms_that_a_capture_meets_first(family, layer_type, rows, warm_rows):
         assert close(static_y, separate(x * scale)), i
         assert close(layer(x), want), i
     assert close(other(x), want)
+
+
+@pytest.mark.parametrize("family", ["mxfp", "minifloat"])
+@pytest.mark.parametrize("layer_type,rows", [("XqWqB", 48), ("XqWqB", 2000), ("XWqB", 12), ("XWqB", 3000), ("XWqB", 100)])
+def test_replays_follow_a_weight_that_is_loaded_in_place(family, layer_type, rows):
+    import mase_hip.minifloat.meta as mf
+    import mase_hip.mxfp.meta as mx
+    from mase_hip.minifloat.layers import MinifloatLinearPTQ
+    from mase_hip.mxfp.layers import MXFPLinearPTQ
+
+    K, N = 4096, 2048
+    g = torch.Generator(device=DEV).manual_seed(rows)
+
+    def make():
+        w = (0.5 * torch.randn(N, K, generator=g, device=DEV)).to(torch.bfloat16)
+        if family == "mxfp":
+            return MXFPLinearPTQ(w, None, mx.MXFP8_E4M3_fn if layer_type == "XqWqB" else None, mx.OCP_MXFP4_E2M1, None, layer_type, "fused")
+        return MinifloatLinearPTQ(weight=w, bias=None, x_minifloat_meta=mf.FP8_E4M3_fn if layer_type == "XqWqB" else None, w_minifloat_meta=mf.FP4_E2M1_fn,
+                                  b_minifloat_meta=None, layer_type=layer_type, backend="fused")
+
+    layers = [make() for _ in range(3)]
+    x = torch.randn(rows, K, generator=g, device=DEV).to(torch.bfloat16)
+    want = [layer(x) for layer in layers]
+    torch.cuda.synchronize()
+    layer, graph = layers[0], torch.cuda.CUDAGraph()
+    states = [{k: v.clone() for k, v in other.state_dict().items()} for other in layers]
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    for i in (0, 1, 2, 1, 0):
+        layer.load_state_dict(states[i])
+        if i == 2:
+            assert torch.equal(layer(x), want[i])
+        junk = [torch.full((N * K,), 255, dtype=torch.uint8, device=DEV) for _ in range(4)]      # what memory that was given back would hold now
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want[i]), i
+        del junk
+    with torch.no_grad():                                       # a write in place, seen with the next call
+        for name, p in layer.named_parameters():
+            p.copy_(states[1][name])
+    assert torch.equal(layer(x), want[1])
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, want[1])

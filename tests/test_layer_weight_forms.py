@@ -27,14 +27,15 @@ class Form:
 
     codes = scales = exp_bits = frac_bits = None
 
-    def __init__(self, elements):
+    def __init__(self, elements, into=None):
+        self.memory = object() if into is None else into.memory
         self.sum = int(elements.sum(dtype=torch.int64))
 
 
 @pytest.fixture
 def layer(monkeypatch):
-    monkeypatch.setattr("mase_hip.mxfp.functional.linear.scaled_weight_operand", lambda scales, elements, meta: Form(elements))
-    monkeypatch.setattr(kernels, "packed_weight_from_mxfp", lambda scales, elements, e, m, rows, k: Form(elements))
+    monkeypatch.setattr("mase_hip.mxfp.functional.linear.scaled_weight_operand", lambda scales, elements, meta, into: Form(elements, into))
+    monkeypatch.setattr(kernels, "packed_weight_from_mxfp", lambda scales, elements, e, m, rows, k, into: Form(elements, into))
     monkeypatch.setattr(kernels, "packed_pays", lambda *a: True)
     monkeypatch.setattr(qlayer, "finish", lambda device, every_stream: None)
     scales, elements = components(0)
@@ -157,3 +158,22 @@ def test_a_call_between_the_steps_of_another(layer, monkeypatch):
     monkeypatch.setattr(MXFPLinearPTQ, "_takes_scaled_route", lambda self, x: asked(self, x) if x is small else (layer(small), asked(self, x))[1])
     layer(large)
     assert taken and set(taken) == {"dense"}
+
+
+def test_what_a_graph_reads_follows_components_written_in_place(layer, monkeypatch):
+    """A captured call reads the kept forms where they lie: a form of new values takes the memory of the one that it replaces, unless the components are others."""
+    before = [f.value.memory for f in both_forms(layer)]
+    state = {k: v + 1 for k, v in layer.state_dict().items()}
+    layer.load_state_dict(state)                                 # (without a call behind it)
+    forms = layer._scaled_w.value, layer._packed_w.value
+    assert [f.memory for f in forms] == before and [f.sum for f in forms] == [int(state["w_elements"].sum(dtype=torch.int64))] * 2
+    with torch.no_grad():
+        layer.w_elements.sub_(1)
+    assert [f.value.memory for f in both_forms(layer)] == before
+    monkeypatch.setattr(qlayer, "capturing", lambda device: True)
+    with torch.no_grad():
+        layer.w_elements.add_(1)
+    assert layer._weight_form("_scaled_w").value.memory not in before                # (a graph's own form)
+    monkeypatch.setattr(qlayer, "capturing", lambda device: False)
+    layer.load_state_dict(state, assign=True)
+    assert not set(f.value.memory for f in both_forms(layer)) & set(before)
