@@ -10,11 +10,14 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <ATen/core/grad_mode.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../../include/mase_hip.h"
 #include "../../../include/mase_hip_scores.h"
@@ -492,6 +495,12 @@ PyObject* linear_plain(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// Would a product through torch.matmul show `left` more than its values: a graph for its gradient, a tangent, a trace, or autocast's type?
+bool followed(const at::Tensor& left) {
+    return (at::GradMode::is_enabled() && left.requires_grad()) || left._fw_grad(/*level=*/0).defined() || at::autocast::is_autocast_enabled(at::kCUDA) ||
+           torch::jit::tracer::isTracing();
+}
+
 // matmul_plain(left [.., M, K], right [.., K, N], format of left or None, format of right): batches of left @ right, the same leading axes on both
 // sides, right contiguous or the transposed view of a contiguous tensor: left quantised to bfloat16 (None: bfloat16 as it is), right to
 // components in [.., N, K] order, one batched product
@@ -524,7 +533,8 @@ PyObject* matmul_plain(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
             seen *= l->size(i);
         }
     }
-    PLAIN((M * N * (dt == 0 ? 4 : 2)) % 16 == 0 || (dt == 2 && N % 16 != 0));
+    // (products whose outputs do not all start on 16 bytes go through torch.matmul otherwise)
+    PLAIN((M * N * (dt == 0 ? 4 : 2)) % 16 == 0 || (dt == 2 && N % 16 != 0 && !followed(*l)));
     void* stream;
     PLAIN(stream_of(*l, &stream));
     Sizes shape = sizes_of(*l);

@@ -112,3 +112,27 @@ def test_batched_products(monkeypatch, batch, M, K, N, lying, l_fmt, r_fmt, dtyp
     if (M * N * y.element_size()) % 16 == 0:                                   # (others went through torch.matmul before)
         _without_extension(monkeypatch, "matmul_plain")
         assert torch.equal(MX.mxfp_matmul(*args), y)
+
+
+def test_products_that_torch_follows_stay_with_torch():
+    """Batches whose outputs do not all start on 16 bytes went through torch.matmul, which is differentiable in a dense left operand, and still do where that
+    shows.  (No backward is run here: it multiplies by a transposed view in bfloat16.)"""
+    import mase_hip.mxfp.functional as MX
+    import mase_hip.mxfp.meta as mx
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    left, right = (torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16) for s in ((2, 5, 64), (2, 64, 7)))
+    product = lambda x: MX.mxfp_matmul(x, right, None, mx.MXFP8_E4M3_fn, "XWq", "fused")      # noqa: E731
+    plain = product(left)
+    leaf = left.clone().requires_grad_()
+    y = product(leaf)
+    assert y.grad_fn is not None and not plain.requires_grad
+    assert ((y.detach().double() - plain.double()).norm() / plain.double().norm()).item() <= 1e-3
+    with torch.no_grad():
+        assert torch.equal(product(leaf), plain)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(left, torch.ones_like(left))
+        assert torch.autograd.forward_ad.unpack_dual(product(dual)).tangent is not None
+    with torch.autocast("cuda", torch.float16):
+        assert product(left).dtype == torch.float16
+    assert torch.equal(product(left), plain)
