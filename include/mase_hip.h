@@ -189,9 +189,8 @@ int mase_hip_mxfp_gemm(const void* a_dense, int a_dtype, const uint8_t* a_scales
  * and rounds to out_dtype.  The library allocates nothing, so the caller brings the memory:
  *
  *   mase_hip_mxfp_gemm_workspace_bytes(a_is_dense, M, N, K)
- *       bytes with which this shape can be split on the current device, 0 if it would not be
- *       (MXFP A, enough tiles, short K, sizes the split kernels do not take).  For N or K that are
- *       no multiples of a tile it may name bytes that the call then leaves alone.
+ *       bytes with which this shape would be split on the current device, 0 if it would not
+ *       (MXFP A, enough tiles, short K, sizes the split kernels do not take).
  *   mase_hip_mxfp_gemm_ws(..., workspace, workspace_bytes, stream)
  *       `workspace`: 16-byte aligned device memory of at least that many bytes, or NULL.  With
  *       NULL, or fewer bytes than the shape asks for, the call is mase_hip_mxfp_gemm.  The

@@ -146,12 +146,5 @@ extern "C" int mase_hip_mxfp_gemm_static_ws(const void* a_dense, int a_dtype, co
 
 extern "C" int64_t mase_hip_mxfp_gemm_workspace_bytes(int a_is_dense, int64_t M, int64_t N, int64_t K) {
     if (!a_is_dense || M < 1 || N < 1 || K < 1 || M > 0x7FFFFFFF || N > 0x7FFFFFFF || K > 0x7FFFFFFF) return 0;
-    const int m = (int)M, n = (int)N, k = (int)K, cus = device_cu_count();
-    const SplitPlan plan = plan_split_k(m, n, k, cus);
-    // (a ragged product that is as well off unsplit: room for two shares all the same, which such shapes have always asked for)
-    if (cus > 0 && plan.splits == 1 && K >= 256 && ragged_shape(m, n, k) && !takes_256(m, n, k)) {
-        const int64_t bytes = SplitPlan{2, k, 3}.workspace_bytes(m, n);
-        return bytes <= 33000000 ? bytes : 0;
-    }
-    return plan.workspace_bytes(m, n);
+    return plan_split_k((int)M, (int)N, (int)K, device_cu_count()).workspace_bytes((int)M, (int)N);
 }

@@ -19,7 +19,7 @@ DEV = "cuda:0"
     ((129, 130, 4128), "OCP_MXFP6_E3M2"),     # 129 steps
     ((120, 500, 800), "OCP_MXFP6_E2M3"),
     ((300, 1000, 4096), "MXFP8_E4M3_fn"),
-    ((257, 4080, 1056), "MXFP8_E4M3_fn"),
+    ((257, 4080, 4128), "MXFP8_E4M3_fn"),     # 128 x 128 tiles, five shares (of K = 1056 one tile's whole walk is as short)
 ])
 def test_ragged_split(MNK, tag):
     import mase_hip.mxfp.kernels as mxk
@@ -60,6 +60,8 @@ def test_ragged_split(MNK, tag):
     call(lib.mase_hip_mxfp_gemm_ws, ws.data_ptr(), need - 1)
     assert torch.equal(y[:M * N].view(M, N), unsplit) and (ws == 0).all()
     call(lib.mase_hip_mxfp_gemm_ws, ws.data_ptr(), need)
+    sums = ws.view(torch.float32).view(-1, pitch)[:, :M * N]
+    assert (sums != 0).any(1).all() and ((sums.double().sum(0).view(M, N) - unsplit).norm() / unsplit.norm()).item() <= 2e-6      # every share in its array
     assert ((y[:M * N].view(M, N) - unsplit).norm() / unsplit.norm()).item() <= 2e-6
     call(lib.mase_hip_mxfp_gemm_static_ws)                     # (does not split these: no scratch shared between streams)
     assert torch.equal(y[:M * N].view(M, N), unsplit)
@@ -70,4 +72,12 @@ def test_shapes_of_other_kernels_are_not_ragged():
 
     ws = _lib.load().mase_hip_mxfp_gemm_workspace_bytes
     for M, N, K in ((16, 4096, 4096), (64, 8192, 4096), (100, 14304, 4096), (2000, 4096, 4096), (300, 4096, 1088), (1, 777, 224), (4096, 4100, 4096), (16384, 14330, 4096)):
+        assert ws(1, M, N, K) == 0, (M, N, K)
+
+
+def test_products_that_are_left_whole_ask_for_no_room():
+    from mase_hip import _lib
+
+    ws = _lib.load().mase_hip_mxfp_gemm_workspace_bytes
+    for M, N, K in ((257, 4080, 1056), (700, 1000, 1024), (1500, 1300, 2048), (2000, 2000, 2080), (16, 2001, 256), (3000, 3001, 4096)):
         assert ws(1, M, N, K) == 0, (M, N, K)
