@@ -157,7 +157,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             tm = self.w_tensor_meta
             bf16 = (self.backend != "fused_scaled" and len(tm.shape) == 2 and kernels.scaled_format_supported(tm.meta) and tm.block_dim % 2 == 1
                     and input.dtype == torch.bfloat16 and getattr(torch, tm.dtype) == input.dtype
-                    and kernels.prepared_w_shape_supported(rows, tm.shape[0], tm.shape[1]))
+                    and kernels.prepared_w_pays(rows, tm.shape[0], tm.shape[1]))
             if not bf16:
                 return None
         return self._weight_form("_scaled_w", needed=scaled)

@@ -559,8 +559,9 @@ def test_prepared_weight_special_blocks_and_refusals(mh):
 
 
 def test_weight_only_layer_keeps_the_prepared_weight(mh):
-    """XWqB (dense bfloat16 activations): from 512 rows on the layer runs the bf16 kernel on its kept prepared weight."""
-    lin = torch.nn.Linear(512, 256, bias=True, dtype=torch.bfloat16, device=DEV)
+    """XWqB (dense bfloat16 activations): from 512 rows on the layer runs the bf16 kernel on its kept prepared weight where that is the faster one, and keeps
+    none where it is not."""
+    lin = torch.nn.Linear(512, 8192, bias=True, dtype=torch.bfloat16, device=DEV)      # (of 256 features the components are faster: no prepared weight)
     wfmt = mh.meta.OCP_MXFP4_E2M1
     fused = mh.MXFPLinearPTQ.from_linear(lin, None, wfmt, None, "XWqB", "fused")
     sep = mh.MXFPLinearPTQ.from_linear(lin, None, wfmt, None, "XWqB", "separate")
@@ -569,8 +570,16 @@ def test_weight_only_layer_keeps_the_prepared_weight(mh):
     big = torch.randn(2, 300, 512, generator=g).to(torch.bfloat16).to(DEV)
     assert rel_fro(fused(small), sep(small)) <= 1e-3 and fused._scaled_w is None
     y = fused(big)
-    assert fused._scaled_w is not None and y.shape == (2, 300, 256)
+    assert fused._scaled_w is not None and y.shape == (2, 300, 8192)
     assert rel_fro(y, sep(big)) <= 1e-3
+    for features, rows in (((512, 256), 600), ((4096, 4096), 1024)):
+        assert not mh.mxk.prepared_w_pays(rows, features[1], features[0])
+        lin = torch.nn.Linear(*features, bias=True, dtype=torch.bfloat16, device=DEV)
+        fused = mh.MXFPLinearPTQ.from_linear(lin, None, wfmt, None, "XWqB", "fused")
+        sep = mh.MXFPLinearPTQ.from_linear(lin, None, wfmt, None, "XWqB", "separate")
+        x = torch.randn(rows, features[0], generator=g).to(torch.bfloat16).to(DEV)
+        assert rel_fro(fused(x), sep(x)) <= 1e-3 and rel_fro(fused(x), sep(x)) <= 1e-3
+        assert fused._scaled_w is None and fused._fast_packed == 3
 
 
 def test_unsupported_shapes_are_refused(mh):

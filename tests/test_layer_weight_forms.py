@@ -177,3 +177,12 @@ def test_what_a_graph_reads_follows_components_written_in_place(layer, monkeypat
     monkeypatch.setattr(qlayer, "capturing", lambda device: False)
     layer.load_state_dict(state, assign=True)
     assert not set(f.value.memory for f in both_forms(layer)) & set(before)
+
+
+def test_no_form_is_built_that_the_call_does_not_read(layer, monkeypatch):
+    """A weight-only call of many rows whose product is faster on the components."""
+    layer.layer_type, layer.x_mxfp_meta = "XWqB", None
+    monkeypatch.setattr(kernels, "prepared_w_shape_supported", lambda *a: True)
+    for pays in (False, True):
+        monkeypatch.setattr(kernels, "prepared_w_pays", lambda *a: pays)
+        assert (layer._weight_operand(OnGpu()) is not None) == pays
