@@ -105,6 +105,13 @@ def test_the_tile_plan_covers_k(lib):
                     assert scaled_plan(lib, M, N, K, False, cus)[1:] == (1, nmac)
 
 
+def test_few_tiles_of_a_long_k_share_it(lib):
+    """The shapes on which the GPU tests compare a product in shares of K with the whole one."""
+    for shape, plan in (((256, 256, 4096), (64, 8)), ((300, 520, 4096), (64, 4)), ((1024, 512, 14336), (128, 8)), ((700, 264, 7168), (64, 8))):
+        assert scaled_plan(lib, *shape)[:2] == plan, shape
+    assert scaled_plan(lib, 300, 520, 2048)[:2] == (64, 1)
+
+
 def test_one_full_round_of_large_tiles_is_not_given_to_two_of_small_ones(lib):
     for M in (65, 96, 128):
         for K in (512, 1024, 2048):
