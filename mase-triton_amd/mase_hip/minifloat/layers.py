@@ -199,7 +199,8 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the codes
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._note == (sig, 0):
+        note = self._note
+        if note == (sig, 0):
             form, w = self._scaled_w, self.w_element
             if form is not None and form.key == (w.data_ptr(), w._version):
                 from ..mxfp import kernels
@@ -243,7 +244,9 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             self._keep_form("_narrowed", narrowed)
         if w_operand is not None:
             self._keep_form("_scaled_w", w_operand)
-        elif not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
+        elif not asked:
+            notes["_no_operand_sig"], notes["_note"] = sig, note
+        elif not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

@@ -224,7 +224,8 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         # A call that looks like the last one that ran on the block-scaled GEMM with the kept weight operand, the weight
         # unchanged since, goes straight to the two kernels: the checks below cost more host time than a decode-sized
         # product takes on the GPU.
-        if self._note == (sig, 0):
+        note = self._note
+        if note == (sig, 0):
             form, w_elements, w_scales = self._scaled_w, self.w_elements, self.w_scales
             if form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
                 from . import kernels
@@ -265,7 +266,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w_operand=None if w_operand is None else w_operand.value)
         if w_operand is not None:
             self._keep_form("_scaled_w", w_operand)
-        elif not (asked and capturing(input.device)):     # (a captured call may have gone without a form that it has a use for)
+        elif not asked:
+            notes["_no_operand_sig"], notes["_note"] = sig, note
+        elif not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

@@ -71,3 +71,19 @@ def test_notes_cost_no_module_assignments(layer_and_calls, monkeypatch):
         layer(torch.zeros(rows, 32))
     assert names == [] and calls["asked"] == 3
     assert layer._no_operand_sig is not None and layer._fast_sig is None
+
+
+def test_what_a_call_is_not_eligible_for_is_not_asked_again(layer_and_calls, monkeypatch):
+    """Calls that the extension does not take (fp16, a format that the kernels do not decode) are looked at once for every look."""
+    import mase_hip.minifloat.functional.linear as MFL
+    import mase_hip.mxfp.functional.linear as MXL
+
+    layer, calls = layer_and_calls
+    asked = []
+    for L in (MXL, MFL):
+        monkeypatch.setattr(L, "_gemm_eligible", lambda *a: asked.append(1))
+    layer.layer_type, layer.backend = "XqWq", "fused"
+    layer.w_tensor_meta = None
+    for rows, times in ((2, 1), (2, 1), (2, 1), (3, 2), (2, 3), (2, 3)):
+        layer(torch.zeros(rows, 32))
+        assert len(asked) == times and layer._fast_sig is None
