@@ -80,3 +80,25 @@ def test_extract_down_the_rows_leaves_room_for_six_wavefronts(tmp_path):
     occupancy = dict(zip(re.findall(r"^(_ZN4mase\w+):\s*; @", text, re.M), re.findall(r"; Occupancy: (\d+)", text)))
     occupancy = {name: int(n) for name, n in occupancy.items() if "mxfp_strided_tile_kernel" in name}
     assert len(occupancy) == 15 and min(occupancy.values()) >= 6, occupancy
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_composing_e5m2_takes_no_comparison_for_each_code(tmp_path):
+    """The one format that the convert instruction does not read.  A test of every code's sign made the kernels depend on how the compiler writes it, two
+    instructions or three by what else a translation unit holds."""
+    probe = tmp_path / "compose.hip"
+    probe.write_text(f"""#include "{CSRC}/mase_device.h"
+#include "{CSRC}/mxfp_compose.h"
+extern "C" __global__ void compose(const uint4* codes, const uint32_t* scales, uint4* out) {{
+    uint4 lo, hi;
+    mase::Composer<mase::SFmt<5, 2>>(scales[threadIdx.x]).run16(codes[threadIdx.x], lo, hi);
+    out[2 * threadIdx.x] = lo;
+    out[2 * threadIdx.x + 1] = hi;
+}}
+""")
+    out = str(tmp_path / "compose.s")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-S", str(probe),
+                    "-o", out], check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL, timeout=300)
+    with open(out) as f:
+        text = f.read()
+    assert text.count("v_cvt_pk_bf16_f32") == 8 and len(re.findall(r"^\s+v_cmp", text, re.M)) <= 1      # (a scale of 2^-127)
