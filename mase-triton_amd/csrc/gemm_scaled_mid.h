@@ -291,6 +291,15 @@ struct ScaledMidPlan {
 // One row of the smaller tiles (up to 128 rows of A) shares nothing of W: a second round adds a wait, up to 1.4 us when it is full (128 x
 // 65536, K = 512 / 1024 / 2048: 14.6 / 19.5 / 29.3 us on 128 x 128 tiles, 12.8 / 17.7 / 27.2 on one round of 256 x 256 ones, fp32 out 18.0 / 23.4 / 33.1
 // and 14.3 / 19.5 / 28.6; K = 4096 53 and 55).
+// the price of `splits` equal shares of K on 256 x 256 tiles
+inline double scaled_256_price(int M, int N, int nmac, int splits, int cus) {
+    const int64_t wgs = (int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN) * splits;
+    const double busy = wgs >= cus ? 1.0 : (double)wgs / cus, sums_mb = (double)M * N * 4.0 / 1e6;
+    return (double)((wgs + cus - 1) / cus) * (nmac / splits * (1.0 + 0.2 * busy)) + 8.0 + (splits > 1 ? 3.0 + (2.0 * splits + 0.5) * sums_mb * 0.16 : 0.0);
+}
+inline bool scaled_256_shares_ok(int M, int N, int nmac, int splits, int cus) {      // (that kernel walks equal shares of pairs of macro steps)
+    return splits == 1 || ((int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN) * splits <= cus && nmac % splits == 0 && nmac / splits % 2 == 0 && nmac / splits >= 4);
+}
 inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
     const int nmac = K / SMAC;
     ScaledMidPlan best{256, 256, 1, nmac};
@@ -298,24 +307,27 @@ inline ScaledMidPlan plan_scaled(int M, int N, int K, int cus, bool may_split) {
     const bool few_columns = M <= 1600 && N <= 8192 && K <= 4096;
     const double mn_mb = (double)M * N * 4.0 / 1e6;
     double best_t = 1e30;
-    for (int bn = 256; bn >= 64; bn /= 2) {
-        const int64_t tiles = bn == 256 ? (int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN) : (int64_t)((M + 127) / 128) * ((N + bn - 1) / bn);
+    for (int want = 1; want <= (may_split ? 16 : 1); ++want) {
+        if (!scaled_256_shares_ok(M, N, nmac, want, cus)) continue;
+        if (const double t = scaled_256_price(M, N, nmac, want, cus); t < best_t) { best_t = t; best = ScaledMidPlan{256, 256, want, nmac / want}; }
+    }
+    for (int bn = 128; bn >= 64; bn /= 2) {
+        const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + bn - 1) / bn);
         for (int want = 1; want <= 16; ++want) {
             if (want > 1 && (!may_split || tiles * want > cus)) break;
             const int per = (nmac + want - 1) / want;
             if (want > 1 && (per < 4 || (nmac + per - 1) / per != want)) continue;
-            if (bn == 256 && want > 1 && (nmac % want != 0 || per % 2 != 0)) continue;      // that kernel walks equal shares of pairs
             const int64_t wgs = tiles * want;
             const double busy = wgs >= cus ? 1.0 : (double)wgs / cus;
-            const double step = bn == 256 ? 1.0 + 0.2 * busy : bn == 128 ? 0.62 : 0.37 + 0.09 * busy;
+            const double step = bn == 128 ? 0.62 : 0.37 + 0.09 * busy;
             const double rounds = (double)((wgs + cus - 1) / cus);
-            const double unshared = bn != 256 && M <= 128 && wgs > cus ? 1.4 * std::min(1.0, (double)(wgs - cus) / cus) : 0.0;
-            double t = rounds * (per * step + (bn == 256 ? 0.0 : 2.5)) + (bn == 256 ? 8.0 : 2.0 + unshared) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
+            const double unshared = M <= 128 && wgs > cus ? 1.4 * std::min(1.0, (double)(wgs - cus) / cus) : 0.0;
+            double t = rounds * (per * step + 2.5) + (2.0 + unshared) + (want > 1 ? 3.0 + (2.0 * want + 0.5) * mn_mb * 0.16 : 0.0);
             if (bn == 128 && few_columns)
                 t = 1.25 * (rounds * (per * (0.292 + 0.195 * busy) + 0.77) + 4.65 + unshared + (want > 1 ? 2.9 + std::max(0.0, 0.55 * want - 0.8) * mn_mb : 0.0));
             else if (bn == 64 && few_columns)
                 t = 1.25 * (rounds * (per * (0.222 + 0.097 * busy) + 1.3) + 3.35 + unshared + (want > 1 ? 2.4 + std::max(0.0, 0.75 * want - 1.0) * mn_mb : 0.0));
-            if (t < best_t) { best_t = t; best = ScaledMidPlan{bn == 256 ? 256 : 128, bn, want, per}; }
+            if (t < best_t) { best_t = t; best = ScaledMidPlan{128, bn, want, per}; }
         }
     }
     return best;

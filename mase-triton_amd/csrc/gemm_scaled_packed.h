@@ -268,18 +268,11 @@ inline ScaledMidPlan plan_packed(bool six, int M, int N, int K, int cus, bool ma
     if (price) *price = best_t;
     return best;
 }
-// the price of 256 x 256 tiles of bytes (plan_scaled's), which many rows are better on
+// the price of 256 x 256 tiles of bytes, which many rows are better on
 inline double price_256(int M, int N, int K, int cus) {
-    const int nmac = K / SMAC;
-    const int64_t tiles = (int64_t)((M + SM - 1) / SM) * ((N + SN - 1) / SN);
     double best = 1e30;
-    for (int want = 1; want <= 16 && (want == 1 || tiles * want <= cus); ++want) {
-        if (want > 1 && (nmac % want != 0 || nmac / want % 2 != 0 || nmac / want < 4)) continue;
-        const int64_t wgs = tiles * want;
-        const double t = (double)((wgs + cus - 1) / cus) * (nmac / want) * (1.0 + 0.2 * std::min(1.0, (double)wgs / cus)) + 8.0 +
-                         (want > 1 ? 3.0 + (2.0 * want + 0.5) * ((double)M * N * 4.0 / 1e6) * 0.16 : 0.0);
-        best = std::min(best, t);
-    }
+    for (int want = 1; want <= 16; ++want)
+        if (scaled_256_shares_ok(M, N, K / SMAC, want, cus)) best = std::min(best, scaled_256_price(M, N, K / SMAC, want, cus));
     return best;
 }
 // Is the packed weight faster than bytes for such a product?  A small weight is launches and latencies either way, and the 6-bit fragments are two loads
