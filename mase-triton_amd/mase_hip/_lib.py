@@ -61,6 +61,7 @@ SCORES_SIGNATURES = {
 
 # include/mase_hip_linear.h
 LINEAR_SIGNATURES = {
+    "mase_hip_event_done": (_i32, [_vp]),
     "mase_hip_mxfp_linear_few_plan": (_i32, [_i64, _i64, _i64]),
     "mase_hip_mxfp_linear_few": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp]),
     "mase_hip_mxfp_packed_dense_plan": (_i32, [_i64, _i64, _i64, _i32, _i32]),
@@ -168,6 +169,11 @@ def stream_ptr(device: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(device.index if device.index is not None else torch.cuda.current_device())
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def event_done(event) -> bool:
+    """Has what a torch event was recorded behind run?  Asked without touching captures, of this thread or another."""
+    return bool(load().mase_hip_event_done(event.cuda_event))
 
 
 _NO_SWITCH = contextlib.nullcontext()

@@ -49,14 +49,13 @@ def narrow_weight_codes(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta, i
     the decode of the reference (src/mase_triton/minifloat/fake.py:97-123).  ``into``: an earlier result whose memory this one takes."""
     assert w_element.dtype == torch.uint16
     low = w_element.contiguous().view(torch.uint8).view(*w_element.shape, 2)[..., 0]
-    if into is not None and (into[1].shape != low.shape or into[1].device != low.device):
-        into = None
-    codes = low.contiguous() if into is None else into[1].copy_(low)
     n_bits = w_tensor_meta.meta.n_bits
+    if into is not None and into[1].shape == low.shape and into[1].device == low.device:
+        into[1].copy_(low & ((1 << n_bits) - 1) if n_bits < 8 else low)      # (in one step: calls may read it)
+        return into
+    codes = low.contiguous()
     if n_bits < 8:
         codes &= (1 << n_bits) - 1
-    if into is not None:
-        return into
     scales = torch.full((w_element.numel() // 32,), _UNIT_SCALE, dtype=torch.uint8, device=w_element.device)
     return scales, codes
 

@@ -124,12 +124,8 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             return MinifloatF.narrow_weight_codes(w_element, tm, into)
         narrowed = self._narrowed_weight()
         if name == "_scaled_w":
-            value = L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value, into)
-        else:
-            value = kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features, into)
-        if narrowed is not None:
-            self._keep_form("_narrowed", narrowed)
-        return value
+            return L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value, into)
+        return kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features, into)
 
     def _weight_operand(self, input: Tensor) -> WeightForm | None:
         """The weight in the block-scaled GEMM's form when this call takes that GEMM (quantised bfloat16 activations, see
@@ -178,7 +174,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         if note is not None and note[0] == sig:
             w, packed = self._parameters.get("w_element"), note[1]     # (none: held otherwise, by a parametrisation)
             form = self._narrowed if packed == 3 else self._packed_w if packed else self._scaled_w
-            if form is not None and w is not None and form.key == (w.data_ptr(), w._version):
+            if form is not None and w is not None and form.key == (w.data_ptr(), w._version) and (form.event is None or form.ready()):
                 xm, bias, op = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, form.value
                 if packed == 3:
                     (scales, codes), m = op, self.w_tensor_meta.meta
@@ -202,7 +198,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         note = self._note
         if note == (sig, 0):
             form, w = self._scaled_w, self.w_element
-            if form is not None and form.key == (w.data_ptr(), w._version):
+            if form is not None and form.key == (w.data_ptr(), w._version) and (form.event is None or form.ready()):
                 from ..mxfp import kernels
 
                 xm = self.x_minifloat_meta
@@ -229,7 +225,6 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:
                 y = kernels.linear_packed(_lib.dense(x2), xm.exp_bits, xm.frac_bits, True, w, None if bias is None else bias.contiguous())
-            self._keep_form("_packed_w", packed[0])
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
@@ -240,13 +235,9 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             _narrowed=None if narrowed is None else narrowed.value, _w_operand=None if w_operand is None else w_operand.value)
-        if narrowed is not None:
-            self._keep_form("_narrowed", narrowed)
-        if w_operand is not None:
-            self._keep_form("_scaled_w", w_operand)
-        elif not asked:
+        if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
-        elif not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
+        elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

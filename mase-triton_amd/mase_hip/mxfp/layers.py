@@ -205,7 +205,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                     if y is not None:
                         return y
             elif (form is not None and w_elements is not None and w_scales is not None
-                  and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version)):
+                  and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version) and (form.event is None or form.ready())):
                 meta, w = self.x_mxfp_meta, form.value
                 bias = None if self.layer_type.endswith("Bq") else self.bias
                 if packed == 2:
@@ -227,7 +227,8 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         note = self._note
         if note == (sig, 0):
             form, w_elements, w_scales = self._scaled_w, self.w_elements, self.w_scales
-            if form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version):
+            if (form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version)
+                    and (form.event is None or form.ready())):
                 from . import kernels
 
                 x2 = input.reshape(-1, self.in_features)
@@ -254,7 +255,6 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:
                 y = kernels.linear_packed(_lib.dense(x2), meta.element_exp_bits, meta.element_frac_bits, False, w, None if bias is None else bias.contiguous())
-            self._keep_form("_packed_w", packed[0])
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
@@ -264,11 +264,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
             w_operand=None if w_operand is None else w_operand.value)
-        if w_operand is not None:
-            self._keep_form("_scaled_w", w_operand)
-        elif not asked:
+        if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
-        elif not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
+        elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 
@@ -295,7 +293,6 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                                                       up.reshape(-1, self.in_features) if up.ndim != 2 else up, self.x_mxfp_meta)
             y = (kernels.mxfp_gemm_scaled(a_op, form.value, self.bias, gate.dtype) if packed is None
                  else kernels.mxfp_gemm_packed(a_op, form.value, self.bias))
-            self._keep_form("_scaled_w" if packed is None else "_packed_w", form)
             return y.view(*gate.shape[:-1], self.out_features)
         return self.forward(torch.nn.functional.silu(gate) * up)
 

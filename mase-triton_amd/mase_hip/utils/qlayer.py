@@ -1,4 +1,6 @@
 """Helpers for the PTQ layers (the first two: same contract as src/mase_triton/utils/qlayer.py:4-21)."""
+import threading
+
 import torch
 
 from .. import _lib
@@ -22,18 +24,6 @@ def devices_equal(device1, device2) -> bool:
     return _canonical(device1) == _canonical(device2)
 
 
-class WeightForm:
-    """A quantised weight in another form than its stored components.
-
-    ``key`` names the components that it was built from, by address and version.  An address names a tensor only until its memory is handed out
-    again, so the form holds an alias of each: whatever replaces a component while the form is kept lies elsewhere."""
-
-    __slots__ = ("value", "key", "components")
-
-    def __init__(self, value, key: tuple, components: tuple):
-        self.value, self.key, self.components = value, key, components
-
-
 def weight_key(components) -> tuple:
     return tuple(v for c in components for v in (c.data_ptr(), c._version))
 
@@ -46,10 +36,42 @@ def capturing(device: torch.device) -> bool:
         return torch.cuda.is_current_stream_capturing()
 
 
-def finish(device: torch.device, every_stream: bool) -> None:
-    """Wait for the current stream of ``device``, or for all its streams."""
+def launched(device: torch.device):
+    """An event behind what the current stream of ``device`` has been given (None: nothing runs behind the host)."""
+    if device.type != "cuda":
+        return None
     with _lib.on_device(device):
-        torch.cuda.synchronize(device) if every_stream else torch.cuda.current_stream(device).synchronize()
+        return torch.cuda.current_stream(device).record_event()
+
+
+class WeightForm:
+    """A quantised weight in another form than its stored components.
+
+    ``key`` names the components that it was built from, by address and version.  An address names a tensor only until its memory is handed out
+    again, so the form holds an alias of each: whatever replaces a component while the form is kept lies elsewhere.  ``event`` is behind the kernels
+    that write the form, None once they are known to have run."""
+
+    __slots__ = ("value", "key", "components", "event")
+
+    def __init__(self, value, key: tuple, components: tuple, event):
+        self.value, self.key, self.components, self.event = value, key, components, event
+
+    def ready(self) -> bool:
+        """Put the current stream behind what writes the form; False where that cannot be (the stream is captured and the form not written yet)."""
+        event, device = self.event, self.components[0].device
+        if event is None:
+            return True
+        if _lib.event_done(event):
+            self.event = None
+            return True
+        if capturing(device):
+            return False
+        with _lib.on_device(device):
+            torch.cuda.current_stream(device).wait_event(event)
+        return True
+
+
+_publish = threading.Lock()
 
 
 class KeepsWeightForms:
@@ -57,9 +79,8 @@ class KeepsWeightForms:
     (``_FORM_COMPONENTS``).  Forms are built on the first call that reads them and again after a change of the components, and are part of
     neither ``state_dict`` nor a copy or pickle of the layer.
 
-    A form is built on the stream of the call and read by calls on any stream and of any thread.  So a call uses what it has built in its stream's
-    order, and once its product is launched waits for the stream and only then shows the form to others (``_keep_form``): once in a form's life,
-    where an event would have to be asked about on every call, and cannot be under capture.
+    A form is built on the stream of one call and read by calls on any stream and of any thread, which wait for its event until it has been seen to have
+    run: ``ready``, asked as long as there is an event.  (The building call could wait for its stream instead: a new layer's first call 63 -> 93 us.)
 
     A captured call reads the forms that were kept then, where they lie.  So components that are written in place are built into the same memory again,
     by the next call or by ``load_state_dict`` itself, and replays follow; a graph is captured again after the components were replaced or moved or
@@ -84,27 +105,28 @@ class KeepsWeightForms:
         raise NotImplementedError
 
     def _weight_form(self, name: str, needed: bool = True) -> WeightForm | None:
-        """The form ``name`` of the weight as it is now: the kept one, or a new one for ``_keep_form``.  One that is built while the stream is captured
-        belongs to that graph, which writes it on every replay; with ``needed`` false, for a call that has another way, None in its place."""
+        """The form ``name`` of the weight as it is now, for the current stream.  One that is built while the stream is captured belongs to that graph, which
+        writes it on every replay; with ``needed`` false, for a call that has another way, None in its place."""
         components = tuple(getattr(self, c) for c in self._FORM_COMPONENTS)
-        kept, key = getattr(self, name), weight_key(components)
-        if kept is not None and kept.key == key:
+        kept, key, device = getattr(self, name), weight_key(components), components[0].device
+        if kept is not None and kept.key == key and kept.ready():
             return kept
-        in_graph = capturing(components[0].device)
+        in_graph = capturing(device)
         if in_graph and not needed:
             return None
-        into = kept.value if kept is not None and kept.key[::2] == key[::2] and not in_graph else None      # (the same tensors, written since)
-        return WeightForm(self._build_form(name, into, *components), key, tuple(c.detach() for c in components))
-
-    def _keep_form(self, name: str, form: WeightForm) -> None:
-        """Keep a form that ``_weight_form`` gave, for calls on every stream."""
-        kept = getattr(self, name)
-        if form is kept or capturing(form.components[0].device):
-            return
-        if any(isinstance(getattr(type(self), c, None), property) for c in self._FORM_COMPONENTS):
-            return                                            # (a parametrisation makes another tensor for every call)
-        finish(form.components[0].device, every_stream=kept is not None)      # (calls on other streams may still read the one that goes)
-        self.__dict__[name] = form
+        written = kept is not None and kept.key[::2] == key[::2] and not in_graph       # the same tensors, written since
+        if written:
+            kept.ready()
+        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, tuple(c.detach() for c in components),
+                          None if in_graph else launched(device))
+        if in_graph or any(isinstance(getattr(type(self), c, None), property) for c in self._FORM_COMPONENTS):
+            return form                                       # (a parametrisation makes another tensor for every call)
+        if kept is not None and not written and device.type == "cuda":
+            torch.cuda.synchronize(device)                    # (calls on other streams may still read the one that goes)
+        with _publish:
+            if getattr(self, name) is kept:                   # (else another thread's call was faster)
+                self.__dict__[name] = form
+        return form
 
     def _drop_forms(self, moved_only: bool = False) -> None:
         """Forget the forms, or those whose components are not the layer's any more."""
@@ -120,7 +142,7 @@ class KeepsWeightForms:
         for name in self._FORMS:
             kept = getattr(self, name)
             if kept is not None and kept.key[::2] == weight_key([getattr(self, c) for c in self._FORM_COMPONENTS])[::2]:
-                self._keep_form(name, self._weight_form(name))
+                self._weight_form(name)
 
     def __getstate__(self):
         return {**self.__dict__, **dict.fromkeys(self._FORMS), "_note": None}

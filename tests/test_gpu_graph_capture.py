@@ -132,3 +132,36 @@ def test_replays_follow_a_weight_that_is_loaded_in_place(family, layer_type, row
     graph.replay()
     torch.cuda.synchronize()
     assert torch.equal(y, want[1])
+
+
+def test_one_call_before_the_capture_is_enough():
+    """The capture finds a form whose event nobody has asked about since: the query does not end the capture, and the form is read, not built again."""
+    import mase_hip.mxfp.meta as mx
+    from mase_hip import _lib
+    from mase_hip.mxfp.layers import MXFPLinearPTQ
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    w = torch.randn(2048, 4096, generator=g, device=DEV).to(torch.bfloat16)
+    x = torch.randn(12, 4096, generator=g, device=DEV).to(torch.bfloat16)
+    layer = MXFPLinearPTQ(w, None, None, mx.OCP_MXFP4_E2M1, None, "XWqB", "fused")
+    want = layer(x)
+    torch.cuda.synchronize()
+    form, graph = layer._packed_w, torch.cuda.CUDAGraph()
+    assert form.event is not None
+    with torch.cuda.graph(graph):
+        y = layer(x)
+    assert layer._packed_w is form and form.event is None
+    side, busy = torch.cuda.Stream(), torch.randn(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):                  # an event that is still to come
+        for _ in range(20):
+            torch.mm(busy, busy)
+        event = side.record_event()
+    early = _lib.event_done(event)
+    side.synchronize()
+    assert not early and _lib.event_done(event)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(layer(x), want)

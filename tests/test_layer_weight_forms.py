@@ -37,7 +37,6 @@ def layer(monkeypatch):
     monkeypatch.setattr("mase_hip.mxfp.functional.linear.scaled_weight_operand", lambda scales, elements, meta, into: Form(elements, into))
     monkeypatch.setattr(kernels, "packed_weight_from_mxfp", lambda scales, elements, e, m, rows, k, into: Form(elements, into))
     monkeypatch.setattr(kernels, "packed_pays", lambda *a: True)
-    monkeypatch.setattr(qlayer, "finish", lambda device, every_stream: None)
     scales, elements = components(0)
     meta = mx.MXFPTensorMeta(device="cpu", dtype="bfloat16", shape=(N, K), block_dim=1, meta=mx.OCP_MXFP4_E2M1)
     return MXFPLinearPTQ.from_quantized(scales, elements, meta, None, None, None, None, mx.MXFP8_E4M3_fn, "XqWqB", "fused")
@@ -56,10 +55,7 @@ class OnGpu:
 
 
 def both_forms(layer):
-    forms = layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
-    layer._keep_form("_scaled_w", forms[0])
-    layer._keep_form("_packed_w", forms[1])
-    return forms
+    return layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
 
 
 def test_forms_go_with_the_components_that_move(layer):
@@ -98,9 +94,7 @@ def test_a_copy_builds_its_own_forms(layer):
 def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
     """What a captured stream is given runs on the replays: nothing is written yet for the calls between."""
     monkeypatch.setattr(qlayer, "capturing", lambda device: True)
-    form = layer._weight_form("_scaled_w")
-    layer._keep_form("_scaled_w", form)
-    assert layer._packed_weight(OnGpu(), True) is None and form.value.sum > 0
+    assert layer._packed_weight(OnGpu(), True) is None and layer._weight_form("_scaled_w").value.sum > 0
     assert layer._scaled_w is None and layer._packed_w is None
     monkeypatch.setattr(qlayer, "capturing", lambda device: False)
     kept = both_forms(layer)
@@ -108,20 +102,59 @@ def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
     assert both_forms(layer) == kept == (layer._scaled_w, layer._packed_w)
 
 
-def test_forms_are_shown_to_other_streams_when_they_are_written(layer, monkeypatch):
-    """The call that builds a form uses it in its stream's order; others see it when that stream has run."""
-    order = []
+class Event:
+    """A stand-in for an event on a GPU."""
+
+    cuda_event, done = 0, False
+
+
+def test_calls_wait_for_a_form_until_it_is_written(layer, monkeypatch):
+    """On whichever stream: each goes behind the event of the call that built the form, until one finds that it has run; none does under capture."""
+    event, waits, products = Event(), [], []
     monkeypatch.setattr(_lib, "dense", lambda t: t)
-    monkeypatch.setattr(kernels, "linear_packed", lambda *a: (order.append("product"), torch.zeros(4, N))[1])
-    monkeypatch.setattr(qlayer, "finish", lambda device, every_stream: order.append((layer._packed_w, every_stream)))
+    monkeypatch.setattr(_lib, "event_done", lambda e: e.done)
+    monkeypatch.setattr(qlayer, "launched", lambda device: event)
+    monkeypatch.setattr(qlayer.torch.cuda, "current_stream", lambda device: type("Stream", (), {"wait_event": lambda self, e: waits.append(e)})())
+    monkeypatch.setattr(kernels, "linear_packed", lambda *a: (products.append("wrappers"), torch.zeros(4, N))[1])
+
+    class Host:
+        linear_packed = staticmethod(lambda *a: products.append("extension") or torch.zeros(4, N))
+
+    monkeypatch.setattr(_lib, "_host", Host)
     layer(OnGpu())
-    first = layer._packed_w
-    assert order == ["product", (None, False)] and first is not None
+    form = layer._packed_w
+    assert form.event is event and waits == [] and products == ["wrappers"]           # (the building call's own stream has the order)
+    layer(OnGpu())
+    layer._forward(OnGpu(), ())
+    assert waits == [event] * 2 and products == ["wrappers", "extension", "wrappers"]
+    monkeypatch.setattr(qlayer, "capturing", lambda device: True)
+    assert layer._packed_weight(OnGpu(), True) is None and layer._packed_w is form and len(waits) == 2
+    event.done = True
+    assert layer._packed_weight(OnGpu(), True)[0] is form and form.event is None
+    monkeypatch.setattr(qlayer, "capturing", lambda device: False)
+    layer(OnGpu())
+    assert len(waits) == 2
+    # written in place: behind what wrote it before
+    form.event, event.done = event, False
     with torch.no_grad():
         layer.w_elements.add_(1)
-    order.clear()
     layer._forward(OnGpu(), ())
-    assert order == ["product", (first, True)] and layer._packed_w is not first      # (a call on another stream may still read the first)
+    assert len(waits) == 3 and layer._packed_w is not form and layer._packed_w.value.memory is form.value.memory
+
+
+def test_of_two_threads_that_build_a_form_one_keeps_its_own(layer, monkeypatch):
+    """The other uses what it has built: a form that calls on other streams may already read is not given back."""
+    build, first = layer._build_form, []
+
+    def build_and_be_overtaken(name, into, *components):
+        if not first:
+            first.append(None)
+            first.append(layer._weight_form(name))
+        return build(name, into, *components)
+
+    monkeypatch.setattr(layer, "_build_form", build_and_be_overtaken)
+    form = layer._weight_form("_scaled_w")
+    assert layer._scaled_w is first[1] is not form and form.value.sum == first[1].value.sum
 
 
 def test_components_that_a_parametrisation_makes_have_no_kept_forms(layer):
