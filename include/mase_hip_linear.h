@@ -88,10 +88,11 @@ int mase_hip_mxfp_gemm_prepared_w_ws(const void* a_dense, int a_dtype, const uin
 int mase_hip_mxfp_prepared_w_pays(int64_t M, int64_t N, int64_t K);
 
 /*
- * For callers that build a prepared or packed weight on one stream and read it on others: has what `event` (a hipEvent_t that was recorded) is behind run?  1: yes,
- * 0: not yet, or not to be known.  May be asked while streams are captured, by this thread or another; no capture is touched.
+ * For callers that build a prepared or packed weight on one stream and read it on others: has all that `stream` was given run, or what `event` (a hipEvent_t that was
+ * recorded on it; or NULL) is behind?  1: yes, 0: not yet, or not to be known (a stream that is captured itself).  May be asked while other streams are captured, by
+ * this thread or another; no capture is touched.
  */
-int mase_hip_event_done(void* event);
+int mase_hip_stream_done(void* stream, void* event);
 
 #ifdef __cplusplus
 }

@@ -61,7 +61,7 @@ SCORES_SIGNATURES = {
 
 # include/mase_hip_linear.h
 LINEAR_SIGNATURES = {
-    "mase_hip_event_done": (_i32, [_vp]),
+    "mase_hip_stream_done": (_i32, [_vp, _vp]),
     "mase_hip_mxfp_linear_few_plan": (_i32, [_i64, _i64, _i64]),
     "mase_hip_mxfp_linear_few": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i64, _vp]),
     "mase_hip_mxfp_packed_dense_plan": (_i32, [_i64, _i64, _i64, _i32, _i32]),
@@ -171,9 +171,10 @@ def stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-def event_done(event) -> bool:
-    """Has what a torch event was recorded behind run?  Asked without touching captures, of this thread or another."""
-    return bool(load().mase_hip_event_done(event.cuda_event))
+def stream_done(stream, event=None) -> bool:
+    """Has all that a torch stream was given run, or what ``event``, recorded on it, is behind?  Asked without touching captures; False of a stream that is
+    captured itself."""
+    return bool(load().mase_hip_stream_done(stream.cuda_stream, None if event is None else event.cuda_event))
 
 
 _NO_SWITCH = contextlib.nullcontext()

@@ -174,7 +174,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         if note is not None and note[0] == sig:
             w, packed = self._parameters.get("w_element"), note[1]     # (none: held otherwise, by a parametrisation)
             form = self._narrowed if packed == 3 else self._packed_w if packed else self._scaled_w
-            if form is not None and w is not None and form.key == (w.data_ptr(), w._version) and (form.event is None or form.ready()):
+            if form is not None and w is not None and form.key == (w.data_ptr(), w._version) and (form.stream is None or form.ready()):
                 xm, bias, op = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, form.value
                 if packed == 3:
                     (scales, codes), m = op, self.w_tensor_meta.meta
@@ -198,7 +198,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         note = self._note
         if note == (sig, 0):
             form, w = self._scaled_w, self.w_element
-            if form is not None and form.key == (w.data_ptr(), w._version) and (form.event is None or form.ready()):
+            if form is not None and form.key == (w.data_ptr(), w._version) and (form.stream is None or form.ready()):
                 from ..mxfp import kernels
 
                 xm = self.x_minifloat_meta
@@ -220,7 +220,14 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
-            xm, bias, x2 = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
+            xm, bias = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias
+            if dense:
+                y = _lib.host().linear_packed_dense(input, w.codes, w.scales, w.exp_bits, w.frac_bits, self.out_features, bias)
+            else:
+                y = _lib.host().linear_packed(input, xm.exp_bits, xm.frac_bits, 1, w.codes, w.scales, w.exp_bits, w.frac_bits, self.out_features, bias)
+            if y is not None:
+                return y
+            x2 = input.reshape(-1, self.in_features)
             if dense:
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:
@@ -229,7 +236,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
         notes["_note"] = None if w_operand is None else (sig, 0)
-        narrowed = self._narrowed_weight()
+        narrowed = self._narrowed_weight() if w_operand is None else None       # (with an operand nothing reads the codes themselves)
         y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,

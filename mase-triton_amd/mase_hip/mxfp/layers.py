@@ -205,7 +205,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                     if y is not None:
                         return y
             elif (form is not None and w_elements is not None and w_scales is not None
-                  and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version) and (form.event is None or form.ready())):
+                  and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version) and (form.stream is None or form.ready())):
                 meta, w = self.x_mxfp_meta, form.value
                 bias = None if self.layer_type.endswith("Bq") else self.bias
                 if packed == 2:
@@ -228,7 +228,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         if note == (sig, 0):
             form, w_elements, w_scales = self._scaled_w, self.w_elements, self.w_scales
             if (form is not None and form.key == (w_elements.data_ptr(), w_elements._version, w_scales.data_ptr(), w_scales._version)
-                    and (form.event is None or form.ready())):
+                    and (form.stream is None or form.ready())):
                 from . import kernels
 
                 x2 = input.reshape(-1, self.in_features)
@@ -250,7 +250,14 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w, dense = packed[0].value, packed[1]
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
-            meta, bias, x2 = self.x_mxfp_meta, None if self.layer_type.endswith("Bq") else self.bias, input.reshape(-1, self.in_features)
+            meta, bias = self.x_mxfp_meta, None if self.layer_type.endswith("Bq") else self.bias
+            if dense:
+                y = _lib.host().linear_packed_dense(input, w.codes, w.scales, w.exp_bits, w.frac_bits, self.out_features, bias)
+            else:
+                y = _lib.host().linear_packed(input, meta.element_exp_bits, meta.element_frac_bits, 0, w.codes, w.scales, w.exp_bits, w.frac_bits, self.out_features, bias)
+            if y is not None:
+                return y
+            x2 = input.reshape(-1, self.in_features)
             if dense:
                 y = kernels.mxfp_gemm_packed_dense(x2, w, bias)
             else:

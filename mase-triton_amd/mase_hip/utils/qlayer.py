@@ -25,7 +25,10 @@ def devices_equal(device1, device2) -> bool:
 
 
 def weight_key(components) -> tuple:
-    return tuple(v for c in components for v in (c.data_ptr(), c._version))
+    key = ()
+    for c in components:
+        key += (c.data_ptr(), c._version)
+    return key
 
 
 def capturing(device: torch.device) -> bool:
@@ -36,38 +39,56 @@ def capturing(device: torch.device) -> bool:
         return torch.cuda.is_current_stream_capturing()
 
 
-def launched(device: torch.device):
-    """An event behind what the current stream of ``device`` has been given (None: nothing runs behind the host)."""
-    if device.type != "cuda":
-        return None
-    with _lib.on_device(device):
-        return torch.cuda.current_stream(device).record_event()
+def stream_captured(stream) -> bool:
+    with torch.cuda.stream(stream):
+        return torch.cuda.is_current_stream_capturing()
+
+
+def current_stream(device: torch.device):
+    """What names the stream that a form built now is written on (None: nothing runs behind the host)."""
+    return torch._C._cuda_getCurrentStream(device.index) if device.type == "cuda" else None
+
+
+def as_stream(name) -> "torch.cuda.Stream":
+    stream_id, device_index, device_type = name
+    return torch.cuda.Stream(stream_id=stream_id, device_index=device_index, device_type=device_type)
 
 
 class WeightForm:
     """A quantised weight in another form than its stored components.
 
     ``key`` names the components that it was built from, by address and version.  An address names a tensor only until its memory is handed out
-    again, so the form holds an alias of each: whatever replaces a component while the form is kept lies elsewhere.  ``event`` is behind the kernels
-    that write the form, None once they are known to have run."""
+    again, so the form holds the memory of each: whatever replaces a component while the form is kept lies elsewhere.  ``stream`` names the one that the
+    kernels which write the form were launched on, None once they are known to have run; ``event`` is behind them, once one was asked for."""
 
-    __slots__ = ("value", "key", "components", "event")
+    __slots__ = ("value", "key", "memory", "device", "stream", "event")
 
-    def __init__(self, value, key: tuple, components: tuple, event):
-        self.value, self.key, self.components, self.event = value, key, components, event
+    def __init__(self, value, key: tuple, components, stream):
+        self.value, self.key, self.memory, self.device = value, key, [c.untyped_storage() for c in components], components[0].device
+        self.stream, self.event = stream, None
 
     def ready(self) -> bool:
-        """Put the current stream behind what writes the form; False where that cannot be (the stream is captured and the form not written yet)."""
-        event, device = self.event, self.components[0].device
-        if event is None:
+        """Put the current stream behind what writes the form; False where that cannot be: one of the two is captured and the form not known to be written.
+
+        The building call records no event (it costs the host 6 us, and the next kernel waits behind it: the first call of a SwiGLU block of two layers, 6 x
+        1024 x 4096, took 139 us without and 159 with); the first call behind it does, on the form's stream, whichever its own is."""
+        stream, device = self.stream, self.device
+        if stream is None:
             return True
-        if _lib.event_done(event):
-            self.event = None
+        stream = as_stream(stream)
+        event, own, captured = self.event, _lib.stream_ptr(device) == stream.cuda_stream, capturing(device)
+        if (event is not None or captured) and _lib.stream_done(stream, event):
+            self.stream = None
             return True
-        if capturing(device):
+        if event is None and not captured:
+            if not own and stream_captured(stream):
+                return False
+            event = self.event = stream.record_event()
+        if captured:
             return False
-        with _lib.on_device(device):
-            torch.cuda.current_stream(device).wait_event(event)
+        if not own:
+            with _lib.on_device(device):
+                torch.cuda.current_stream(device).wait_event(event)
         return True
 
 
@@ -79,8 +100,8 @@ class KeepsWeightForms:
     (``_FORM_COMPONENTS``).  Forms are built on the first call that reads them and again after a change of the components, and are part of
     neither ``state_dict`` nor a copy or pickle of the layer.
 
-    A form is built on the stream of one call and read by calls on any stream and of any thread, which wait for its event until it has been seen to have
-    run: ``ready``, asked as long as there is an event.  (The building call could wait for its stream instead: a new layer's first call 63 -> 93 us.)
+    A form is built on the stream of one call and read by calls on any stream and of any thread, which go behind what writes it until that is known to
+    have run (``WeightForm.ready``).  (The building call could wait for its stream instead: a new layer's first call 63 -> 93 us.)
 
     A captured call reads the forms that were kept then, where they lie.  So components that are written in place are built into the same memory again,
     by the next call or by ``load_state_dict`` itself, and replays follow; a graph is captured again after the components were replaced or moved or
@@ -107,26 +128,33 @@ class KeepsWeightForms:
     def _weight_form(self, name: str, needed: bool = True) -> WeightForm | None:
         """The form ``name`` of the weight as it is now, for the current stream.  One that is built while the stream is captured belongs to that graph, which
         writes it on every replay; with ``needed`` false, for a call that has another way, None in its place."""
-        components = tuple(getattr(self, c) for c in self._FORM_COMPONENTS)
+        held = self._parameters
+        components = [held[c] if held.get(c) is not None else getattr(self, c) for c in self._FORM_COMPONENTS]
         kept, key, device = getattr(self, name), weight_key(components), components[0].device
         if kept is not None and kept.key == key and kept.ready():
             return kept
         in_graph = capturing(device)
         if in_graph and not needed:
             return None
-        written = kept is not None and kept.key[::2] == key[::2] and not in_graph       # the same tensors, written since
-        if written:
-            kept.ready()
-        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, tuple(c.detach() for c in components),
-                          None if in_graph else launched(device))
-        if in_graph or any(isinstance(getattr(type(self), c, None), property) for c in self._FORM_COMPONENTS):
-            return form                                       # (a parametrisation makes another tensor for every call)
+        same = kept is not None and kept.key == key                                     # (... which this stream cannot be put behind)
+        written = not same and kept is not None and kept.key[::2] == key[::2] and not in_graph and kept.ready()       # the same tensors, written since
+        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, components, None if in_graph else current_stream(device))
+        if in_graph or same or self._computed_components():
+            return form
         if kept is not None and not written and device.type == "cuda":
             torch.cuda.synchronize(device)                    # (calls on other streams may still read the one that goes)
         with _publish:
             if getattr(self, name) is kept:                   # (else another thread's call was faster)
                 self.__dict__[name] = form
         return form
+
+    def _computed_components(self) -> bool:
+        """Does a parametrisation make the components anew for every call?"""
+        cls = type(self)
+        for c in self._FORM_COMPONENTS:
+            if isinstance(getattr(cls, c, None), property):
+                return True
+        return False
 
     def _drop_forms(self, moved_only: bool = False) -> None:
         """Forget the forms, or those whose components are not the layer's any more."""

@@ -135,7 +135,7 @@ def test_replays_follow_a_weight_that_is_loaded_in_place(family, layer_type, row
 
 
 def test_one_call_before_the_capture_is_enough():
-    """The capture finds a form whose event nobody has asked about since: the query does not end the capture, and the form is read, not built again."""
+    """The capture finds a form that no other call has asked about since: the query does not end the capture, and the form is read, not built again."""
     import mase_hip.mxfp.meta as mx
     from mase_hip import _lib
     from mase_hip.mxfp.layers import MXFPLinearPTQ
@@ -147,19 +147,24 @@ def test_one_call_before_the_capture_is_enough():
     want = layer(x)
     torch.cuda.synchronize()
     form, graph = layer._packed_w, torch.cuda.CUDAGraph()
-    assert form.event is not None
+    assert form.stream is not None
     with torch.cuda.graph(graph):
         y = layer(x)
-    assert layer._packed_w is form and form.event is None
+    assert layer._packed_w is form and form.stream is None
     side, busy = torch.cuda.Stream(), torch.randn(4096, 4096, device=DEV)
     torch.cuda.synchronize()
     with torch.cuda.stream(side):                  # an event that is still to come
         for _ in range(20):
             torch.mm(busy, busy)
         event = side.record_event()
-    early = _lib.event_done(event)
+    early = _lib.stream_done(side, event), _lib.stream_done(side)
     side.synchronize()
-    assert not early and _lib.event_done(event)
+    assert early == (False, False) and _lib.stream_done(side, event) and _lib.stream_done(side)
+    again = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(again, stream=side):     # a stream that is captured has not run what it was given
+        x.add_(0)
+        assert not _lib.stream_done(side) and not _lib.stream_done(side, event) and _lib.stream_done(torch.cuda.default_stream())
+    again.replay()
     for _ in range(3):
         y.zero_()
         graph.replay()

@@ -102,44 +102,95 @@ def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
     assert both_forms(layer) == kept == (layer._scaled_w, layer._packed_w)
 
 
+class Stream:
+    """A stand-in for a stream on a GPU: the events recorded on it, and those that it waits for."""
+
+    def __init__(self, number):
+        self.cuda_stream, self.recorded, self.waits, self.done, self.captured = number, [], [], False, False
+
+    def record_event(self):
+        self.recorded.append(Event())
+        return self.recorded[-1]
+
+    def wait_event(self, event):
+        self.waits.append(event)
+
+
 class Event:
-    """A stand-in for an event on a GPU."""
-
-    cuda_event, done = 0, False
+    done = False
 
 
-def test_calls_wait_for_a_form_until_it_is_written(layer, monkeypatch):
-    """On whichever stream: each goes behind the event of the call that built the form, until one finds that it has run; none does under capture."""
-    event, waits, products = Event(), [], []
+def test_calls_go_behind_what_writes_a_form(layer, monkeypatch):
+    """Calls on the stream that the form is written on have the order; of others each waits for an event of that stream, until one is found to have run."""
+    a, b, products = Stream(1), Stream(2), []
+    at = [a]
     monkeypatch.setattr(_lib, "dense", lambda t: t)
-    monkeypatch.setattr(_lib, "event_done", lambda e: e.done)
-    monkeypatch.setattr(qlayer, "launched", lambda device: event)
-    monkeypatch.setattr(qlayer.torch.cuda, "current_stream", lambda device: type("Stream", (), {"wait_event": lambda self, e: waits.append(e)})())
-    monkeypatch.setattr(kernels, "linear_packed", lambda *a: (products.append("wrappers"), torch.zeros(4, N))[1])
+    monkeypatch.setattr(_lib, "stream_ptr", lambda device: at[0].cuda_stream)
+    monkeypatch.setattr(_lib, "stream_done", lambda stream, event=None: (stream if event is None else event).done and not stream.captured)
+    monkeypatch.setattr(qlayer, "current_stream", lambda device: at[0])
+    monkeypatch.setattr(qlayer, "as_stream", lambda name: name)
+    monkeypatch.setattr(qlayer, "capturing", lambda device: at[0].captured)
+    monkeypatch.setattr(qlayer, "stream_captured", lambda stream: stream.captured)
+    monkeypatch.setattr(qlayer.torch.cuda, "current_stream", lambda device: at[0])
+    monkeypatch.setattr(kernels, "linear_packed", lambda *args: (products.append("wrappers"), torch.zeros(4, N))[1])
 
     class Host:
-        linear_packed = staticmethod(lambda *a: products.append("extension") or torch.zeros(4, N))
+        linear_packed = staticmethod(lambda *args: products.append("extension") or (torch.zeros(4, N) if takes else None))
 
+    def build(written=False):
+        layer._drop_forms()
+        layer(OnGpu())
+        if written:
+            a.done = True
+        return layer._packed_w
+
+    takes = False
     monkeypatch.setattr(_lib, "_host", Host)
-    layer(OnGpu())
-    form = layer._packed_w
-    assert form.event is event and waits == [] and products == ["wrappers"]           # (the building call's own stream has the order)
+    form = build()
+    assert form.stream is a and not a.recorded and products == ["extension", "wrappers"]
+    takes = True
+    # another stream first: the event is recorded there and then, on the form's stream
+    at[0] = b
     layer(OnGpu())
     layer._forward(OnGpu(), ())
-    assert waits == [event] * 2 and products == ["wrappers", "extension", "wrappers"]
-    monkeypatch.setattr(qlayer, "capturing", lambda device: True)
-    assert layer._packed_weight(OnGpu(), True) is None and layer._packed_w is form and len(waits) == 2
-    event.done = True
-    assert layer._packed_weight(OnGpu(), True)[0] is form and form.event is None
-    monkeypatch.setattr(qlayer, "capturing", lambda device: False)
+    assert len(a.recorded) == 1 and b.waits == a.recorded * 2 and not b.recorded and products[2:] == ["extension"] * 2
+    at[0] = a
     layer(OnGpu())
-    assert len(waits) == 2
-    # written in place: behind what wrote it before
-    form.event, event.done = event, False
+    assert not a.waits and form.stream is a
+    a.recorded[0].done = True
+    at[0] = b
+    layer(OnGpu())
+    assert form.stream is None and len(b.waits) == 2 and len(a.recorded) == 1
+    # its own stream first
+    at[0] = a
+    form = build()
+    layer(OnGpu())
+    assert form.event is a.recorded[1] and not a.waits
+    # captured calls: one on another stream asks the form's stream or its event, one on the form's own only the event
+    b.captured, at[0] = True, b
+    assert layer._packed_weight(OnGpu(), True) is None and len(b.waits) == 2
+    a.recorded[1].done = True
+    assert layer._packed_weight(OnGpu(), True)[0] is form and form.stream is None
+    at[0] = a
+    form = build()
+    at[0] = b
+    assert layer._packed_weight(OnGpu(), True) is None and layer._packed_w is form
+    a.done = True
+    assert layer._packed_weight(OnGpu(), True)[0] is form and form.stream is None and len(a.recorded) == 2
+    at[0], a.done = a, False
+    form = build(written=True)
+    a.captured = True
+    assert layer._packed_weight(OnGpu(), True) is None
+    # an eager call while the form's stream is captured by another thread: a form of its own
+    b.captured, at[0] = False, b
+    other = layer._packed_weight(OnGpu(), True)[0]
+    assert other is not form and layer._packed_w is form and other.value.memory is not form.value.memory and len(a.recorded) == 2
+    # written in place: in the same memory, behind what wrote it before
+    a.captured = False
     with torch.no_grad():
         layer.w_elements.add_(1)
     layer._forward(OnGpu(), ())
-    assert len(waits) == 3 and layer._packed_w is not form and layer._packed_w.value.memory is form.value.memory
+    assert b.waits[-1] is a.recorded[2] and layer._packed_w is not form and layer._packed_w.value.memory is form.value.memory and layer._packed_w.stream is b
 
 
 def test_of_two_threads_that_build_a_form_one_keeps_its_own(layer, monkeypatch):
