@@ -41,3 +41,8 @@ extern "C" int mase_bench_strided_pair_tiles(int64_t inner, int64_t columns, int
 extern "C" int mase_bench_short_k(int64_t M, int64_t N, int64_t K, int64_t batches) {
     return mase::short_k_shape_ok((int)M, (int)N, (int)K, (int)batches) ? 1 : 0;
 }
+
+// do products that no kernel of whole macro steps takes go to the tiles of any shape?  (else to the 256 x 256 kernel)
+extern "C" int mase_bench_any_shape(int64_t M, int64_t N, int64_t K, int64_t batches, int cus) {
+    return mase::any_pays(mase::plan_any((int)M, (int)N, (int)K, (int)batches, cus, 1), (int)M, (int)N, (int)K, (int)batches, cus) ? 1 : 0;
+}

@@ -191,3 +191,13 @@ def test_few_rows_stay_with_the_weight_streaming_kernel_where_it_is_ahead(lib):
         assert scaled_plan(lib, *shape)[0] == 0, shape
     for shape in ((1, 12288, 1024), (16, 14336, 768), (17, 65536, 512), (32, 8192, 1536), (33, 8192, 2048), (64, 8192, 2048), (48, 4096, 14336), (64, 14336, 4096)):
         assert scaled_plan(lib, *shape)[0] == 64, shape
+
+
+def test_large_products_of_any_shape_stay_on_the_large_tiles(lib):
+    """(batches, rows, columns, k) on both sides of the line; the first is the batch of odd products of the GPU tests."""
+    rule = lib.mase_bench_any_shape
+    rule.argtypes = [ctypes.c_int64] * 4 + [ctypes.c_int]
+    for b, M, N, K in ((2, 4033, 2005, 2368), (1, 2759, 2961, 3648), (1, 16384, 14330, 4096)):
+        assert not rule(M, N, K, b, 256), (b, M, N, K)
+    for b, M, N, K in ((2, 1001, 1003, 2368), (1, 4033, 2005, 160), (40, 257, 259, 96), (1, 700, 1000, 4096)):
+        assert rule(M, N, K, b, 256), (b, M, N, K)

@@ -59,6 +59,23 @@ def test_any_shape(MNK, name):
         assert bool((y[:shift] == 7.0).all()) and bool((y[shift + M * N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("odt", [torch.bfloat16, torch.float16])
+def test_batch_of_large_odd_products(odt):
+    """On the 256 x 256 kernel (test_dispatch_rules.py): the second product's outputs start on an odd multiple of two bytes."""
+    B, M, N, K = 2, 4033, 2005, 2368
+    meta = mx_meta.MXFP8_E4M3_fn
+    g = torch.Generator(device=DEV).manual_seed(9)
+    a = torch.randn(B, M, K, generator=g, device=DEV).to(torch.bfloat16)
+    sc, el, tm = extract_mxfp_components((0.02 * torch.randn(B * N, K, generator=g, device=DEV)).to(torch.bfloat16), block_dim=1, mxfp_meta=meta)
+    w = compose_mxfp_tensor(sc, el, tm).view(B, N, K)
+    y = torch.full((B * M * N + 64,), 7.0, dtype=odt, device=DEV)
+    _lib.check(_lib.load().mase_hip_mxfp_matmul_batched(a.data_ptr(), sc.data_ptr(), el.data_ptr(), meta.element_exp_bits, meta.element_frac_bits, y.data_ptr() + 32,
+                                                        {torch.float16: 1, torch.bfloat16: 2}[odt], M, N, K, B, _lib.stream_ptr(y.device)))
+    for b in range(B):
+        _check(y[16 + b * M * N:16 + (b + 1) * M * N].view(M, N), a[b], w[b], None, odt)
+    assert bool((y[:16] == 7.0).all()) and bool((y[16 + B * M * N:] == 7.0).all())
+
+
 @pytest.mark.parametrize("shape", [(3, 1, 64, 160), (5, 33, 65, 224), (2, 64, 128, 416), (2, 65, 1, 96), (3, 130, 64, 352), (40, 200, 127, 160), (70, 257, 128, 256)])
 @pytest.mark.parametrize("name", FORMATS)
 def test_product_that_quantises(shape, name):

@@ -29,7 +29,8 @@ def _without_extension(monkeypatch, name):
     ("XqWqB", "bfloat16", "E5M2", "E4M3", (2, 1024), 996, True), ("XqWqB", "bfloat16", "E4M3", "E5M2", (3, 50, 4096), 4096, True),
     ("XqWqB", "float32", "E4M3", "E3M2", (29, 1408), 768, False), ("XqWqB", "float32", "E2M3", "E2M1", (600, 512), 256, True),
     ("XWqB", "bfloat16", None, "E4M3", (5, 7, 544), 72, True), ("XWqB", "bfloat16", None, "E5M2", (70, 2048), 1000, False),
-    ("XqWqBq", "bfloat16", "E5M2", "E5M2", (9, 96), 40, True)])
+    ("XqWqBq", "bfloat16", "E5M2", "E5M2", (9, 96), 40, True),
+    ("XqWqBq", "bfloat16", "E5M2", "E4M3", (9, 96), 64, True)])      # (the MXFP layer has its quantised bias as well: whole blocks of 32)
 def test_layers_on_the_components(monkeypatch, kind, layer_type, dtype, x_fmt, w_fmt, shape, N, bias):
     import mase_hip.minifloat.layers as ML
     import mase_hip.minifloat.meta as mf
@@ -51,6 +52,7 @@ def test_layers_on_the_components(monkeypatch, kind, layer_type, dtype, x_fmt, w
         F = {"E4M3": mf.FP8_E4M3_fn, "E5M2": mf.FP8_E5M2_fn, "E2M3": mf.FP6_E2M3_fn, "E3M2": mf.FP6_E3M2_fn, "E2M1": mf.FP4_E2M1_fn, None: None}
         layer = ML.MinifloatLinearPTQ(weight=w, bias=b, x_minifloat_meta=F[x_fmt], w_minifloat_meta=F[w_fmt],
                                       b_minifloat_meta=mf.FP8_E4M3_fn if layer_type.endswith("Bq") else None, layer_type=layer_type, backend="fused")
+    assert not layer_type.endswith("Bq") or kind == "minifloat" or (layer.b_elements is not None) == (N % 32 == 0)
     first, repeated = layer(x), layer(x)
     assert layer._fast_packed == 3 and first.dtype == dt
     moved = layer(x.transpose(0, 1).contiguous().transpose(0, 1)) if x.dim() > 2 else first       # rows that are not contiguous
