@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm, capturing
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, capturing
 from . import functional as MinifloatF
 from .meta import MinifloatMeta, MinifloatTensorMeta
 
@@ -106,14 +106,14 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             self.b_tensor_meta = self.b_tensor_meta.create(device=self.b_element.device)
         return result
 
-    def _narrowed_weight(self) -> WeightForm | None:
+    def _narrowed_weight(self):
         """One-byte copy of the weight codes for the fused GEMM (not part of ``state_dict``),
         rebuilt when ``w_element`` is replaced, written in place or moved."""
         w = self.w_element
         if (self.backend == "separate" or w is None or w.device.type != "cuda"
                 or not MinifloatF.gemm_weight_eligible(self.w_tensor_meta)):
             return None
-        return self._weight_form("_narrowed")
+        return self._weight_form("_narrowed").value
 
     def _build_form(self, name: str, into, w_element: Tensor):
         from ..mxfp import kernels
@@ -124,10 +124,10 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             return MinifloatF.narrow_weight_codes(w_element, tm, into)
         narrowed = self._narrowed_weight()
         if name == "_scaled_w":
-            return L.scaled_weight_operand(w_element, tm, None if narrowed is None else narrowed.value, into)
-        return kernels.packed_weight_from_mxfp(*narrowed.value, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features, into)
+            return L.scaled_weight_operand(w_element, tm, narrowed, into)
+        return kernels.packed_weight_from_mxfp(*narrowed, tm.meta.exp_bits, tm.meta.frac_bits, self.out_features, self.in_features, into)
 
-    def _weight_operand(self, input: Tensor) -> WeightForm | None:
+    def _weight_operand(self, input: Tensor):
         """The weight in the block-scaled GEMM's form when this call takes that GEMM (quantised bfloat16 activations, see
         ``minifloat_linear``), else None.  Not part of ``state_dict``; rebuilt like the one-byte copy."""
         from ..mxfp.functional.linear import takes_scaled_route
@@ -141,9 +141,9 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         if not ((self.backend == "fused_scaled" or takes_scaled_route(rows, True))
                 and L._scaled_eligible(input, self.x_minifloat_meta, self.w_tensor_meta, bias)):
             return None
-        return self._weight_form("_scaled_w")
+        return self._weight_form("_scaled_w").value
 
-    def _packed_weight(self, input: Tensor) -> tuple[WeightForm, bool] | None:
+    def _packed_weight(self, input: Tensor):
         """The weight packed at its own width when that is the fastest form for this call, and whether the activations are dense (``MXFPLinearPTQ``);
         else None."""
         from ..mxfp import kernels
@@ -162,7 +162,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
                   and L._scaled_eligible(input, self.x_minifloat_meta, tm, bias)):
             return None
         form = self._weight_form("_packed_w", needed=False)
-        return None if form is None else (form, dense)
+        return None if form is None else (form.value, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_minifloat_meta)
@@ -217,7 +217,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         if packed is not None:
             from ..mxfp import kernels
 
-            w, dense = packed[0].value, packed[1]
+            w, dense = packed
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
             xm, bias = self.x_minifloat_meta, None if self.layer_type.endswith("Bq") else self.bias
@@ -241,7 +241,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
-            _narrowed=None if narrowed is None else narrowed.value, _w_operand=None if w_operand is None else w_operand.value)
+            _narrowed=narrowed, _w_operand=w_operand)
         if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
         elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)

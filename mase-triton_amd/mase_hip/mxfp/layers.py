@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, WeightForm, capturing
+from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, capturing
 from . import functional as MXFP_F
 from .meta import MXFPMeta, MXFPTensorMeta
 
@@ -143,7 +143,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         return ((self.backend == "fused_scaled" or L.takes_scaled_route(rows, True))
                 and L._scaled_eligible(input, self.x_mxfp_meta, self.w_tensor_meta, bias))
 
-    def _weight_operand(self, input: Tensor) -> WeightForm | None:
+    def _weight_operand(self, input: Tensor):
         """The weight in the block-scaled GEMM's form when this call has a kernel that reads it (the block-scaled GEMM for
         quantised bfloat16 activations, the large-tile bf16 kernel from 512 rows on), else None."""
         from . import kernels
@@ -160,9 +160,10 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                     and kernels.prepared_w_pays(rows, tm.shape[0], tm.shape[1]))
             if not bf16:
                 return None
-        return self._weight_form("_scaled_w", needed=scaled)
+        form = self._weight_form("_scaled_w", needed=scaled)
+        return None if form is None else form.value
 
-    def _packed_weight(self, input: Tensor, scaled: bool = False) -> tuple[WeightForm, bool] | None:
+    def _packed_weight(self, input: Tensor, scaled: bool = False):
         """The weight packed at its own width when that is the fastest form for this call, and whether the call is one of dense activations
         (weight-only layers) or of quantised ones; else None.  ``scaled``: the caller knows that the call takes the block-scaled route."""
         from . import kernels
@@ -184,7 +185,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                   and (scaled or self._takes_scaled_route(input))):
             return None
         form = self._weight_form("_packed_w", needed=False)
-        return None if form is None else (form, dense)
+        return None if form is None else (form.value, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta)
@@ -247,7 +248,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         if packed is not None:
             from . import kernels
 
-            w, dense = packed[0].value, packed[1]
+            w, dense = packed
             assert input.shape[-1] == self.in_features
             notes["_no_operand_sig"], notes["_note"] = None, (sig, 2 if dense else 1)
             meta, bias = self.x_mxfp_meta, None if self.layer_type.endswith("Bq") else self.bias
@@ -270,7 +271,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             x=input, x_meta=self.x_mxfp_meta, w=self.weight, w_scales=self.w_scales, w_elements=self.w_elements,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_scales=self.b_scales, b_elements=self.b_elements,
             b_tensor_meta=self.b_tensor_meta, layer_type=self.layer_type, backend=self.backend,
-            w_operand=None if w_operand is None else w_operand.value)
+            w_operand=w_operand)
         if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
         elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
@@ -295,11 +296,10 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         if (gate.shape == up.shape and gate.dtype == up.dtype and gate.device == up.device and gate.shape[-1] == self.in_features
                 and self.layer_type == "XqWqB" and self._takes_scaled_route(gate)):
             packed = self._packed_weight(gate, True)
-            form = self._weight_form("_scaled_w") if packed is None else packed[0]
+            w_op = self._weight_form("_scaled_w").value if packed is None else packed[0]
             a_op = kernels.scaled_operand_from_swiglu(gate.reshape(-1, self.in_features) if gate.ndim != 2 else gate,
                                                       up.reshape(-1, self.in_features) if up.ndim != 2 else up, self.x_mxfp_meta)
-            y = (kernels.mxfp_gemm_scaled(a_op, form.value, self.bias, gate.dtype) if packed is None
-                 else kernels.mxfp_gemm_packed(a_op, form.value, self.bias))
+            y = kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype) if packed is None else kernels.mxfp_gemm_packed(a_op, w_op, self.bias)
             return y.view(*gate.shape[:-1], self.out_features)
         return self.forward(torch.nn.functional.silu(gate) * up)
 

@@ -55,7 +55,7 @@ class OnGpu:
 
 
 def both_forms(layer):
-    return layer._weight_form("_scaled_w"), layer._packed_weight(OnGpu(), True)[0]
+    return layer._weight_form("_scaled_w"), layer._weight_form("_packed_w")
 
 
 def test_forms_go_with_the_components_that_move(layer):
@@ -170,13 +170,13 @@ def test_calls_go_behind_what_writes_a_form(layer, monkeypatch):
     b.captured, at[0] = True, b
     assert layer._packed_weight(OnGpu(), True) is None and len(b.waits) == 2
     a.recorded[1].done = True
-    assert layer._packed_weight(OnGpu(), True)[0] is form and form.stream is None
+    assert layer._packed_weight(OnGpu(), True)[0] is form.value and layer._packed_w is form and form.stream is None
     at[0] = a
     form = build()
     at[0] = b
     assert layer._packed_weight(OnGpu(), True) is None and layer._packed_w is form
     a.done = True
-    assert layer._packed_weight(OnGpu(), True)[0] is form and form.stream is None and len(a.recorded) == 2
+    assert layer._packed_weight(OnGpu(), True)[0] is form.value and layer._packed_w is form and form.stream is None and len(a.recorded) == 2
     at[0], a.done = a, False
     form = build(written=True)
     a.captured = True
@@ -184,7 +184,7 @@ def test_calls_go_behind_what_writes_a_form(layer, monkeypatch):
     # an eager call while the form's stream is captured by another thread: a form of its own
     b.captured, at[0] = False, b
     other = layer._packed_weight(OnGpu(), True)[0]
-    assert other is not form and layer._packed_w is form and other.value.memory is not form.value.memory and len(a.recorded) == 2
+    assert layer._packed_w is form and other.memory is not form.value.memory and len(a.recorded) == 2
     # written in place: in the same memory, behind what wrote it before
     a.captured = False
     with torch.no_grad():
