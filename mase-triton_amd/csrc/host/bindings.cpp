@@ -244,6 +244,26 @@ PyObject* minifloat(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// what the linears have in common beside x and W: the bias (a vector of N, or None), the stream, the shape of the outputs
+struct LinearRest {
+    const void* bias = nullptr;
+    int bias_dtype = 0;
+    void* stream = nullptr;
+    Sizes shape;
+};
+bool linear_rest(const at::Tensor& x, int64_t N, PyObject* bias, LinearRest& r) {
+    if (bias != Py_None) {
+        const at::Tensor* const b = THPVariable_Check(bias) ? &THPVariable_Unpack(bias) : nullptr;
+        if (!b || !b->is_cuda() || b->device() != x.device() || !b->unsafeGetTensorImpl()->has_storage() || !b->is_contiguous() || b->numel() != N) return false;
+        r.bias_dtype = dtype_code(b->scalar_type());
+        if (r.bias_dtype < 0) return false;
+        r.bias = b->data_ptr();
+    }
+    r.shape = sizes_of(x);
+    r.shape.back() = N;
+    return stream_of(x, &r.stream);
+}
+
 // linear_scaled(x [.., K] bf16, exp_bits, frac_bits, minifloat, w_codes, w_scales, N, bias or None) -> [.., N]
 PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     HANDLE_TH_ERRORS
@@ -255,19 +275,8 @@ PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     PLAIN(whole(a[1], e) && whole(a[2], m) && whole(a[3], mini) && whole(a[6], N));
     const int64_t K = x->size(-1), M = K > 0 ? x->numel() / K : 0;
     PLAIN(M > 0 && N > 0 && codes->size(1) == K && codes->size(0) >= N && w_sc->numel() >= K / 128 * codes->size(0));
-    const void* b_ptr = nullptr;
-    int b_dt = 0;
-    if (a[7] != Py_None) {
-        const at::Tensor* const b = THPVariable_Check(a[7]) ? &THPVariable_Unpack(a[7]) : nullptr;
-        PLAIN(b && b->is_cuda() && b->device() == x->device() && b->unsafeGetTensorImpl()->has_storage() && b->is_contiguous() && b->numel() == N);
-        b_dt = dtype_code(b->scalar_type());
-        PLAIN(b_dt >= 0);
-        b_ptr = b->data_ptr();
-    }
-    void* stream;
-    PLAIN(stream_of(*x, &stream));
-    Sizes shape = sizes_of(*x);
-    shape.back() = N;
+    LinearRest r;
+    PLAIN(linear_rest(*x, N, a[7], r));
     const void* const data = x->data_ptr();
     const uint8_t* const code_data = codes->data_ptr<uint8_t>();
     const uint32_t* const scale_data = reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>());
@@ -277,12 +286,12 @@ PyObject* linear_scaled(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     {
         const WithoutGil released;
         if (mase_hip_mxfp_linear_few_plan(M, N, K)) {
-            y = empty(shape, at::kBFloat16, device);
-            rc = mase_hip_mxfp_linear_few(data, (int)e, (int)m, (int)mini, code_data, scale_data, b_ptr, b_dt, y.data_ptr(), M, N, K, stream);
+            y = empty(r.shape, at::kBFloat16, device);
+            rc = mase_hip_mxfp_linear_few(data, (int)e, (int)m, (int)mini, code_data, scale_data, r.bias, r.bias_dtype, y.data_ptr(), M, N, K, r.stream);
         } else if (const int64_t bytes = mase_hip_mxfp_linear_scaled_scratch_bytes(M, N, K); bytes > 0) {
             scratch = empty({bytes}, at::kByte, device);
-            y = empty(shape, at::kBFloat16, device);
-            rc = mase_hip_mxfp_linear_scaled(data, 2, (int)e, (int)m, (int)mini, code_data, scale_data, b_ptr, b_dt, y.data_ptr(), 2, M, N, K, scratch.data_ptr(), bytes, stream);
+            y = empty(r.shape, at::kBFloat16, device);
+            rc = mase_hip_mxfp_linear_scaled(data, 2, (int)e, (int)m, (int)mini, code_data, scale_data, r.bias, r.bias_dtype, y.data_ptr(), 2, M, N, K, scratch.data_ptr(), bytes, r.stream);
         }
     }
     PLAIN(rc == 0);
@@ -303,19 +312,8 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     PLAIN(M > 0 && N > 0 && K < (1 << 27));
     const int64_t code_bytes = mase_hip_packed_weight_bytes(N, K, (int)we, (int)wm);
     PLAIN(code_bytes > 0 && codes->numel() == code_bytes && w_sc->numel() == K / 128 * ((N + 255) / 256 * 256));
-    const void* b_ptr = nullptr;
-    int b_dt = 0;
-    if (a[9] != Py_None) {
-        const at::Tensor* const b = THPVariable_Check(a[9]) ? &THPVariable_Unpack(a[9]) : nullptr;
-        PLAIN(b && b->is_cuda() && b->device() == x->device() && b->unsafeGetTensorImpl()->has_storage() && b->is_contiguous() && b->numel() == N);
-        b_dt = dtype_code(b->scalar_type());
-        PLAIN(b_dt >= 0);
-        b_ptr = b->data_ptr();
-    }
-    void* stream;
-    PLAIN(stream_of(*x, &stream));
-    Sizes shape = sizes_of(*x);
-    shape.back() = N;
+    LinearRest r;
+    PLAIN(linear_rest(*x, N, a[9], r));
     const void* const data = x->data_ptr();
     const uint8_t* const code_data = codes->data_ptr<uint8_t>();
     const uint32_t* const scale_data = reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>());
@@ -326,9 +324,9 @@ PyObject* linear_packed(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         const WithoutGil released;
         const int64_t bytes = mase_hip_mxfp_linear_packed_scratch_bytes(M, N, K, (int)we, (int)wm);
         if (bytes > 0) scratch = empty({bytes}, at::kByte, device);
-        y = empty(shape, at::kBFloat16, device);
-        rc = mase_hip_mxfp_linear_packed(data, (int)e, (int)m, (int)mini, code_data, scale_data, (int)we, (int)wm, b_ptr, b_dt, y.data_ptr(), M, N, K,
-                                         bytes > 0 ? scratch.data_ptr() : nullptr, bytes, stream);
+        y = empty(r.shape, at::kBFloat16, device);
+        rc = mase_hip_mxfp_linear_packed(data, (int)e, (int)m, (int)mini, code_data, scale_data, (int)we, (int)wm, r.bias, r.bias_dtype, y.data_ptr(), M, N, K,
+                                         bytes > 0 ? scratch.data_ptr() : nullptr, bytes, r.stream);
     }
     PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(y));
@@ -348,19 +346,8 @@ PyObject* linear_packed_dense(PyObject*, PyObject* const* a, Py_ssize_t n_args) 
     PLAIN(M > 0 && N > 0 && K < (1 << 27));
     const int64_t code_bytes = mase_hip_packed_weight_bytes(N, K, (int)we, (int)wm);
     PLAIN(code_bytes > 0 && codes->numel() == code_bytes && w_sc->numel() == K / 128 * ((N + 255) / 256 * 256));
-    const void* b_ptr = nullptr;
-    int b_dt = 0;
-    if (a[6] != Py_None) {
-        const at::Tensor* const b = THPVariable_Check(a[6]) ? &THPVariable_Unpack(a[6]) : nullptr;
-        PLAIN(b && b->is_cuda() && b->device() == x->device() && b->unsafeGetTensorImpl()->has_storage() && b->is_contiguous() && b->numel() == N);
-        b_dt = dtype_code(b->scalar_type());
-        PLAIN(b_dt >= 0);
-        b_ptr = b->data_ptr();
-    }
-    void* stream;
-    PLAIN(stream_of(*x, &stream));
-    Sizes shape = sizes_of(*x);
-    shape.back() = N;
+    LinearRest r;
+    PLAIN(linear_rest(*x, N, a[6], r));
     const void* const data = x->data_ptr();
     const uint8_t* const code_data = codes->data_ptr<uint8_t>();
     const uint32_t* const scale_data = reinterpret_cast<const uint32_t*>(w_sc->data_ptr<int>());
@@ -371,9 +358,9 @@ PyObject* linear_packed_dense(PyObject*, PyObject* const* a, Py_ssize_t n_args) 
         const WithoutGil released;
         const int64_t bytes = mase_hip_mxfp_packed_dense_workspace_bytes(M, N, K);
         if (bytes > 0) workspace = empty({bytes}, at::kByte, device);
-        y = empty(shape, at::kBFloat16, device);
-        rc = mase_hip_mxfp_gemm_packed_dense(data, code_data, scale_data, (int)we, (int)wm, b_ptr, b_dt, y.data_ptr(), M, N, K, bytes > 0 ? workspace.data_ptr() : nullptr, bytes,
-                                             stream);
+        y = empty(r.shape, at::kBFloat16, device);
+        rc = mase_hip_mxfp_gemm_packed_dense(data, code_data, scale_data, (int)we, (int)wm, r.bias, r.bias_dtype, y.data_ptr(), M, N, K, bytes > 0 ? workspace.data_ptr() : nullptr, bytes,
+                                             r.stream);
     }
     PLAIN(rc == 0);
     return THPVariable_Wrap(std::move(y));
@@ -453,19 +440,8 @@ PyObject* linear_plain(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     const int64_t K = x->size(-1), n = x->numel(), M = K > 0 ? n / K : 0;
     PLAIN(M > 0 && N > 0 && N <= INT32_MAX && M <= INT32_MAX && K <= INT32_MAX && K % 32 == 0 && w_el->numel() == N * K && w_sc->numel() == N * K / 32);
     PLAIN(!cast || mini || (f5[0] > 0 && n % f5[0] == 0));
-    const void* b_ptr = nullptr;
-    int b_dt = 0;
-    if (a[8] != Py_None) {
-        const at::Tensor* const b = THPVariable_Check(a[8]) ? &THPVariable_Unpack(a[8]) : nullptr;
-        PLAIN(b && b->is_cuda() && b->device() == x->device() && b->unsafeGetTensorImpl()->has_storage() && b->is_contiguous() && b->numel() == N);
-        b_dt = dtype_code(b->scalar_type());
-        PLAIN(b_dt >= 0);
-        b_ptr = b->data_ptr();
-    }
-    void* stream;
-    PLAIN(stream_of(*x, &stream));
-    Sizes shape = sizes_of(*x);
-    shape.back() = N;
+    LinearRest r;
+    PLAIN(linear_rest(*x, N, a[8], r));
     const void* const data = x->data_ptr();
     const uint8_t *const scale_data = w_sc->data_ptr<uint8_t>(), *const code_data = w_el->data_ptr<uint8_t>();
     const at::Device device = x->device();
@@ -477,17 +453,17 @@ PyObject* linear_plain(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
         if (cast) {
             x_q = empty({n}, at::kBFloat16, device);
             left = x_q.data_ptr();
-            rc = mini ? mase_hip_qdq_minifloat(data, dt, x_q.data_ptr(), 2, n, (int)f4[0], (int)f4[1], (int)f4[2], (int)f4[3], stream)
-                      : mase_hip_qdq_mxfp(data, dt, x_q.data_ptr(), 2, n, (int)f5[0], (int)f5[1], (int)f5[2], (int)f5[3], (int)f5[4], stream);
+            rc = mini ? mase_hip_qdq_minifloat(data, dt, x_q.data_ptr(), 2, n, (int)f4[0], (int)f4[1], (int)f4[2], (int)f4[3], r.stream)
+                      : mase_hip_qdq_mxfp(data, dt, x_q.data_ptr(), 2, n, (int)f5[0], (int)f5[1], (int)f5[2], (int)f5[3], (int)f5[4], r.stream);
         }
         if (rc == 0) {
             // (which products are given room for partial sums: kernels._workspace_bytes)
             const bool whole_k = K < (M <= 64 ? 1344 : 1024) && (M <= 64 || N % 128 != 0 || K % 128 != 0);
             const int64_t bytes = whole_k ? 0 : mase_hip_mxfp_gemm_workspace_bytes(1, M, N, K);
             if (bytes > 0) workspace = empty({bytes}, at::kByte, device);
-            y = empty(shape, kDtypes[dt], device);
-            rc = mase_hip_mxfp_gemm_ws(left, 2, nullptr, nullptr, 0, 0, scale_data, code_data, (int)we, (int)wm, b_ptr, b_dt, y.data_ptr(), dt, M, N, K, 32,
-                                       bytes > 0 ? workspace.data_ptr() : nullptr, bytes, stream);
+            y = empty(r.shape, kDtypes[dt], device);
+            rc = mase_hip_mxfp_gemm_ws(left, 2, nullptr, nullptr, 0, 0, scale_data, code_data, (int)we, (int)wm, r.bias, r.bias_dtype, y.data_ptr(), dt, M, N, K, 32,
+                                       bytes > 0 ? workspace.data_ptr() : nullptr, bytes, r.stream);
         }
     }
     PLAIN(rc == 0);
