@@ -25,7 +25,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
     reference, ``backend="fused"`` (the default) works: it runs the fused MFMA GEMMs.  Where the block-scaled route
     applies, the layer keeps the weight a second time in that kernel's form (``N * K * 33 / 32`` bytes, built on the
     first such forward and rebuilt when the components change or move; not part of ``state_dict``), and weights of 4- and
-    6-bit codes for up to hundreds of rows packed at their own width, in the same way.
+    6-bit codes for up to hundreds of rows (weight-only: 32) packed at their own width, in the same way: ``N * K / 2`` or ``N * K * 3 / 4``
+    bytes and the scales.  With the components (``N * K * 33 / 32``) a 4-bit layer called with few and with many rows holds 2.5 bytes
+    a weight, a weight-only one with few rows 1.5.
     """
 
     in_features: int
