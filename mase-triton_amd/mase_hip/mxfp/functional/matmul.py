@@ -179,7 +179,7 @@ def mxfp_matmul(
         plain = _lib.host().scores(input, other, other_meta._codes)     # queries and keys, as a model has them
         if plain is not None:
             return plain
-    if fused and quantised_other and other.ndim > 2 and input.dtype != torch.float16:
+    if fused and quantised_other and other.ndim > 2:
         plain = _lib.host().matmul_plain(input, other, input_meta._codes if quantised_input else None, other_meta._codes)
         if plain is not None:
             return plain
