@@ -51,7 +51,8 @@ def narrow_weight_codes(w_element: Tensor, w_tensor_meta: MinifloatTensorMeta, i
     low = w_element.contiguous().view(torch.uint8).view(*w_element.shape, 2)[..., 0]
     n_bits = w_tensor_meta.meta.n_bits
     if into is not None and into[1].shape == low.shape and into[1].device == low.device:
-        into[1].copy_(low & ((1 << n_bits) - 1) if n_bits < 8 else low)      # (in one step: calls may read it)
+        with torch.inference_mode(into[1].is_inference()):
+            into[1].copy_(low & ((1 << n_bits) - 1) if n_bits < 8 else low)      # (in one step: calls may read it)
         return into
     codes = low.contiguous()
     if n_bits < 8:

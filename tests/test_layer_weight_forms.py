@@ -270,3 +270,19 @@ def test_no_form_is_built_that_the_call_does_not_read(layer, monkeypatch):
     for pays in (False, True):
         monkeypatch.setattr(kernels, "prepared_w_pays", lambda *a: pays)
         assert (layer._weight_operand(OnGpu()) is not None) == pays
+
+
+@pytest.mark.parametrize("built_in,written_in", [(True, False), (False, True), (True, True), (False, False)])
+def test_narrowed_codes_are_written_again_in_either_mode(built_in, written_in):
+    """Codes that a call in inference mode built, written again by one outside of it, and the other way round."""
+    import mase_hip.minifloat.functional as MF
+    import mase_hip.minifloat.meta as mf
+
+    meta = mf.MinifloatTensorMeta(device="cpu", dtype="bfloat16", shape=(4, 64), meta=mf.FP6_E3M2_fn)
+    first, second = (torch.randint(0, 64, (4, 64), dtype=torch.int16).view(torch.uint16) for _ in range(2))
+    with torch.inference_mode(built_in):
+        kept = MF.narrow_weight_codes(first, meta)
+    at = kept[1].data_ptr()
+    with torch.inference_mode(written_in), torch.no_grad():
+        again = MF.narrow_weight_codes(second, meta, kept)
+    assert again[1].data_ptr() == at and torch.equal(again[1].to(torch.int16), second.view(torch.int16))
