@@ -25,6 +25,7 @@ def devices_equal(device1, device2) -> bool:
 
 
 def weight_key(components) -> tuple:
+    """Address and version of each.  (Tensors made in inference mode have no version; asking for it raises.)"""
     key = ()
     for c in components:
         key += (c.data_ptr(), c._version)
@@ -158,18 +159,21 @@ class KeepsWeightForms:
 
     def _drop_forms(self, moved_only: bool = False) -> None:
         """Forget the forms, or those whose components are not the layer's any more."""
-        components = [getattr(self, c) for c in self._FORM_COMPONENTS]
-        key = None if any(c is None for c in components) else weight_key(components)
+        addresses = self._component_addresses()
         for name in self._FORMS:
             kept = getattr(self, name)
-            if kept is not None and not (moved_only and kept.key == key):
+            if kept is not None and not (moved_only and kept.key[::2] == addresses):
                 self.__dict__[name] = self.__dict__["_note"] = None
+
+    def _component_addresses(self) -> tuple:
+        components = [getattr(self, c) for c in self._FORM_COMPONENTS]
+        return tuple(None if c is None else c.data_ptr() for c in components)
 
     def _load_from_state_dict(self, *args, **kwargs):
         super()._load_from_state_dict(*args, **kwargs)
         for name in self._FORMS:
             kept = getattr(self, name)
-            if kept is not None and kept.key[::2] == weight_key([getattr(self, c) for c in self._FORM_COMPONENTS])[::2]:
+            if kept is not None and kept.key[::2] == self._component_addresses():
                 self._weight_form(name)
 
     def __getstate__(self):

@@ -272,6 +272,21 @@ def test_no_form_is_built_that_the_call_does_not_read(layer, monkeypatch):
         assert (layer._weight_operand(OnGpu()) is not None) == pays
 
 
+def test_layers_of_inference_tensors_move_and_load(layer):
+    """Their components have no versions."""
+    with torch.inference_mode():
+        scales, elements = components(1)
+        made = MXFPLinearPTQ.from_quantized(scales, elements, layer.w_tensor_meta, None, None, None, None, None, "XWqB", "fused")
+        assert made.w_elements.is_inference() and made.to("cpu") is made
+        made.load_state_dict(layer.state_dict())
+        assert torch.equal(made.w_elements, layer.w_elements)
+        both_forms(layer)
+        layer.w_scales, layer.w_elements = made.w_scales, made.w_elements       # forms of what it had before
+        layer.load_state_dict(layer.state_dict())
+        layer.to("cpu")
+        assert layer._scaled_w is None and layer._packed_w is None
+
+
 @pytest.mark.parametrize("built_in,written_in", [(True, False), (False, True), (True, True), (False, False)])
 def test_narrowed_codes_are_written_again_in_either_mode(built_in, written_in):
     """Codes that a call in inference mode built, written again by one outside of it, and the other way round."""
