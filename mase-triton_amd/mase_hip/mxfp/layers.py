@@ -180,7 +180,8 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             from .functional import linear as L
 
             bias = None if self.layer_type.endswith("Bq") else self.bias
-            if (rows > 32 or not kernels.packed_dense_pays(rows, self.out_features, self.in_features, m.element_exp_bits, m.element_frac_bits)
+            # (components that were made or moved in inference mode: writes to them are not counted, so they are read themselves)
+            if (rows > 32 or self.w_elements.is_inference() or self.w_scales.is_inference() or not kernels.packed_dense_pays(rows, self.out_features, self.in_features, m.element_exp_bits, m.element_frac_bits)
                     or m.scale_exp_bits != 8 or not L._gemm_eligible(input, False, tm, bias)):
                 return None
         elif not (kernels.packed_pays(rows, self.out_features, self.in_features, m.element_exp_bits, m.element_frac_bits, input.device)

@@ -287,6 +287,22 @@ def test_layers_of_inference_tensors_move_and_load(layer):
         assert layer._scaled_w is None and layer._packed_w is None
 
 
+def test_weight_only_calls_read_components_whose_writes_are_not_counted(layer, monkeypatch):
+    """A layer that was moved in inference mode, and one that was built in it: a packed form would not follow a write in place."""
+    monkeypatch.setattr(kernels, "packed_dense_pays", lambda *a: True)
+    layer.layer_type, layer.x_mxfp_meta = "XWqB", None
+    assert layer._packed_weight(OnGpu())[1]
+    with torch.inference_mode():
+        for name in ("w_scales", "w_elements"):
+            getattr(layer, name).data = getattr(layer, name).clone()
+        before = layer.w_elements._version
+        layer.w_elements.add_(1)
+        assert layer.w_elements._version == before and layer._packed_weight(OnGpu()) is None
+        scales, elements = components(1)
+        made = MXFPLinearPTQ.from_quantized(scales, elements, layer.w_tensor_meta, None, None, None, None, None, "XWqB", "fused")
+        assert made._packed_weight(OnGpu()) is None
+
+
 @pytest.mark.parametrize("built_in,written_in", [(True, False), (False, True), (True, True), (False, False)])
 def test_narrowed_codes_are_written_again_in_either_mode(built_in, written_in):
     """Codes that a call in inference mode built, written again by one outside of it, and the other way round."""
