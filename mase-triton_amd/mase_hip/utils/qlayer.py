@@ -55,6 +55,12 @@ def as_stream(name) -> "torch.cuda.Stream":
     return torch.cuda.Stream(stream_id=stream_id, device_index=device_index, device_type=device_type)
 
 
+def owned_elsewhere(name) -> bool:
+    """Is it a stream that torch was handed (``ExternalStream``), whose owner may destroy it?  (torch's own are never destroyed; their numbers are odd, and
+    0 for the default one, where a stream of another owner is named by its handle.)"""
+    return name is not None and name[0] != 0 and name[0] % 2 == 0
+
+
 class WeightForm:
     """A quantised weight in another form than its stored components.
 
@@ -139,7 +145,11 @@ class KeepsWeightForms:
             return None
         same = kept is not None and kept.key == key                                     # (... which this stream cannot be put behind)
         written = not same and kept is not None and kept.key[::2] == key[::2] and not in_graph and kept.ready()       # the same tensors, written since
-        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, components, None if in_graph else current_stream(device))
+        stream = None if in_graph else current_stream(device)
+        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, components, stream)
+        if owned_elsewhere(stream):                           # (it may be gone when the next call would record an event on it)
+            as_stream(stream).synchronize()
+            form.stream = None
         if in_graph or same or self._computed_components():
             return form
         if kept is not None and not written and device.type == "cuda":

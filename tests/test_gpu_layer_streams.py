@@ -53,6 +53,25 @@ def test_forms_built_behind_other_work_of_their_stream(family, layer_type, rows)
 
 
 @pytest.mark.parametrize("family", ["mxfp", "minifloat"])
+def test_forms_built_on_a_stream_of_another_owner(family):
+    """No later call asks anything of such a stream, which may be gone by then."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    w = (0.5 * torch.randn(2048, 4096, generator=g, device=DEV)).to(torch.bfloat16)
+    x = torch.randn(48, 4096, generator=g, device=DEV).to(torch.bfloat16)
+    layer, warm = _make(family, "XqWqB", w), _make(family, "XqWqB", w)
+    want, own = warm(x), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    assert warm._packed_w.stream is not None
+    with torch.cuda.stream(torch.cuda.ExternalStream(own.cuda_stream)):
+        y = layer(x)
+    assert layer._packed_w.stream is None and (layer._scaled_w is None) == (warm._scaled_w is None)
+    with torch.cuda.stream(own):
+        z = layer(x)
+    torch.cuda.synchronize()
+    assert torch.equal(y, want) and torch.equal(z, want)
+
+
+@pytest.mark.parametrize("family", ["mxfp", "minifloat"])
 def test_threads_with_streams_of_their_own(family):
     """Decode-sized and prefill-sized calls of the same fresh layers, each thread with its own mix."""
     K, N, rows = 4096, 2048, (1, 12, 48, 600, 3000)

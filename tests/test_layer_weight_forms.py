@@ -108,6 +108,9 @@ class Stream:
     def __init__(self, number):
         self.cuda_stream, self.recorded, self.waits, self.done, self.captured = number, [], [], False, False
 
+    def __getitem__(self, i):      # (as torch names it: its number, its device, ..)
+        return self.cuda_stream * 2 + 1
+
     def record_event(self):
         self.recorded.append(Event())
         return self.recorded[-1]
@@ -191,6 +194,26 @@ def test_calls_go_behind_what_writes_a_form(layer, monkeypatch):
         layer.w_elements.add_(1)
     layer._forward(OnGpu(), ())
     assert b.waits[-1] is a.recorded[2] and layer._packed_w is not form and layer._packed_w.value.memory is form.value.memory and layer._packed_w.stream is b
+
+
+def test_no_event_is_recorded_on_a_stream_that_its_owner_may_have_destroyed(layer, monkeypatch):
+    """The call that builds a form on a stream that torch was handed waits for it."""
+    waited = []
+
+    class External:
+        synchronize = staticmethod(lambda: waited.append("stream"))
+
+        def __getattr__(self, name):
+            raise AssertionError(name)
+
+    at = [(0x55550010, 0, 1)]
+    monkeypatch.setattr(qlayer, "current_stream", lambda device: at[0])
+    monkeypatch.setattr(qlayer, "as_stream", lambda name: External())
+    form = layer._weight_form("_packed_w")
+    assert waited == ["stream"] and form.stream is None and layer._weight_form("_packed_w") is form
+    for at[0] in ((0, 0, 1), (0x23, 0, 1), None):                 # torch's own
+        layer._drop_forms()
+        assert layer._weight_form("_packed_w").stream == at[0] and len(waited) == 1
 
 
 def test_of_two_threads_that_build_a_form_one_keeps_its_own(layer, monkeypatch):
