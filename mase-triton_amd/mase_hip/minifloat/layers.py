@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, capturing
+from ..utils.qlayer import NOT_NOW, ChangeDtypeError, KeepsWeightForms
 from . import functional as MinifloatF
 from .meta import MinifloatMeta, MinifloatTensorMeta
 
@@ -130,12 +130,12 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
     def _weight_operand(self, input: Tensor):
         """The weight in the block-scaled GEMM's form when this call takes that GEMM (quantised bfloat16 activations, see
         ``minifloat_linear``), else None.  Not part of ``state_dict``; rebuilt like the one-byte copy."""
+        w = self.w_element
+        if input.dtype != torch.bfloat16 or self.backend in ("separate", "fused_bf16") or w is None or not self.layer_type.startswith("XqWq") or input.device.type != "cuda":
+            return None
         from ..mxfp.functional.linear import takes_scaled_route
         from .functional import linear as L
 
-        w = self.w_element
-        if self.backend in ("separate", "fused_bf16") or w is None or not self.layer_type.startswith("XqWq") or input.device.type != "cuda":
-            return None
         rows = input.numel() // input.shape[-1] if input.numel() else 0
         bias = self.bias if not self.layer_type.endswith("Bq") else None
         if not ((self.backend == "fused_scaled" or takes_scaled_route(rows, True))
@@ -146,12 +146,14 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
     def _packed_weight(self, input: Tensor):
         """The weight packed at its own width when that is the fastest form for this call, and whether the activations are dense (``MXFPLinearPTQ``);
         else None."""
+        w, tm = self.w_element, self.w_tensor_meta
+        if input.dtype != torch.bfloat16 or self.backend != "fused" or w is None or input.device.type != "cuda" or tm.meta.round_mode != "rn":
+            return None
+        if tm.meta.exp_bits + tm.meta.frac_bits > 5:            # (nothing to pack)
+            return None
         from ..mxfp import kernels
         from .functional import linear as L
 
-        w, tm = self.w_element, self.w_tensor_meta
-        if self.backend != "fused" or w is None or input.device.type != "cuda" or tm.meta.round_mode != "rn":
-            return None
         rows = input.numel() // input.shape[-1] if input.numel() else 0
         bias = self.bias if not self.layer_type.endswith("Bq") else None
         E, M, dense = tm.meta.exp_bits, tm.meta.frac_bits, self.layer_type.startswith("XWq")
@@ -162,7 +164,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
                   and L._scaled_eligible(input, self.x_minifloat_meta, tm, bias)):
             return None
         form = self._weight_form("_packed_w", needed=False)
-        return None if form is None else (form.value, dense)
+        return NOT_NOW if form is None else (form.value, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_minifloat_meta)
@@ -214,7 +216,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         asked = self._no_operand_sig != sig
         notes = self.__dict__
         packed = self._packed_weight(input) if asked else None
-        if packed is not None:
+        if packed:
             from ..mxfp import kernels
 
             w, dense = packed
@@ -236,7 +238,8 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
         w_operand = self._weight_operand(input) if asked else None
         notes["_no_operand_sig"] = None
         notes["_note"] = None if w_operand is None else (sig, 0)
-        narrowed = self._narrowed_weight() if w_operand is None else None       # (with an operand nothing reads the codes themselves)
+        # (with an operand nothing reads the codes themselves, and of fp16 calls nothing reads them in one byte)
+        narrowed = self._narrowed_weight() if w_operand is None and input.dtype != torch.float16 else None
         y = MinifloatF.minifloat_linear(
             x=input, x_meta=self.x_minifloat_meta, w=self.weight, w_element=self.w_element,
             w_tensor_meta=self.w_tensor_meta, b=self.bias, b_element=self.b_element,
@@ -244,7 +247,7 @@ class MinifloatLinearPTQ(KeepsWeightForms, nn.Module):
             _narrowed=narrowed, _w_operand=w_operand)
         if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
-        elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
+        elif w_operand is None and packed is not NOT_NOW:
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 

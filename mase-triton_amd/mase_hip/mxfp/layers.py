@@ -8,7 +8,7 @@ import torch
 from torch import Tensor, nn
 
 from .. import _lib
-from ..utils.qlayer import ChangeDtypeError, KeepsWeightForms, capturing
+from ..utils.qlayer import NOT_NOW, ChangeDtypeError, KeepsWeightForms
 from . import functional as MXFP_F
 from .meta import MXFPMeta, MXFPTensorMeta
 
@@ -147,33 +147,35 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
 
     def _weight_operand(self, input: Tensor):
         """The weight in the block-scaled GEMM's form when this call has a kernel that reads it (the block-scaled GEMM for
-        quantised bfloat16 activations, the large-tile bf16 kernel from 512 rows on), else None."""
+        quantised bfloat16 activations, the large-tile bf16 kernel from 512 rows on), else None (``NOT_NOW``: a captured call that has to do without)."""
+        if input.dtype != torch.bfloat16 or self.backend == "separate" or "Wq" not in self.layer_type or input.device.type != "cuda":
+            return None
         from . import kernels
         from .functional import linear as L
 
-        if self.backend == "separate" or "Wq" not in self.layer_type or input.device.type != "cuda":
-            return None
         rows = input.numel() // input.shape[-1] if input.numel() else 0
         scaled = self._takes_scaled_route(input)
         if not scaled:
             tm = self.w_tensor_meta
             bf16 = (self.backend != "fused_scaled" and len(tm.shape) == 2 and kernels.scaled_format_supported(tm.meta) and tm.block_dim % 2 == 1
-                    and input.dtype == torch.bfloat16 and getattr(torch, tm.dtype) == input.dtype
+                    and getattr(torch, tm.dtype) == input.dtype
                     and kernels.prepared_w_pays(rows, tm.shape[0], tm.shape[1]))
             if not bf16:
                 return None
         form = self._weight_form("_scaled_w", needed=scaled)
-        return None if form is None else form.value
+        return NOT_NOW if form is None else form.value
 
     def _packed_weight(self, input: Tensor, scaled: bool = False):
         """The weight packed at its own width when that is the fastest form for this call, and whether the call is one of dense activations
         (weight-only layers) or of quantised ones; else None.  ``scaled``: the caller knows that the call takes the block-scaled route."""
-        from . import kernels
-
         tm = self.w_tensor_meta
-        if self.backend != "fused" or tm is None or input.device.type != "cuda":
+        if input.dtype != torch.bfloat16 or self.backend != "fused" or tm is None or input.device.type != "cuda":
             return None
         m = tm.meta
+        if m.element_exp_bits + m.element_frac_bits > 5:        # (8-bit codes: there is nothing to pack)
+            return None
+        from . import kernels
+
         rows = input.numel() // input.shape[-1] if input.numel() else 0
         dense = self.layer_type.startswith("XWq")
         if dense:
@@ -188,7 +190,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                   and (scaled or self._takes_scaled_route(input))):
             return None
         form = self._weight_form("_packed_w", needed=False)
-        return None if form is None else (form.value, dense)
+        return NOT_NOW if form is None else (form.value, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
         return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta)
@@ -248,7 +250,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         asked = self._no_operand_sig != sig
         notes = self.__dict__
         packed = self._packed_weight(input) if asked else None
-        if packed is not None:
+        if packed:
             from . import kernels
 
             w, dense = packed
@@ -268,6 +270,9 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
                 y = kernels.linear_packed(_lib.dense(x2), meta.element_exp_bits, meta.element_frac_bits, False, w, None if bias is None else bias.contiguous())
             return y.view(*input.shape[:-1], self.out_features)
         w_operand = self._weight_operand(input) if asked else None
+        missed = packed is NOT_NOW or w_operand is NOT_NOW
+        if w_operand is NOT_NOW:
+            w_operand = None
         notes["_no_operand_sig"] = None
         notes["_note"] = (sig, 0) if w_operand is not None and self._takes_scaled_route(input) else None
         y = MXFP_F.mxfp_linear(
@@ -277,7 +282,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
             w_operand=w_operand)
         if w_operand is None and not asked:
             notes["_no_operand_sig"], notes["_note"] = sig, note
-        elif w_operand is None and not capturing(input.device):     # (a captured call may have gone without a form that it has a use for)
+        elif w_operand is None and not missed:
             notes["_no_operand_sig"] = sig
             from .functional import linear as L
 
@@ -299,10 +304,10 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         if (gate.shape == up.shape and gate.dtype == up.dtype and gate.device == up.device and gate.shape[-1] == self.in_features
                 and self.layer_type == "XqWqB" and self._takes_scaled_route(gate)):
             packed = self._packed_weight(gate, True)
-            w_op = self._weight_form("_scaled_w").value if packed is None else packed[0]
+            w_op = packed[0] if packed else self._weight_form("_scaled_w").value
             a_op = kernels.scaled_operand_from_swiglu(gate.reshape(-1, self.in_features) if gate.ndim != 2 else gate,
                                                       up.reshape(-1, self.in_features) if up.ndim != 2 else up, self.x_mxfp_meta)
-            y = kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype) if packed is None else kernels.mxfp_gemm_packed(a_op, w_op, self.bias)
+            y = kernels.mxfp_gemm_packed(a_op, w_op, self.bias) if packed else kernels.mxfp_gemm_scaled(a_op, w_op, self.bias, gate.dtype)
             return y.view(*gate.shape[:-1], self.out_features)
         return self.forward(torch.nn.functional.silu(gate) * up)
 

@@ -94,12 +94,29 @@ def test_a_copy_builds_its_own_forms(layer):
 def test_forms_built_for_a_graph_are_not_kept(layer, monkeypatch):
     """What a captured stream is given runs on the replays: nothing is written yet for the calls between."""
     monkeypatch.setattr(qlayer, "capturing", lambda device: True)
-    assert layer._packed_weight(OnGpu(), True) is None and layer._weight_form("_scaled_w").value.sum > 0
+    assert layer._packed_weight(OnGpu(), True) is qlayer.NOT_NOW and layer._weight_form("_scaled_w").value.sum > 0
     assert layer._scaled_w is None and layer._packed_w is None
     monkeypatch.setattr(qlayer, "capturing", lambda device: False)
     kept = both_forms(layer)
     monkeypatch.setattr(qlayer, "capturing", lambda device: True)
     assert both_forms(layer) == kept == (layer._scaled_w, layer._packed_w)
+
+
+def test_only_calls_that_have_a_use_for_a_form_ask_about_captures(layer, monkeypatch):
+    """fp16 calls, and those of many rows on the components, whatever their shape was last; of the others a captured one that went without is not noted."""
+    layer.layer_type, layer.x_mxfp_meta, asked = "XWqB", None, []
+    monkeypatch.setattr(qlayer, "capturing", lambda device: asked.append(device) or True)
+    monkeypatch.setattr(kernels, "packed_dense_pays", lambda rows, *a: rows <= 32)
+    monkeypatch.setattr(kernels, "prepared_w_pays", lambda rows, *a: rows >= 1000)
+    monkeypatch.setattr(OnGpu, "numel", lambda self: self.shape.numel())
+    monkeypatch.setattr(MX, "mxfp_linear", lambda **kw: torch.zeros(1))
+    for rows, dtype, has_use in ((4, torch.float16, False), (8, torch.float16, False), (40, torch.bfloat16, False), (60, torch.bfloat16, False), (4, torch.bfloat16, True),
+                                 (1000, torch.bfloat16, True)):
+        x = OnGpu()
+        x.shape, x.dtype = torch.Size((rows, K)), dtype
+        asked.clear()
+        layer(x)
+        assert bool(asked) == has_use and (layer._no_operand_sig is None) == has_use
 
 
 class Stream:
@@ -171,19 +188,19 @@ def test_calls_go_behind_what_writes_a_form(layer, monkeypatch):
     assert form.event is a.recorded[1] and not a.waits
     # captured calls: one on another stream asks the form's stream or its event, one on the form's own only the event
     b.captured, at[0] = True, b
-    assert layer._packed_weight(OnGpu(), True) is None and len(b.waits) == 2
+    assert layer._packed_weight(OnGpu(), True) is qlayer.NOT_NOW and len(b.waits) == 2
     a.recorded[1].done = True
     assert layer._packed_weight(OnGpu(), True)[0] is form.value and layer._packed_w is form and form.stream is None
     at[0] = a
     form = build()
     at[0] = b
-    assert layer._packed_weight(OnGpu(), True) is None and layer._packed_w is form
+    assert layer._packed_weight(OnGpu(), True) is qlayer.NOT_NOW and layer._packed_w is form
     a.done = True
     assert layer._packed_weight(OnGpu(), True)[0] is form.value and layer._packed_w is form and form.stream is None and len(a.recorded) == 2
     at[0], a.done = a, False
     form = build(written=True)
     a.captured = True
-    assert layer._packed_weight(OnGpu(), True) is None
+    assert layer._packed_weight(OnGpu(), True) is qlayer.NOT_NOW
     # an eager call while the form's stream is captured by another thread: a form of its own
     b.captured, at[0] = False, b
     other = layer._packed_weight(OnGpu(), True)[0]
