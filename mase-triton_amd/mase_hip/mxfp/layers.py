@@ -106,7 +106,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
     def _apply(self, fn, recurse=True):
         before = {n: getattr(self, n).dtype for n in self._CODE_PARAMS if getattr(self, n) is not None}
         result = super()._apply(fn, recurse)
-        self._no_operand_sig = None
+        self._no_operand_sig = self._note = None
         self._drop_forms(moved_only=True)
         for name, dt in before.items():
             now = getattr(self, name).dtype
@@ -193,7 +193,7 @@ class MXFPLinearPTQ(KeepsWeightForms, nn.Module):
         return NOT_NOW if form is None else (form.value, dense)
 
     def _call_signature(self, input: Tensor) -> tuple:
-        return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta)
+        return (input.shape, input.dtype, input.device, self.backend, self.layer_type, self.x_mxfp_meta, self.w_tensor_meta)
 
     def forward(self, input: Tensor) -> Tensor:
         # (no autograd either way: the extension's outputs have none, and it costs less than entering no_grad)

@@ -70,13 +70,13 @@ class WeightForm:
     """A quantised weight in another form than its stored components.
 
     ``key`` names the components that it was built from, by address and version.  An address names a tensor only until its memory is handed out
-    again, so the form holds the memory of each: whatever replaces a component while the form is kept lies elsewhere.  ``stream`` names the one that the
+    again, so the form holds the memory of each: whatever replaces a component while the form is kept lies elsewhere.  ``format`` is what their codes meant.  ``stream`` names the one that the
     kernels which write the form were launched on, None once they are known to have run; ``event`` is behind them, once one was asked for."""
 
-    __slots__ = ("value", "key", "memory", "device", "stream", "event")
+    __slots__ = ("value", "key", "format", "memory", "device", "stream", "event")
 
-    def __init__(self, value, key: tuple, components, stream):
-        self.value, self.key, self.memory, self.device = value, key, [c.untyped_storage() for c in components], components[0].device
+    def __init__(self, value, key: tuple, format, components, stream):
+        self.value, self.key, self.format, self.memory, self.device = value, key, format, [c.untyped_storage() for c in components], components[0].device
         self.stream, self.event = stream, None
 
     def ready(self) -> bool:
@@ -142,16 +142,17 @@ class KeepsWeightForms:
         writes it on every replay; with ``needed`` false, for a call that has another way, None in its place."""
         held = self._parameters
         components = [held[c] if held.get(c) is not None else getattr(self, c) for c in self._FORM_COMPONENTS]
-        kept, key, device = getattr(self, name), weight_key(components), components[0].device
-        if kept is not None and kept.key == key and kept.ready():
+        kept, key, device, format = getattr(self, name), weight_key(components), components[0].device, self.w_tensor_meta.meta
+        same = kept is not None and kept.key == key and (kept.format is format or kept.format == format)
+        if same and kept.ready():
             return kept
         in_graph = capturing(device)
         if in_graph and not needed:
             return None
-        same = kept is not None and kept.key == key                                     # (... which this stream cannot be put behind)
-        written = not same and kept is not None and kept.key[::2] == key[::2] and not in_graph and kept.ready()       # the same tensors, written since
+        # (the same, which this stream cannot be put behind; or the same tensors, written since or of another format)
+        written = not same and kept is not None and kept.key[::2] == key[::2] and not in_graph and kept.ready()
         stream = None if in_graph else current_stream(device)
-        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, components, stream)
+        form = WeightForm(self._build_form(name, kept.value if written else None, *components), key, format, components, stream)
         if owned_elsewhere(stream):                           # (it may be gone when the next call would record an event on it)
             as_stream(stream).synchronize()
             form.stream = None

@@ -119,6 +119,35 @@ def test_only_calls_that_have_a_use_for_a_form_ask_about_captures(layer, monkeyp
         assert bool(asked) == has_use and (layer._no_operand_sig is None) == has_use
 
 
+def test_a_layer_that_is_given_a_weight_of_another_format(layer, monkeypatch):
+    """Neither the way of the last call nor a form outlives what the codes meant then."""
+    kept, taken = both_forms(layer), []
+    layer.w_tensor_meta = layer.w_tensor_meta.create(meta=mx.OCP_MXFP6_E3M2)
+    assert not set(both_forms(layer)) & set(kept) and layer._scaled_w.format is mx.OCP_MXFP6_E3M2
+    kept = both_forms(layer)
+    layer.w_tensor_meta = layer.w_tensor_meta.create(meta=mx.MXFPMeta(**vars(mx.OCP_MXFP6_E3M2)))       # the same, another object
+    assert both_forms(layer) == kept
+
+    class Host:
+        linear_plain = staticmethod(lambda *a: taken.append(a[5:7]) or torch.zeros(4, N))
+
+    monkeypatch.setattr(_lib, "_host", Host)
+    monkeypatch.setattr(kernels, "packed_dense_pays", lambda *a: False)
+    monkeypatch.setattr(kernels, "prepared_w_pays", lambda *a: False)
+    monkeypatch.setattr("mase_hip.mxfp.functional.linear._gemm_eligible", lambda x, quantised, tm, b: tm.meta.element_is_finite)
+    monkeypatch.setattr(MX, "mxfp_linear", lambda **kw: torch.zeros(4, N))
+    layer.layer_type, layer.x_mxfp_meta = "XWqB", None
+    for _ in range(3):
+        layer(OnGpu())
+    assert taken == [(3, 2)] * 2
+    scales, elements = components(1)
+    layer.w_scales, layer.w_elements = (torch.nn.Parameter(t, requires_grad=False) for t in (scales, elements))
+    layer.w_tensor_meta = layer.w_tensor_meta.create(meta=mx.MXFPMeta(32, 8, 5, 2, False, "rn"))        # its top exponent field is inf / NaN, which the kernels do not know
+    for _ in range(3):
+        layer(OnGpu())
+    assert len(taken) == 2
+
+
 class Stream:
     """A stand-in for a stream on a GPU: the events recorded on it, and those that it waits for."""
 
