@@ -1,6 +1,7 @@
 """The further forms of a quantised weight that a layer keeps, with stand-ins for the kernels that build and read them: what becomes of them when the
 components move or change."""
 import copy
+import dataclasses
 import pickle
 
 import pytest
@@ -125,7 +126,7 @@ def test_a_layer_that_is_given_a_weight_of_another_format(layer, monkeypatch):
     layer.w_tensor_meta = layer.w_tensor_meta.create(meta=mx.OCP_MXFP6_E3M2)
     assert not set(both_forms(layer)) & set(kept) and layer._scaled_w.format is mx.OCP_MXFP6_E3M2
     kept = both_forms(layer)
-    layer.w_tensor_meta = layer.w_tensor_meta.create(meta=mx.MXFPMeta(**vars(mx.OCP_MXFP6_E3M2)))       # the same, another object
+    layer.w_tensor_meta = layer.w_tensor_meta.create(meta=dataclasses.replace(mx.OCP_MXFP6_E3M2))       # the same, another object
     assert both_forms(layer) == kept
 
     class Host:
